@@ -84,7 +84,7 @@ typedef struct reef_hal_completion {
     uint64_t* exit_ticks;
     uint32_t* exit_count;
     uint32_t seq;
-    uint32_t reserved;
+    uint32_t user;   /* the caller's: kept as it is */
 } reef_hal_completion;
 enum { REEF_COMPLETE_STREAM_WRITE = 0, REEF_COMPLETE_IN_KERNEL = 1 };
 
@@ -213,6 +213,37 @@ int reef_hal_graph_end(reef_stream_t s, reef_graph_t* out);
 int reef_hal_graph_launch(reef_graph_t g, reef_stream_t s);
 int reef_hal_graph_destroy(reef_graph_t g);
 
+/* A recorded pass: the same launches with the same arguments, run over and over (a model's
+ * inference).  The argument blocks stay in device memory and the launches go to a hardware queue
+ * of this library's own as ready-made packets, so a pass costs the host microseconds and no
+ * kernel waits for arguments the host has just written.
+ *   pass_create: copies the launches and assigns every launch a block of device memory: its arguments
+ *                and `tail_bytes` of the caller's behind them.  Returns 2 where the backend cannot
+ *                record a pass (the caller then launches kernel by kernel).
+ *   pass_block:  device address and size of the block of launch `i`, the host copy that pass_commit
+ *                uploads (the caller may still write into it), and where in it the tail starts.
+ *   pass_commit: uploads the blocks; needed before the first run.
+ *   pass_run:    waits for what `after` (may be NULL: the default stream) has been given, runs the
+ *                launches in order and returns when the last has finished. */
+typedef struct reef_pass_s* reef_pass_t;
+typedef struct reef_pass_launch {
+    reef_function_t fn;
+    uint32_t grid[3], block[3];
+    uint32_t dyn_lds;
+    const void* kernarg;
+    size_t kernarg_bytes;
+} reef_pass_launch;
+typedef struct reef_pass_block {
+    char* device;
+    char* host;
+    size_t bytes, tail;
+} reef_pass_block;
+int reef_hal_pass_create(const reef_pass_launch* launches, size_t n, size_t tail_bytes, reef_pass_t* out);
+int reef_hal_pass_block(reef_pass_t p, size_t i, reef_pass_block* out);
+int reef_hal_pass_commit(reef_pass_t p);
+int reef_hal_pass_run(reef_pass_t p, reef_stream_t after);
+int reef_hal_pass_destroy(reef_pass_t p);
+
 /*
  * Backend table.  The functions above forward to the active backend; the HIP
  * backend is the default and the only one the library ships.  Host-logic tests
@@ -263,6 +294,11 @@ typedef struct reef_hal_backend {
     int (*module_kernel_entry)(reef_module_t, const char*, uint64_t*);
     int (*host_fill32)(reef_devptr_t, int32_t, size_t);
     int (*stream_drained)(reef_stream_t, int*);
+    int (*pass_create)(const reef_pass_launch*, size_t, size_t, reef_pass_t*);
+    int (*pass_block)(reef_pass_t, size_t, reef_pass_block*);
+    int (*pass_commit)(reef_pass_t);
+    int (*pass_run)(reef_pass_t, reef_stream_t);
+    int (*pass_destroy)(reef_pass_t);
 } reef_hal_backend;
 
 const reef_hal_backend* reef_hal_hip_backend(void);

@@ -60,6 +60,22 @@ typedef struct ReefOpDesc {
     int32_t attr[REEF_MAX_ATTRS];  /* JSON `attrs` order */
 } ReefOpDesc;
 
+/* What the workgroups behind a launch's tasks bring into the L2 of their XCD while the tasks run: the
+ * parameters of the launch that follows (its weights, then up to five small operands and its argument
+ * block).  In device memory; its address travels in the last pointer slot of the descriptor, which such
+ * a launch does not use otherwise.  Weights are `chunks` pieces of chunk_bytes (the consumer's tiles of
+ * output rows): XCD x of 8 needs pieces [x chunks / 8, (x + 1) chunks / 8] of them (contiguous runs of
+ * tiles per XCD), or every eighth piece (interleaved). */
+#define REEF_PREFETCH_SLOT (REEF_MAX_PTRS - 1)
+#define REEF_PREFETCH_SMALL 6
+#define REEF_PREFETCH_WGS_UNIT 8 /* workgroups come in eights: one per XCD each */
+typedef struct ReefPrefetch {
+    const char* base;
+    uint32_t chunks, chunk_bytes, total, interleaved;
+    uint32_t wgs, reserved;
+    struct { const char* p; uint64_t bytes; } small_[REEF_PREFETCH_SMALL];
+} ReefPrefetch;
+
 /* Argument block of the best-effort flavour.  The first 32 bytes are the
  * reef_hal_completion of reef_hal.h (all zero: nothing is signalled). */
 typedef struct ReefBeArgs {
@@ -67,7 +83,7 @@ typedef struct ReefBeArgs {
     uint64_t* exit_ticks;
     uint32_t* exit_count;
     uint32_t seq;
-    uint32_t reserved;
+    uint32_t tasks;       /* workgroups from this one on are the prefetching ones; 0: there are none */
     int32_t* preempted;
     int32_t* task_slot;
     ReefOpDesc desc;
@@ -89,7 +105,7 @@ typedef struct ReefDkpArgs {
     int32_t cu_partition;  /* virtual CUs given to side l, multiple of num_xcds */
     int32_t num_cus;       /* virtual CUs per layer (grid = layers * num_cus) */
     int32_t num_xcds;      /* 8 on MI355X; 1 reproduces the reference's flat mapping */
-    int32_t reserved;
+    int32_t prefetch_at;   /* workgroups from this one on prefetch (descriptor of side l); 0: there are none */
     int32_t* task_slot_r;  /* unused, null */
     /* First instruction of each side's own kernel (the reference's func_l / func_r,
      * transform_kernel.py:345-352): read by the merge_framework_<n> proxies only, which jump

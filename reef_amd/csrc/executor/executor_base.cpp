@@ -1,6 +1,9 @@
 #include "executor/executor_base.h"
 #include "executor/op_extents.h"
+#include "executor/prefetch.h"
 
+#include <algorithm>
+#include <cstddef>
 #include <cstdlib>
 
 #include <cstring>
@@ -14,6 +17,7 @@ ExecutorBase::ExecutorBase()
 
 ExecutorBase::~ExecutorBase() {
     drop_graph();
+    drop_pass(model_pass);
     if (owns_stream && s) reef_hal_stream_destroy(s);
     if (arena) reef_hal_free(arena, REEF_MEM_DEVICE);
     if (sync_mem) reef_hal_free(sync_mem, REEF_MEM_DEVICE_FINEGRAINED);
@@ -210,8 +214,14 @@ Status ExecutorBase::execute(GPUStream_t stream) { return execute_to((int)num_ke
 
 Status ExecutorBase::execute_to(int idx, GPUStream_t stream) {
     if (idx < 0 || (size_t)idx > num_kernels()) RETURN_STATUS(Status::OutOfRange);
-    if ((size_t)idx == num_kernels()) RETURN_STATUS(launch_model(stream));
-    else for (int i = 0; i < idx; i++) RETURN_STATUS(launch_kernel(i, stream));
+    if ((size_t)idx == num_kernels()) {
+        if (!use_graph) {
+            bool ran = false;
+            RETURN_STATUS(run_pass(model_pass, [this](int i, Launch& l) { return make_launch(i, l); }, stream, &ran));
+            if (ran) return Status::Succ;
+        }
+        RETURN_STATUS(launch_model(stream));
+    } else for (int i = 0; i < idx; i++) RETURN_STATUS(launch_kernel(i, stream));
     GPU_RETURN_STATUS(reef_hal_stream_sync(stream));
     return Status::Succ;
 }
@@ -258,11 +268,67 @@ Status ExecutorBase::launch_range(int begin, int end, GPUStream_t stream) {
     return Status::Succ;
 }
 
-Status ExecutorBase::launch_kernel(int i, GPUStream_t stream) {
+Status ExecutorBase::make_launch(int i, Launch& l) const {
     const uint32_t* lp = model->kernels[i].launch_params;
-    GPU_RETURN_STATUS(reef_hal_launch(kernel_funcs[i], lp, lp + 3, 0, stream, &descs[i],
-                                      sizeof(ReefOpDesc)));
+    l.fn = kernel_funcs[i];
+    std::copy(lp, lp + 3, l.grid);
+    std::copy(lp + 3, lp + 6, l.block);
+    l.bytes = sizeof(ReefOpDesc);
+    std::memcpy(l.args, &descs[i], l.bytes);
     return Status::Succ;
+}
+
+Status ExecutorBase::launch_kernel(int i, GPUStream_t stream) {
+    Launch l;
+    RETURN_STATUS(make_launch(i, l));
+    GPU_RETURN_STATUS(reef_hal_launch(l.fn, l.grid, l.block, 0, stream, l.args, l.bytes));
+    return Status::Succ;
+}
+
+size_t ExecutorBase::add_prefetch(Launch& l, uint32_t wgs) const {
+    l.grid[0] += wgs;
+    return offsetof(ReefOpDesc, ptr) + REEF_PREFETCH_SLOT * sizeof(void*);
+}
+
+Status ExecutorBase::record_pass(Pass& p, std::vector<Launch>& l) {
+    const size_t n = l.size();
+    if (n == 0) return Status::Succ;
+    std::vector<ReefPrefetch> pf = plan_prefetch(*model, storage);
+    std::vector<size_t> slot(n, 0);
+    for (size_t i = 0; i < n; i++)
+        if (pf[i].wgs) slot[i] = add_prefetch(l[i], pf[i].wgs);
+    std::vector<reef_pass_launch> r(n);
+    for (size_t i = 0; i < n; i++) {
+        r[i].fn = l[i].fn;
+        std::copy(l[i].grid, l[i].grid + 3, r[i].grid);
+        std::copy(l[i].block, l[i].block + 3, r[i].block);
+        r[i].dyn_lds = 0;
+        r[i].kernarg = l[i].args;
+        r[i].kernarg_bytes = l[i].bytes;
+    }
+    // A launch's record lies right behind its arguments: the launch in front brings both in, as one
+    // more thing the next launch would wait for.
+    const int rc = reef_hal_pass_create(r.data(), n, sizeof(ReefPrefetch), &p.handle);
+    if (rc == 2) return Status::Succ;
+    GPU_RETURN_STATUS(rc);
+    reef_pass_block cur, next;
+    for (size_t i = 0; i < n; i++) {
+        if (!pf[i].wgs) continue;
+        GPU_RETURN_STATUS(reef_hal_pass_block(p.handle, i, &cur));
+        GPU_RETURN_STATUS(reef_hal_pass_block(p.handle, i + 1, &next));
+        pf[i].small_[REEF_PREFETCH_SMALL - 1].p = next.device;
+        pf[i].small_[REEF_PREFETCH_SMALL - 1].bytes = next.bytes;
+        std::memcpy(cur.host + cur.tail, &pf[i], sizeof(ReefPrefetch));
+        const void* rec = cur.device + cur.tail;
+        std::memcpy(cur.host + slot[i], &rec, sizeof(rec));
+    }
+    GPU_RETURN_STATUS(reef_hal_pass_commit(p.handle));
+    return Status::Succ;
+}
+
+void ExecutorBase::drop_pass(Pass& p) {
+    if (p.handle) reef_hal_pass_destroy(p.handle);
+    p = Pass();
 }
 
 }  // namespace executor

@@ -67,7 +67,29 @@ public:
 
 protected:
     Status init_executor_base(const char* json_file_path, GPUModule_t module);
-    virtual Status launch_kernel(int kernel_offset, GPUStream_t stream);
+    // One launch of a kernel call: function, geometry and argument block.
+    struct Launch {
+        GPUFunction_t fn;
+        uint32_t grid[3], block[3];
+        size_t bytes;
+        alignas(16) char args[512];
+    };
+    virtual Status make_launch(int kernel_offset, Launch& l) const;
+    // Appends the workgroups that prefetch for the next launch.
+    // Returns the place of that address in the argument block.
+    virtual size_t add_prefetch(Launch& l, uint32_t wgs) const;
+    Status launch_kernel(int kernel_offset, GPUStream_t stream);
+    // A whole run recorded once (reef_hal_pass_create) and submitted as ready-made packets from then on.
+    struct Pass {
+        reef_pass_t handle = nullptr;
+        bool tried = false;
+    };
+    // Runs the pass behind what `stream` has been given and waits for it.  *ran = false, and nothing done,
+    // where the backend cannot record one.
+    template <class Make>
+    Status run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran);
+    Status record_pass(Pass& p, std::vector<Launch>& launches);
+    static void drop_pass(Pass& p);
     Status find_storage_idx(const std::string& name, size_t& idx);
     size_t storage_bytes(size_t idx) const;
 
@@ -84,8 +106,24 @@ protected:
     bool owns_stream;
     bool use_graph;
     reef_graph_t model_graph;
+    Pass model_pass;
     void drop_graph();
 };
+
+template <class Make>
+Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran) {
+    *ran = false;
+    if (!p.tried) {
+        std::vector<Launch> l(num_kernels());
+        for (size_t i = 0; i < l.size(); i++) RETURN_STATUS(make((int)i, l[i]));
+        RETURN_STATUS(record_pass(p, l));
+        p.tried = true;
+    }
+    if (!p.handle) return Status::Succ;
+    *ran = true;
+    GPU_RETURN_STATUS(reef_hal_pass_run(p.handle, stream));
+    return Status::Succ;
+}
 
 }  // namespace executor
 }  // namespace reef

@@ -1,5 +1,6 @@
 #include "executor/hybrid_executor.h"
 
+#include <algorithm>
 #include <cstddef>
 #include <cstring>
 
@@ -15,6 +16,7 @@ HybridExecutor::HybridExecutor()
       sync_ptr(nullptr), sync_bytes(0) {}
 
 HybridExecutor::~HybridExecutor() {
+    drop_pass(preempt_pass);
     if (owns_flag && preempt_flag) reef_hal_free(preempt_flag, REEF_MEM_DEVICE_FINEGRAINED);
     if (task_slot_base) reef_hal_free(task_slot_base, REEF_MEM_DEVICE);
     if (task_slots_host) reef_hal_free(task_slots_host, REEF_MEM_HOST_PINNED);
@@ -102,10 +104,14 @@ Status HybridExecutor::set_preempt_flag(GPUDevicePtr_t flag) {
     if (owns_flag && preempt_flag) GPU_RETURN_STATUS(reef_hal_free(preempt_flag, REEF_MEM_DEVICE_FINEGRAINED));
     owns_flag = false;
     preempt_flag = flag;
+    drop_pass(preempt_pass);   // its argument blocks name the old flag
     return Status::Succ;
 }
 
 Status HybridExecutor::execute_preemptale(GPUStream_t stream) {
+    bool ran = false;
+    RETURN_STATUS(run_pass(preempt_pass, [this](int i, Launch& l) { return make_preempt_launch(i, l); }, stream, &ran));
+    if (ran) return Status::Succ;
     for (size_t i = 0; i < model->kernels.size(); i++) {
         Status ret = launch_preempt_kernel((int)i, stream);
         if (ret != Status::Succ) return ret;
@@ -161,16 +167,37 @@ Status HybridExecutor::reset_sync_storage_from_host(GPUStream_t fallback) {
     return reset_sync_storage(fallback);
 }
 
-Status HybridExecutor::launch_preempt_kernel(int i, GPUStream_t stream) {
+Status HybridExecutor::make_preempt_launch(int i, Launch& l) const {
     const KernelArg& ka = trans_args[i];
     ReefBeArgs arg;
+    static_assert(sizeof(arg) <= sizeof(l.args), "a launch record holds the best-effort flavour's arguments");
     std::memset(&arg, 0, sizeof(reef_hal_completion));   // filled by the layer on a windowed stream
     arg.preempted = (int*)preempt_flag;
     arg.task_slot = (int*)((char*)task_slot_base + i * 4);
     arg.desc = descs[i];
+    l.fn = preempt_kernels[i];
     const uint32_t grid[3] = {ka.task_dim.x, ka.task_dim.y, ka.task_dim.z};
     const uint32_t block[3] = {ka.thread_dim.x, ka.thread_dim.y, ka.thread_dim.z};
-    GPU_RETURN_STATUS(reef_hal_launch(preempt_kernels[i], grid, block, 0, stream, &arg, sizeof(arg)));
+    std::copy(grid, grid + 3, l.grid);
+    std::copy(block, block + 3, l.block);
+    l.bytes = sizeof(arg);
+    std::memcpy(l.args, &arg, sizeof(arg));
+    return Status::Succ;
+}
+
+// A pass of this model is one of the padding flavour or one of the best-effort flavour.
+size_t HybridExecutor::add_prefetch(Launch& l, uint32_t wgs) const {
+    if (l.bytes != sizeof(ReefBeArgs)) return TransExecutor::add_prefetch(l, wgs);
+    static_assert(sizeof(ReefBeArgs) != sizeof(ReefDkpArgs), "the two flavours' argument blocks are told apart by size");
+    ((ReefBeArgs*)l.args)->tasks = l.grid[0];
+    l.grid[0] += wgs;
+    return offsetof(ReefBeArgs, desc) + offsetof(ReefOpDesc, ptr) + REEF_PREFETCH_SLOT * sizeof(void*);
+}
+
+Status HybridExecutor::launch_preempt_kernel(int i, GPUStream_t stream) {
+    Launch l;
+    RETURN_STATUS(make_preempt_launch(i, l));
+    GPU_RETURN_STATUS(reef_hal_launch(l.fn, l.grid, l.block, 0, stream, l.args, l.bytes));
     return Status::Succ;
 }
 

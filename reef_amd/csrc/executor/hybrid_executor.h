@@ -35,6 +35,8 @@ public:
     int get_be_kernel_offset(int begin);
 
     Status launch_preempt_kernel(int kernel_offset, GPUStream_t stream);
+    Status make_preempt_launch(int kernel_offset, Launch& l) const;
+    virtual size_t add_prefetch(Launch& l, uint32_t wgs) const override;
     // Zeroes the model's "reef_sync" storage (the arrival counters of kernels that
     // fold split-K internally) in stream order.  Needed before kernels of this model
     // run again after an interrupted run; a no-op for models without that storage.
@@ -59,6 +61,7 @@ protected:
     std::shared_ptr<ModelProfile> model_profile;
     GPUDevicePtr_t sync_ptr;
     size_t sync_bytes;
+    Pass preempt_pass;
 };
 
 }  // namespace executor

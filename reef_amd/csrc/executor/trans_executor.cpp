@@ -1,6 +1,7 @@
 #include "executor/trans_executor.h"
 #include "executor/op_extents.h"
 
+#include <cstddef>
 #include <cstring>
 
 namespace reef {
@@ -80,10 +81,11 @@ void TransExecutor::fill_side(ReefDkpSide& side, int i, int layers, int task_num
 
 // Single-sided launch: the whole grid belongs to side l (trans_executor.cpp:143-171
 // passes cu_partition = num_cus and duplicates the left side into the right one).
-Status TransExecutor::launch_kernel(int i, GPUStream_t stream) {
+Status TransExecutor::make_launch(int i, Launch& l) const {
     const KernelArg& ka = trans_args[i];
     const int num_cus = (int)GPUConfig::get_num_cus();
     ReefDkpArgs a;
+    static_assert(sizeof(a) <= sizeof(l.args), "a launch record holds the padding flavour's arguments");
     std::memset(&a, 0, sizeof(a));
     fill_side(a.l, i, ka.min_occupancy, ka.block_num, ka.block_offset);
     a.r = a.l;
@@ -92,10 +94,19 @@ Status TransExecutor::launch_kernel(int i, GPUStream_t stream) {
     a.num_cus = num_cus;
     a.num_xcds = (int)GPUConfig::get_num_xcds();
     a.task_slot_r = nullptr;
-    const uint32_t grid[3] = {(uint32_t)(num_cus * ka.min_occupancy), 1, 1};
-    const uint32_t block[3] = {ka.thread_dim.count(), 1, 1};
-    GPU_RETURN_STATUS(reef_hal_launch(ka.kernel, grid, block, 0, stream, &a, sizeof(a)));
+    l.fn = ka.kernel;
+    l.grid[0] = (uint32_t)(num_cus * ka.min_occupancy);
+    l.block[0] = ka.thread_dim.count();
+    l.grid[1] = l.grid[2] = l.block[1] = l.block[2] = 1;
+    l.bytes = sizeof(a);
+    std::memcpy(l.args, &a, sizeof(a));
     return Status::Succ;
+}
+
+size_t TransExecutor::add_prefetch(Launch& l, uint32_t wgs) const {
+    ((ReefDkpArgs*)l.args)->prefetch_at = (int32_t)l.grid[0];
+    l.grid[0] += wgs;
+    return offsetof(ReefDkpArgs, l) + offsetof(ReefDkpSide, desc) + offsetof(ReefOpDesc, ptr) + REEF_PREFETCH_SLOT * sizeof(void*);
 }
 
 // One single-sided launch with an explicit layer count and task range (profiling).  cus > 0:

@@ -69,7 +69,8 @@ public:
 
 protected:
     Status init_rt_executor(const char* json_file_path, GPUModule_t module);
-    virtual Status launch_kernel(int kernel_offset, GPUStream_t stream) override;
+    virtual Status make_launch(int kernel_offset, Launch& l) const override;
+    virtual size_t add_prefetch(Launch& l, uint32_t wgs) const override;
     GPUFunction_t get_proxy_kernel(int index);
     void fill_side(ReefDkpSide& side, int kernel_offset, int layers, int task_num, int task_offset) const;
 

@@ -1,0 +1,349 @@
+#include "hal/aql.h"
+
+#include <hip/hip_runtime.h>
+#include <hsa/hsa.h>
+#include <hsa/hsa_ext_amd.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <vector>
+
+#include "hal/code_object.h"
+
+namespace reef {
+namespace hal {
+
+namespace {
+
+std::string hsa_text(hsa_status_t s, const char* what) {
+    const char* m = nullptr;
+    hsa_status_string(s, &m);
+    return std::string(what) + ": " + (m ? m : "HSA error");
+}
+
+// One hardware queue; passes of several threads interleave whole (the mutex is held while a
+// pass's packets are written, not while they run).
+struct Queue {
+    hsa_queue_t* q = nullptr;
+    std::mutex mtx;
+    std::atomic<int> error{0};
+};
+void on_queue_error(hsa_status_t s, hsa_queue_t*, void* data) { ((Queue*)data)->error.store((int)s); }
+
+constexpr int kMaxQueues = 4;      // as many as the runtime itself opens per process
+constexpr uint32_t kQueuePackets = 1024;
+
+struct Device {
+    bool tried = false, ok = false;
+    hsa_agent_t agent{};
+    Queue* queues[kMaxQueues] = {};   // opened as passes need them, kept for the life of the process
+    unsigned next = 0;
+};
+constexpr int kMaxDevices = 16;
+Device g_devices[kMaxDevices];
+std::mutex g_mtx;
+
+struct FindAgent {
+    uint32_t bdf, domain;
+    hsa_agent_t agent;
+    bool found;
+};
+hsa_status_t match_agent(hsa_agent_t a, void* data) {
+    FindAgent* f = (FindAgent*)data;
+    hsa_device_type_t type;
+    if (hsa_agent_get_info(a, HSA_AGENT_INFO_DEVICE, &type) != HSA_STATUS_SUCCESS || type != HSA_DEVICE_TYPE_GPU)
+        return HSA_STATUS_SUCCESS;
+    uint32_t bdf = 0, domain = 0;
+    if (hsa_agent_get_info(a, (hsa_agent_info_t)HSA_AMD_AGENT_INFO_BDFID, &bdf) != HSA_STATUS_SUCCESS) return HSA_STATUS_SUCCESS;
+    hsa_agent_get_info(a, (hsa_agent_info_t)HSA_AMD_AGENT_INFO_DOMAIN, &domain);
+    // the function number is no part of the runtime's device properties
+    if ((bdf & ~7u) == f->bdf && domain == f->domain && !f->found) {
+        f->agent = a;
+        f->found = true;
+    }
+    return HSA_STATUS_SUCCESS;
+}
+
+// Caller holds g_mtx.
+bool set_up(int device) {
+    if (device < 0 || device >= kMaxDevices) return false;
+    Device& d = g_devices[device];
+    if (d.tried) return d.ok;
+    d.tried = true;
+    if (const char* v = std::getenv("REEF_HAL_AQL"))
+        if (std::atoi(v) == 0) return false;
+    if (hsa_init() != HSA_STATUS_SUCCESS) return false;
+    hipDeviceProp_t p;
+    if (hipGetDeviceProperties(&p, device) != hipSuccess) return false;
+    FindAgent f{(uint32_t)((p.pciBusID << 8) | (p.pciDeviceID << 3)), (uint32_t)p.pciDomainID, hsa_agent_t{}, false};
+    hsa_iterate_agents(match_agent, &f);
+    if (!f.found) return false;
+    d.agent = f.agent;
+    d.ok = true;
+    return true;
+}
+
+// The next queue in turn.  Caller holds g_mtx.
+Queue* take_queue(Device& d, std::string* err) {
+    Queue*& q = d.queues[d.next % kMaxQueues];
+    if (!q) {
+        Queue* nq = new Queue;
+        const hsa_status_t s = hsa_queue_create(d.agent, kQueuePackets, HSA_QUEUE_TYPE_MULTI, on_queue_error, nq, UINT32_MAX,
+                                                UINT32_MAX, &nq->q);
+        if (s != HSA_STATUS_SUCCESS) {
+            delete nq;
+            *err = hsa_text(s, "hsa_queue_create");
+            return nullptr;
+        }
+        q = nq;
+    }
+    d.next++;
+    return q;
+}
+
+}  // namespace
+
+struct AqlKernel {
+    uint64_t object;
+    uint32_t lds, scratch, kernarg;
+};
+
+// The implicit arguments a kernel may read behind its own (code object version 5): block counts and
+// block sizes; everything else is zero.
+struct HiddenArgs {
+    uint32_t block_count[3];
+    uint16_t group_size[3], remainder[3];
+    uint64_t reserved[2], global_offset[3];
+    uint16_t grid_dims;
+};
+
+struct AqlCode {
+    std::vector<uint8_t> elf;
+    std::mutex mtx;
+    bool loaded = false;
+    int device = -1;
+    hsa_code_object_reader_t reader{};
+    hsa_executable_t exe{};
+    std::map<std::string, AqlKernel> kernels;
+
+    ~AqlCode() {
+        if (!loaded) return;
+        hsa_executable_destroy(exe);
+        hsa_code_object_reader_destroy(reader);
+    }
+    // Caller holds mtx.
+    bool load(int dev, hsa_agent_t agent, std::string* err) {
+        if (loaded) {
+            if (device != dev) *err = "code object is loaded on another device";
+            return device == dev;
+        }
+        hsa_status_t s = hsa_code_object_reader_create_from_memory(elf.data(), elf.size(), &reader);
+        if (s != HSA_STATUS_SUCCESS) { *err = hsa_text(s, "hsa_code_object_reader_create_from_memory"); return false; }
+        s = hsa_executable_create_alt(HSA_PROFILE_FULL, HSA_DEFAULT_FLOAT_ROUNDING_MODE_DEFAULT, nullptr, &exe);
+        if (s != HSA_STATUS_SUCCESS) {
+            hsa_code_object_reader_destroy(reader);
+            *err = hsa_text(s, "hsa_executable_create_alt");
+            return false;
+        }
+        s = hsa_executable_load_agent_code_object(exe, agent, reader, nullptr, nullptr);
+        if (s == HSA_STATUS_SUCCESS) s = hsa_executable_freeze(exe, nullptr);
+        if (s != HSA_STATUS_SUCCESS) {
+            hsa_executable_destroy(exe);
+            hsa_code_object_reader_destroy(reader);
+            *err = hsa_text(s, "hsa_executable_load_agent_code_object");
+            return false;
+        }
+        loaded = true;
+        device = dev;
+        return true;
+    }
+    bool find(const std::string& name, hsa_agent_t agent, AqlKernel* out, std::string* err) {
+        auto it = kernels.find(name);
+        if (it == kernels.end()) {
+            hsa_executable_symbol_t sym;
+            hsa_status_t s = hsa_executable_get_symbol_by_name(exe, (name + ".kd").c_str(), &agent, &sym);
+            AqlKernel k{};
+            if (s == HSA_STATUS_SUCCESS) s = hsa_executable_symbol_get_info(sym, HSA_EXECUTABLE_SYMBOL_INFO_KERNEL_OBJECT, &k.object);
+            if (s == HSA_STATUS_SUCCESS)
+                s = hsa_executable_symbol_get_info(sym, HSA_EXECUTABLE_SYMBOL_INFO_KERNEL_GROUP_SEGMENT_SIZE, &k.lds);
+            if (s == HSA_STATUS_SUCCESS)
+                s = hsa_executable_symbol_get_info(sym, HSA_EXECUTABLE_SYMBOL_INFO_KERNEL_PRIVATE_SEGMENT_SIZE, &k.scratch);
+            if (s == HSA_STATUS_SUCCESS)
+                s = hsa_executable_symbol_get_info(sym, HSA_EXECUTABLE_SYMBOL_INFO_KERNEL_KERNARG_SEGMENT_SIZE, &k.kernarg);
+            if (s != HSA_STATUS_SUCCESS) { *err = hsa_text(s, ("kernel " + name).c_str()); return false; }
+            it = kernels.emplace(name, k).first;
+        }
+        *out = it->second;
+        return true;
+    }
+};
+
+std::shared_ptr<AqlCode> aql_code_from_file(const char* path) {
+    // model directories carry copies of the same three code objects: one load serves them all
+    static std::mutex mtx;
+    static std::vector<std::weak_ptr<AqlCode>> live;
+    std::vector<uint8_t> elf;
+    std::string err;
+    if (!read_code_object_image(path, &elf, &err)) return nullptr;
+    std::lock_guard<std::mutex> lock(mtx);
+    for (size_t i = 0; i < live.size();) {
+        if (std::shared_ptr<AqlCode> c = live[i].lock()) {
+            if (c->elf == elf) return c;
+            ++i;
+        } else {
+            live.erase(live.begin() + (long)i);
+        }
+    }
+    auto c = std::make_shared<AqlCode>();
+    c->elf.swap(elf);
+    live.push_back(c);
+    return c;
+}
+
+bool aql_available(int device) {
+    std::lock_guard<std::mutex> lock(g_mtx);
+    return set_up(device);
+}
+
+struct AqlPass {
+    Queue* queue = nullptr;
+    hsa_signal_t done{};
+    void* kernargs = nullptr;    // device memory, one 64-byte aligned block per launch
+    std::vector<char> host;      // the same as it is uploaded
+    std::vector<size_t> at, tail;    // where a launch's block starts, and the caller's part inside it
+    bool committed = false;
+    std::vector<hsa_kernel_dispatch_packet_t> packets;
+    std::mutex mtx;
+    ~AqlPass() {
+        if (done.handle) hsa_signal_destroy(done);
+        if (kernargs) (void)hipFree(kernargs);
+    }
+};
+
+AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t tail_bytes, std::string* err) {
+    std::unique_ptr<AqlPass> p(new AqlPass);
+    std::lock_guard<std::mutex> lock(g_mtx);
+    if (!set_up(device)) { *err = "no packet queue on this device"; return nullptr; }
+    Device& d = g_devices[device];
+    std::vector<AqlKernel> kernels(n);
+    std::vector<size_t>& at = p->at;
+    at.resize(n + 1);
+    p->tail.resize(n);
+    size_t bytes = 0;
+    for (size_t i = 0; i < n; ++i) {
+        const AqlLaunch& l = launches[i];
+        std::lock_guard<std::mutex> code_lock(l.code->mtx);
+        if (!l.code->load(device, d.agent, err) || !l.code->find(l.name, d.agent, &kernels[i], err)) return nullptr;
+        if (l.kernarg_bytes > kernels[i].kernarg) { *err = std::string(l.name) + ": argument block larger than the kernel's"; return nullptr; }
+        at[i] = bytes;
+        p->tail[i] = ((size_t)kernels[i].kernarg + 15) / 16 * 16;
+        bytes += (p->tail[i] + tail_bytes + 63) / 64 * 64;
+    }
+    at[n] = bytes;
+    std::vector<char>& host = p->host;
+    host.assign(bytes + 64, 0);
+    for (size_t i = 0; i < n; ++i) {
+        const AqlLaunch& l = launches[i];
+        std::memcpy(host.data() + at[i], l.kernarg, l.kernarg_bytes);
+        HiddenArgs h;
+        std::memset(&h, 0, sizeof(h));
+        for (int x = 0; x < 3; ++x) {
+            h.block_count[x] = l.grid[x];
+            h.group_size[x] = (uint16_t)l.block[x];
+        }
+        h.grid_dims = 3;
+        const size_t behind = (l.kernarg_bytes + 7) / 8 * 8;
+        if (kernels[i].kernarg > behind) std::memcpy(host.data() + at[i] + behind, &h, std::min(sizeof(h), kernels[i].kernarg - behind));
+    }
+    const hipError_t e = hipMalloc(&p->kernargs, host.size());
+    if (e != hipSuccess) { *err = std::string("argument blocks: ") + hipGetErrorString(e); return nullptr; }
+    for (size_t i = 0; i < n; ++i) {
+        const AqlLaunch& l = launches[i];
+        const AqlKernel& k = kernels[i];
+        hsa_kernel_dispatch_packet_t a;
+        std::memset(&a, 0, sizeof(a));
+        // Launches follow one another (barrier) and see each other's results; the first also sees what
+        // the host and the copy engines wrote, the last makes its results visible to them.
+        const int acquire = i == 0 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
+        const int release = i == n - 1 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
+        a.header = (uint16_t)((HSA_PACKET_TYPE_KERNEL_DISPATCH << HSA_PACKET_HEADER_TYPE) | (1 << HSA_PACKET_HEADER_BARRIER) |
+                              (acquire << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE) |
+                              (release << HSA_PACKET_HEADER_SCRELEASE_FENCE_SCOPE));
+        a.setup = (uint16_t)(3 << HSA_KERNEL_DISPATCH_PACKET_SETUP_DIMENSIONS);
+        a.workgroup_size_x = (uint16_t)l.block[0];
+        a.workgroup_size_y = (uint16_t)l.block[1];
+        a.workgroup_size_z = (uint16_t)l.block[2];
+        a.grid_size_x = l.grid[0] * l.block[0];
+        a.grid_size_y = l.grid[1] * l.block[1];
+        a.grid_size_z = l.grid[2] * l.block[2];
+        a.private_segment_size = k.scratch;
+        a.group_segment_size = k.lds + l.dyn_lds;
+        a.kernel_object = k.object;
+        a.kernarg_address = (char*)p->kernargs + at[i];
+        p->packets.push_back(a);
+    }
+    const hsa_status_t s = hsa_signal_create(0, 0, nullptr, &p->done);
+    if (s != HSA_STATUS_SUCCESS) { *err = hsa_text(s, "hsa_signal_create"); return nullptr; }
+    if (n) p->packets.back().completion_signal = p->done;
+    p->queue = take_queue(d, err);
+    return p->queue ? p.release() : nullptr;
+}
+
+bool aql_pass_block(AqlPass* p, size_t i, char** device, char** host, size_t* bytes, size_t* tail) {
+    if (i >= p->packets.size()) return false;
+    *device = (char*)p->kernargs + p->at[i];
+    *host = p->host.data() + p->at[i];
+    *bytes = p->at[i + 1] - p->at[i];
+    *tail = p->tail[i];
+    return true;
+}
+
+bool aql_pass_commit(AqlPass* p, std::string* err) {
+    const hipError_t e = hipMemcpy(p->kernargs, p->host.data(), p->host.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) *err = hipGetErrorString(e);
+    p->committed = e == hipSuccess;
+    return p->committed;
+}
+
+bool aql_pass_run(AqlPass* p, std::string* err) {
+    if (p->packets.empty()) return true;
+    if (!p->committed) { *err = "the pass has not been committed"; return false; }
+    std::lock_guard<std::mutex> lock(p->mtx);
+    Queue& w = *p->queue;
+    hsa_signal_store_relaxed(p->done, 1);
+    {
+        std::lock_guard<std::mutex> submit(w.mtx);
+        hsa_queue_t* q = w.q;
+        const size_t n = p->packets.size();
+        for (size_t i = 0; i < n; ++i) {
+            const uint64_t idx = hsa_queue_add_write_index_relaxed(q, 1);
+            while (idx - hsa_queue_load_read_index_scacquire(q) >= q->size) {
+                hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)(idx - 1));   // the device works the ring down
+                if (w.error.load()) { *err = hsa_text((hsa_status_t)w.error.load(), "queue"); return false; }
+            }
+            char* slot = (char*)q->base_address + (idx & (q->size - 1)) * sizeof(hsa_kernel_dispatch_packet_t);
+            const char* src = (const char*)&p->packets[i];
+            // the first four bytes (header and setup) hand the packet to the device: last, in one store
+            std::memcpy(slot + 4, src + 4, sizeof(hsa_kernel_dispatch_packet_t) - 4);
+            uint32_t head;
+            std::memcpy(&head, src, 4);
+            __atomic_store_n((uint32_t*)slot, head, __ATOMIC_RELEASE);
+            // The device starts on the first packets while the rest are written.  No doorbell covers packets
+            // on both sides of the ring's end: a profiler's interception takes such a run for contiguous.
+            if (i == n - 1 || (i & 31) == 3 || ((idx + 1) & (q->size - 1)) == 0) hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)idx);
+        }
+    }
+    // the wait looks at the queue's error word once a second, so that a failed queue ends it
+    while (hsa_signal_wait_scacquire(p->done, HSA_SIGNAL_CONDITION_LT, 1, 1000000000ull, HSA_WAIT_STATE_ACTIVE) >= 1)
+        if (w.error.load()) { *err = hsa_text((hsa_status_t)w.error.load(), "queue"); return false; }
+    return true;
+}
+
+void aql_pass_destroy(AqlPass* p) { delete p; }
+
+}  // namespace hal
+}  // namespace reef

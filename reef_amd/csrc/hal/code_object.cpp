@@ -146,8 +146,7 @@ bool parse_elf(const uint8_t* b, size_t n, std::map<std::string, KernelMeta>* ou
 
 }  // namespace
 
-bool read_code_object_metadata(const char* path, std::map<std::string, KernelMeta>* out,
-                               std::string* err) {
+bool read_code_object_image(const char* path, std::vector<uint8_t>* elf, std::string* err) {
     std::string dummy;
     if (!err) err = &dummy;
     FILE* fp = std::fopen(path, "rb");
@@ -155,32 +154,42 @@ bool read_code_object_metadata(const char* path, std::map<std::string, KernelMet
     std::fseek(fp, 0, SEEK_END);
     long sz = std::ftell(fp);
     std::fseek(fp, 0, SEEK_SET);
-    std::vector<uint8_t> buf(sz > 0 ? (size_t)sz : 0);
+    std::vector<uint8_t>& buf = *elf;
+    buf.assign(sz > 0 ? (size_t)sz : 0, 0);
     size_t got = buf.empty() ? 0 : std::fread(buf.data(), 1, buf.size(), fp);
     std::fclose(fp);
     if (got != buf.size() || buf.size() < 32) { *err = "short read"; return false; }
 
     static const char kBundle[] = "__CLANG_OFFLOAD_BUNDLE__";
-    if (std::memcmp(buf.data(), kBundle, 24) == 0) {
-        uint64_t n;
-        std::memcpy(&n, buf.data() + 24, 8);
-        size_t off = 32;
-        for (uint64_t i = 0; i < n && off + 24 <= buf.size(); ++i) {
-            uint64_t o, s, ts;
-            std::memcpy(&o, buf.data() + off, 8);
-            std::memcpy(&s, buf.data() + off + 8, 8);
-            std::memcpy(&ts, buf.data() + off + 16, 8);
-            off += 24;
-            if (off + ts > buf.size()) break;
-            std::string triple((const char*)buf.data() + off, ts);
-            off += ts;
-            if (triple.find("amdgcn") != std::string::npos && s > 0 && o + s <= buf.size())
-                return parse_elf(buf.data() + o, s, out, err);
+    if (std::memcmp(buf.data(), kBundle, 24) != 0) return true;
+    uint64_t n;
+    std::memcpy(&n, buf.data() + 24, 8);
+    size_t off = 32;
+    for (uint64_t i = 0; i < n && off + 24 <= buf.size(); ++i) {
+        uint64_t o, s, ts;
+        std::memcpy(&o, buf.data() + off, 8);
+        std::memcpy(&s, buf.data() + off + 8, 8);
+        std::memcpy(&ts, buf.data() + off + 16, 8);
+        off += 24;
+        if (off + ts > buf.size()) break;
+        std::string triple((const char*)buf.data() + off, ts);
+        off += ts;
+        if (triple.find("amdgcn") != std::string::npos && s > 0 && o + s <= buf.size()) {
+            buf.erase(buf.begin(), buf.begin() + (long)o);
+            buf.resize(s);
+            return true;
         }
-        *err = "offload bundle holds no amdgcn code object";
-        return false;
     }
-    return parse_elf(buf.data(), buf.size(), out, err);
+    *err = "offload bundle holds no amdgcn code object";
+    return false;
+}
+
+bool read_code_object_metadata(const char* path, std::map<std::string, KernelMeta>* out,
+                               std::string* err) {
+    std::string dummy;
+    if (!err) err = &dummy;
+    std::vector<uint8_t> elf;
+    return read_code_object_image(path, &elf, err) && parse_elf(elf.data(), elf.size(), out, err);
 }
 
 }  // namespace hal

@@ -10,6 +10,7 @@
 #include <cstdint>
 #include <map>
 #include <string>
+#include <vector>
 
 namespace reef {
 namespace hal {
@@ -23,6 +24,9 @@ struct KernelMeta {
     int kernarg = 0;  // kernarg segment bytes
     int max_threads = 0;
 };
+
+// The ELF image in `path`: the file itself, or the device part of an offload bundle.
+bool read_code_object_image(const char* path, std::vector<uint8_t>* elf, std::string* err);
 
 // name -> metadata.  Returns false and fills err when the file cannot be parsed.
 bool read_code_object_metadata(const char* path, std::map<std::string, KernelMeta>* out,

@@ -102,6 +102,13 @@ int reef_hal_stream_clear_queue(reef_stream_t s, uint64_t* n_dropped) {
     return be()->stream_clear_queue(s, n_dropped);
 }
 int reef_hal_reset_cus(void) { return be()->reset_cus(); }
+int reef_hal_pass_create(const reef_pass_launch* launches, size_t n, size_t tail_bytes, reef_pass_t* out) {
+    return be()->pass_create ? be()->pass_create(launches, n, tail_bytes, out) : 2;
+}
+int reef_hal_pass_block(reef_pass_t p, size_t i, reef_pass_block* out) { return be()->pass_block ? be()->pass_block(p, i, out) : 1; }
+int reef_hal_pass_commit(reef_pass_t p) { return be()->pass_commit ? be()->pass_commit(p) : 1; }
+int reef_hal_pass_run(reef_pass_t p, reef_stream_t after) { return be()->pass_run ? be()->pass_run(p, after) : 1; }
+int reef_hal_pass_destroy(reef_pass_t p) { return p && be()->pass_destroy ? be()->pass_destroy(p) : 0; }
 int reef_hal_event_create(reef_event_t* out) { return be()->event_create(out); }
 int reef_hal_event_destroy(reef_event_t e) { return be()->event_destroy(e); }
 int reef_hal_event_record(reef_event_t e, reef_stream_t s) { return be()->event_record(e, s); }

@@ -5,15 +5,18 @@
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
 
+#include "hal/aql.h"
 #include "hal/code_object.h"
 #include "reef_hal.h"
 
@@ -26,12 +29,14 @@ struct reef_module_s {
     hipModule_t mod;
     std::map<std::string, reef::hal::KernelMeta> meta;
     std::vector<reef_function_s*> fns;
+    std::shared_ptr<reef::hal::AqlCode> code;   // the same code object for recorded passes
 };
 struct reef_function_s {
     hipFunction_t fn;
     reef::hal::KernelMeta meta;
     bool has_meta;
     std::string name;
+    reef_module_s* mod;
 };
 
 namespace {
@@ -105,6 +110,7 @@ struct reef_stream_s {
     std::atomic<size_t> held_count{0};   // mirror of held.size(), readable without mtx
     std::atomic<uint32_t> enqueued{0};   // highest seq whose runtime calls have returned
     bool has_feeder = false;
+    std::atomic<bool> pending{false};    // runtime work enqueued since the last synchronisation
 };
 
 struct reef_graph_s {
@@ -203,6 +209,7 @@ int h_module_load(const char* path, reef_module_t* out) {
     }
     std::string err;
     if (!reef::hal::read_code_object_metadata(path, &m->meta, &err)) m->meta.clear();
+    m->code = reef::hal::aql_code_from_file(path);
     *out = m;
     return 0;
 }
@@ -222,6 +229,7 @@ int h_module_get_function(reef_module_t m, const char* name, reef_function_t* ou
     reef_function_s* f = new reef_function_s;
     f->fn = fn;
     f->name = name;
+    f->mod = m;
     auto it = m->meta.find(name);
     f->has_meta = it != m->meta.end();
     if (f->has_meta) f->meta = it->second;
@@ -278,10 +286,12 @@ int h_memset(reef_devptr_t p, int byte, size_t n) { HIPCHK(hipMemset(p, byte, n)
 int h_h2d(reef_devptr_t d, const void* s, size_t n) { HIPCHK(hipMemcpy(d, s, n, hipMemcpyHostToDevice)); return 0; }
 int h_d2h(void* d, reef_devptr_t s, size_t n) { HIPCHK(hipMemcpy(d, s, n, hipMemcpyDeviceToHost)); return 0; }
 int h_h2d_async(reef_devptr_t d, const void* s, size_t n, reef_stream_t st) {
+    if (st) st->pending.store(true, std::memory_order_release);
     HIPCHK(hipMemcpyAsync(d, s, n, hipMemcpyHostToDevice, st ? st->s : nullptr));
     return 0;
 }
 int h_d2h_async(void* d, reef_devptr_t s, size_t n, reef_stream_t st) {
+    if (st) st->pending.store(true, std::memory_order_release);
     HIPCHK(hipMemcpyAsync(d, s, n, hipMemcpyDeviceToHost, st ? st->s : nullptr));
     return 0;
 }
@@ -498,12 +508,13 @@ int submit(reef_stream_t st, hipFunction_t fn, const uint32_t* g, const uint32_t
         c.exit_ticks = (uint64_t*)&st->exit_ticks[seq % kExitRing];
         c.exit_count = st->exit_count;
         c.seq = seq;
-        c.reserved = 0;
+        std::memcpy(&c.user, (const char*)kernarg + offsetof(reef_hal_completion, user), sizeof(c.user));
         std::memcpy(patched, &c, sizeof(c));
         kernarg = patched;
     }
     void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, const_cast<void*>(kernarg),
                      HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz, HIP_LAUNCH_PARAM_END};
+    if (st) st->pending.store(true, std::memory_order_release);
     HIPCHK(hipModuleLaunchKernel(fn, g[0], g[1], g[2], b[0], b[1], b[2], lds, st ? st->s : nullptr,
                                  nullptr, extra));
     if (seq != 0) {
@@ -567,6 +578,7 @@ int h_stream_sync(reef_stream_t st) {
         if (int rc = drain_ring(st)) return rc;
         std::lock_guard<std::mutex> sub(st->submit_mtx);   // a launch the feeder has in hand is enqueued
     }
+    if (st) st->pending.store(false, std::memory_order_release);   // what is enqueued from now on counts again
     HIPCHK(hipStreamSynchronize(st ? st->s : nullptr));
     return 0;
 }
@@ -597,6 +609,7 @@ int h_stream_query(reef_stream_t st, int* idle) {
 int h_device_sync() { HIPCHK(hipDeviceSynchronize()); return 0; }
 
 int h_write_value32(reef_stream_t st, reef_devptr_t p, int32_t v) {
+    if (st) st->pending.store(true, std::memory_order_release);
     HIPCHK(hipStreamWriteValue32(st ? st->s : nullptr, p, (uint32_t)v, 0));
     return 0;
 }
@@ -703,6 +716,7 @@ int h_graph_launch(reef_graph_t g, reef_stream_t st) {
         reef_hal_set_error("reef_hal_graph_launch: bad graph or windowed stream");
         return 1;
     }
+    if (st) st->pending.store(true, std::memory_order_release);
     HIPCHK(hipGraphLaunch(g->exec, st ? st->s : nullptr));
     return 0;
 }
@@ -711,6 +725,52 @@ int h_graph_destroy(reef_graph_t g) {
     hipGraphExecDestroy(g->exec);
     hipGraphDestroy(g->graph);
     delete g;
+    return 0;
+}
+int h_pass_create(const reef_pass_launch* l, size_t n, size_t tail_bytes, reef_pass_t* out) {
+    if (!out || (n && !l)) { reef_hal_set_error("reef_hal_pass_create: null argument"); return 1; }
+    if (!reef::hal::aql_available(g_device)) return 2;
+    std::vector<reef::hal::AqlLaunch> a(n);
+    for (size_t i = 0; i < n; ++i) {
+        reef_module_s* m = l[i].fn->mod;
+        if (!m->code) return 2;
+        a[i].code = m->code.get();
+        a[i].name = l[i].fn->name.c_str();
+        std::memcpy(a[i].grid, l[i].grid, sizeof(a[i].grid));
+        std::memcpy(a[i].block, l[i].block, sizeof(a[i].block));
+        a[i].dyn_lds = l[i].dyn_lds;
+        a[i].kernarg = l[i].kernarg;
+        a[i].kernarg_bytes = l[i].kernarg_bytes;
+    }
+    std::string err;
+    reef::hal::AqlPass* p = reef::hal::aql_pass_create(g_device, a.data(), n, tail_bytes, &err);
+    if (!p) { reef_hal_set_error(("reef_hal_pass_create: " + err).c_str()); return 1; }
+    *out = (reef_pass_t)p;
+    return 0;
+}
+int h_pass_run(reef_pass_t p, reef_stream_t after) {
+    if (!p) { reef_hal_set_error("reef_hal_pass_run: null argument"); return 1; }
+    // whatever the stream was given runs first (the queue of the pass knows nothing of it)
+    if (!after || after->window > 0 || after->pending.load(std::memory_order_acquire))
+        if (int rc = h_stream_sync(after)) return rc;
+    std::string err;
+    if (reef::hal::aql_pass_run((reef::hal::AqlPass*)p, &err)) return 0;
+    reef_hal_set_error(("reef_hal_pass_run: " + err).c_str());
+    return 1;
+}
+int h_pass_block(reef_pass_t p, size_t i, reef_pass_block* out) {
+    if (p && out && reef::hal::aql_pass_block((reef::hal::AqlPass*)p, i, &out->device, &out->host, &out->bytes, &out->tail)) return 0;
+    reef_hal_set_error("reef_hal_pass_block: no such launch");
+    return 1;
+}
+int h_pass_commit(reef_pass_t p) {
+    std::string err;
+    if (p && reef::hal::aql_pass_commit((reef::hal::AqlPass*)p, &err)) return 0;
+    reef_hal_set_error(("reef_hal_pass_commit: " + err).c_str());
+    return 1;
+}
+int h_pass_destroy(reef_pass_t p) {
+    reef::hal::aql_pass_destroy((reef::hal::AqlPass*)p);
     return 0;
 }
 int h_clear_queue(reef_stream_t st, uint64_t* n) {
@@ -736,6 +796,7 @@ int fill_async(reef_devptr_t p, int byte, size_t n, hipStream_t s) {
 }
 
 int h_memset_async(reef_devptr_t p, int byte, size_t n, reef_stream_t st) {
+    if (st) st->pending.store(true, std::memory_order_release);
     // a windowed stream may hold launches on the host: the fill must not overtake them
     if (st && st->window > 0) {
         if (int rc = drain_ring(st)) return rc;
@@ -753,6 +814,7 @@ int h_event_create(reef_event_t* out) {
 }
 int h_event_destroy(reef_event_t e) { HIPCHK(hipEventDestroy((hipEvent_t)e)); return 0; }
 int h_event_record(reef_event_t e, reef_stream_t st) {
+    if (st) st->pending.store(true, std::memory_order_release);
     HIPCHK(hipEventRecord((hipEvent_t)e, st ? st->s : nullptr));
     return 0;
 }
@@ -774,6 +836,7 @@ const reef_hal_backend kHip = {
     h_graph_begin, h_graph_end, h_graph_launch, h_graph_destroy,
     h_stream_set_completion, h_stream_progress, h_stream_exit_ticks, h_clock_sync,
     h_module_kernel_entry, h_host_fill32, h_stream_drained,
+    h_pass_create, h_pass_block, h_pass_commit, h_pass_run, h_pass_destroy,
 };
 
 }  // namespace

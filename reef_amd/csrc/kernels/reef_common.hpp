@@ -127,6 +127,71 @@ __device__ __forceinline__ float gelu_erf(float x) {
     return x * (0.5f + 0.5f * erff(x * 0.70710678f));
 }
 
+// ---- prefetching workgroups --------------------------------------------------------
+// A layer's weights are read once per inference and its kernels last a few microseconds: the first
+// use of every line is a trip to HBM, through translations nobody has used since the last
+// inference, in front of everything else (1x1 1024 -> 256 at 14x14: 5.6 us per launch with the
+// weights cold, 3.8 with them in L2).  The launch in front has idle CUs and an idle memory system
+// while it computes, so a few workgroups behind its tasks touch one word of every 128-byte line of
+// the slice that this XCD will need (L2 keeps its lines across launches): 4.0 us per launch.
+// 16 to 64 of them measured the same, 8 leave 0.7 us of it (a CU's share gets too long); as a
+// launch of its own beside the kernel it costs a packet, 1.4 us.
+// All of a thread's loads are issued together and waited for once, at the end of the workgroup (which
+// must not outlast the tasks); their values are not used.  A thread without a line repeats its first.
+__device__ __forceinline__ void touch4(const char* a, const char* b, const char* c, const char* d) {
+    unsigned t0, t1, t2, t3;
+    asm volatile("global_load_dword %0, %4, off\n\tglobal_load_dword %1, %5, off\n\t"
+                 "global_load_dword %2, %6, off\n\tglobal_load_dword %3, %7, off\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3) : "v"(a), "v"(b), "v"(c), "v"(d) : "memory");
+}
+// j: number of this workgroup among the prefetching ones.  The last of an XCD takes the small
+// operands, the others the XCD's slice of the weights.
+__device__ __forceinline__ void prefetch_lines(const ReefPrefetch* r, int j) {
+    constexpr int X = REEF_PREFETCH_WGS_UNIT;
+    const unsigned slot = (unsigned)j / X, per = r->wgs / X - 1, x = blockIdx.x % X, tid = threadIdx.x;
+    const char* at[REEF_PREFETCH_SMALL];
+    if (slot == per) {
+        static_assert(REEF_PREFETCH_SMALL == 6, "two rounds of four below");
+#pragma unroll
+        for (int s = 0; s < REEF_PREFETCH_SMALL; ++s) {
+            const char* p = r->small_[s].p;
+            const unsigned bytes = (unsigned)r->small_[s].bytes;
+            p = bytes ? p : (const char*)r;
+            at[s] = tid * 128u < bytes ? p + tid * 128u : p;
+        }
+        touch4(at[0], at[1], at[2], at[3]);
+        touch4(at[4], at[5], at[5], at[5]);
+        return;
+    }
+    const unsigned step = per * kThreads * 128u, first = (slot * kThreads + tid) * 128u;
+    const unsigned chunks = r->chunks, chunk_bytes = r->chunk_bytes, total = r->total;
+    if (r->interleaved) {
+        // every eighth piece, as if they lay one behind the other
+        const unsigned mine = (chunks - x + X - 1) / X, bytes = mine * chunk_bytes;
+        for (unsigned o = first; o < bytes; o += 4 * step) {
+            const char* q[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned ou = o + u * step < bytes ? o + u * step : o;
+                const unsigned c = div_small((int)(ou / 16u), (int)(chunk_bytes / 16u));
+                const unsigned p = (c * X + x) * chunk_bytes + (ou - c * chunk_bytes);
+                q[u] = r->base + (p < total ? p : 0u);
+            }
+            touch4(q[0], q[1], q[2], q[3]);
+        }
+        return;
+    }
+    const unsigned lo = min(x * chunks / X * chunk_bytes, total);
+    const unsigned bytes = min(((x + 1) * chunks + X - 1) / X * chunk_bytes, total) - lo;
+    const char* base = r->base + lo;
+    for (unsigned o = first; o < bytes; o += 4 * step) {
+        const char* q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = base + (o + u * step < bytes ? o + u * step : o);
+        touch4(q[0], q[1], q[2], q[3]);
+    }
+}
+
 // Optional operands of the conv / reduce epilogue follow the fixed pointers in
 // flag-bit order: bias, residual, scale, shift.
 struct Epilogue {

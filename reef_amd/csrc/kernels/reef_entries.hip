@@ -27,9 +27,30 @@ using namespace reef_dev;
 
 namespace {
 
+// Tasks of a plain launch, from its attributes: workgroups behind them prefetch for the next launch.
+// Ops without a count here are never given any.
+__device__ __forceinline__ int conv_tasks(const ReefOpDesc& d) {
+    return d.attr[REEF_CONV_SPLIT_K] * d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
+}
+__device__ __forceinline__ int gemm_tasks(const ReefOpDesc& d) {
+    const int s = d.attr[REEF_GEMM_SPLIT_K];
+    return d.attr[REEF_GEMM_BATCH] * d.attr[REEF_GEMM_M_TILES] * d.attr[REEF_GEMM_N_TILES] * (s > 1 ? s : 1);
+}
+__device__ __forceinline__ int attention_tasks(const ReefOpDesc& d) {
+    return d.attr[REEF_AT_HEADS] * ((d.attr[REEF_AT_SEQ] + REEF_AT_ROWS - 1) / REEF_AT_ROWS);
+}
+__device__ __forceinline__ int pool_tasks(const ReefOpDesc& d) {
+    return (d.attr[REEF_POOL_C] * d.attr[REEF_POOL_HO] * d.attr[REEF_POOL_WO] + kThreads - 1) / kThreads;
+}
+__device__ __forceinline__ int gap_tasks(const ReefOpDesc& d) { return (d.attr[REEF_GAP_C] + 3) / 4; }
+__device__ __forceinline__ int no_tasks(const ReefOpDesc&) { return 0x7fffffff; }
+#define REEF_TASKS(FN) \
+    static __device__ __forceinline__ int tasks(const ReefOpDesc& d) { return FN(d); }
+
 // ---- op functors: LDS need + body ------------------------------------------
 template <class T, int MODE = CONV_GENERAL>
 struct OpConv {
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = T::LDS_BYTES;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
@@ -38,6 +59,7 @@ struct OpConv {
 };
 template <int R, int TN = 1, int TM = 1, bool PRE = false, bool ROWS = false, bool PACKED = false>
 struct OpConvDirect {
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;   // the body makes the wrapper's first flag check
     template <class P>
@@ -56,6 +78,7 @@ using OpConvRows = OpConvDirect<9, G, TM, false, true>;
 // 1x1 convolution and the depthwise 3x3 convolution (stride S) behind it in one launch
 template <int G, int S = 1>
 struct OpConvXdw {
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileXdw<G, S>::LDS_BYTES;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
@@ -66,6 +89,7 @@ struct OpConvXdw {
 // projection in one launch, every channel in one workgroup
 template <int G, int S, bool STEM, int MT, int KC>
 struct OpConvBlock {
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileBlk<G, S, STEM, MT, KC>::LDS_BYTES;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
@@ -74,6 +98,7 @@ struct OpConvBlock {
 };
 // 7x7 stride-2 convolution and the 3x3 stride-2 max-pool behind it in one launch
 struct OpConvStemPool {
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileSp7::LDS_BYTES;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
@@ -82,6 +107,7 @@ struct OpConvStemPool {
 };
 template <class T, bool TRANS_B, bool LN_A = false>
 struct OpGemm {
+    REEF_TASKS(gemm_tasks)
     static constexpr int LDS = T::LDS_BYTES + (LN_A ? 2 * T::BM * 4 : 0);   // + mean, rstd of the tile's rows
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
@@ -90,6 +116,7 @@ struct OpGemm {
 };
 template <int TM, int TN>
 struct OpGemmNtDirect {
+    REEF_TASKS(gemm_tasks)
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
@@ -97,8 +124,9 @@ struct OpGemmNtDirect {
         return gemm_nt_direct_body<TM, TN>(d, task, smem, p);
     }
 };
-#define REEF_SIMPLE_OP(STRUCT, CALL)                                                            \
+#define REEF_SIMPLE_OP(STRUCT, CALL, TASKS)                                                     \
     struct STRUCT {                                                                             \
+        REEF_TASKS(TASKS)                                                                       \
         static constexpr int LDS = 0;                                                           \
         template <class P>                                                                      \
         static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char*, const P&) { \
@@ -107,6 +135,7 @@ struct OpGemmNtDirect {
         }                                                                                       \
     };
 struct OpAttention {
+    REEF_TASKS(attention_tasks)
     static constexpr int LDS = REEF_AT_LDS_BYTES;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P&) {
@@ -114,22 +143,23 @@ struct OpAttention {
         return true;
     }
 };
-REEF_SIMPLE_OP(OpSplitKReduce, splitk_reduce_body<8>)
-REEF_SIMPLE_OP(OpDwConv, dwconv2d_body)
-REEF_SIMPLE_OP(OpPool, pool2d_body)
-REEF_SIMPLE_OP(OpGap, global_avgpool_body)
-REEF_SIMPLE_OP(OpEltwise, eltwise_body)
-REEF_SIMPLE_OP(OpDense, dense_body)
-REEF_SIMPLE_OP(OpSoftmax, softmax_body)
-REEF_SIMPLE_OP(OpLayerNorm, layernorm_body)
-REEF_SIMPLE_OP(OpBiasGelu, bias_gelu_body)
-REEF_SIMPLE_OP(OpEmbedding, embedding_body)
-REEF_SIMPLE_OP(OpCopy, copy_body)
-REEF_SIMPLE_OP(OpTranspose, transpose_body)
+REEF_SIMPLE_OP(OpSplitKReduce, splitk_reduce_body<8>, no_tasks)
+REEF_SIMPLE_OP(OpDwConv, dwconv2d_body, no_tasks)
+REEF_SIMPLE_OP(OpPool, pool2d_body, pool_tasks)
+REEF_SIMPLE_OP(OpGap, global_avgpool_body, gap_tasks)
+REEF_SIMPLE_OP(OpEltwise, eltwise_body, no_tasks)
+REEF_SIMPLE_OP(OpDense, dense_body, no_tasks)
+REEF_SIMPLE_OP(OpSoftmax, softmax_body, no_tasks)
+REEF_SIMPLE_OP(OpLayerNorm, layernorm_body, no_tasks)
+REEF_SIMPLE_OP(OpBiasGelu, bias_gelu_body, no_tasks)
+REEF_SIMPLE_OP(OpEmbedding, embedding_body, no_tasks)
+REEF_SIMPLE_OP(OpCopy, copy_body, no_tasks)
+REEF_SIMPLE_OP(OpTranspose, transpose_body, no_tasks)
 
 // The mocked kernels keep the reference's 128 logical threads per block.
 template <bool MUL>
 struct OpMocked {
+    REEF_TASKS(no_tasks)
     static constexpr int LDS = 0;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char*, const P&) {
@@ -234,7 +264,13 @@ __device__ __forceinline__ bool dkp_walk(const ReefDkpArgs& a, DkpWalk& w) {
     extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS) NAME(ReefOpDesc) {  \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];               \
         kernarg_warm<sizeof(ReefOpDesc)>();                                           \
-        OP::run(kernarg_at<ReefOpDesc>(0), (int)blockIdx.x, smem, NoPoll{true});      \
+        const ReefOpDesc& d = kernarg_at<ReefOpDesc>(0);                              \
+        const int behind = (int)blockIdx.x - OP::tasks(d);                            \
+        if (behind >= 0) {                                                            \
+            prefetch_lines((const ReefPrefetch*)d.ptr[REEF_PREFETCH_SLOT], behind);   \
+            return;                                                                   \
+        }                                                                             \
+        OP::run(d, (int)blockIdx.x, smem, NoPoll{true});                              \
     }
 #elif REEF_FLAVOUR == 1
 namespace {
@@ -273,7 +309,9 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         const int t = threadIdx.x + threadIdx.y * blockDim.x + threadIdx.z * blockDim.x * blockDim.y; \
         FlagPoll poll{a.preempted};                                                       \
         bool done = false;                                                                \
-        if (ChecksFlagItself<OP>::value) {                                                \
+        if (a.tasks != 0 && blockIdx.x >= a.tasks) {                                      \
+            prefetch_lines((const ReefPrefetch*)a.desc.ptr[REEF_PREFETCH_SLOT], (int)(blockIdx.x - a.tasks)); \
+        } else if (ChecksFlagItself<OP>::value) {                                                \
             done = OP::run(a.desc, (int)blockIdx.x, smem, poll);                          \
         } else {                                                                          \
             if (t == 0) s_pre = poll.load();                                              \
@@ -293,6 +331,10 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];                \
         kernarg_warm<sizeof(ReefDkpArgs)>();                                           \
         const ReefDkpArgs& a = kernarg_at<ReefDkpArgs>(0);                             \
+        if (a.prefetch_at != 0 && (int)blockIdx.x >= a.prefetch_at) {                  \
+            prefetch_lines((const ReefPrefetch*)a.l.desc.ptr[REEF_PREFETCH_SLOT], (int)blockIdx.x - a.prefetch_at); \
+            return;                                                                    \
+        }                                                                              \
         DkpWalk w;                                                                     \
         if (!dkp_walk(a, w)) return;                                                   \
         const ReefDkpSide& side = w.right ? a.r : a.l;                                 \
