@@ -234,7 +234,7 @@ class GraphBuilder:
         t = force or tiling.choose(M, N, K, fused=fused_reduce, pointwise=(kh, kw) == (1, 1),
                                    taps=kh * kw, direct=tiling.direct_ok(cin, kh, kw),
                                    rows=tiling.rows_ok(kh, kw, sh, sw, ph, pw), image=(Ho, Wo),
-                                   under_load=self.under_load)
+                                   under_load=self.under_load, stride=max(sh, sw), pre_act=pre_act)
         if t.get("fused"):
             fused_reduce = True       # the measured table asks for the split folded into the launch
         pre = []

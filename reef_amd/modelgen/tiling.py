@@ -162,12 +162,15 @@ def _steps_time(bm, bn, eff, steps):
 
 
 def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, pointwise=False,
-           taps=1, direct=False, rows=False, image=None, under_load=False):
+           taps=1, direct=False, rows=False, image=None, under_load=False, stride=1, pre_act=False):
     """Returns dict(tile, tile_id, BM, BN, split_k, k_chunk, m_tiles, n_tiles, tasks).
     Measured choices (tuned.py) win over the analytic model for the shapes they cover; an entry
     that names the direct tile counts only if the caller says the filter qualifies.
     under_load: the layer belongs to a model that shares the device with other streams; the
-    entries measured for that case (TUNED_UNDER_LOAD) come before those measured alone."""
+    entries measured for that case (TUNED_UNDER_LOAD) come before those measured alone.
+    image: output rows and columns of a convolution (with stride, pre_act: the input goes through an
+    activation of its own); shapes outside the table are then chosen by the measured cost of every
+    tile (CONV_COST), those of a bare matrix product by the analytic model."""
     if allow_split and tiles is None and not fused:
         key = (M, N, K, 1 if pointwise else 0)
         hit = TUNED.get(key)
@@ -186,9 +189,9 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
             t["est_us"] = hit[2]
             t["fused"] = hit[1] < 0
             return t
+    if allow_split and tiles is None and (image is not None or direct and M * N <= NUM_CUS * 4096):
+        return _choose_conv(M, N, K, taps, direct, rows and image is not None, image, stride, pointwise, pre_act)
     best = None
-    if allow_split and tiles is None and direct:
-        best = _choose_direct(M, N, K, taps, fused, rows, image)
     for name in (tiles or [t for t in TILES if t not in DIRECT_TILES and t not in ROW_TILES]):
         tid, bm, bn, eff, occ = TILES[name]
         m_tiles, n_tiles = math.ceil(M / bm), math.ceil(N / bn)
@@ -213,67 +216,118 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
             cand = (t, name, s_eff, k_chunk, m_tiles, n_tiles)
             if best is None or cand[0] < best[0] - 1e-9:
                 best = cand
-    if len(best) == 2:          # a direct or row-form geometry, complete already
-        return best[1]
     t, name, s, k_chunk, m_tiles, n_tiles = best
     tid, bm, bn, _, _ = TILES[name]
     return dict(tile=name, tile_id=tid, BM=bm, BN=bn, split_k=s, k_chunk=k_chunk,
                 m_tiles=m_tiles, n_tiles=n_tiles, tasks=s * m_tiles * n_tiles, est_us=t)
 
 
-# Cost of a direct-family launch in microseconds, for shapes the measured table does not cover.
-# Linear in what the batch-1 sweeps showed to matter: the cache lines a workgroup pulls in,
-# (BM + BN) K_chunk / 32, times the rounds of workgroups the device needs; the workgroups per
-# CU; and what a split of K adds (folded inside the launch, or as a launch of its own).  The
-# constants are a least-squares fit over the 4095 direct candidates of the sweeps behind
-# tuned.py (181 shapes of four networks, rms error 12 %); choosing by this model instead of by
-# measurement costs 7 % on average over those shapes (worst case 1.5x), where the staged tiles
-# alone cost 62 % (worst 2.8x).
-DIRECT_COST = dict(fixed=3.57, per_line_round=0.00377, fused_split=2.20, separate_split=2.92,
-                   per_wg_per_cu=0.689, per_split=0.172)
+# Cost of a convolution launch in microseconds, for shapes the measured table does not cover: per
+# tile and kind of filter,
+#     c0 + w (c1 + c2 (r + ceil(r)) / 2 + c3 max(1, r)) + c4 r   (+ c5 + c6 split / 10 where K is split)
+# with w = a workgroup's share of K in thousands and r = workgroups per CU.  c1 is the serial chain
+# of one workgroup, c2 and c3 what the CU's matrix pipes and loads need for all of its workgroups,
+# c4 the start and end of each, c5 and c6 the fold of a split inside the launch.  Fitted (non-negative
+# least squares on relative error, candidates near the best of their shape weighted up) to 21 600
+# candidates over 782 layer shapes of the image networks at image sizes of 64 to 448 and twelve
+# device-filling layers, timed as launches of one long model.  Choosing by it costs 5 % on average
+# against the measured best of every shape (the linear model of the direct family alone with the
+# staged tiles' estimate scaled by 3, which was fitted at 224: 18 %, and up to 3x on layers of more
+# than 500 pixels, which it left to the staged tiles).
+# Kinds: "1" 1x1 stride 1 and "s" 1x1 strided on the direct tiles; on the staged ones "p" the
+# pointwise loader, "q" a 1x1 filter it cannot take, "s" strided; "9" 3x3; "n" any other filter.
+CONV_COST = {
+    ("16x16k4", "1"): (3.864, 0, 2.361, 0, 0.176, 0, 0.87),
+    ("16x16k4", "s"): (3.929, 0, 2.743, 0.246, 0.445, 0, 0),
+    ("16x16k4", "9"): (3.08, 1.304, 1.368, 0, 0.564, 0.17, 2.749),
+    ("16x16k4", "n"): (3.329, 0.182, 1.761, 0.453, 0.274, 0, 2.575),
+    ("16x32k4", "1"): (3.902, 0, 3.553, 0.038, 0.222, 0, 1.036),
+    ("16x32k4", "s"): (3.863, 0, 4.739, 0, 0.57, 0, 0),
+    ("16x32k4", "9"): (3.636, 2.107, 2.124, 0, 0.83, 0.389, 2.679),
+    ("16x32k4", "n"): (2.934, 0.083, 3.144, 1.977, 0.306, 0.583, 2.758),
+    ("16x64k4", "1"): (3.953, 0.388, 3.741, 2.128, 0.669, 0, 2.147),
+    ("16x64k4", "s"): (4.082, 0, 8.982, 0, 1.094, 0, 0),
+    ("16x64k4", "9"): (4.756, 3.955, 4.628, 0.196, 1.746, 0.241, 2.752),
+    ("32x32d4", "1"): (3.907, 1.517, 4.385, 0.45, 0.818, 0, 3.727),
+    ("32x32d4", "s"): (4.102, 0, 8.38, 0, 0.884, 0.202, 0.67),
+    ("32x32d4", "9"): (4.484, 2.719, 3.542, 0.286, 1.081, 0.01, 4.04),
+    ("g1", "9"): (3.549, 0.474, 1.311, 0, 0.248, 0.102, 2.009),
+    ("g2", "9"): (3.727, 1.089, 1.993, 0, 0.351, 0.025, 2.573),
+    ("g4", "9"): (4.29, 1.461, 2.599, 1.143, 0.715, 0.103, 3.085),
+    ("64x64", "s"): (9.068, 14.79, 19.38, 5.296, 1.646, 6.436, 0),
+    ("64x64", "9"): (9.626, 17.47, 18.78, 4.938, 0.945, 6.364, 0),
+    ("64x64", "n"): (6.715, 32.23, 13.12, 0, 0.74, 6.959, 0),
+    ("64x64", "p"): (6.828, 8.68, 7.25, 6.944, 1.996, 7.122, 0),
+    ("64x64", "q"): (7.02, 30.34, 15.1, 0, 2.243, 6.398, 0),
+    ("128x32", "s"): (8.123, 18.61, 10.09, 2.462, 2.242, 7.287, 0),
+    ("128x32", "9"): (8.851, 11.91, 12.4, 8.535, 1.186, 5.927, 0),
+    ("128x32", "n"): (7.783, 29.36, 1.753, 0, 0, 6.173, 0),
+    ("128x32", "p"): (6.496, 10.34, 6.87, 6.631, 2.695, 6.766, 0),
+    ("128x32", "q"): (6.557, 3.254, 2.007, 27.51, 3.213, 6.061, 0),
+    ("64x32k2", "s"): (6.11, 5.167, 6.082, 8.086, 1.944, 3.971, 0),
+    ("64x32k2", "9"): (6.353, 6.917, 6.546, 7.894, 1.763, 3.457, 0),
+    ("64x32k2", "n"): (5.643, 19.9, 0, 0, 1.828, 4.177, 0),
+    ("64x32k2", "p"): (4.947, 4.238, 5.818, 3.177, 1.217, 4.379, 0),
+    ("64x32k2", "q"): (5.417, 0, 2.793, 18.77, 1.872, 3.878, 0),
+    ("32x64k2", "s"): (7.462, 8.888, 17.1, 2.856, 0.841, 3.958, 0),
+    ("32x64k2", "9"): (8.526, 12.45, 15.32, 2.858, 0.694, 3.183, 0),
+    ("32x64k2", "n"): (5.941, 28.4, 0, 0, 1.546, 4.225, 0),
+    ("32x64k2", "p"): (5.524, 1.379, 3.516, 6.325, 1.184, 4.288, 0),
+    ("32x64k2", "q"): (6.407, 11.94, 2.272, 13.94, 2.239, 3.673, 0),
+    ("32x32k4", "s"): (6.845, 0, 6.321, 5.181, 1.577, 1.65, 0),
+    ("32x32k4", "9"): (6.803, 4.635, 1.99, 8.083, 1.942, 1.107, 0),
+    ("32x32k4", "n"): (5.74, 0, 5.897, 11.65, 0.09, 1.704, 1.883),
+    ("32x32k4", "p"): (4.406, 1, 2.163, 3.927, 1.29, 2.115, 0),
+    ("32x32k4", "q"): (6.071, 2.839, 0, 10.58, 2.008, 1.917, 0),
+}
+PRE_ACT_LAUNCH_US = 6.0   # a pre-activation launch of its own, in front of a tile without the form
 
 
-def direct_cost(tile, geom, fused):
-    _, bm, bn, _, _ = TILES[tile]
-    c = DIRECT_COST
+def conv_kind(tile, taps, stride=1, pointwise=True):
+    if taps != 1:
+        return "9" if taps == 9 else "n"
+    if stride > 1:
+        return "s"
+    return "1" if tile in DIRECT_TILES else "p" if pointwise else "q"
+
+
+def direct_cost(tile, geom, fused=True, kind="1"):
+    """Microseconds of a launch of this geometry (forced, forced_rows) by CONV_COST."""
+    c = CONV_COST[(tile, kind)]
     s = geom["split_k"]
-    lines = (bm + bn) * geom["k_chunk"] / 32.0
-    t = c["fixed"] + c["per_line_round"] * lines * math.ceil(geom["tasks"] / NUM_CUS) \
-        + c["per_wg_per_cu"] * geom["tasks"] / NUM_CUS
+    w, r = geom["k_chunk"] / 1000.0, geom["tasks"] / NUM_CUS
+    t = c[0] + (c[1] + c[2] * (r + math.ceil(r)) / 2 + c[3] * max(1.0, r)) * w + c[4] * r
     if s > 1:
-        t += (c["fused_split"] if fused else c["separate_split"]) + c["per_split"] * s
+        t += c[5] + 0.1 * c[6] * s + (0.0 if fused else T_REDUCE_LAUNCH)
     return t
 
 
-def _choose_direct(M, N, K, taps, fused, rows, image):
-    """Best direct (or row-form) tile and split by direct_cost; (cost, geometry)."""
+def _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act):
+    """Cheapest tile and split of a convolution by CONV_COST; a split is folded inside the launch."""
     best = None
-    for tile in DIRECT_TILES:
-        if taps not in DIRECT_TAPS[tile]:
+    pointwise = pointwise and stride == 1 and N % 4 == 0 and K % 4 == 0
+    for tile in TILES:
+        if tile in ROW_TILES and not rows:
             continue
-        for s in (1, 2, 3, 4, 6, 8, 12, 16):
-            g = forced(tile, M, N, K, s, taps)
+        if tile in DIRECT_TILES and not (direct and taps in DIRECT_TAPS[tile]):
+            continue
+        kind = conv_kind(tile, taps, stride, pointwise)
+        if (tile, kind) not in CONV_COST:
+            continue
+        for s in (1, 2, 3, 4, 6, 8):
+            g = forced_rows(tile, M, image[0], image[1], K, s) if tile in ROW_TILES else forced(tile, M, N, K, s, taps)
             if g["split_k"] != s:
                 continue
-            t = direct_cost(tile, g, fused)
+            t = direct_cost(tile, dict(g, k_chunk=min(g["k_chunk"], K)), True, kind)
+            if pre_act and tile not in PRE_ACT_TILES:
+                t += PRE_ACT_LAUNCH_US
+            if image is None:
+                t *= 1.0 + 0.04 * max(0.0, 1.0 - g["tasks"] / NUM_CUS)   # of two alike, the one that leaves fewer CUs idle
             if best is None or t < best[0] - 1e-9:
                 g["est_us"] = t
-                g["fused"] = fused and s > 1
+                g["fused"] = s > 1
                 best = (t, g)
-    if rows and image is not None and best is not None:
-        # the row form of the same nominal tile loads each input value once instead of once per
-        # tap: measured 5 to 10 % ahead of the tap form on the 3x3 layers of the table
-        for tile in ("g2", "g4"):
-            for s in (1, 2, 3, 4, 6, 8):
-                g = forced_rows(tile, M, image[0], image[1], K, s)
-                if g["split_k"] != s:
-                    continue
-                t = 0.93 * direct_cost(tile, g, fused)
-                if t < best[0] - 1e-9:
-                    g["est_us"] = t
-                    g["fused"] = fused and s > 1
-                    best = (t, g)
-    return best
+    return best[1]
 
 
 def lds_bytes(tile):

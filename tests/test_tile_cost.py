@@ -1,0 +1,59 @@
+"""Tile choice by the measured cost of every tile (tiling.CONV_COST), for layers the measured table
+does not hold: the choice is a kernel that exists for the filter, and on the GPU it computes the
+convolution (split folded inside the launch, ragged last tiles, row form, strides)."""
+import json
+import os
+
+import numpy as np
+import pytest
+
+from reef_amd.modelgen import tiling
+from reef_amd.modelgen.builder import GraphBuilder, ACT_RELU
+from tests.helpers import max_rel_err, REL_TOL
+
+# cin, H, W, cout, k, stride, pad: one workgroup's worth, a split, just past a round of workgroups,
+# many rounds; a filter no direct tile has; channels and pixels that fill no tile
+LAYERS = [(8, 5, 5, 12, 1, 1, 0), (520, 9, 9, 130, 1, 1, 0), (36, 31, 33, 70, 1, 1, 0), (64, 57, 57, 250, 1, 2, 0),
+          (128, 13, 13, 200, 3, 1, 1), (96, 45, 43, 100, 3, 1, 1), (72, 63, 61, 130, 3, 1, 1), (256, 15, 15, 96, 3, 2, 1),
+          (40, 23, 23, 48, 5, 1, 2), (12, 21, 21, 20, (1, 7), 1, (0, 3)), (16, 20, 20, 24, 4, 2, 1)]
+
+
+def build(layer):
+    cin, H, W, cout, k, s, p = layer
+    g = GraphBuilder("layer", seed=3)
+    x = g.input("data", (cin, H, W))
+    g.mark_output(g.conv2d(x, cout, k, s, p, bias=True, act=ACT_RELU))
+    return g
+
+
+@pytest.mark.parametrize("layer", LAYERS)
+def test_choice_has_a_kernel_and_covers_the_layer(layer):
+    g = build(layer)
+    assert len(g.kernels) == 1                      # a split of K is folded inside the launch
+    a = g.kernels[0]["attrs"]
+    assert a[15] * a[16] >= a[0] * a[6] * a[7]      # split_k * k_chunk covers K
+    assert g.kernels[0]["launch_params"][0] == a[15] * a[17] * a[18]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layer", LAYERS)
+def test_choice_computes_the_layer(layer, tmp_path):
+    from oracle import oracle as O
+    from reef_amd import binding as B
+    g = build(layer)
+    g.write(str(tmp_path))
+    x = np.random.default_rng(5).standard_normal(layer[:3]).astype(np.float32)
+    exe = B.Executor.from_dir(str(tmp_path), g.name, B.BASE)
+    exe.set_input_checked("data", x)
+    for _ in range(2):                              # the counters of a fold are ready for the next run
+        exe.execute()
+        got = exe.get_output()
+        orc = O.GraphOracle(json.load(open(os.path.join(str(tmp_path), g.name + ".json"))), os.path.join(str(tmp_path), g.name + ".param"))
+        orc.set_input("data", x)
+        assert max_rel_err(got, orc.run()) <= REL_TOL
+    exe.close()
+
+
+def test_cost_table_names_tiles_and_kinds():
+    for tile, kind in tiling.CONV_COST:
+        assert tile in tiling.TILES and kind in "1s9npq"
