@@ -202,16 +202,17 @@ typedef struct {
 } reef_conv2d_desc;
 /* Loads the gfx950 kernels (a reef_kernels.raw.co) for the current device. */
 int reef_ops_init(const char* kernels_co_path);
-/* Takes the partial-tile workspace and the counters from hipMalloc for the duration of the call
- * and returns them before it returns (it waits for the stream then). */
+/* Takes the partial-tile workspace and the counters from a pool of the library's for the duration of
+ * the call (it waits for the stream then); the pool keeps at most four workspaces of 4 MiB per GPU,
+ * more calls at once allocate and free their own.  reef_ops_release gives the pool back. */
 int reef_ops_conv2d(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
                     const float* residual, float* out, void* stream);
 /* The same convolution for callers that cannot allocate (code under stream capture, tight
  * serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.
  * The partial tiles and arrival counters of a split K live in a fixed array in device memory
  * that belongs to this library (4 MiB of partial tiles + 16384 counters per GPU, held until the
- * process ends); the call allocates and frees nothing, enqueues a small fill kernel that zeroes
- * the counters it needs and then the convolution, and returns without waiting.  A layer whose
+ * process ends; the counters are zero between calls); the call allocates and frees nothing,
+ * enqueues the convolution and returns without waiting.  A layer whose
  * split needs more than the array holds is refused with Status::Fail and a message saying so
  * (reef_ops_scratch_bytes() = bytes of partial tiles the array holds; the library's own choice
  * of split stays within it for every shape it accepts).  reef_ops_init must have
@@ -221,6 +222,12 @@ int reef_ops_conv2d(const reef_conv2d_desc* c, const float* in, const float* w, 
 int reef_ops_conv2d_noalloc(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
                             const float* residual, float* out, void* stream);
 size_t reef_ops_scratch_bytes(void);
+/* reef_ops_conv2d (noalloc 0) or reef_ops_conv2d_noalloc (1) on the default stream, behind everything the
+ * device was given before; the output is complete when it returns. */
+int reef_ops_conv2d_wait(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
+                         const float* residual, float* out, int noalloc);
+/* Frees the idle workspaces of reef_ops_conv2d. */
+int reef_ops_release(void);
 
 /* GPUConfig (src/reef/executor/hip/hip_impl.cpp:9-74) */
 int reef_gpuconfig_num_cus(void);

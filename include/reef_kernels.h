@@ -241,6 +241,9 @@ enum {
  *                           straight into 16x16x4 MFMAs, the four wavefronts split the input
  *                           channels.  d1 needs Cin % 8 == 0 (any stride); K_CHUNK is a multiple
  *                           of R (R > 1) or 8 (d1) and splits K on channel boundaries.
+ *   reef_conv2d_f<R>_<direct tile>  (raw code object) direct, R = kw taps a filter row (3, 5, 7), any kh;
+ *                           K_CHUNK is a multiple of 16 R.
+ *   reef_conv2d_o1_<direct tile>    (raw code object) direct, 1x1, any Cin; K_CHUNK a multiple of 128.
  *   reef_conv2d_r9_g<G>[m2] row form of the direct 3x3 / stride 1 / padding 1 convolution: every input value
  *                           is loaded once per tile and the horizontal taps come from neighbouring lanes. */
 #define REEF_F_POOL_OUTPUT 256  /* symbol reef_conv2d_sp7_g2: a 7x7 convolution (stride 2, padding 3, Cin <= 3; + bias,

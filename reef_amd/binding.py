@@ -449,10 +449,6 @@ def ops_init(kernels_co=None):
 
 
 def ops_conv2d(desc, inp, w, bias, residual, out, noalloc=False):
-    """reef_ops_conv2d / reef_ops_conv2d_noalloc on DeviceBuffers, default stream; returns the status."""
-    fn = lib().reef_ops_conv2d_noalloc if noalloc else lib().reef_ops_conv2d
-    st = fn(ctypes.byref(desc), inp.ptr, w.ptr, bias.ptr if bias is not None else None,
-            residual.ptr if residual is not None else None, out.ptr, None)
-    if st == 0:
-        _check("device_sync", lib().reef_hal_device_sync())
-    return st
+    """reef_ops_conv2d / reef_ops_conv2d_noalloc on DeviceBuffers, default stream, waited for; returns the status."""
+    return lib().reef_ops_conv2d_wait(ctypes.byref(desc), inp.ptr, w.ptr, bias.ptr if bias is not None else None,
+                                      residual.ptr if residual is not None else None, out.ptr, 1 if noalloc else 0)

@@ -37,11 +37,20 @@ void on_queue_error(hsa_status_t s, hsa_queue_t*, void* data) { ((Queue*)data)->
 constexpr int kMaxQueues = 4;      // as many as the runtime itself opens per process
 constexpr uint32_t kQueuePackets = 1024;
 
+// What one call in flight owns: its completion signal and its argument block (host memory).
+struct Call {
+    hsa_signal_t done{};
+    char* kernarg = nullptr;
+    Queue* queue = nullptr;
+};
+
 struct Device {
     bool tried = false, ok = false;
     hsa_agent_t agent{};
     Queue* queues[kMaxQueues] = {};   // opened as passes need them, kept for the life of the process
     unsigned next = 0;
+    std::vector<Call*> idle;     // calls that have ended, for the next ones: as many as ever ran at once
+    std::mutex idle_mtx;
 };
 constexpr int kMaxDevices = 16;
 Device g_devices[kMaxDevices];
@@ -209,6 +218,152 @@ bool aql_available(int device) {
     return set_up(device);
 }
 
+const AqlKernel* aql_kernel(AqlCode* code, int device, const char* name, std::string* err) {
+    std::lock_guard<std::mutex> lock(g_mtx);
+    if (!set_up(device)) { *err = "no packet queue on this device"; return nullptr; }
+    const hsa_agent_t agent = g_devices[device].agent;
+    std::lock_guard<std::mutex> code_lock(code->mtx);
+    AqlKernel k;
+    if (!code->load(device, agent, err) || !code->find(name, agent, &k, err)) return nullptr;
+    return &code->kernels.find(name)->second;
+}
+
+namespace {
+
+// The arguments, and behind them what the kernel may read of its launch.
+void fill_kernarg(char* at, const AqlKernel& k, const void* args, size_t bytes, const uint32_t grid[3], const uint32_t block[3]) {
+    std::memcpy(at, args, bytes);
+    HiddenArgs h;
+    std::memset(&h, 0, sizeof(h));
+    for (int x = 0; x < 3; ++x) {
+        h.block_count[x] = grid[x];
+        h.group_size[x] = (uint16_t)block[x];
+    }
+    h.grid_dims = 3;
+    const size_t behind = (bytes + 7) / 8 * 8;
+    if (k.kernarg > behind) std::memcpy(at + behind, &h, std::min(sizeof(h), (size_t)k.kernarg - behind));
+}
+
+hsa_kernel_dispatch_packet_t dispatch_packet(const AqlKernel& k, const uint32_t grid[3], const uint32_t block[3], uint32_t dyn_lds,
+                                             void* kernarg, int acquire, int release) {
+    hsa_kernel_dispatch_packet_t a;
+    std::memset(&a, 0, sizeof(a));
+    a.header = (uint16_t)((HSA_PACKET_TYPE_KERNEL_DISPATCH << HSA_PACKET_HEADER_TYPE) | (1 << HSA_PACKET_HEADER_BARRIER) |
+                          (acquire << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE) |
+                          (release << HSA_PACKET_HEADER_SCRELEASE_FENCE_SCOPE));
+    a.setup = (uint16_t)(3 << HSA_KERNEL_DISPATCH_PACKET_SETUP_DIMENSIONS);
+    a.workgroup_size_x = (uint16_t)block[0];
+    a.workgroup_size_y = (uint16_t)block[1];
+    a.workgroup_size_z = (uint16_t)block[2];
+    a.grid_size_x = grid[0] * block[0];
+    a.grid_size_y = grid[1] * block[1];
+    a.grid_size_z = grid[2] * block[2];
+    a.private_segment_size = k.scratch;
+    a.group_segment_size = k.lds + dyn_lds;
+    a.kernel_object = k.object;
+    a.kernarg_address = kernarg;
+    return a;
+}
+
+// Hands one packet to the device; `ring`: with the doorbell.  Caller holds w.mtx.
+bool put_packet(Queue& w, const hsa_kernel_dispatch_packet_t& packet, bool ring, std::string* err) {
+    hsa_queue_t* q = w.q;
+    const uint64_t idx = hsa_queue_add_write_index_relaxed(q, 1);
+    while (idx - hsa_queue_load_read_index_scacquire(q) >= q->size) {
+        hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)(idx - 1));   // the device works the ring down
+        if (w.error.load()) { *err = hsa_text((hsa_status_t)w.error.load(), "queue"); return false; }
+    }
+    char* slot = (char*)q->base_address + (idx & (q->size - 1)) * sizeof(packet);
+    const char* src = (const char*)&packet;
+    // the first four bytes (header and setup) hand the packet to the device: last, in one store
+    std::memcpy(slot + 4, src + 4, sizeof(packet) - 4);
+    uint32_t head;
+    std::memcpy(&head, src, 4);
+    __atomic_store_n((uint32_t*)slot, head, __ATOMIC_RELEASE);
+    // No doorbell covers packets on both sides of the ring's end: a profiler's interception takes such
+    // a run for contiguous.
+    if (ring || ((idx + 1) & (q->size - 1)) == 0) hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)idx);
+    return true;
+}
+
+// The wait looks at the queue's error word once a second, so that a failed queue ends it.
+bool wait_done(Queue& w, hsa_signal_t done, std::string* err) {
+    while (hsa_signal_wait_scacquire(done, HSA_SIGNAL_CONDITION_LT, 1, 1000000000ull, HSA_WAIT_STATE_ACTIVE) >= 1)
+        if (w.error.load()) { *err = hsa_text((hsa_status_t)w.error.load(), "queue"); return false; }
+    return true;
+}
+
+Call* take_call(int device, std::string* err) {
+    Device& d = g_devices[device];
+    {
+        std::lock_guard<std::mutex> lock(d.idle_mtx);
+        if (!d.idle.empty()) {
+            Call* c = d.idle.back();
+            d.idle.pop_back();
+            return c;
+        }
+    }
+    std::unique_ptr<Call> c(new Call);
+    void* p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, kAqlCallArgs, hipHostMallocDefault);
+    if (e != hipSuccess) { *err = std::string("argument block: ") + hipGetErrorString(e); return nullptr; }
+    c->kernarg = (char*)p;
+    const hsa_status_t s = hsa_signal_create(0, 0, nullptr, &c->done);
+    if (s == HSA_STATUS_SUCCESS) {
+        std::lock_guard<std::mutex> lock(g_mtx);
+        c->queue = take_queue(d, err);
+    } else {
+        *err = hsa_text(s, "hsa_signal_create");
+    }
+    if (!c->queue) {
+        if (s == HSA_STATUS_SUCCESS) hsa_signal_destroy(c->done);
+        (void)hipHostFree(p);
+        return nullptr;
+    }
+    return c.release();
+}
+
+}  // namespace
+
+bool aql_call_prepare(int device, std::string* err) {
+    Call* c = take_call(device, err);
+    if (!c) return false;
+    std::lock_guard<std::mutex> lock(g_devices[device].idle_mtx);
+    g_devices[device].idle.push_back(c);
+    return true;
+}
+
+void aql_call_args(const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
+                   char (&image)[kAqlCallArgs]) {
+    const uint32_t grid[3] = {groups, 1, 1}, block[3] = {threads, 1, 1};
+    std::memset(image, 0, sizeof(image));
+    fill_kernarg(image, *kernel, kernarg, kernarg_bytes, grid, block);
+}
+
+bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
+              const void* resident, std::string* err) {
+    if (std::max<size_t>(kernel->kernarg, kernarg_bytes) + sizeof(HiddenArgs) > kAqlCallArgs) { *err = "argument block too large"; return false; }
+    Call* c = take_call(device, err);
+    if (!c) return false;
+    const uint32_t grid[3] = {groups, 1, 1}, block[3] = {threads, 1, 1};
+    if (!resident) fill_kernarg(c->kernarg, *kernel, kernarg, kernarg_bytes, grid, block);
+    hsa_kernel_dispatch_packet_t packet =
+        dispatch_packet(*kernel, grid, block, 0, resident ? const_cast<void*>(resident) : c->kernarg, HSA_FENCE_SCOPE_SYSTEM, HSA_FENCE_SCOPE_SYSTEM);
+    packet.completion_signal = c->done;
+    hsa_signal_store_relaxed(c->done, 1);
+    bool ok;
+    {
+        std::lock_guard<std::mutex> submit(c->queue->mtx);
+        ok = put_packet(*c->queue, packet, true, err);
+    }
+    ok = ok && wait_done(*c->queue, c->done, err);
+    if (!ok) return false;      // the device may still use what the call owns: it is not handed on
+    Device& d = g_devices[device];
+    std::lock_guard<std::mutex> lock(d.idle_mtx);
+    d.idle.push_back(c);
+    return true;
+}
+
 struct AqlPass {
     Queue* queue = nullptr;
     hsa_signal_t done{};
@@ -248,43 +403,17 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
     host.assign(bytes + 64, 0);
     for (size_t i = 0; i < n; ++i) {
         const AqlLaunch& l = launches[i];
-        std::memcpy(host.data() + at[i], l.kernarg, l.kernarg_bytes);
-        HiddenArgs h;
-        std::memset(&h, 0, sizeof(h));
-        for (int x = 0; x < 3; ++x) {
-            h.block_count[x] = l.grid[x];
-            h.group_size[x] = (uint16_t)l.block[x];
-        }
-        h.grid_dims = 3;
-        const size_t behind = (l.kernarg_bytes + 7) / 8 * 8;
-        if (kernels[i].kernarg > behind) std::memcpy(host.data() + at[i] + behind, &h, std::min(sizeof(h), kernels[i].kernarg - behind));
+        fill_kernarg(host.data() + at[i], kernels[i], l.kernarg, l.kernarg_bytes, l.grid, l.block);
     }
     const hipError_t e = hipMalloc(&p->kernargs, host.size());
     if (e != hipSuccess) { *err = std::string("argument blocks: ") + hipGetErrorString(e); return nullptr; }
     for (size_t i = 0; i < n; ++i) {
         const AqlLaunch& l = launches[i];
-        const AqlKernel& k = kernels[i];
-        hsa_kernel_dispatch_packet_t a;
-        std::memset(&a, 0, sizeof(a));
         // Launches follow one another (barrier) and see each other's results; the first also sees what
         // the host and the copy engines wrote, the last makes its results visible to them.
         const int acquire = i == 0 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
         const int release = i == n - 1 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
-        a.header = (uint16_t)((HSA_PACKET_TYPE_KERNEL_DISPATCH << HSA_PACKET_HEADER_TYPE) | (1 << HSA_PACKET_HEADER_BARRIER) |
-                              (acquire << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE) |
-                              (release << HSA_PACKET_HEADER_SCRELEASE_FENCE_SCOPE));
-        a.setup = (uint16_t)(3 << HSA_KERNEL_DISPATCH_PACKET_SETUP_DIMENSIONS);
-        a.workgroup_size_x = (uint16_t)l.block[0];
-        a.workgroup_size_y = (uint16_t)l.block[1];
-        a.workgroup_size_z = (uint16_t)l.block[2];
-        a.grid_size_x = l.grid[0] * l.block[0];
-        a.grid_size_y = l.grid[1] * l.block[1];
-        a.grid_size_z = l.grid[2] * l.block[2];
-        a.private_segment_size = k.scratch;
-        a.group_segment_size = k.lds + l.dyn_lds;
-        a.kernel_object = k.object;
-        a.kernarg_address = (char*)p->kernargs + at[i];
-        p->packets.push_back(a);
+        p->packets.push_back(dispatch_packet(kernels[i], l.grid, l.block, l.dyn_lds, (char*)p->kernargs + at[i], acquire, release));
     }
     const hsa_status_t s = hsa_signal_create(0, 0, nullptr, &p->done);
     if (s != HSA_STATUS_SUCCESS) { *err = hsa_text(s, "hsa_signal_create"); return nullptr; }
@@ -317,30 +446,12 @@ bool aql_pass_run(AqlPass* p, std::string* err) {
     hsa_signal_store_relaxed(p->done, 1);
     {
         std::lock_guard<std::mutex> submit(w.mtx);
-        hsa_queue_t* q = w.q;
         const size_t n = p->packets.size();
-        for (size_t i = 0; i < n; ++i) {
-            const uint64_t idx = hsa_queue_add_write_index_relaxed(q, 1);
-            while (idx - hsa_queue_load_read_index_scacquire(q) >= q->size) {
-                hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)(idx - 1));   // the device works the ring down
-                if (w.error.load()) { *err = hsa_text((hsa_status_t)w.error.load(), "queue"); return false; }
-            }
-            char* slot = (char*)q->base_address + (idx & (q->size - 1)) * sizeof(hsa_kernel_dispatch_packet_t);
-            const char* src = (const char*)&p->packets[i];
-            // the first four bytes (header and setup) hand the packet to the device: last, in one store
-            std::memcpy(slot + 4, src + 4, sizeof(hsa_kernel_dispatch_packet_t) - 4);
-            uint32_t head;
-            std::memcpy(&head, src, 4);
-            __atomic_store_n((uint32_t*)slot, head, __ATOMIC_RELEASE);
-            // The device starts on the first packets while the rest are written.  No doorbell covers packets
-            // on both sides of the ring's end: a profiler's interception takes such a run for contiguous.
-            if (i == n - 1 || (i & 31) == 3 || ((idx + 1) & (q->size - 1)) == 0) hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)idx);
-        }
+        // the device starts on the first packets while the rest are written
+        for (size_t i = 0; i < n; ++i)
+            if (!put_packet(w, p->packets[i], i == n - 1 || (i & 31) == 3, err)) return false;
     }
-    // the wait looks at the queue's error word once a second, so that a failed queue ends it
-    while (hsa_signal_wait_scacquire(p->done, HSA_SIGNAL_CONDITION_LT, 1, 1000000000ull, HSA_WAIT_STATE_ACTIVE) >= 1)
-        if (w.error.load()) { *err = hsa_text((hsa_status_t)w.error.load(), "queue"); return false; }
-    return true;
+    return wait_done(w, p->done, err);
 }
 
 void aql_pass_destroy(AqlPass* p) { delete p; }

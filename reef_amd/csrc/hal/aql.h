@@ -16,9 +16,25 @@ namespace hal {
 
 struct AqlCode;   // one code object, loaded on the device on first use
 struct AqlPass;
+struct AqlKernel; // one of its kernels
 
 // The code object of `path` (read now; modules with the same contents share one copy).  nullptr: unreadable.
 std::shared_ptr<AqlCode> aql_code_from_file(const char* path);
+
+// A kernel of `code` (loaded on `device` if it is not yet), valid as long as the code is.  nullptr and *err: not found.
+const AqlKernel* aql_kernel(AqlCode* code, int device, const char* name, std::string* err);
+// One launch of `groups` workgroups of `threads`, waited for: it sees what host, copy engines and finished
+// kernels have written, and its results are visible everywhere when this returns.  Calls of several
+// threads run beside each other.  `resident`: device memory that holds aql_call_args' image of the same
+// arguments, or null (they are read from host memory then, 1.2 us later).
+constexpr size_t kAqlCallArgs = 512;
+bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
+              const void* resident, std::string* err);
+// The argument block of such a launch.
+void aql_call_args(const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
+                   char (&image)[kAqlCallArgs]);
+// Makes what one call in flight needs, so that a first call allocates nothing (one beside another does).
+bool aql_call_prepare(int device, std::string* err);
 
 struct AqlLaunch {
     AqlCode* code;

@@ -57,14 +57,14 @@ struct OpConv {
         return conv2d_body<T, MODE>(d, task, smem, p);
     }
 };
-template <int R, int TN = 1, int TM = 1, bool PRE = false, bool ROWS = false, bool PACKED = false>
+template <int R, int TN = 1, int TM = 1, bool PRE = false, bool ROWS = false, bool PACKED = false, bool FROWS = false, bool ODDC = false>
 struct OpConvDirect {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;   // the body makes the wrapper's first flag check
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
-        return conv2d_direct_body<R, TN, TM, PRE, ROWS, PACKED>(d, task, smem, p);
+        return conv2d_direct_body<R, TN, TM, PRE, ROWS, PACKED, FROWS, ODDC>(d, task, smem, p);
     }
 };
 // the same with the weights read from their packed copy
@@ -75,6 +75,11 @@ using OpConvRowsK = OpConvDirect<9, G, TM, false, true, true>;
 // row form of the 3x3 convolution: G image rows x one 14-column segment per workgroup
 template <int G, int TM = 1>
 using OpConvRows = OpConvDirect<9, G, TM, false, true>;
+// filters of any height whose rows have R taps; 1x1 filters on any number of channels
+template <int R, int TN = 1, int TM = 1>
+using OpConvFilterRows = OpConvDirect<R, TN, TM, false, false, false, true>;
+template <int TN = 1, int TM = 1>
+using OpConvOdd = OpConvDirect<1, TN, TM, false, false, false, false, true>;
 // 1x1 convolution and the depthwise 3x3 convolution (stride S) behind it in one launch
 template <int G, int S = 1>
 struct OpConvXdw {
@@ -408,6 +413,24 @@ REEF_ENTRY(reef_conv2d_d25k_16x16k4, OpConvDirectK<25>)
 REEF_ENTRY(reef_conv2d_d25k_16x32k4, OpConvDirectK<25 REEF_COMMA 2>)
 REEF_ENTRY(reef_conv2d_d7k_16x16k4, OpConvDirectK<7>)
 REEF_ENTRY(reef_conv2d_d7k_16x32k4, OpConvDirectK<7 REEF_COMMA 2>)
+#if REEF_FLAVOUR == 0   // the single-convolution entry points' own: no model launches them
+REEF_ENTRY(reef_conv2d_f3_16x16k4, OpConvFilterRows<3>)
+REEF_ENTRY(reef_conv2d_f3_16x32k4, OpConvFilterRows<3 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_f3_16x64k4, OpConvFilterRows<3 REEF_COMMA 4>)
+REEF_ENTRY(reef_conv2d_f3_32x32d4, OpConvFilterRows<3 REEF_COMMA 2 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_f5_16x16k4, OpConvFilterRows<5>)
+REEF_ENTRY(reef_conv2d_f5_16x32k4, OpConvFilterRows<5 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_f5_16x64k4, OpConvFilterRows<5 REEF_COMMA 4>)
+REEF_ENTRY(reef_conv2d_f5_32x32d4, OpConvFilterRows<5 REEF_COMMA 2 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_f7_16x16k4, OpConvFilterRows<7>)
+REEF_ENTRY(reef_conv2d_f7_16x32k4, OpConvFilterRows<7 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_f7_16x64k4, OpConvFilterRows<7 REEF_COMMA 4>)
+REEF_ENTRY(reef_conv2d_f7_32x32d4, OpConvFilterRows<7 REEF_COMMA 2 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_o1_16x16k4, OpConvOdd<>)
+REEF_ENTRY(reef_conv2d_o1_16x32k4, OpConvOdd<2>)
+REEF_ENTRY(reef_conv2d_o1_16x64k4, OpConvOdd<4>)
+REEF_ENTRY(reef_conv2d_o1_32x32d4, OpConvOdd<2 REEF_COMMA 2>)
+#endif
 REEF_ENTRY(reef_conv2d_xdw_g2, OpConvXdw<2>)
 REEF_ENTRY(reef_conv2d_xdw_g4, OpConvXdw<4>)
 REEF_ENTRY(reef_conv2d_sp7_g2, OpConvStemPool)

@@ -847,12 +847,23 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane i <- lane (
 // (zero-padded to whole groups): the 64 lanes of a wavefront read 1 KiB contiguous, aligned, per
 // group of four taps.  Measured on the 3x3 layers of ResNet-152: 1.4 us less per launch.  The
 // model generator writes the copy as a parameter of its own; attr WPACK names its pointer slot.
-template <int R, int TN, int TM, bool PRE, bool ROWS, bool PACKED, class Poll>
+//
+// FROWS (symbols reef_conv2d_f<R>_*): R is the width of the filter and a k slot's channel is one row of one
+// channel's filter, number c * kh + ky.  The weights of a row of W are contiguous in that order too, so the
+// A side does not change; the B side finds the image row of its slot by counting (c, ky) up from step
+// to step.  Any filter height, and no idle slots for the channels that a short input lacks: 7x7 on 12
+// channels is 84 slots of 7 taps.
+//
+// ODDC (1-tap kernels; symbols reef_conv2d_o1_*): Cin is no multiple of 4.  The last 128-bit load of a row
+// of weights reaches into the next row; those values are dropped in front of the MFMAs.
+template <int R, int TN, int TM, bool PRE, bool ROWS, bool PACKED, bool FROWS, bool ODDC, class Poll>
 __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int task, char* smem_raw,
                                                    const Poll& poll) {
     static_assert(!PRE || R == 1, "the pre-activation form exists for 1-tap filters only");
     static_assert(!ROWS || R == 9, "the row form exists for 3x3 filters only");
     static_assert(!PACKED || R > 1, "1-tap filters are read from OIHW as they are");
+    static_assert(!FROWS || !(PRE || ROWS || PACKED), "filter rows are read from OIHW, tap by tap");
+    static_assert(!ODDC || R == 1, "only the 1-tap kernels load several channels at once");
     typedef DirectGeom<R, TN, TM, PRE, ROWS> G;
     typedef TileD16<TN, TM> TD;
     constexpr int RC = G::RC, NS = G::NS;
@@ -862,7 +873,8 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
     const int* a = d.attr;
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int M = a[REEF_CONV_COUT], C = a[REEF_CONV_CIN];
+    const int kh = FROWS ? a[REEF_CONV_KH] : 1;
+    const int M = a[REEF_CONV_COUT], C = FROWS ? a[REEF_CONV_CIN] * kh : a[REEF_CONV_CIN];
     const int H = a[REEF_CONV_H], W = a[REEF_CONV_W], Wo = a[REEF_CONV_WO];
     const int N = a[REEF_CONV_HO] * Wo;
     const int K = C * R;
@@ -918,7 +930,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
                                     ((flags & REEF_F_AFFINE) ? 2 : 0) + ((flags & REEF_F_DUAL) ? 2 : 0);
     // per-lane operand offsets
     const rsrc_t rs_a = make_rsrc(d.ptr[1], (unsigned)M * (unsigned)K * 4u);
-    const rsrc_t rs_b = make_rsrc(d.ptr[0], (unsigned)C * HW4);
+    const rsrc_t rs_b = make_rsrc(d.ptr[0], (unsigned)(FROWS ? a[REEF_CONV_CIN] : C) * HW4);
     const int lane_c = cb + (wave * 4 + kq) * G::CPL;     // first channel of this lane's k slot
     constexpr int G4 = (R + 3) / 4;                 // groups of four taps in the packed copy
     const unsigned C4 = (unsigned)(C + 3) / 4u;
@@ -986,7 +998,30 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
         asm volatile("" ::: "memory");
     }
     unsigned vb[ROWS ? TN + 2 : TN][ROWS ? 1 : R];
-    if (ROWS) {
+    // FROWS: filter row ky of this lane's slot in the next step, byte offset of (its channel, filter row), and
+    // how both go on; per pixel group the image row of ky = 0 (vb: column taps alone)
+    int f_ky = 0, f_iy[FROWS ? TN : 1];
+    unsigned f_off = 0, f_step = 0;
+    const int f_dky = FROWS ? 16 - div_small(16, kh) * kh : 0;
+    if (FROWS) {
+        const int c = div_small(lane_c, kh);
+        f_ky = lane_c - c * kh;
+        f_off = (unsigned)c * HW4 + (unsigned)(f_ky * W) * 4u;
+        f_step = (unsigned)div_small(16, kh) * HW4 + (unsigned)(f_dky * W) * 4u;
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+            const int n = n0 + 16 * g + i16;
+            const int oy = div_small(n, Wo), ox = n - oy * Wo;
+            const int iy = oy * a[REEF_CONV_SH] - a[REEF_CONV_PH];
+            f_iy[FROWS ? g : 0] = iy;
+#pragma unroll
+            for (int t = 0; t < R; ++t) {
+                const int ix = ox * a[REEF_CONV_SW] + t - a[REEF_CONV_PW];
+                const bool ok = n < N && (unsigned)ix < (unsigned)W;
+                vb[ROWS ? 0 : g][ROWS ? 0 : t] = ok ? (unsigned)(iy * W + ix) * 4u : kOutside;   // (a negative row: with ky it is none)
+            }
+        }
+    } else if (ROWS) {
         // one value per input row: column of this lane (lane 15: left of the segment)
         const int ix = i16 == 15 ? x0 - 1 : x0 + i16;
 #pragma unroll
@@ -1037,7 +1072,23 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
                 }
             }
         }
-        if (ROWS) {
+        if (FROWS) {
+#pragma unroll
+            for (int g = 0; g < TN; ++g) {
+                const bool in = step < lane_steps && (unsigned)(f_iy[FROWS ? g : 0] + f_ky) < (unsigned)H;
+#pragma unroll
+                for (int q = 0; q < RC; ++q) {
+                    const unsigned x = vb[ROWS ? 0 : g][ROWS ? 0 : q];
+                    rb[s][ROWS ? 0 : g * RC + q] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(rs_b, (int)(in && x != kOutside ? x + f_off : kOutside), 0, 0));
+                }
+            }
+            f_ky += f_dky;
+            f_off += f_step;
+            const bool wrap = f_ky >= kh;
+            f_ky -= wrap ? kh : 0;
+            f_off += wrap ? HW4 - (unsigned)(kh * W) * 4u : 0u;
+        } else if (ROWS) {
 #pragma unroll
             for (int r = 0; r < NB; ++r)
                 rb[s][r] = __builtin_bit_cast(
@@ -1109,7 +1160,15 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
             acc[h][g][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             acc[h][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
+    int odd_left = C - lane_c;      // ODDC: channels of this lane's row from its slot of the next step on
     auto mma_stage = [&](int s) {
+        if (ODDC) {
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int q = 1; q < RC; ++q) ra[s][h][q] = q < odd_left ? ra[s][h][q] : 0.0f;
+            odd_left -= G::STEP_C;
+        }
         if (ROWS) {
             // taps of input row r: the loaded value and its two neighbours within the 16-lane row
             float bt[NB][3];
