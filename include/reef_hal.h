@@ -223,8 +223,14 @@ int reef_hal_graph_destroy(reef_graph_t g);
  *   pass_block:  device address and size of the block of launch `i`, the host copy that pass_commit
  *                uploads (the caller may still write into it), and where in it the tail starts.
  *   pass_commit: uploads the blocks; needed before the first run.
+ *   pass_mirror: (before pass_commit) adds a last launch that copies ranges of device memory to host
+ *                memory of the pass's; host[i] is where range i is found after a run.
  *   pass_run:    waits for what `after` (may be NULL: the default stream) has been given, runs the
- *                launches in order and returns when the last has finished. */
+ *                launches in order and returns when the last has finished.  `fresh`: the caches may hold
+ *                what the host or launches outside passes have changed since the last run.
+ *   host_write:  stores into device memory from the host (device memory behind the PCIe window); returns 2
+ *                where the backend cannot.  Nothing that reads the memory may be running; a pass run
+ *                with `fresh` sees the bytes, and so does any launch after host_write_fence. */
 typedef struct reef_pass_s* reef_pass_t;
 typedef struct reef_pass_launch {
     reef_function_t fn;
@@ -241,7 +247,12 @@ typedef struct reef_pass_block {
 int reef_hal_pass_create(const reef_pass_launch* launches, size_t n, size_t tail_bytes, reef_pass_t* out);
 int reef_hal_pass_block(reef_pass_t p, size_t i, reef_pass_block* out);
 int reef_hal_pass_commit(reef_pass_t p);
-int reef_hal_pass_run(reef_pass_t p, reef_stream_t after);
+typedef struct reef_pass_range { const void* src; size_t bytes; } reef_pass_range;
+#define REEF_PASS_MAX_RANGES 8
+int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* ranges, size_t n, const char** host);
+int reef_hal_pass_run(reef_pass_t p, reef_stream_t after, int fresh);
+int reef_hal_host_write(reef_devptr_t dst, const void* src, size_t bytes);
+int reef_hal_host_write_fence(void);
 int reef_hal_pass_destroy(reef_pass_t p);
 
 /*
@@ -297,8 +308,11 @@ typedef struct reef_hal_backend {
     int (*pass_create)(const reef_pass_launch*, size_t, size_t, reef_pass_t*);
     int (*pass_block)(reef_pass_t, size_t, reef_pass_block*);
     int (*pass_commit)(reef_pass_t);
-    int (*pass_run)(reef_pass_t, reef_stream_t);
+    int (*pass_run)(reef_pass_t, reef_stream_t, int);
     int (*pass_destroy)(reef_pass_t);
+    int (*pass_mirror)(reef_pass_t, const reef_pass_range*, size_t, const char**);
+    int (*host_write)(reef_devptr_t, const void*, size_t);
+    int (*host_write_fence)(void);
 } reef_hal_backend;
 
 const reef_hal_backend* reef_hal_hip_backend(void);

@@ -83,13 +83,20 @@ protected:
     struct Pass {
         reef_pass_t handle = nullptr;
         bool tried = false;
+        // what a run leaves in host memory besides device memory: the output, and storages that the
+        // caller has fetched after run upon run
+        struct Mirrored { size_t idx, bytes; const char* host; };
+        std::vector<Mirrored> mirrored;
+        size_t watched = 0;    // how many of `watch` it holds
     };
     // Runs the pass behind what `stream` has been given and waits for it.  *ran = false, and nothing done,
     // where the backend cannot record one.
     template <class Make>
     Status run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran);
     Status record_pass(Pass& p, std::vector<Launch>& launches);
-    static void drop_pass(Pass& p);
+    void drop_pass(Pass& p);
+    // Called in front of every launch of a kernel of this model that is no part of a pass.
+    Status leave_passes();
     Status find_storage_idx(const std::string& name, size_t& idx);
     size_t storage_bytes(size_t idx) const;
 
@@ -107,12 +114,21 @@ protected:
     bool use_graph;
     reef_graph_t model_graph;
     Pass model_pass;
+    // State of the storages as passes know them.  after_pass: the last thing that ran on them was a pass (which has
+    // finished); host_wrote: since then the host has stored into them past the caches; current: the pass whose
+    // mirrored storages are those of the device.
+    bool after_pass = false, host_wrote = false;
+    Pass* current = nullptr;
+    std::vector<size_t> watch;         // storages fetched again and again
+    size_t asked_idx = 0, asked_run = 0, runs = 0;
+    void note_fetch(size_t idx);
     void drop_graph();
 };
 
 template <class Make>
 Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran) {
     *ran = false;
+    if (p.handle && p.watched != watch.size()) drop_pass(p);
     if (!p.tried) {
         std::vector<Launch> l(num_kernels());
         for (size_t i = 0; i < l.size(); i++) RETURN_STATUS(make((int)i, l[i]));
@@ -121,7 +137,14 @@ Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, boo
     }
     if (!p.handle) return Status::Succ;
     *ran = true;
-    GPU_RETURN_STATUS(reef_hal_pass_run(p.handle, stream));
+    current = nullptr;
+    const int fresh = host_wrote || !after_pass;
+    after_pass = false;
+    GPU_RETURN_STATUS(reef_hal_pass_run(p.handle, stream, fresh));
+    after_pass = true;
+    host_wrote = false;
+    current = &p;
+    runs++;
     return Status::Succ;
 }
 

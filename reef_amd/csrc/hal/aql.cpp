@@ -4,6 +4,8 @@
 #include <hsa/hsa.h>
 #include <hsa/hsa_ext_amd.h>
 
+#include <emmintrin.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
@@ -12,6 +14,7 @@
 #include <mutex>
 #include <vector>
 
+#include "hal/blit.h"
 #include "hal/code_object.h"
 
 namespace reef {
@@ -47,6 +50,7 @@ struct Call {
 struct Device {
     bool tried = false, ok = false;
     hsa_agent_t agent{};
+    volatile uint32_t* flush = nullptr;   // a store here pushes out what the host has stored into device memory
     Queue* queues[kMaxQueues] = {};   // opened as passes need them, kept for the life of the process
     unsigned next = 0;
     std::vector<Call*> idle;     // calls that have ended, for the next ones: as many as ever ran at once
@@ -92,6 +96,8 @@ bool set_up(int device) {
     hsa_iterate_agents(match_agent, &f);
     if (!f.found) return false;
     d.agent = f.agent;
+    hsa_amd_hdp_flush_t hdp{};
+    if (hsa_agent_get_info(d.agent, (hsa_agent_info_t)HSA_AMD_AGENT_INFO_HDP_FLUSH, &hdp) == HSA_STATUS_SUCCESS) d.flush = hdp.HDP_MEM_FLUSH_CNTL;
     d.ok = true;
     return true;
 }
@@ -212,6 +218,22 @@ std::shared_ptr<AqlCode> aql_code_from_file(const char* path) {
     live.push_back(c);
     return c;
 }
+
+namespace {
+
+// The library's own kernels (hal/blit.hip), linked in as they were built.
+extern "C" const char reef_blit_code[], reef_blit_code_end[];
+
+std::shared_ptr<AqlCode> blit_code() {
+    static std::shared_ptr<AqlCode> code = [] {
+        auto c = std::make_shared<AqlCode>();
+        c->elf.assign((const uint8_t*)reef_blit_code, (const uint8_t*)reef_blit_code_end);
+        return c;
+    }();
+    return code;
+}
+
+}  // namespace
 
 bool aql_available(int device) {
     std::lock_guard<std::mutex> lock(g_mtx);
@@ -348,7 +370,7 @@ bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t thr
     const uint32_t grid[3] = {groups, 1, 1}, block[3] = {threads, 1, 1};
     if (!resident) fill_kernarg(c->kernarg, *kernel, kernarg, kernarg_bytes, grid, block);
     hsa_kernel_dispatch_packet_t packet =
-        dispatch_packet(*kernel, grid, block, 0, resident ? const_cast<void*>(resident) : c->kernarg, HSA_FENCE_SCOPE_SYSTEM, HSA_FENCE_SCOPE_SYSTEM);
+        dispatch_packet(*kernel, grid, block, 0, resident ? const_cast<void*>(resident) : c->kernarg, HSA_FENCE_SCOPE_AGENT, HSA_FENCE_SCOPE_SYSTEM);
     packet.completion_signal = c->done;
     hsa_signal_store_relaxed(c->done, 1);
     bool ok;
@@ -368,6 +390,7 @@ struct AqlPass {
     Queue* queue = nullptr;
     hsa_signal_t done{};
     void* kernargs = nullptr;    // device memory, one 64-byte aligned block per launch
+    char* mirror = nullptr;      // host memory, what aql_pass_mirror's launch fills
     std::vector<char> host;      // the same as it is uploaded
     std::vector<size_t> at, tail;    // where a launch's block starts, and the caller's part inside it
     bool committed = false;
@@ -376,6 +399,7 @@ struct AqlPass {
     ~AqlPass() {
         if (done.handle) hsa_signal_destroy(done);
         if (kernargs) (void)hipFree(kernargs);
+        if (mirror) (void)hipHostFree(mirror);
     }
 };
 
@@ -400,7 +424,7 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
     }
     at[n] = bytes;
     std::vector<char>& host = p->host;
-    host.assign(bytes + 64, 0);
+    host.assign(bytes + 64 + kAqlCallArgs, 0);       // the last block: aql_pass_mirror's
     for (size_t i = 0; i < n; ++i) {
         const AqlLaunch& l = launches[i];
         fill_kernarg(host.data() + at[i], kernels[i], l.kernarg, l.kernarg_bytes, l.grid, l.block);
@@ -409,9 +433,9 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
     if (e != hipSuccess) { *err = std::string("argument blocks: ") + hipGetErrorString(e); return nullptr; }
     for (size_t i = 0; i < n; ++i) {
         const AqlLaunch& l = launches[i];
-        // Launches follow one another (barrier) and see each other's results; the first also sees what
-        // the host and the copy engines wrote, the last makes its results visible to them.
-        const int acquire = i == 0 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
+        // Launches follow one another (barrier) and see each other's results; the last makes its results
+        // visible to host and copy engines.
+        const int acquire = HSA_FENCE_SCOPE_AGENT;
         const int release = i == n - 1 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
         p->packets.push_back(dispatch_packet(kernels[i], l.grid, l.block, l.dyn_lds, (char*)p->kernargs + at[i], acquire, release));
     }
@@ -438,11 +462,83 @@ bool aql_pass_commit(AqlPass* p, std::string* err) {
     return p->committed;
 }
 
-bool aql_pass_run(AqlPass* p, std::string* err) {
+bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, const char** host, std::string* err) {
+    if (p->mirror || p->packets.empty() || n == 0 || n > kBlitRanges) { *err = "bad number of ranges, or a second mirror"; return false; }
+    const AqlKernel* k = aql_kernel(blit_code().get(), device, "reef_blit_ranges", err);
+    if (!k) return false;
+    BlitArgs a;
+    std::memset(&a, 0, sizeof(a));
+    size_t total = 0;
+    for (size_t i = 0; i < n; ++i) total += (bytes[i] + 255) / 256 * 256;
+    void* m = nullptr;
+    const hipError_t e = hipHostMalloc(&m, total, hipHostMallocDefault);
+    if (e != hipSuccess) { *err = std::string("mirror: ") + hipGetErrorString(e); return false; }
+    p->mirror = (char*)m;
+    size_t at = 0;
+    uint32_t blocks = 0;
+    for (size_t i = 0; i < n; ++i) {
+        host[i] = p->mirror + at;
+        a.range[i].src = (const char*)src[i];
+        a.range[i].dst = p->mirror + at;
+        a.range[i].bytes = (uint32_t)bytes[i];
+        blocks += (uint32_t)((bytes[i] + kBlitBlock - 1) / kBlitBlock);
+        a.range[i].end = blocks;
+        at += (bytes[i] + 255) / 256 * 256;
+    }
+    a.ranges = (uint32_t)n;
+    const uint32_t grid[3] = {blocks, 1, 1}, block[3] = {256, 1, 1};
+    const size_t off = p->at.back();
+    fill_kernarg(p->host.data() + off, *k, &a, sizeof(a), grid, block);
+    hsa_kernel_dispatch_packet_t packet =
+        dispatch_packet(*k, grid, block, 0, (char*)p->kernargs + off, HSA_FENCE_SCOPE_AGENT, HSA_FENCE_SCOPE_SYSTEM);
+    packet.completion_signal = p->done;
+    p->packets.back().completion_signal = hsa_signal_t{};
+    p->packets.push_back(packet);
+    return true;
+}
+
+bool aql_host_write(int device, void* dst, const void* src, size_t bytes) {
+    volatile uint32_t* flush = g_devices[device].flush;
+    if (!flush || bytes < 4) return false;
+    std::memcpy(dst, src, bytes);
+    _mm_sfence();
+    *flush = 1;
+    (void)*(volatile uint32_t*)(((uintptr_t)dst + bytes - 4) & ~(uintptr_t)3);   // comes back behind the stores
+    return true;
+}
+
+bool aql_fence(int device, std::string* err) {
+    Call* c = take_call(device, err);
+    if (!c) return false;
+    hsa_barrier_and_packet_t b;
+    std::memset(&b, 0, sizeof(b));
+    b.header = (uint16_t)((HSA_PACKET_TYPE_BARRIER_AND << HSA_PACKET_HEADER_TYPE) | (1 << HSA_PACKET_HEADER_BARRIER) |
+                          (HSA_FENCE_SCOPE_SYSTEM << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE) |
+                          (HSA_FENCE_SCOPE_SYSTEM << HSA_PACKET_HEADER_SCRELEASE_FENCE_SCOPE));
+    b.completion_signal = c->done;
+    static_assert(sizeof(b) == sizeof(hsa_kernel_dispatch_packet_t), "packets are of one size");
+    hsa_kernel_dispatch_packet_t packet;
+    std::memcpy(&packet, &b, sizeof(b));
+    hsa_signal_store_relaxed(c->done, 1);
+    bool ok;
+    {
+        std::lock_guard<std::mutex> submit(c->queue->mtx);
+        ok = put_packet(*c->queue, packet, true, err);
+    }
+    if (!ok || !wait_done(*c->queue, c->done, err)) return false;
+    std::lock_guard<std::mutex> lock(g_devices[device].idle_mtx);
+    g_devices[device].idle.push_back(c);
+    return true;
+}
+
+bool aql_pass_run(AqlPass* p, bool fresh, std::string* err) {
     if (p->packets.empty()) return true;
     if (!p->committed) { *err = "the pass has not been committed"; return false; }
     std::lock_guard<std::mutex> lock(p->mtx);
     Queue& w = *p->queue;
+    uint16_t& first = p->packets[0].header;
+    first = (uint16_t)((first & ~(3 << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE)) |
+                       ((fresh ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT) << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE));
     hsa_signal_store_relaxed(p->done, 1);
     {
         std::lock_guard<std::mutex> submit(w.mtx);

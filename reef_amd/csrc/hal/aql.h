@@ -23,9 +23,10 @@ std::shared_ptr<AqlCode> aql_code_from_file(const char* path);
 
 // A kernel of `code` (loaded on `device` if it is not yet), valid as long as the code is.  nullptr and *err: not found.
 const AqlKernel* aql_kernel(AqlCode* code, int device, const char* name, std::string* err);
-// One launch of `groups` workgroups of `threads`, waited for: it sees what host, copy engines and finished
-// kernels have written, and its results are visible everywhere when this returns.  Calls of several
-// threads run beside each other.  `resident`: device memory that holds aql_call_args' image of the same
+// One launch of `groups` workgroups of `threads`, waited for: it sees what finished kernels and the
+// runtime's copies have written (what a launch through the runtime sees; the runtime empties the caches in
+// front of a copy), and its results are visible everywhere when this returns.  Calls of several threads
+// run beside each other.  `resident`: device memory that holds aql_call_args' image of the same
 // arguments, or null (they are read from host memory then, 1.2 us later).
 constexpr size_t kAqlCallArgs = 512;
 bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
@@ -51,10 +52,20 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
 bool aql_pass_block(AqlPass* p, size_t i, char** device, char** host, size_t* bytes, size_t* tail);
 // Uploads the blocks.
 bool aql_pass_commit(AqlPass* p, std::string* err);
+// Adds a last launch that copies device ranges to host memory of the pass's: host[i] for range i.
+bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, const char** host, std::string* err);
 // Runs the recorded launches one after the other and returns when the last has finished.
+// fresh: the first launch drops what the caches hold of memory that others than finished kernels and
+// the runtime's copies have written (3 us: code and weights are fetched anew as well).
 // false and *err when the queue reported an error.
-bool aql_pass_run(AqlPass* p, std::string* err);
+bool aql_pass_run(AqlPass* p, bool fresh, std::string* err);
 void aql_pass_destroy(AqlPass* p);
+
+// Stores into device memory through the PCIe window, 45 GB/s; all of it has arrived when this returns.
+// Caches may still hold the old bytes.  false: the device says nothing of how to flush the window.
+bool aql_host_write(int device, void* dst, const void* src, size_t bytes);
+// Drops them.
+bool aql_fence(int device, std::string* err);
 
 }  // namespace hal
 }  // namespace reef

@@ -748,13 +748,13 @@ int h_pass_create(const reef_pass_launch* l, size_t n, size_t tail_bytes, reef_p
     *out = (reef_pass_t)p;
     return 0;
 }
-int h_pass_run(reef_pass_t p, reef_stream_t after) {
+int h_pass_run(reef_pass_t p, reef_stream_t after, int fresh) {
     if (!p) { reef_hal_set_error("reef_hal_pass_run: null argument"); return 1; }
     // whatever the stream was given runs first (the queue of the pass knows nothing of it)
     if (!after || after->window > 0 || after->pending.load(std::memory_order_acquire))
         if (int rc = h_stream_sync(after)) return rc;
     std::string err;
-    if (reef::hal::aql_pass_run((reef::hal::AqlPass*)p, &err)) return 0;
+    if (reef::hal::aql_pass_run((reef::hal::AqlPass*)p, fresh != 0, &err)) return 0;
     reef_hal_set_error(("reef_hal_pass_run: " + err).c_str());
     return 1;
 }
@@ -767,6 +767,25 @@ int h_pass_commit(reef_pass_t p) {
     std::string err;
     if (p && reef::hal::aql_pass_commit((reef::hal::AqlPass*)p, &err)) return 0;
     reef_hal_set_error(("reef_hal_pass_commit: " + err).c_str());
+    return 1;
+}
+int h_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char** host) {
+    const void* src[REEF_PASS_MAX_RANGES];
+    size_t bytes[REEF_PASS_MAX_RANGES];
+    if (!p || !r || !host || n > REEF_PASS_MAX_RANGES) { reef_hal_set_error("reef_hal_pass_mirror: bad argument"); return 1; }
+    for (size_t i = 0; i < n; ++i) { src[i] = r[i].src; bytes[i] = r[i].bytes; }
+    std::string err;
+    if (reef::hal::aql_pass_mirror((reef::hal::AqlPass*)p, g_device, src, bytes, n, host, &err)) return 0;
+    reef_hal_set_error(("reef_hal_pass_mirror: " + err).c_str());
+    return 1;
+}
+int h_host_write(reef_devptr_t dst, const void* src, size_t n) {
+    return g_host_visible && reef::hal::aql_host_write(g_device, dst, src, n) ? 0 : 2;
+}
+int h_host_write_fence() {
+    std::string err;
+    if (reef::hal::aql_fence(g_device, &err)) return 0;
+    reef_hal_set_error(("reef_hal_host_write_fence: " + err).c_str());
     return 1;
 }
 int h_pass_destroy(reef_pass_t p) {
@@ -837,6 +856,7 @@ const reef_hal_backend kHip = {
     h_stream_set_completion, h_stream_progress, h_stream_exit_ticks, h_clock_sync,
     h_module_kernel_entry, h_host_fill32, h_stream_drained,
     h_pass_create, h_pass_block, h_pass_commit, h_pass_run, h_pass_destroy,
+    h_pass_mirror, h_host_write, h_host_write_fence,
 };
 
 }  // namespace
