@@ -230,7 +230,11 @@ int reef_hal_graph_destroy(reef_graph_t g);
  *                what the host or launches outside passes have changed since the last run.
  *   host_write:  stores into device memory from the host (device memory behind the PCIe window); returns 2
  *                where the backend cannot.  Nothing that reads the memory may be running; a pass run
- *                with `fresh` sees the bytes, and so does any launch after host_write_fence. */
+ *                with `fresh` sees the bytes, and so does any launch after host_write_fence (which does
+ *                nothing when no host_write came since the last one).
+ *   fetch:       copies ranges of device memory, one behind the other at multiples of 256 bytes, into
+ *                pinned host memory with one launch, and waits for it; what has written them has finished.
+ *                Returns 2 where the backend cannot. */
 typedef struct reef_pass_s* reef_pass_t;
 typedef struct reef_pass_launch {
     reef_function_t fn;
@@ -253,6 +257,7 @@ int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* ranges, size_t n,
 int reef_hal_pass_run(reef_pass_t p, reef_stream_t after, int fresh);
 int reef_hal_host_write(reef_devptr_t dst, const void* src, size_t bytes);
 int reef_hal_host_write_fence(void);
+int reef_hal_fetch(const reef_pass_range* ranges, size_t n, void* host);
 int reef_hal_pass_destroy(reef_pass_t p);
 
 /*
@@ -313,6 +318,7 @@ typedef struct reef_hal_backend {
     int (*pass_mirror)(reef_pass_t, const reef_pass_range*, size_t, const char**);
     int (*host_write)(reef_devptr_t, const void*, size_t);
     int (*host_write_fence)(void);
+    int (*fetch)(const reef_pass_range*, size_t, void*);
 } reef_hal_backend;
 
 const reef_hal_backend* reef_hal_hip_backend(void);

@@ -9,6 +9,7 @@
 // `attrs` integers (include/reef_kernels.h).
 #pragma once
 #include <memory>
+#include <mutex>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -80,14 +81,22 @@ protected:
     virtual size_t add_prefetch(Launch& l, uint32_t wgs) const;
     Status launch_kernel(int kernel_offset, GPUStream_t stream);
     // A whole run recorded once (reef_hal_pass_create) and submitted as ready-made packets from then on.
+    // Storages as they are in host memory besides device memory: the output, and what the caller has fetched
+    // after run upon run.
+    struct Mirror {
+        struct Entry { size_t idx, bytes; const char* host; };
+        std::vector<Entry> entries;
+        size_t watched = 0;    // how many of `watch` it holds
+        const Entry* find(size_t idx) const {
+            for (const Entry& e : entries)
+                if (e.idx == idx) return &e;
+            return nullptr;
+        }
+    };
     struct Pass {
         reef_pass_t handle = nullptr;
         bool tried = false;
-        // what a run leaves in host memory besides device memory: the output, and storages that the
-        // caller has fetched after run upon run
-        struct Mirrored { size_t idx, bytes; const char* host; };
-        std::vector<Mirrored> mirrored;
-        size_t watched = 0;    // how many of `watch` it holds
+        Mirror mirror;         // filled by every run
     };
     // Runs the pass behind what `stream` has been given and waits for it.  *ran = false, and nothing done,
     // where the backend cannot record one.
@@ -95,8 +104,12 @@ protected:
     Status run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran);
     Status record_pass(Pass& p, std::vector<Launch>& launches);
     void drop_pass(Pass& p);
+public:
     // Called in front of every launch of a kernel of this model that is no part of a pass.
     Status leave_passes();
+    // Called when a run is asked for: what set_input has stored is there for whatever launches follow.
+    Status inputs_ready();
+protected:
     Status find_storage_idx(const std::string& name, size_t& idx);
     size_t storage_bytes(size_t idx) const;
 
@@ -114,21 +127,28 @@ protected:
     bool use_graph;
     reef_graph_t model_graph;
     Pass model_pass;
-    // State of the storages as passes know them.  after_pass: the last thing that ran on them was a pass (which has
-    // finished); host_wrote: since then the host has stored into them past the caches; current: the pass whose
-    // mirrored storages are those of the device.
+    // State of the storages (io_mtx: a client fetches results while the scheduler's thread runs the model).
+    // after_pass: the last thing that ran on them was a pass (which has finished); host_wrote: the host has stored
+    // into them past the caches; current: the mirror that is equal to them, or null.
+    std::mutex io_mtx;
     bool after_pass = false, host_wrote = false;
-    Pass* current = nullptr;
+    const Mirror* current = nullptr;
+    Mirror fetched;                    // of the last fetch that was no pass's
+    GPUDevicePtr_t fetch_mem = nullptr;   // pinned
+    size_t fetch_bytes = 0;
     std::vector<size_t> watch;         // storages fetched again and again
     size_t asked_idx = 0, asked_run = 0, runs = 0;
     void note_fetch(size_t idx);
+    void list_mirrored(Mirror& m) const;
+    Status fetch(size_t idx, void* out);
     void drop_graph();
 };
 
 template <class Make>
 Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran) {
     *ran = false;
-    if (p.handle && p.watched != watch.size()) drop_pass(p);
+    std::unique_lock<std::mutex> lock(io_mtx);
+    if (p.handle && p.mirror.watched != watch.size()) drop_pass(p);
     if (!p.tried) {
         std::vector<Launch> l(num_kernels());
         for (size_t i = 0; i < l.size(); i++) RETURN_STATUS(make((int)i, l[i]));
@@ -139,12 +159,13 @@ Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, boo
     *ran = true;
     current = nullptr;
     const int fresh = host_wrote || !after_pass;
-    after_pass = false;
-    GPU_RETURN_STATUS(reef_hal_pass_run(p.handle, stream, fresh));
-    after_pass = true;
-    host_wrote = false;
-    current = &p;
+    after_pass = host_wrote = false;
     runs++;
+    lock.unlock();
+    GPU_RETURN_STATUS(reef_hal_pass_run(p.handle, stream, fresh));
+    lock.lock();
+    after_pass = true;
+    current = &p.mirror;
     return Status::Succ;
 }
 

@@ -462,30 +462,48 @@ bool aql_pass_commit(AqlPass* p, std::string* err) {
     return p->committed;
 }
 
+namespace {
+
+// Workgroups of the launch.
+uint32_t blit_args(BlitArgs* a, const void* const* src, const size_t* bytes, size_t n, char* host) {
+    std::memset(a, 0, sizeof(*a));
+    uint32_t blocks = 0;
+    for (size_t i = 0; i < n; ++i) {
+        a->range[i].src = (const char*)src[i];
+        a->range[i].dst = host;
+        a->range[i].bytes = (uint32_t)bytes[i];
+        blocks += (uint32_t)((bytes[i] + kBlitBlock - 1) / kBlitBlock);
+        a->range[i].end = blocks;
+        host += (bytes[i] + 255) / 256 * 256;
+    }
+    a->ranges = (uint32_t)n;
+    return blocks;
+}
+
+}  // namespace
+
+bool aql_fetch(int device, const void* const* src, const size_t* bytes, size_t n, char* host, std::string* err) {
+    if (n == 0 || n > kBlitRanges) { *err = "bad number of ranges"; return false; }
+    const AqlKernel* k = aql_kernel(blit_code().get(), device, "reef_blit_ranges", err);
+    if (!k) return false;
+    BlitArgs a;
+    const uint32_t blocks = blit_args(&a, src, bytes, n, host);
+    return aql_call(device, k, blocks, 256, &a, sizeof(a), nullptr, err);
+}
+
 bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, const char** host, std::string* err) {
     if (p->mirror || p->packets.empty() || n == 0 || n > kBlitRanges) { *err = "bad number of ranges, or a second mirror"; return false; }
     const AqlKernel* k = aql_kernel(blit_code().get(), device, "reef_blit_ranges", err);
     if (!k) return false;
     BlitArgs a;
-    std::memset(&a, 0, sizeof(a));
     size_t total = 0;
     for (size_t i = 0; i < n; ++i) total += (bytes[i] + 255) / 256 * 256;
     void* m = nullptr;
     const hipError_t e = hipHostMalloc(&m, total, hipHostMallocDefault);
     if (e != hipSuccess) { *err = std::string("mirror: ") + hipGetErrorString(e); return false; }
     p->mirror = (char*)m;
-    size_t at = 0;
-    uint32_t blocks = 0;
-    for (size_t i = 0; i < n; ++i) {
-        host[i] = p->mirror + at;
-        a.range[i].src = (const char*)src[i];
-        a.range[i].dst = p->mirror + at;
-        a.range[i].bytes = (uint32_t)bytes[i];
-        blocks += (uint32_t)((bytes[i] + kBlitBlock - 1) / kBlitBlock);
-        a.range[i].end = blocks;
-        at += (bytes[i] + 255) / 256 * 256;
-    }
-    a.ranges = (uint32_t)n;
+    const uint32_t blocks = blit_args(&a, src, bytes, n, p->mirror);
+    for (size_t i = 0; i < n; ++i) host[i] = a.range[i].dst;
     const uint32_t grid[3] = {blocks, 1, 1}, block[3] = {256, 1, 1};
     const size_t off = p->at.back();
     fill_kernarg(p->host.data() + off, *k, &a, sizeof(a), grid, block);

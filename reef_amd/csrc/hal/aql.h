@@ -64,7 +64,9 @@ void aql_pass_destroy(AqlPass* p);
 // Stores into device memory through the PCIe window, 45 GB/s; all of it has arrived when this returns.
 // Caches may still hold the old bytes.  false: the device says nothing of how to flush the window.
 bool aql_host_write(int device, void* dst, const void* src, size_t bytes);
-// Drops them.
+// Copies device ranges to pinned host memory, one behind the other at multiples of 256 bytes, and waits for it.
+bool aql_fetch(int device, const void* const* src, const size_t* bytes, size_t n, char* host, std::string* err);
+// Drops what the caches hold of bytes that aql_host_write has replaced.
 bool aql_fence(int device, std::string* err);
 
 }  // namespace hal

@@ -113,6 +113,7 @@ int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, cons
 int reef_hal_pass_run(reef_pass_t p, reef_stream_t after, int fresh) { return be()->pass_run ? be()->pass_run(p, after, fresh) : 1; }
 int reef_hal_host_write(reef_devptr_t dst, const void* src, size_t bytes) { return be()->host_write ? be()->host_write(dst, src, bytes) : 2; }
 int reef_hal_host_write_fence(void) { return be()->host_write_fence ? be()->host_write_fence() : 0; }
+int reef_hal_fetch(const reef_pass_range* r, size_t n, void* host) { return be()->fetch ? be()->fetch(r, n, host) : 2; }
 int reef_hal_pass_destroy(reef_pass_t p) { return p && be()->pass_destroy ? be()->pass_destroy(p) : 0; }
 int reef_hal_event_create(reef_event_t* out) { return be()->event_create(out); }
 int reef_hal_event_destroy(reef_event_t e) { return be()->event_destroy(e); }

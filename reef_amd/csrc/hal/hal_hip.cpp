@@ -779,13 +779,37 @@ int h_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char*
     reef_hal_set_error(("reef_hal_pass_mirror: " + err).c_str());
     return 1;
 }
+std::atomic<uint64_t> g_host_writes{0}, g_host_writes_seen{0};   // how many there were, how many of them the last fence covers
 int h_host_write(reef_devptr_t dst, const void* src, size_t n) {
-    return g_host_visible && reef::hal::aql_host_write(g_device, dst, src, n) ? 0 : 2;
+    if (!g_host_visible || !reef::hal::aql_available(g_device)) return 2;
+    // what the default stream still does with the memory comes first, as in front of a copy
+    HIPCHK(hipStreamSynchronize(nullptr));
+    if (!reef::hal::aql_host_write(g_device, dst, src, n)) return 2;
+    g_host_writes.fetch_add(1);
+    return 0;
 }
 int h_host_write_fence() {
+    const uint64_t n = g_host_writes.load();
+    if (g_host_writes_seen.load() >= n) return 0;
     std::string err;
-    if (reef::hal::aql_fence(g_device, &err)) return 0;
+    if (reef::hal::aql_fence(g_device, &err)) {
+        uint64_t seen = g_host_writes_seen.load();
+        while (seen < n && !g_host_writes_seen.compare_exchange_weak(seen, n)) {}
+        return 0;
+    }
     reef_hal_set_error(("reef_hal_host_write_fence: " + err).c_str());
+    return 1;
+}
+int h_fetch(const reef_pass_range* r, size_t n, void* host) {
+    const void* src[REEF_PASS_MAX_RANGES];
+    size_t bytes[REEF_PASS_MAX_RANGES];
+    if (!r || !host || n > REEF_PASS_MAX_RANGES) { reef_hal_set_error("reef_hal_fetch: bad argument"); return 1; }
+    if (!reef::hal::aql_available(g_device)) return 2;
+    HIPCHK(hipStreamSynchronize(nullptr));
+    for (size_t i = 0; i < n; ++i) { src[i] = r[i].src; bytes[i] = r[i].bytes; }
+    std::string err;
+    if (reef::hal::aql_fetch(g_device, src, bytes, n, (char*)host, &err)) return 0;
+    reef_hal_set_error(("reef_hal_fetch: " + err).c_str());
     return 1;
 }
 int h_pass_destroy(reef_pass_t p) {
@@ -856,7 +880,7 @@ const reef_hal_backend kHip = {
     h_stream_set_completion, h_stream_progress, h_stream_exit_ticks, h_clock_sync,
     h_module_kernel_entry, h_host_fill32, h_stream_drained,
     h_pass_create, h_pass_block, h_pass_commit, h_pass_run, h_pass_destroy,
-    h_pass_mirror, h_host_write, h_host_write_fence,
+    h_pass_mirror, h_host_write, h_host_write_fence, h_fetch,
 };
 
 }  // namespace

@@ -158,6 +158,8 @@ Status REEFScheduler::new_task(const ModelID& mid, TaskID& tid) {
     if (model_pool_size.load() <= mid) RETURN_STATUS(Status::OutOfRange);
     auto& model = model_pool[mid];
     if (model->qid == rt_queue_id && !rt_queue) RETURN_STATUS(Status::NotFound);
+    // here, in the client's thread: the scheduler's would do it in front of the first launch
+    RETURN_STATUS(model->executor.inputs_ready());
     std::shared_ptr<Task> task(new Task);
     task->model = model;
     task->id = task_idx_pool.fetch_add(1);
@@ -616,6 +618,7 @@ void REEFScheduler::dynamic_kernel_padding(std::shared_ptr<Task>& rt_task) {
     const std::vector<TransExecutor::Proxy>& proxies = rt_exe.proxies();
 
     const int n_rt = (int)rt_exe.num_kernels();
+    rt_exe.leave_passes();
     for (int i = 0; i < n_rt; i++) {
         const auto sel_start = std::chrono::steady_clock::now();
         const TransExecutor::KernelArg& rt_args = rt_exe.trans_args[i];
@@ -687,6 +690,7 @@ void REEFScheduler::dynamic_kernel_padding(std::shared_ptr<Task>& rt_task) {
             a.entry_l = (const void*)(uintptr_t)rt_args.entry;
             a.entry_r = (const void*)(uintptr_t)be_args->entry;
             if (be_task->start.time_since_epoch().count() == 0) be_task->start = current_time_point;
+            be_exe.leave_passes();
             executor::GPUFunction_t proxy = rt_exe.get_proxy_kernel(proxy_idx);
             const uint32_t grid[3] = {(uint32_t)(dec.final_occupancy * num_cus), 1, 1};
             const uint32_t block[3] = {(uint32_t)dec.merged_block_size, 1, 1};
