@@ -153,6 +153,7 @@ enum {
 #define REEF_K_TRANSPOSE "reef_transpose"
 #define REEF_K_GEMM "reef_gemm"
 #define REEF_K_ATTENTION "reef_attention"
+#define REEF_K_ATTENTION_MM "reef_attention_m16"
 /* The reference's mocked model (resource/mocked_kernel/mocked_kernel.json)
  * keeps its own names and its (64,1,1)x(4,8,4) launch. */
 #define REEF_K_MOCK_ADD "add"
@@ -307,6 +308,9 @@ enum {
     REEF_TILE_R9G7 = 16,
     REEF_TILE_R9G2M2 = 17,   /* 32 channels x 2, 4 image rows */
     REEF_TILE_R9G4M2 = 18,
+    REEF_TILE_32x48d4 = 19,  /* matrix products, direct family */
+    REEF_TILE_48x48d4 = 20,
+    REEF_TILE_64x64d4 = 21,
     REEF_TILE_COUNT
 };
 
@@ -388,6 +392,12 @@ enum {
 #define REEF_AT_LDS_BYTES \
     (4 * (REEF_AT_ROWS * REEF_AT_MAX_HEAD_DIM + REEF_AT_MAX_SEQ * REEF_AT_KV_STRIDE + REEF_AT_ROWS * (REEF_AT_MAX_SEQ + 4)))
 
+/* reef_attention_m16: the same operands, attributes and result on the matrix cores, 16 query rows per workgroup,
+ * for sequences of up to REEF_AT_MM_MAX_SEQ.  tasks = heads * ceil(seq / REEF_AT_MM_ROWS). */
+#define REEF_AT_MM_ROWS 16
+#define REEF_AT_MM_MAX_SEQ 512
+#define REEF_AT_MM_LDS_BYTES (4 * (REEF_AT_MM_ROWS * (REEF_AT_MM_MAX_SEQ + 4) + REEF_AT_MM_ROWS))
+
 /* ---- reef_bias_gelu: out = gelu_erf(x + bias[col]).  ptr: x, out, bias(optional).
  * attr: rows, cols, flags.  tasks = ceil(rows*cols / 1024). */
 enum { REEF_GELU_ROWS = 0, REEF_GELU_COLS, REEF_GELU_FLAGS, REEF_GELU_NATTR };
@@ -408,7 +418,7 @@ enum { REEF_TR_D0 = 0, REEF_TR_D1, REEF_TR_D2, REEF_TR_FLAGS, REEF_TR_NATTR };
 /* ---- reef_gemm_nt_<tile> / reef_gemm_ntd_<tile> / reef_gemm_nn_<tile>: batched fp32 GEMM on MFMA ----
  * nt: trans_b = 1 (K, lda, ldb and the batch strides must be multiples of 4);
  * ntd: trans_b = 1, operands straight from memory into 16x16x4 MFMAs (tiles 16x16k4, 16x32k4,
- *      32x32d4; K a multiple of 8, lda, ldb and the batch strides multiples of 4);
+ *      32x32d4, 32x48d4, 48x48d4, 64x64d4; K a multiple of 8, lda, ldb and the batch strides multiples of 4);
  * nn: trans_b = 0 (K and lda multiples of 4).
  * C[b][m][n] = act(alpha * sum_k A[b][m][k] * B(b,k,n) (+bias[n])) (+R[b][m][n])
  * trans_b = 1: B stored [b][n][k] (dense layers, Q.K^T); 0: [b][k][n] (P.V).
@@ -421,7 +431,7 @@ enum { REEF_TR_D0 = 0, REEF_TR_D1, REEF_TR_D2, REEF_TR_FLAGS, REEF_TR_NATTR };
  *       one [tokens][3 * hidden] projection.
  * tasks = batch * m_tiles * n_tiles.
  *
- * reef_gemm_ntl_<tile> (staged tiles, trans_b = 1, batch 1, flags has REEF_GEMM_F_LN): the product
+ * reef_gemm_ntl_<tile> (staged tiles; direct tiles with K a multiple of 8; trans_b = 1, batch 1, flags has REEF_GEMM_F_LN): the product
  * behind a LayerNorm of the rows of A,
  *   A'[m][k] = (A[m][k] - mean[m]) / sqrt(var[m] + eps) * gamma[k] + beta[k]
  * (mean and variance over the K columns of the row), C = act(alpha * A' x W^T (+bias)) (+R), computed

@@ -475,7 +475,7 @@ class GraphOracle:
                     c = c + np.lib.stride_tricks.as_strided(R[bi * sC:], (M, N), (ldc * 4, 4))
                 Cm = np.lib.stride_tricks.as_strided(C[bi * sC:], (M, N), (ldc * 4, 4))
                 Cm[:, :] = c
-        elif name == "reef_attention":
+        elif name in ("reef_attention", "reef_attention_m16"):
             # softmax(alpha Q K^T (masked)) V per head; Q, K, V column blocks of one [seq][ld] tensor
             S, HD, heads, ld, ldo, oq, ok, ov, alpha_bits, flags = a[:10]
             alpha = _bits_to_float(alpha_bits)

@@ -19,7 +19,7 @@ int op_from_symbol(const std::string& n) {
         {REEF_K_BIAS_GELU, REEF_OP_BIAS_GELU}, {REEF_K_EMBEDDING, REEF_OP_EMBEDDING},
         {REEF_K_COPY, REEF_OP_COPY}, {REEF_K_TRANSPOSE, REEF_OP_TRANSPOSE},
         {REEF_K_MOCK_ADD, REEF_OP_MOCK_ADD}, {REEF_K_MOCK_MULTIPLY, REEF_OP_MOCK_MULTIPLY},
-        {REEF_K_ATTENTION, REEF_OP_ATTENTION},
+        {REEF_K_ATTENTION, REEF_OP_ATTENTION}, {REEF_K_ATTENTION_MM, REEF_OP_ATTENTION},
     };
     for (auto& e : table) {
         const size_t len = std::strlen(e.prefix);
@@ -285,13 +285,14 @@ void gemm(const std::string& symbol, const Attrs& a, Needs& n) {
     if (n.tasks >= kDivSmallLimit) n.bad = "4 Mi workgroups or more (the kernels' index arithmetic is exact below that)";
 }
 
-void attention(const Attrs& a, Needs& n) {
+void attention(const std::string& symbol, const Attrs& a, Needs& n) {
+    const bool mma = symbol == REEF_K_ATTENTION_MM;
     if (!all_positive(a, {REEF_AT_SEQ, REEF_AT_HEAD_DIM, REEF_AT_HEADS, REEF_AT_LD, REEF_AT_LDO}) ||
         a[REEF_AT_OFF_Q] < 0 || a[REEF_AT_OFF_K] < 0 || a[REEF_AT_OFF_V] < 0) {
         n.bad = "a dimension of the attention is not positive";
         return;
     }
-    if (a[REEF_AT_SEQ] > REEF_AT_MAX_SEQ || a[REEF_AT_HEAD_DIM] > REEF_AT_MAX_HEAD_DIM) {
+    if (a[REEF_AT_SEQ] > (mma ? REEF_AT_MM_MAX_SEQ : REEF_AT_MAX_SEQ) || a[REEF_AT_HEAD_DIM] > REEF_AT_MAX_HEAD_DIM) {
         n.bad = "the sequence or the head is larger than the kernel's staging area";
         return;
     }
@@ -306,7 +307,7 @@ void attention(const Attrs& a, Needs& n) {
     n.f32("queries, keys and values", last + (seq - 1) * a[REEF_AT_LD] + width);
     n.f32("context", (seq - 1) * a[REEF_AT_LDO] + width);
     if (a[REEF_AT_FLAGS] & 1) n.raw("mask", seq);
-    n.tasks = a[REEF_AT_HEADS] * cdiv(seq, REEF_AT_ROWS);
+    n.tasks = a[REEF_AT_HEADS] * cdiv(seq, mma ? REEF_AT_MM_ROWS : REEF_AT_ROWS);
 }
 
 // Fills `n` for the ops that are a few lines each; false for an op that is not judged.
@@ -456,7 +457,7 @@ bool kernel_fits_storages(const Model& m, size_t index, std::string* why) {
     case REEF_OP_CONV2D: conv2d(symbol, a, n); break;
     case REEF_OP_SPLITK_REDUCE: splitk_reduce(a, n); break;
     case REEF_OP_GEMM: gemm(symbol, a, n); break;
-    case REEF_OP_ATTENTION: attention(a, n); break;
+    case REEF_OP_ATTENTION: attention(symbol, a, n); break;
     default:
         if (!small_op(op, a, grid, n)) return true;
     }

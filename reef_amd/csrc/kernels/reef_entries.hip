@@ -39,6 +39,9 @@ __device__ __forceinline__ int gemm_tasks(const ReefOpDesc& d) {
 __device__ __forceinline__ int attention_tasks(const ReefOpDesc& d) {
     return d.attr[REEF_AT_HEADS] * ((d.attr[REEF_AT_SEQ] + REEF_AT_ROWS - 1) / REEF_AT_ROWS);
 }
+__device__ __forceinline__ int attention_mma_tasks(const ReefOpDesc& d) {
+    return d.attr[REEF_AT_HEADS] * ((d.attr[REEF_AT_SEQ] + REEF_AT_MM_ROWS - 1) / REEF_AT_MM_ROWS);
+}
 __device__ __forceinline__ int pool_tasks(const ReefOpDesc& d) {
     return (d.attr[REEF_POOL_C] * d.attr[REEF_POOL_HO] * d.attr[REEF_POOL_WO] + kThreads - 1) / kThreads;
 }
@@ -119,14 +122,14 @@ struct OpGemm {
         return gemm_body<T, TRANS_B, LN_A>(d, task, smem, p);
     }
 };
-template <int TM, int TN>
+template <int TM, int TN, bool LN = false>
 struct OpGemmNtDirect {
     REEF_TASKS(gemm_tasks)
-    static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
+    static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES + (LN ? 9 * 16 * TM * 4 : 0);   // + the rows' sums per wavefront, pivots
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
-        return gemm_nt_direct_body<TM, TN>(d, task, smem, p);
+        return gemm_nt_direct_body<TM, TN, LN>(d, task, smem, p);
     }
 };
 #define REEF_SIMPLE_OP(STRUCT, CALL, TASKS)                                                     \
@@ -145,6 +148,15 @@ struct OpAttention {
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P&) {
         attention_body(d, task, smem);
+        return true;
+    }
+};
+struct OpAttentionMma {
+    REEF_TASKS(attention_mma_tasks)
+    static constexpr int LDS = REEF_AT_MM_LDS_BYTES;
+    template <class P>
+    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P&) {
+        attention_mma_body(d, task, smem);
         return true;
     }
 };
@@ -449,6 +461,14 @@ REEF_ENTRY(reef_gemm_ntl_64x32k2, OpGemm<Tile64x32k2 REEF_COMMA true REEF_COMMA 
 REEF_ENTRY(reef_gemm_ntd_16x16k4, OpGemmNtDirect<1 REEF_COMMA 1>)
 REEF_ENTRY(reef_gemm_ntd_16x32k4, OpGemmNtDirect<1 REEF_COMMA 2>)
 REEF_ENTRY(reef_gemm_ntd_32x32d4, OpGemmNtDirect<2 REEF_COMMA 2>)
+REEF_ENTRY(reef_gemm_ntd_32x48d4, OpGemmNtDirect<2 REEF_COMMA 3>)
+REEF_ENTRY(reef_gemm_ntd_48x48d4, OpGemmNtDirect<3 REEF_COMMA 3>)
+REEF_ENTRY(reef_gemm_ntd_64x64d4, OpGemmNtDirect<4 REEF_COMMA 4>)
+REEF_ENTRY(reef_gemm_ntl_16x16k4, OpGemmNtDirect<1 REEF_COMMA 1 REEF_COMMA true>)
+REEF_ENTRY(reef_gemm_ntl_16x32k4, OpGemmNtDirect<1 REEF_COMMA 2 REEF_COMMA true>)
+REEF_ENTRY(reef_gemm_ntl_32x48d4, OpGemmNtDirect<2 REEF_COMMA 3 REEF_COMMA true>)
+REEF_ENTRY(reef_gemm_ntl_48x48d4, OpGemmNtDirect<3 REEF_COMMA 3 REEF_COMMA true>)
+REEF_ENTRY(reef_gemm_ntl_64x64d4, OpGemmNtDirect<4 REEF_COMMA 4 REEF_COMMA true>)
 REEF_ENTRY(reef_gemm_nn_128x128, OpGemm<Tile128x128 REEF_COMMA false>)
 REEF_ENTRY(reef_gemm_nn_64x64, OpGemm<Tile64x64 REEF_COMMA false>)
 REEF_ENTRY(reef_gemm_nn_32x128, OpGemm<Tile32x128 REEF_COMMA false>)
@@ -464,6 +484,7 @@ REEF_ENTRY(reef_softmax, OpSoftmax)
 REEF_ENTRY(reef_layernorm, OpLayerNorm)
 REEF_ENTRY(reef_bias_gelu, OpBiasGelu)
 REEF_ENTRY(reef_attention, OpAttention)
+REEF_ENTRY(reef_attention_m16, OpAttentionMma)
 REEF_ENTRY(reef_embedding, OpEmbedding)
 REEF_ENTRY(reef_copy, OpCopy)
 REEF_ENTRY(reef_transpose, OpTranspose)

@@ -2154,6 +2154,74 @@ __device__ __forceinline__ bool conv2d_stem_pool_body(const ReefOpDesc& d, int t
     return true;
 }
 
+// The rows of A behind their LayerNorm, written by the products that read A through one (REEF_GEMM_F_LN_OUT):
+// the BM * K / 4 float4s of a row block in n_tiles contiguous runs, one for every column tile (one
+// workgroup writing it all would be the launch's straggler).  What a thread needs for the first float4 of
+// its share (the only one for rows of up to 256 n_tiles / BM float4s) is loaded by init, ahead of the
+// K loop, so that after the loop only arithmetic and a store are left.
+struct LnOut {
+    float* out;
+    int end, row4, r, next, m0, M;
+    unsigned off, koff, lda4, bytes;
+    f32x4 v, g, b;
+    rsrc_t ra, rg, rb;
+    // p: first of c1, c2, gamma, beta, A' in the pointer slots
+    __device__ __forceinline__ void init(const ReefOpDesc& d, int p, const float* A, int M_, int K, int lda, int m0_, int BM, int nt, int n_tiles) {
+        out = (d.attr[REEF_GEMM_FLAGS] & REEF_GEMM_F_LN_OUT) ? (float*)d.ptr[p + 4] : nullptr;
+        M = M_;
+        m0 = m0_;
+        lda4 = (unsigned)lda * 4u;
+        bytes = (unsigned)(M - 1) * lda4 + (unsigned)K * 4u;
+        ra = make_rsrc(A, out ? bytes : 0u);
+        rg = make_rsrc(d.ptr[p + 2], out ? (unsigned)K * 4u : 0u);
+        rb = make_rsrc(d.ptr[p + 3], out ? (unsigned)K * 4u : 0u);
+        row4 = K / 4;
+        const int total = BM * row4, share = (total + n_tiles - 1) / n_tiles;
+        end = (nt + 1) * share < total ? (nt + 1) * share : total;
+        const int id = nt * share + (int)threadIdx.x;
+        next = id + kThreads;
+        off = koff = kOutside;
+        r = 0;
+        if (out && id < end) {
+            r = div_small(id, row4);
+            if (m0 + r < M) {
+                koff = (unsigned)(id - r * row4) * 16u;
+                off = (unsigned)(m0 + r) * lda4 + koff;
+            }
+        }
+        v = buf_load4(ra, off);
+        g = buf_load4(rg, koff);
+        b = buf_load4(rb, koff);
+    }
+    // stats(row of the tile, mean, 1 / std)
+    template <class Stats>
+    __device__ __forceinline__ void write(const Stats& stats) const {
+        if (!out) return;
+        const rsrc_t ro = make_rsrc(out, bytes);
+        {   // the float4 whose operands have been waiting since before the K loop
+            float mu, rs;
+            stats(r, mu, rs);
+            f32x4 y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = (v[e] - mu) * rs * g[e] + b[e];
+            buf_store4(ro, off, y);      // no share, or a row outside M: an offset outside the buffer
+        }
+        for (int id = next; id < end; id += kThreads) {
+            const int rr = div_small(id, row4), k4 = (id - rr * row4) * 4;
+            if (m0 + rr < M) {
+                const unsigned o = (unsigned)(m0 + rr) * lda4 + (unsigned)k4 * 4u;
+                const f32x4 x = buf_load4(ra, o), gm = buf_load4(rg, (unsigned)k4 * 4u), bt = buf_load4(rb, (unsigned)k4 * 4u);
+                float mu, rs;
+                stats(rr, mu, rs);
+                f32x4 y;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] = (x[e] - mu) * rs * gm[e] + bt[e];
+                buf_store4(ro, o, y);
+            }
+        }
+    }
+};
+
 // ---- reef_gemm ----------------------------------------------------------------
 // TRANS_B: B stored [N][K] (dense layers, Q.K^T) -- both operands take 128-bit row
 // loads, so K, lda, ldb and the batch strides must be multiples of 4 floats.
@@ -2210,38 +2278,10 @@ __device__ __forceinline__ bool gemm_body(const ReefOpDesc& d, int task, char* s
                          : nullptr;
     const int lnp = 3 + (bias ? 1 : 0) + (R ? 1 : 0);      // LN_A: first of c1, c2, gamma, beta, A'
     float e_c1[T::TN], e_c2[T::TN];
-    // LN_A with REEF_GEMM_F_LN_OUT: the normalised rows go to memory as well, a share per column
-    // tile -- the BM * K / 4 float4s of the row block in n_tiles contiguous runs (one workgroup
-    // writing it all would be the launch's straggler).  What a thread needs for the first float4
-    // of its share (the only one for rows of up to 256 n_tiles / BM float4s) is loaded here, ahead
-    // of the K loop, so that after the loop only arithmetic and a store are left.
-    float* Aout = nullptr;
-    int o_share = 0, o_end = 0, o_row4 = 1, o_r = 0;
-    unsigned o_off = kOutside, o_koff = kOutside;
-    f32x4 o_v, o_g, o_b;
-    rsrc_t rs_oa, rs_og, rs_ob;
+    LnOut ln_out;
     if (LN_A) {
         la.init_ln();
-        if (fl & REEF_GEMM_F_LN_OUT) Aout = (float*)d.ptr[lnp + 4];
-        const unsigned bytes = ((unsigned)(M - 1) * (unsigned)lda + (unsigned)K) * 4u;
-        rs_oa = make_rsrc(A, Aout ? bytes : 0u);
-        rs_og = make_rsrc(d.ptr[lnp + 2], Aout ? (unsigned)K * 4u : 0u);
-        rs_ob = make_rsrc(d.ptr[lnp + 3], Aout ? (unsigned)K * 4u : 0u);
-        o_row4 = K / 4;
-        const int total = T::BM * o_row4;
-        o_share = (total + n_tiles - 1) / n_tiles;
-        o_end = (nt + 1) * o_share < total ? (nt + 1) * o_share : total;
-        const int id = nt * o_share + (int)threadIdx.x;
-        if (Aout && id < o_end) {
-            o_r = div_small(id, o_row4);
-            if (m0 + o_r < M) {
-                o_koff = (unsigned)(id - o_r * o_row4) * 16u;
-                o_off = (unsigned)(m0 + o_r) * (unsigned)lda * 4u + o_koff;
-            }
-        }
-        o_v = buf_load4(rs_oa, o_off);
-        o_g = buf_load4(rs_og, o_koff);
-        o_b = buf_load4(rs_ob, o_koff);
+        ln_out.init(d, lnp, A, M, K, lda, m0, T::BM, nt, n_tiles);
         // c1 and c2 of this thread's output columns, on their way before the K loop
         const float* c1 = (const float*)d.ptr[lnp];
         const float* c2 = (const float*)d.ptr[lnp + 1];
@@ -2286,29 +2326,10 @@ __device__ __forceinline__ bool gemm_body(const ReefOpDesc& d, int task, char* s
             }
         }
         __syncthreads();
-        if (Aout) {
-            const rsrc_t rs_o = make_rsrc(Aout, ((unsigned)(M - 1) * (unsigned)lda + (unsigned)K) * 4u);
-            {   // the float4 whose operands have been waiting since before the K loop
-                const float mu = stats[2 * o_r], rs = stats[2 * o_r + 1];
-                f32x4 y;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[e] = (o_v[e] - mu) * rs * o_g[e] + o_b[e];
-                buf_store4(rs_o, o_off, y);      // no share, or a row outside M: an offset outside the buffer
-            }
-            for (int id = nt * o_share + (int)threadIdx.x + kThreads; id < o_end; id += kThreads) {
-                const int r = div_small(id, o_row4), k4 = (id - r * o_row4) * 4;
-                if (m0 + r < M) {
-                    const unsigned off = ((unsigned)(m0 + r) * (unsigned)lda + (unsigned)k4) * 4u;
-                    const f32x4 v = buf_load4(rs_oa, off);
-                    const f32x4 gm = buf_load4(rs_og, (unsigned)k4 * 4u), bt = buf_load4(rs_ob, (unsigned)k4 * 4u);
-                    const float mu = stats[2 * r], rs = stats[2 * r + 1];
-                    f32x4 y;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = (v[e] - mu) * rs * gm[e] + bt[e];
-                    buf_store4(rs_o, off, y);
-                }
-            }
-        }
+        ln_out.write([&](int r, float& mu, float& rs) {
+            mu = stats[2 * r];
+            rs = stats[2 * r + 1];
+        });
     }
     float res[T::TM][T::TN][T::RPW];
     const int r0 = finish_tile<T>(acc, res, smem);
@@ -2348,11 +2369,23 @@ __device__ __forceinline__ bool gemm_body(const ReefOpDesc& d, int task, char* s
 // every slot.  The four wavefronts split K (a step is 128 k values), the partial tiles meet in
 // LDS, thread t writes element (t / 16, t % 16) of every 16 x 16 sub-tile.  K % 8 == 0, lda, ldb
 // and the batch strides multiples of 4.  No split of K across workgroups.
-template <int TM, int TN, class Poll>
+//
+// LN (symbols reef_gemm_ntl_<direct tile>): the product behind a LayerNorm of the rows of A, as reef_gemm_ntl on the
+// staged tiles.  A lane adds what it loads of a row to sums of (a - p) and (a - p)^2 around a pivot p
+// (element 0 of the row); the sixteen lanes that share a row -- four k slots, four wavefronts -- meet in LDS.
+//
+// Tiles of more than four sub-tiles (32x48, 48x48, 64x64) load four k values per lane and step instead of
+// eight and keep one accumulator per sub-tile.  A CU's loads are what bounds these products (384 x 2304 x 768
+// on 32x32: 170 MB out of L2, 6.3 TB/s), and they go with (BM + BN) / (BM BN): 64x64 22.0 -> 17.9 us there,
+// 32x48 12.1 -> 10.2 at 128 x 2304 x 768, 48x48 27.4 -> 22.4 at 384 x 3072 x 768.
+template <int TM, int TN, bool LN, class Poll>
 __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int task, char* smem_raw,
                                                     const Poll& poll) {
     typedef TileD16<TN, TM> TD;
-    constexpr int LOADS = 2 * (TM + TN);
+    constexpr bool BIG = TM * TN > 4;
+    constexpr int KL = BIG ? 4 : 8;        // k values per lane and step
+    constexpr int KSTEP = 16 * KL;         // k values of a step
+    constexpr int AC = BIG ? 1 : 2;        // accumulators per sub-tile: enough for no MFMA to wait for the one in front
     constexpr int NS = 3;      // steps of loads in flight (6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * TD::SUBS * TD::PART);
@@ -2363,7 +2396,7 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
     const int n_tiles = a[REEF_GEMM_N_TILES];
     const int tiles = a[REEF_GEMM_M_TILES] * n_tiles;
     // K split across workgroups (batch 1): the split_k workgroups of a tile are neighbours in the task order
-    const int split_k = a[REEF_GEMM_SPLIT_K] > 1 ? a[REEF_GEMM_SPLIT_K] : 1;
+    const int split_k = !LN && a[REEF_GEMM_SPLIT_K] > 1 ? a[REEF_GEMM_SPLIT_K] : 1;
     const int tile_task = split_k > 1 ? div_small(task, split_k) : task;
     const int split = task - tile_task * split_k;
     const int b = div_small(tile_task, tiles);
@@ -2401,21 +2434,40 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
         }
     }
 
+    // LN: the pivots of this lane's rows of A (for the sums) and of its output rows, c1 and c2 of its columns
+    const int lnp = 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0);
+    LnOut ln_out;
+    float pivot[LN ? TM : 1], ls1[LN ? TM : 1], ls2[LN ? TM : 1], e_c1[LN ? TN : 1], e_c2[LN ? TN : 1];
+    if (LN) {
+        const rsrc_t rs_c1 = make_rsrc(d.ptr[lnp], (unsigned)N * 4u), rs_c2 = make_rsrc(d.ptr[lnp + 1], (unsigned)N * 4u);
+#pragma unroll
+        for (int h = 0; h < TM; ++h) {
+            pivot[LN ? h : 0] = buf_load(rs_a, (unsigned)(m0 + 16 * h + i16) * lda * 4u);
+            ls1[LN ? h : 0] = ls2[LN ? h : 0] = 0.0f;
+        }
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+            const unsigned n4 = (unsigned)(n0 + 16 * g + ocol) * 4u;
+            e_c1[LN ? g : 0] = buf_load(rs_c1, n4);
+            e_c2[LN ? g : 0] = buf_load(rs_c2, n4);
+        }
+        ln_out.init(d, lnp, (const float*)d.ptr[0], M, K, (int)lda, m0, TD::BM, nt, n_tiles);
+    }
     const int k_lo = split_k > 1 ? split * a[REEF_GEMM_K_CHUNK] : 0;        // this workgroup's part of K
     const int k_hi = split_k > 1 ? min(K, k_lo + a[REEF_GEMM_K_CHUNK]) : K;
-    const int lane_k = k_lo + (wave * 4 + kq) * 8;   // first k of this lane's slot
-    const int nsteps = (k_hi - k_lo + 127) / 128;
-    const int lane_steps = lane_k < k_hi ? (k_hi - lane_k + 127) / 128 : 0;
+    const int lane_k = k_lo + (wave * 4 + kq) * KL;  // first k of this lane's slot
+    const int nsteps = (k_hi - k_lo + KSTEP - 1) / KSTEP;
+    const int lane_steps = lane_k < k_hi ? (k_hi - lane_k + KSTEP - 1) / KSTEP : 0;
     unsigned va[TM], vb[TN];
 #pragma unroll
     for (int h = 0; h < TM; ++h) va[h] = ((unsigned)(m0 + 16 * h + i16) * lda + (unsigned)lane_k) * 4u;
 #pragma unroll
     for (int g = 0; g < TN; ++g) vb[g] = ((unsigned)(n0 + 16 * g + i16) * ldb + (unsigned)lane_k) * 4u;
 
-    float ra[NS][TM][8], rb[NS][TN][8];
-    auto load8 = [&](float (&dst)[8], rsrc_t rs, unsigned off, unsigned soff) {
+    float ra[NS][TM][KL], rb[NS][TN][KL];
+    auto load_slot = [&](float (&dst)[KL], rsrc_t rs, unsigned off, unsigned soff) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < KL / 4; ++q) {
             const f32x4 v = __builtin_bit_cast(
                 f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off + 16u * q), (int)soff, 0));
             dst[4 * q] = v[0]; dst[4 * q + 1] = v[1]; dst[4 * q + 2] = v[2]; dst[4 * q + 3] = v[3];
@@ -2423,11 +2475,11 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
     };
     auto load_step = [&](int s, int step) {
         const unsigned outm = step < lane_steps ? 0u : kOutside;
-        const unsigned so = (unsigned)step * 512u;   // 128 k values, uniform
+        const unsigned so = (unsigned)step * (unsigned)KSTEP * 4u;   // uniform
 #pragma unroll
-        for (int h = 0; h < TM; ++h) load8(ra[s][h], rs_a, va[h] | outm, so);
+        for (int h = 0; h < TM; ++h) load_slot(ra[s][h], rs_a, va[h] | outm, so);
 #pragma unroll
-        for (int g = 0; g < TN; ++g) load8(rb[s][g], rs_b, vb[g] | outm, so);
+        for (int g = 0; g < TN; ++g) load_slot(rb[s][g], rs_b, vb[g] | outm, so);
     };
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -2443,23 +2495,37 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
         __syncthreads();
         if (*sflag) return false;
     }
-    f32x4 acc[TM][TN][2];
+    f32x4 acc[TM][TN][AC];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) {
-            acc[h][g][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            acc[h][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    auto mma_stage = [&](int s) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
+            for (int e = 0; e < AC; ++e) acc[h][g][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    int ln_step = 0;
+    auto mma_stage = [&](int s) {
+        if (LN) {
+            const float in = ln_step++ < lane_steps ? 1.0f : 0.0f;     // values outside K were loaded as zeros: 0 - 0
+#pragma unroll
+            for (int h = 0; h < TM; ++h) {
+                const float pv = pivot[LN ? h : 0] * in;
+#pragma unroll
+                for (int q = 0; q < KL; ++q) {
+                    const float dl = ra[s][h][q] - pv;
+                    ls1[LN ? h : 0] += dl;
+                    ls2[LN ? h : 0] = fmaf(dl, dl, ls2[LN ? h : 0]);
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < KL; ++q)
 #pragma unroll
             for (int h = 0; h < TM; ++h)
 #pragma unroll
                 for (int g = 0; g < TN; ++g)
-                    acc[h][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][g][q],
-                                                                            acc[h][g][q & 1], 0, 0, 0);
+                    acc[h][g][q % AC] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][g][q],
+                                                                             acc[h][g][q % AC], 0, 0, 0);
     };
     int pf = 0, it = 0;
     bool left = false;
@@ -2502,6 +2568,23 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
             if (it + s < nsteps) mma_stage(s);
     }
 
+    float* sums = smem + 4 * TD::SUBS * TD::PART + 4;      // LN: [wavefront][row][2], then the pivots [row]
+    if (LN) {
+#pragma unroll
+        for (int h = 0; h < TM; ++h) {
+            float t1 = ls1[LN ? h : 0], t2 = ls2[LN ? h : 0];
+            t1 += __shfl_xor(t1, 16, 64);
+            t2 += __shfl_xor(t2, 16, 64);
+            t1 += __shfl_xor(t1, 32, 64);
+            t2 += __shfl_xor(t2, 32, 64);
+            if (kq == 0) {
+                const int r = 16 * h + i16;
+                sums[(wave * TD::BM + r) * 2] = t1;
+                sums[(wave * TD::BM + r) * 2 + 1] = t2;
+                if (wave == 0) sums[4 * TD::BM * 2 + r] = pivot[LN ? h : 0];
+            }
+        }
+    }
     float* part = smem + wave * (TD::SUBS * TD::PART);
 #pragma unroll
     for (int h = 0; h < TM; ++h)
@@ -2509,14 +2592,32 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
         for (int g = 0; g < TN; ++g)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = acc[h][g][0][j] + acc[h][g][1][j];
+                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = AC == 2 ? acc[h][g][0][j] + acc[h][g][AC - 1][j] : acc[h][g][0][j];
     __syncthreads();
     if (Poll::enabled && *sflag) return false;
     const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
     constexpr int WSTRIDE = TD::SUBS * TD::PART;
     const float alpha = __int_as_float(a[REEF_GEMM_ALPHA_BITS]);
     const int act = a[REEF_GEMM_ACT];
+    auto row_stats = [&](int r, float& mu, float& rs) {
+        float t1 = 0.0f, t2 = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            t1 += sums[(w * TD::BM + r) * 2];
+            t2 += sums[(w * TD::BM + r) * 2 + 1];
+        }
+        const float m1 = t1 / (float)K;                    // mean of a - pivot
+        mu = sums[4 * TD::BM * 2 + r] + m1;
+        rs = 1.0f / sqrtf(fmaxf(t2 / (float)K - m1 * m1, 0.0f) + __int_as_float(a[REEF_GEMM_LN_EPS_BITS]));
+    };
+    float e_mu[LN ? TM : 1], e_rs[LN ? TM : 1];
+    if (LN) {
+#pragma unroll
+        for (int h = 0; h < TM; ++h) row_stats(16 * h + orow, e_mu[LN ? h : 0], e_rs[LN ? h : 0]);
+        ln_out.write(row_stats);
+    }
     auto finish = [&](float sum, int h, int g) {
+        if (LN) sum = e_rs[LN ? h : 0] * (sum - e_mu[LN ? h : 0] * e_c1[LN ? g : 0]) + e_c2[LN ? g : 0];
         float v = sum * alpha + e_bias[g];
         if (act == REEF_ACT_RELU) v = fmaxf(v, 0.0f);
         else if (act == REEF_ACT_GELU) v = gelu_erf(v);
@@ -2616,6 +2717,172 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int tas
     if (threadIdx.x == 0)  // ready for the next run
         __hip_atomic_store(&counters[rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
+}
+
+// ---- reef_attention_m16: softmax(alpha Q K^T (masked)) V of all heads in one launch, on the matrix cores ----
+// For sequences of up to REEF_AT_MM_MAX_SEQ.  A workgroup takes 16 query rows of one head.
+//   scores   the wavefronts take the key tiles (16 keys) in turn; Q and K come straight from memory into
+//            16x16x4 MFMAs, k slot kq holding elements 16 u + 4 kq .. + 3 of the head (a load of a wavefront
+//            reads 64 consecutive bytes of every row); the scores of the 16
+//            rows go to LDS (row stride 4 mod 64 floats: the four k slots' rows lie in different banks).
+//   softmax  16 threads a row; what stays in LDS is exp(s - max), its sum divides the result at the end.
+//   context  a wavefront forms 16 columns of the head for all rows: A = four probabilities per lane and
+//            128-bit LDS read, B = values straight from memory (64-byte pieces of their rows), the next 64
+//            keys' values on their way while these multiply, the first before the scores are formed.
+// Bound by latency (Q, K, V of a layer are in L2): 384 tokens, 12 heads of 64: 16.4 us against 14.5 + 6.3 + 9.4
+// for scores, softmax and context as launches of their own around two [12][384][384] tensors.
+template <int NT>
+__device__ __forceinline__ void attention_scores(rsrc_t rk, const f32x4 (&q)[4], const unsigned (&koff)[4], int ld, int S, int kq, int i16,
+                                                 int wave, int tiles, float alpha, const unsigned char* mask, float* P, int SP) {
+    // NT: 128-bit loads per k slot (HD <= 16 NT)
+    // two pairs of tiles: one is loaded while the other is multiplied
+    f32x4 kb[2][2][NT];
+    auto load = [&](f32x4 (&r)[2][NT], int tile) {
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const unsigned row = (unsigned)((tile + 4 * v) * 16) * (unsigned)ld * 4u;     // uniform
+#pragma unroll
+            for (int u = 0; u < NT; ++u) r[v][u] = buf_load4(rk, koff[u] + row);
+        }
+    };
+    auto multiply = [&](const f32x4 (&r)[2][NT], int tile) {
+        f32x4 acc[2][2];
+#pragma unroll
+        for (int v = 0; v < 2; ++v) acc[v][0] = acc[v][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int v = 0; v < 2; ++v) acc[v][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[u][e], r[v][u][e], acc[v][e & 1], 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            if (tile + 4 * v < tiles) {
+                const int key = (tile + 4 * v) * 16 + i16;
+                const bool in = key < S && !(mask && mask[key]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) P[(4 * kq + j) * SP + key] = in ? (acc[v][0][j] + acc[v][1][j]) * alpha : -INFINITY;
+            }
+        }
+    };
+    load(kb[0], wave);
+    for (int tile = wave; tile < tiles; tile += 16) {
+        if (tile + 8 < tiles) load(kb[1], tile + 8);
+        multiply(kb[0], tile);
+        if (tile + 8 < tiles) {
+            if (tile + 16 < tiles) load(kb[0], tile + 16);
+            multiply(kb[1], tile + 8);
+        }
+    }
+}
+
+__device__ __forceinline__ void attention_mma_body(const ReefOpDesc& d, int task, char* smem_raw) {
+    constexpr int ROWS = REEF_AT_MM_ROWS;
+    const int* a = d.attr;
+    const int S = a[REEF_AT_SEQ], HD = a[REEF_AT_HEAD_DIM], heads = a[REEF_AT_HEADS];
+    const int ld = a[REEF_AT_LD], ldo = a[REEF_AT_LDO];
+    const int row_blocks = (S + ROWS - 1) / ROWS;
+    task = xcd_chunked(task, heads * row_blocks);     // the row blocks of a head share keys and values
+    const int h = div_small(task, row_blocks);
+    const int m0 = (task - h * row_blocks) * ROWS;
+    const float alpha = __int_as_float(a[REEF_AT_ALPHA_BITS]);
+    const unsigned char* mask = (a[REEF_AT_FLAGS] & 1) ? (const unsigned char*)d.ptr[2] : nullptr;
+    // the head's columns of Q, K and V as buffers that end with row S - 1: later rows are outside by themselves
+    const unsigned bytes = (unsigned)((S - 1) * ld + HD) * 4u;
+    const float* base = (const float*)d.ptr[0] + h * HD;
+    const rsrc_t rq = make_rsrc(base + a[REEF_AT_OFF_Q], bytes), rk = make_rsrc(base + a[REEF_AT_OFF_K], bytes),
+                 rv = make_rsrc(base + a[REEF_AT_OFF_V], bytes);
+    const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int chunks = (S + 63) / 64, tiles = chunks * 4;     // keys in whole chunks of 64: those past S are -inf, their values 0
+    const int SP = chunks * 64 + 4;
+    float* P = (float*)smem_raw;                              // [16][SP]
+    float* inv = P + ROWS * SP;                               // [16]
+
+    const int nt = (HD + 15) / 16;
+    f32x4 q[4];
+    unsigned koff[4];         // this lane's pieces of a row of its tile (offsets that are added, not selected: no branch per load)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const unsigned k = (unsigned)(16 * u + 4 * kq);
+        koff[u] = ((unsigned)i16 * (unsigned)ld + k) * 4u + (k < (unsigned)HD ? 0u : kOutside);
+        q[u] = buf_load4(rq, koff[u] + (unsigned)m0 * (unsigned)ld * 4u);
+    }
+    const int col = wave * 16 + i16;                          // column of the head this lane forms
+    float vb[2][16];                                          // two chunks: one is loaded while the other is multiplied
+    const unsigned voff = ((unsigned)(kq * 4) * (unsigned)ld + (unsigned)col) * 4u + (col < HD ? 0u : kOutside);
+    auto load_v = [&](float (&v)[16], int chunk) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) v[g * 4 + t] = buf_load(rv, voff + (unsigned)((chunk * 64 + g * 16 + t) * ld) * 4u);
+    };
+    load_v(vb[0], 0);
+    load_v(vb[1], 1);
+
+    if (nt == 4) attention_scores<4>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
+    else if (nt == 3) attention_scores<3>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
+    else if (nt == 2) attention_scores<2>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
+    else attention_scores<1>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
+    __syncthreads();
+
+    {
+        // a thread's columns: four of every chunk, all of them in registers
+        constexpr int MAXC = REEF_AT_MM_MAX_SEQ / 64;
+        float* row = P + (threadIdx.x >> 4) * SP + (threadIdx.x & 15) * 4;
+        f32x4 x[MAXC];
+        float m = -FLT_MAX;
+#pragma unroll
+        for (int c = 0; c < MAXC; ++c)
+            if (c < chunks) {
+                x[c] = *(const f32x4*)(row + c * 64);
+                m = fmaxf(m, fmaxf(fmaxf(x[c][0], x[c][1]), fmaxf(x[c][2], x[c][3])));
+            }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 16));
+        float sum = 0.0f;
+#pragma unroll
+        for (int c = 0; c < MAXC; ++c)
+            if (c < chunks) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x[c][e] = expf(x[c][e] - m);              // -inf - m -> 0 for masked and missing columns
+                    sum += x[c][e];
+                }
+                *(f32x4*)(row + c * 64) = x[c];
+            }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 16);
+        if ((threadIdx.x & 15) == 0) inv[threadIdx.x >> 4] = 1.0f / sum;
+    }
+    __syncthreads();
+
+    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    const float* pr = P + i16 * SP + kq * 4;
+    auto multiply_v = [&](const float (&v)[16], int c) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const f32x4 p = *(const f32x4*)(pr + c * 64 + g * 16);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], v[g * 4 + t], acc[t & 1], 0, 0, 0);
+        }
+    };
+    for (int c = 0; c < chunks; c += 2) {
+        multiply_v(vb[0], c);
+        if (c + 2 < chunks) load_v(vb[0], c + 2);
+        if (c + 1 < chunks) {
+            multiply_v(vb[1], c + 1);
+            if (c + 3 < chunks) load_v(vb[1], c + 3);
+        }
+    }
+    if (col < HD) {
+        float* out = (float*)d.ptr[1] + h * HD + col;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = 4 * kq + j;
+            if (m0 + r < S) out[(size_t)(m0 + r) * ldo] = (acc[0][j] + acc[1][j]) * inv[r];
+        }
+    }
 }
 
 }  // namespace reef_dev

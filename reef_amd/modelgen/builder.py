@@ -586,24 +586,31 @@ class GraphBuilder:
         return out
 
     ATTENTION_MAX_SEQ, ATTENTION_MAX_HEAD_DIM, ATTENTION_ROWS = 128, 64, 8    # REEF_AT_* of include/reef_kernels.h
+    ATTENTION_MMA_MAX_SEQ, ATTENTION_MMA_ROWS = 512, 16
+    ATTENTION_MMA_FROM = 12      # workgroups from which the matrix cores' form is taken; fewer: twice as many of eight rows
 
     @classmethod
     def attention_ok(cls, seq, head_dim, ld, ldo, offs):
-        """Whether reef_attention takes this shape (all keys of a head fit a workgroup's LDS)."""
-        return (seq <= cls.ATTENTION_MAX_SEQ and head_dim <= cls.ATTENTION_MAX_HEAD_DIM
+        """Whether an attention kernel takes this shape (the scores of a row block fit a workgroup's LDS)."""
+        return (seq <= cls.ATTENTION_MMA_MAX_SEQ and head_dim <= cls.ATTENTION_MAX_HEAD_DIM
                 and all(v % 4 == 0 for v in (head_dim, ld, ldo) + tuple(offs)))
 
-    def attention(self, qkv, seq, heads, head_dim, ld, off_q, off_k, off_v, alpha, mask=None, out=None, ldo=None):
+    def attention(self, qkv, seq, heads, head_dim, ld, off_q, off_k, off_v, alpha, mask=None, out=None, ldo=None, mma=None):
         """softmax(alpha Q K^T (masked)) V for every head in one launch; Q, K, V are column blocks
         of qkv [seq][ld] (head h at columns off + h * head_dim), the context goes to
-        out [seq][ldo] at columns h * head_dim."""
+        out [seq][ldo] at columns h * head_dim.
+        mma: on the matrix cores (reef_attention_m16; None: from ATTENTION_MMA_FROM workgroups on)."""
+        if mma is None:
+            mma = seq > self.ATTENTION_MAX_SEQ or heads * math.ceil(seq / self.ATTENTION_MMA_ROWS) >= self.ATTENTION_MMA_FROM
+        assert mma or seq <= self.ATTENTION_MAX_SEQ
         ldo = heads * head_dim if ldo is None else ldo
         assert self.attention_ok(seq, head_dim, ld, ldo, (off_q, off_k, off_v))
         out = Tensor(out.idx, (seq, ldo)) if out is not None else self.temp((seq, ldo))
         args = [qkv.idx, out.idx] + ([mask.idx] if mask is not None else [])
         flops = 4 * heads * seq * seq * head_dim
         self.flops += flops
-        self._emit("reef_attention", heads * math.ceil(seq / self.ATTENTION_ROWS), args,
+        self._emit("reef_attention_m16" if mma else "reef_attention",
+                   heads * math.ceil(seq / (self.ATTENTION_MMA_ROWS if mma else self.ATTENTION_ROWS)), args,
                    [seq, head_dim, heads, ld, ldo, off_q, off_k, off_v, float_bits(alpha), 1 if mask is not None else 0],
                    "attention", flops, 4 * (3 * seq * heads * head_dim + seq * ldo), 4.0)
         return out
@@ -629,12 +636,12 @@ class GraphBuilder:
         """C[b] = act(alpha * A[b] x B[b] (+bias)) (+res[b]); operands are storages with explicit strides.
         res: a residual laid out as C is.
         split_k: K split across workgroups and folded inside the launch (direct tiles, batch 1);
-        None = what tiling.choose_gemm finds (1 or 2).
-        force_tile: a staged tile name or, for trans_b, one of tiling.GEMM_DIRECT_TILES.
+        None = what tiling.choose_product finds.
+        force_tile: a staged tile name or, for trans_b, one of tiling.GEMM_DIRECT_TILES or GEMM_WIDE_TILES.
         off_a / off_b / off_c: element at which the first matrix starts inside its storage.
         ln: dict(gamma=, beta=, eps=1e-12, out=None) -- the product behind a LayerNorm of the rows
-        of A; `out`, if given, receives the normalised rows (kernels reef_gemm_ntl_<tile>: staged
-        tiles, one K-contiguous B).  b, gamma and beta must be parameters: the kernel works from
+        of A; `out`, if given, receives the normalised rows (kernels reef_gemm_ntl_<tile> of
+        LN_GEMM_TILES, one K-contiguous B).  b, gamma and beta must be parameters: the kernel works from
         b scaled by gamma and two vectors derived from them (include/reef_kernels.h)."""
         lda = K if lda is None else lda
         ldb = (K if trans_b else N) if ldb is None else ldb
@@ -646,15 +653,12 @@ class GraphBuilder:
                      and stride_b % 4 == 0)
         if ln is not None:
             assert trans_b and batch == 1 and off_a == 0, "the LayerNorm form: one K-contiguous B, A without offset"
-            direct_ok = False
-            if force_tile is None:
-                force_tile = self.LN_GEMM_TILE
-            assert force_tile in self.LN_GEMM_TILES, "no LayerNorm form of this tile"
+            assert force_tile is None or force_tile in self.LN_GEMM_TILES, "no LayerNorm form of this tile"
         if force_tile is not None:
             t = tiling.forced(force_tile, M, N, K, 1)
         else:
-            t = tiling.choose_gemm(M, N, K, batch, direct_ok, under_load=self.under_load)
-        direct = t["tile"] in tiling.GEMM_DIRECT_TILES
+            t = tiling.choose_product(M, N, K, batch, direct_ok, under_load=self.under_load, ln=ln is not None)
+        direct = t["tile"] in tiling.GEMM_DIRECT_TILES or t["tile"] in tiling.GEMM_WIDE_TILES
         assert direct_ok or not direct, "this GEMM has no direct form"
         args = [a.idx, b.idx, out.idx]
         if ln is not None:
@@ -712,8 +716,8 @@ class GraphBuilder:
                    "gemm", flops, 4 * batch * (M * K + N * K + M * N), t["est_us"])
         return out
 
-    LN_GEMM_TILES = ("32x32k4", "64x32k2")     # tiles that exist as reef_gemm_ntl_<tile>
-    LN_GEMM_TILE = "32x32k4"
+    # tiles that exist as reef_gemm_ntl_<tile>
+    LN_GEMM_TILES = ("32x32k4", "64x32k2", "16x16k4", "16x32k4", "32x48d4", "48x48d4", "64x64d4")
 
     def mocked(self, name, a, b, out):
         self._emit(name, 64, [a.idx, b.idx, out.idx], [], "mocked", 0, 3 * 8192 * 4, 14.0,
@@ -745,7 +749,12 @@ class GraphBuilder:
             elif sym.startswith("reef_conv2d_") or sym.startswith("reef_gemm_"):
                 shared[n] = tiling.lds_bytes(sym.split("_")[-1])
                 if sym.startswith("reef_gemm_ntl_"):
-                    shared[n] += 2 * tiling.TILES[sym.split("_")[-1]][1] * 4    # mean, 1/std of the tile's rows
+                    # mean, 1/std of the tile's rows; direct tiles: the rows' sums per wavefront and their pivots
+                    t = sym.split("_")[-1]
+                    if t in tiling.GEMM_WIDE_TILES or t in tiling.DIRECT_TILES:
+                        shared[n] += 9 * 4 * (tiling.GEMM_WIDE_TILES[t] if t in tiling.GEMM_WIDE_TILES else tiling.TILES[t])[1]
+                    else:
+                        shared[n] += 2 * tiling.TILES[t][1] * 4
             else:
                 shared[n] = 4   # the reference's floor (generate_final_schedule.py:117-143)
         return {"storage": self.storage, "kernels": self.kernels, "args": self.graph_args,

@@ -38,6 +38,8 @@ TILES = {
     "g2m2": (17, 32, 32, 0.40, 2),
     "g4m2": (18, 32, 64, 0.40, 2),
 }
+# matrix products only (reef_gemm_ntd_<tile>, reef_gemm_ntl_<tile>): name -> (id, BM, BN)
+GEMM_WIDE_TILES = {"32x48d4": (19, 32, 48), "48x48d4": (20, 48, 48), "64x64d4": (21, 64, 64)}
 # row form: image rows per tile
 ROW_TILES = {"g1": 1, "g2": 2, "g4": 4, "g7": 7, "g2m2": 2, "g4m2": 4}
 ROW_SEG = 14
@@ -91,6 +93,54 @@ def choose_gemm(M, N, K, batch=1, direct_ok=False, under_load=False):
     return t
 
 
+# Microseconds of a product (tile, reads its rows through a LayerNorm), fitted as CONV_COST is, in the form
+# of _cost with whole rounds of workgroups: 16 sequence lengths of 8 to 512 times 13 layer shapes of 256 to 4096 columns and
+# a depth of 256 to 4096, splits of 1 to 6, 3100 launches on MI355X; it picks within 0.3 % of the fastest
+# launch on average (worst 7 %).  Without the three wide direct tiles it would lose 4 to 5 %.
+GEMM_COST = {
+    ("16x16k4", False): (2.534, 0.3324, 2.843, 0.4488, 0.2743, 1.799, 1.127),
+    ("16x16k4", True): (3.635, 0.17, 3.258, 0.04108, 0.4272, 0, 0),
+    ("16x32k4", False): (2.691, 0.6074, 4.59, 0.2421, 0.4406, 1.636, 2.151),
+    ("16x32k4", True): (3.518, 1.365, 4.748, 0, 0.5508, 0, 0),
+    ("32x32d4", False): (2.801, 0, 5.975, 1.091, 1.507, 1.92, 1.86),
+    ("32x48d4", False): (3.211, 0.1859, 8.06, 0.3396, 1.479, 2.465, 2.754),
+    ("32x48d4", True): (4.578, 0.2621, 8.58, 0, 1.171, 0, 0),
+    ("48x48d4", False): (3.424, 0.6952, 9.742, 0, 2.909, 2.943, 2.692),
+    ("48x48d4", True): (5.234, 0, 11.05, 0, 1.908, 0, 0),
+    ("64x64d4", False): (4.323, 0, 15.27, 0, 6.721, 2.321, 5.733),
+    ("64x64d4", True): (6.322, 0, 18.41, 0, 2.093, 0, 0),
+    ("32x32k4", False): (3.647, 2.504, 3.621, 0.3601, 0.5328, 0, 0),
+    ("32x32k4", True): (5.233, 0.809, 4.395, 2.123, 0.502, 0, 0),
+    ("64x32k2", False): (4.431, 12.06, 0, 0, 0.5025, 0, 0),
+    ("64x32k2", True): (5.956, 3.589, 7.457, 1.34, 0.4235, 0, 0),
+}
+GEMM_COST_MIN, GEMM_COST_MAX_OUT = 256, 512 * 4096     # columns and depth from which, outputs up to which it was measured
+
+
+def choose_product(M, N, K, batch=1, direct_ok=False, under_load=False, ln=False):
+    """Tile (and split of K, gemm_split) of a matrix product: inside the measured range by GEMM_COST, outside
+    it by choose_gemm (behind a LayerNorm: the staged 32x32k4, which takes every shape).
+    under_load: as in choose_gemm."""
+    if under_load and direct_ok and not ln and batch == 1 and (M, N, K) in GEMM_UNDER_LOAD:
+        return choose_gemm(M, N, K, batch, direct_ok, under_load)
+    if batch == 1 and direct_ok and min(N, K) >= GEMM_COST_MIN and M * N <= GEMM_COST_MAX_OUT:
+        best = None
+        for (tile, through_ln), c in GEMM_COST.items():
+            if through_ln != ln:
+                continue
+            staged = tile not in DIRECT_TILES and tile not in GEMM_WIDE_TILES
+            for s in (1,) if ln or staged else (1, 2, 3, 4, 6):
+                t = forced(tile, M, N, K, s)
+                if t["split_k"] == s:
+                    us = _cost(c, t["k_chunk"] if s > 1 else K, t["tasks"], s, math.ceil(t["tasks"] / NUM_CUS))
+                    if best is None or us < best[0]:
+                        best = (us, dict(t, gemm_split=s, est_us=us))
+        return best[1]
+    if ln:
+        return forced("32x32k4", M, N, K, 1)
+    return choose_gemm(M, N, K, batch, direct_ok, under_load)
+
+
 GEMM_PAIR_FOLD_LINES = 900.0    # what a split of two costs, in the cost rule's cache lines
 GEMM_STAGED_BONUS = 1.0
 
@@ -99,7 +149,7 @@ def step_k(tile, taps=1):
     """Granularity of a split's share of K (taps = kh*kw, direct family only: 16 channels of a
     filter with taps > 1, one K step; 128 channels of a 1x1 filter, two of its 64-channel steps --
     rounding to 64 instead was measured on DenseNet-201 and changes nothing)."""
-    if tile in DIRECT_TILES:
+    if tile in DIRECT_TILES or tile in GEMM_WIDE_TILES:
         return 128 if taps == 1 else 16 * taps
     return BK * KW.get(tile, 1)
 
@@ -133,7 +183,7 @@ def forced_rows(tile, M, H, W, K, split=1):
 def forced(tile, M, N, K, split=1, taps=1):
     """The launch geometry of a given tile and split-K factor (no cost model)."""
     assert tile not in ROW_TILES, "row-form tiles take the image shape: forced_rows"
-    tid, bm, bn, _, _ = TILES[tile]
+    tid, bm, bn = GEMM_WIDE_TILES[tile] if tile in GEMM_WIDE_TILES else TILES[tile][:3]
     bk = step_k(tile, taps)
     k_chunk = math.ceil(math.ceil(K / split) / bk) * bk
     s = math.ceil(K / k_chunk)
@@ -293,13 +343,17 @@ def conv_kind(tile, taps, stride=1, pointwise=True):
 
 def direct_cost(tile, geom, fused=True, kind="1"):
     """Microseconds of a launch of this geometry (forced, forced_rows) by CONV_COST."""
-    c = CONV_COST[(tile, kind)]
     s = geom["split_k"]
-    w, r = geom["k_chunk"] / 1000.0, geom["tasks"] / NUM_CUS
-    t = c[0] + (c[1] + c[2] * (r + math.ceil(r)) / 2 + c[3] * max(1.0, r)) * w + c[4] * r
-    if s > 1:
-        t += c[5] + 0.1 * c[6] * s + (0.0 if fused else T_REDUCE_LAUNCH)
-    return t
+    r = geom["tasks"] / NUM_CUS
+    us = _cost(CONV_COST[(tile, kind)], geom["k_chunk"], geom["tasks"], s, (r + math.ceil(r)) / 2)
+    return us + T_REDUCE_LAUNCH if s > 1 and not fused else us
+
+
+def _cost(c, depth, tasks, split, rounds):
+    """The fitted form of CONV_COST and GEMM_COST: `tasks` workgroups over `depth` values of K each."""
+    w, r = depth / 1000.0, tasks / NUM_CUS
+    t = c[0] + (c[1] + c[2] * rounds + c[3] * max(1.0, r)) * w + c[4] * r
+    return t + c[5] + 0.1 * c[6] * split if split > 1 else t
 
 
 def _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act):
@@ -331,6 +385,8 @@ def _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act)
 
 
 def lds_bytes(tile):
+    if tile in GEMM_WIDE_TILES:
+        return 4 * (GEMM_WIDE_TILES[tile][1] // 16) * (GEMM_WIDE_TILES[tile][2] // 16) * 320 * 4 + 16
     if tile in DIRECT_TILES or tile in ROW_TILES:
         # four wavefronts x (BM/16)(BN/16) partial 16x16 tiles (skewed rows) + leave / last-arrival flags
         return 4 * (TILES[tile][1] // 16) * (TILES[tile][2] // 16) * 320 * 4 + 16
