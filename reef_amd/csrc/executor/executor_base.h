@@ -8,6 +8,7 @@
 // ReefOpDesc by value: storage pointers in JSON `args` order plus the JSON
 // `attrs` integers (include/reef_kernels.h).
 #pragma once
+#include <algorithm>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -106,7 +107,9 @@ protected:
     void drop_pass(Pass& p);
 public:
     // Called in front of every launch of a kernel of this model that is no part of a pass.
-    Status leave_passes();
+    Status leave_passes(GPUStream_t stream);
+    // Called by whoever has waited for `stream`: what it was given of this model has run.
+    void launches_done(GPUStream_t stream);
     // Called when a run is asked for: what set_input has stored is there for whatever launches follow.
     Status inputs_ready();
 protected:
@@ -130,9 +133,16 @@ protected:
     // State of the storages (io_mtx: a client fetches results while the scheduler's thread runs the model).
     // after_pass: the last thing that ran on them was a pass (which has finished); host_wrote: the host has stored
     // into them past the caches; current: the mirror that is equal to them, or null.
+    // A launch outside a pass returns before it has run, and only who has waited for its stream knows when it has:
+    // busy holds the streams that may still run some.  While there are any, or a pass runs (passes_running), what a fetch
+    // copies is good for that fetch only.  inputs_set counts set_input.
     std::mutex io_mtx;
     bool after_pass = false, host_wrote = false;
     const Mirror* current = nullptr;
+    std::vector<GPUStream_t> busy;
+    int passes_running = 0;
+    size_t inputs_set = 0;
+    bool at_rest() const { return busy.empty() && passes_running == 0; }
     Mirror fetched;                    // of the last fetch that was no pass's
     GPUDevicePtr_t fetch_mem = nullptr;   // pinned
     size_t fetch_bytes = 0;
@@ -161,11 +171,18 @@ Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, boo
     const int fresh = host_wrote || !after_pass;
     after_pass = host_wrote = false;
     runs++;
+    passes_running++;
+    const size_t inputs_before = inputs_set;
     lock.unlock();
-    GPU_RETURN_STATUS(reef_hal_pass_run(p.handle, stream, fresh));
+    const int rc = reef_hal_pass_run(p.handle, stream, fresh);
     lock.lock();
+    passes_running--;
+    current = nullptr;
+    GPU_RETURN_STATUS(rc);
+    busy.erase(std::remove(busy.begin(), busy.end(), stream), busy.end());   // the pass has waited for it
     after_pass = true;
-    current = &p.mirror;
+    // (an input stored meanwhile may be one of what is mirrored)
+    if (at_rest() && inputs_set == inputs_before) current = &p.mirror;
     return Status::Succ;
 }
 

@@ -117,6 +117,7 @@ Status HybridExecutor::execute_preemptale(GPUStream_t stream) {
         if (ret != Status::Succ) return ret;
     }
     GPU_RETURN_STATUS(reef_hal_stream_sync(stream));
+    launches_done(stream);
     return Status::Succ;
 }
 
@@ -195,7 +196,7 @@ size_t HybridExecutor::add_prefetch(Launch& l, uint32_t wgs) const {
 }
 
 Status HybridExecutor::launch_preempt_kernel(int i, GPUStream_t stream) {
-    RETURN_STATUS(leave_passes());
+    RETURN_STATUS(leave_passes(stream));
     Launch l;
     RETURN_STATUS(make_preempt_launch(i, l));
     GPU_RETURN_STATUS(reef_hal_launch(l.fn, l.grid, l.block, 0, stream, l.args, l.bytes));

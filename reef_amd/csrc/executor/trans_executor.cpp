@@ -114,7 +114,7 @@ size_t TransExecutor::add_prefetch(Launch& l, uint32_t wgs) const {
 // (the right side of a partition with nothing on the left), so `layers` workgroups really share
 // each of those CUs.
 Status TransExecutor::launch_kernel_dkp(int i, int layers, int task_num, GPUStream_t stream, int cus) {
-    RETURN_STATUS(leave_passes());
+    RETURN_STATUS(leave_passes(stream));
     const KernelArg& ka = trans_args[i];
     const int num_cus = (int)GPUConfig::get_num_cus();
     const int num_xcds = (int)GPUConfig::get_num_xcds();

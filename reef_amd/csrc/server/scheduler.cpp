@@ -539,7 +539,6 @@ void REEFScheduler::execute_rt_task(std::shared_ptr<Task>& task) {
     if (be_waiting) {
         // something to pad with: one launch per kernel, each with its own decision
         dynamic_kernel_padding(task);
-        reef_hal_stream_sync(rt_queue->stream);
     } else {
         task->model->executor.execute(rt_queue->stream);
     }
@@ -614,11 +613,12 @@ void REEFScheduler::dynamic_kernel_padding(std::shared_ptr<Task>& rt_task) {
     const int num_cus = (int)GPUConfig::get_num_cus();
     const int num_xcds = (int)GPUConfig::get_num_xcds();
     std::vector<std::shared_ptr<Task>> complete_be_tasks;
+    std::vector<std::shared_ptr<Model>> padded_models;
     TimePoint current_time_point = Clock::now();
     const std::vector<TransExecutor::Proxy>& proxies = rt_exe.proxies();
 
     const int n_rt = (int)rt_exe.num_kernels();
-    rt_exe.leave_passes();
+    rt_exe.leave_passes(rt_queue->stream);
     for (int i = 0; i < n_rt; i++) {
         const auto sel_start = std::chrono::steady_clock::now();
         const TransExecutor::KernelArg& rt_args = rt_exe.trans_args[i];
@@ -690,7 +690,8 @@ void REEFScheduler::dynamic_kernel_padding(std::shared_ptr<Task>& rt_task) {
             a.entry_l = (const void*)(uintptr_t)rt_args.entry;
             a.entry_r = (const void*)(uintptr_t)be_args->entry;
             if (be_task->start.time_since_epoch().count() == 0) be_task->start = current_time_point;
-            be_exe.leave_passes();
+            be_exe.leave_passes(rt_queue->stream);
+            if (padded_models.empty() || padded_models.back() != be_task->model) padded_models.push_back(be_task->model);
             executor::GPUFunction_t proxy = rt_exe.get_proxy_kernel(proxy_idx);
             const uint32_t grid[3] = {(uint32_t)(dec.final_occupancy * num_cus), 1, 1};
             const uint32_t block[3] = {(uint32_t)dec.merged_block_size, 1, 1};
@@ -722,9 +723,15 @@ void REEFScheduler::dynamic_kernel_padding(std::shared_ptr<Task>& rt_task) {
     }
     // Tasks that finished inside real-time shadows are reported once the
     // real-time stream has drained (their last workgroups run on it).
-    if (!complete_be_tasks.empty()) {
-        reef_hal_stream_sync(rt_queue->stream);
-        for (auto& t : complete_be_tasks) finish_task(t, t->end);
+    if (reef_hal_stream_sync(rt_queue->stream) != 0) REEF_LOG_ERROR("real-time stream: %s", reef_hal_last_error());
+    rt_exe.launches_done(rt_queue->stream);
+    for (auto& m : padded_models) m->executor.launches_done(rt_queue->stream);
+    for (auto& t : complete_be_tasks) {
+        // what the task left on its own stream when it was preempted may still be leaving
+        int drained = 0;
+        const executor::GPUStream_t own = be_queues[t->qid]->stream;
+        if (reef_hal_stream_drained(own, &drained) == 0 && drained) t->model->executor.launches_done(own);
+        finish_task(t, t->end);
     }
 }
 
@@ -738,6 +745,7 @@ void REEFScheduler::execute_be_task(std::shared_ptr<Task>& task, std::shared_ptr
             if (executor::GPUStreamEmpty(tqueue->stream)) {
                 task->kernel_offset = 0;
                 task->block_offset = 0;
+                task->model->executor.launches_done(tqueue->stream);
                 finish_task(task, Clock::now());
             }
             return;
@@ -755,6 +763,7 @@ void REEFScheduler::execute_be_task(std::shared_ptr<Task>& task, std::shared_ptr
             if (task->kernel_offset >= num_kernels) {
                 task->kernel_offset = 0;
                 task->block_offset = 0;
+                task->model->executor.launches_done(tqueue->stream);
                 finish_task(task, Clock::now());
                 return;
             }

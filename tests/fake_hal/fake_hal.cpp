@@ -9,6 +9,12 @@
 // Launch-window semantics match the HIP backend: at most `window` kernels of a
 // windowed stream are in flight, the rest wait in a host-side queue that
 // stream_clear_queue drops.
+//
+// Recorded passes, stores past the caches and fetches are there when a test asks for them
+// (fake_hal_set_passes).  A pass runs whole inside pass_run; a fetch copies at once, whatever is in
+// flight, as the device's does.  What others than kernels have stored into device memory (copies, fills,
+// host_write, a pass's argument blocks) counts as not yet seen by packets until a launch through the
+// runtime, a fence or a fresh pass drops the caches; packets that run before that are counted.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -43,6 +49,13 @@ struct reef_stream_s {
 };
 struct reef_event_s { int dummy; };
 struct reef_graph_s { std::vector<Op> ops; };
+struct reef_pass_s {
+    struct Launch { Op op; size_t at, tail; };
+    std::vector<Launch> launches;
+    std::vector<char> host, device;   // argument blocks: as the caller fills them, as they were committed
+    std::vector<reef_pass_range> ranges;
+    std::vector<char> mirror;
+};
 
 namespace {
 
@@ -65,6 +78,9 @@ long g_launches = 0, g_completed = 0, g_dropped = 0;
 struct LogEntry { std::string symbol; int stream; uint32_t grid, block, lds; };
 std::vector<LogEntry> g_log;
 int g_auto_progress = 1;  // kernels completed per stream_query
+bool g_passes = false, g_unseen = false;
+long g_pass_creates = 0, g_pass_runs = 0, g_fetches = 0, g_stale = 0, g_mallocs = 0, g_frees = 0;
+void (*g_pass_hook)(int) = nullptr;   // called with 0 in the middle of every pass and with 1 at its end
 
 reef_stream_s* S(reef_stream_t s) { return s ? s : &g_null_stream; }
 
@@ -159,6 +175,7 @@ int f_function_resource(reef_function_t f, reef_kernel_resource* out) {
 std::map<char*, size_t> g_allocs;
 int f_malloc(size_t bytes, int, reef_devptr_t* out) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    ++g_mallocs;
     if (!bytes) bytes = 4;
     *out = std::calloc(1, bytes);
     if (!*out) return 1;
@@ -167,12 +184,13 @@ int f_malloc(size_t bytes, int, reef_devptr_t* out) {
 }
 int f_free(reef_devptr_t p, int) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    ++g_frees;
     g_allocs.erase((char*)p);
     std::free(p);
     return 0;
 }
-int f_memset(reef_devptr_t p, int b, size_t n) { std::memset(p, b, n); return 0; }
-int f_h2d(reef_devptr_t d, const void* s, size_t n) { std::memcpy(d, s, n); return 0; }
+int f_memset(reef_devptr_t p, int b, size_t n) { std::memset(p, b, n); g_unseen = true; return 0; }
+int f_h2d(reef_devptr_t d, const void* s, size_t n) { std::memcpy(d, s, n); g_unseen = true; return 0; }
 int f_d2h(void* d, reef_devptr_t s, size_t n) { std::memcpy(d, s, n); return 0; }
 int f_copy_async(void* d, const void* s, size_t n, reef_stream_t st) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
@@ -227,6 +245,7 @@ int f_launch(reef_function_t f, const uint32_t* g, const uint32_t* b, uint32_t l
         return 0;
     }
     ++g_launches;
+    g_unseen = false;
     g_log.push_back(LogEntry{f->name, S(st)->id, g[0] * g[1] * g[2], b[0] * b[1] * b[2], lds});
     enqueue(S(st), std::move(op));
     return 0;
@@ -300,6 +319,99 @@ int f_graph_launch(reef_graph_t g, reef_stream_t st) {
     return 0;
 }
 int f_graph_destroy(reef_graph_t g) { delete g; return 0; }
+// ---- recorded passes
+int f_pass_create(const reef_pass_launch* l, size_t n, size_t tail, reef_pass_t* out) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    if (!g_passes) return 2;
+    ++g_pass_creates;
+    reef_pass_s* p = new reef_pass_s;
+    for (size_t i = 0; i < n; ++i) {
+        Op op{};
+        op.fn = l[i].fn;
+        op.lds = l[i].dyn_lds;
+        std::memcpy(op.grid, l[i].grid, sizeof(op.grid));
+        std::memcpy(op.block, l[i].block, sizeof(op.block));
+        op.bytes = l[i].kernarg_bytes;
+        const size_t at = p->host.size(), args = (l[i].kernarg_bytes + 15) / 16 * 16;
+        p->host.resize(at + (args + tail + 63) / 64 * 64);
+        std::memcpy(p->host.data() + at, l[i].kernarg, l[i].kernarg_bytes);
+        p->launches.push_back({op, at, args});
+    }
+    p->device.resize(p->host.size());
+    *out = p;
+    return 0;
+}
+int f_pass_block(reef_pass_t p, size_t i, reef_pass_block* out) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    if (i >= p->launches.size()) return 1;
+    const size_t at = p->launches[i].at, end = i + 1 < p->launches.size() ? p->launches[i + 1].at : p->host.size();
+    *out = reef_pass_block{p->device.data() + at, p->host.data() + at, end - at, p->launches[i].tail};
+    return 0;
+}
+int f_pass_commit(reef_pass_t p) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    p->device.assign(p->host.begin(), p->host.end());
+    g_unseen = true;
+    return 0;
+}
+int f_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char** host) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    p->ranges.assign(r, r + n);
+    size_t total = 0;
+    for (size_t i = 0; i < n; ++i) total += (r[i].bytes + 255) / 256 * 256;
+    p->mirror.assign(total, 0);
+    total = 0;
+    for (size_t i = 0; i < n; ++i) {
+        host[i] = p->mirror.data() + total;
+        total += (r[i].bytes + 255) / 256 * 256;
+    }
+    return 0;
+}
+int f_pass_run(reef_pass_t p, reef_stream_t after, int fresh) {
+    std::unique_lock<std::recursive_mutex> lock(g_mtx);
+    drain(S(after));
+    if (fresh) g_unseen = false;
+    if (g_unseen) ++g_stale;
+    ++g_pass_runs;
+    auto call_hook = [&](int where) {
+        if (!g_pass_hook) return;
+        lock.unlock();
+        g_pass_hook(where);
+        lock.lock();
+    };
+    for (size_t i = 0; i < p->launches.size(); ++i) {
+        const Op& o = p->launches[i].op;
+        if (g_cb) g_cb(o.fn->name.c_str(), o.fn->module_path.c_str(), p->device.data() + p->launches[i].at, o.bytes, o.grid,
+                       o.block, o.lds, 0);
+        if (i == 0) call_hook(0);
+    }
+    for (size_t i = 0, at = 0; i < p->ranges.size(); ++i) {
+        std::memcpy(p->mirror.data() + at, p->ranges[i].src, p->ranges[i].bytes);
+        at += (p->ranges[i].bytes + 255) / 256 * 256;
+    }
+    call_hook(1);
+    return 0;
+}
+int f_pass_destroy(reef_pass_t p) { delete p; return 0; }
+int f_host_write(reef_devptr_t d, const void* s, size_t n) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    if (!g_passes) return 2;
+    std::memcpy(d, s, n);
+    g_unseen = true;
+    return 0;
+}
+int f_host_write_fence() { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_unseen = false; return 0; }
+int f_fetch(const reef_pass_range* r, size_t n, void* host) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    if (!g_passes) return 2;
+    ++g_fetches;
+    if (g_unseen) ++g_stale;
+    for (size_t i = 0, at = 0; i < n; ++i) {
+        std::memcpy((char*)host + at, r[i].src, r[i].bytes);
+        at += (r[i].bytes + 255) / 256 * 256;
+    }
+    return 0;
+}
 int f_event_create(reef_event_t* out) { *out = new reef_event_s{0}; return 0; }
 int f_event_destroy(reef_event_t e) { delete e; return 0; }
 int f_event_record(reef_event_t, reef_stream_t) { return 0; }
@@ -313,6 +425,9 @@ const reef_hal_backend kFake = {
     f_write_value32, f_clear_queue, f_reset_cus, f_event_create, f_event_destroy, f_event_record,
     f_event_sync, f_event_elapsed, f_memset_async, f_host_write32, f_stream_wait_device,
     f_graph_begin, f_graph_end, f_graph_launch, f_graph_destroy,
+    nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+    f_pass_create, f_pass_block, f_pass_commit, f_pass_run, f_pass_destroy,
+    f_pass_mirror, f_host_write, f_host_write_fence, f_fetch,
 };
 
 }  // namespace
@@ -341,6 +456,17 @@ void fake_hal_reset(void) {
     g_missing.clear();
     g_info_set = false;
     g_auto_progress = 1;
+    g_passes = g_unseen = false;
+    g_pass_creates = g_pass_runs = g_fetches = g_stale = g_mallocs = g_frees = 0;
+    g_pass_hook = nullptr;
+}
+void fake_hal_set_passes(int on) { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_passes = on != 0; }
+void fake_hal_set_pass_hook(void (*hook)(int)) { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_pass_hook = hook; }
+// pass_create, pass_run, fetch calls; packets that ran before the caches had been dropped; malloc, free calls
+void fake_hal_pass_counts(long out[6]) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    const long v[6] = {g_pass_creates, g_pass_runs, g_fetches, g_stale, g_mallocs, g_frees};
+    std::memcpy(out, v, sizeof(v));
 }
 // Bytes from `p` to the end of the allocation that holds it (0 when unknown).
 size_t fake_hal_extent(const void* p) {

@@ -54,6 +54,8 @@ CB_TYPE = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.c_char_p, ctypes.c_void
                            ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_uint32),
                            ctypes.c_uint32, ctypes.c_int)
 
+HOOK_TYPE = ctypes.CFUNCTYPE(None, ctypes.c_int)
+
 
 class FakeHal:
     def __init__(self):
@@ -106,6 +108,20 @@ class FakeHal:
 
     def set_missing(self, name):
         self.lib.fake_hal_set_missing(name.encode())
+
+    def set_passes(self, on=True):
+        """The backend records passes, stores past the caches and fetches (off after install)."""
+        self.lib.fake_hal_set_passes(int(on))
+
+    def set_pass_hook(self, fn):
+        """`fn(0)` runs in the middle of every pass from now on, `fn(1)` at its end."""
+        self._hook = HOOK_TYPE(fn)
+        self.lib.fake_hal_set_pass_hook(self._hook)
+
+    def pass_counts(self):
+        out = (ctypes.c_long * 6)()
+        self.lib.fake_hal_pass_counts(out)
+        return dict(zip(("creates", "runs", "fetches", "stale", "mallocs", "frees"), out))
 
     def log(self):
         out = []

@@ -1,0 +1,91 @@
+"""What a model keeps between a run and the fetches behind it -- the mirror of the last run, what a fetch has copied --
+on the recording backend with passes switched on: a fetch returns what the storages hold, whenever it comes."""
+import time
+
+import numpy as np
+import pytest
+
+from reef_amd import binding as B
+from reef_amd.modelgen import nets
+from tests.fakehal import FakeHal
+from tests.helpers import write_model
+
+N = 8192
+
+
+@pytest.fixture()
+def fake():
+    f = FakeHal().install()
+    f.set_passes()
+    yield f
+    f.remove()
+
+
+@pytest.fixture(scope="module")
+def mocked(tmp_path_factory):
+    g = nets.mocked_kernel()
+    return g.name, write_model(g, tmp_path_factory.mktemp("mocked"))
+
+
+def set_inputs(set_input, v):
+    for k in "abc":
+        set_input(k, np.full(N, v, np.float32))
+
+
+def wait_for(cond):
+    end = time.time() + 20
+    while not cond():
+        assert time.time() < end
+        time.sleep(0.001)
+
+
+def test_a_fetch_during_a_best_effort_run_leaves_nothing_for_the_one_after_it(fake, mocked):
+    name, d = mocked
+    s = B.Scheduler(B.MODE_REEF)
+    m = s.load_model(d, name)
+    s.bind_model_queue(s.create_queue(B.QUEUE_BE), m)
+    for v in (3.0, 4.0):
+        set_inputs(lambda k, x: s.set_input(m, x, k), v)
+        fake.lib.fake_hal_set_auto_progress(0)             # launched, and nothing ends
+        launched = len(fake.log())
+        t = s.new_task(m)
+        if v == 3.0:
+            s.run()
+        wait_for(lambda: len(fake.log()) == launched + 2)
+        early = s.get_output(m, N)
+        assert not np.array_equal(early, np.full(N, 2 * v * v))
+        fake.lib.fake_hal_set_auto_progress(1)
+        s.wait_task(t)
+        before = fake.pass_counts()["fetches"]
+        for _ in range(3):
+            np.testing.assert_array_equal(s.get_output(m, N), np.full(N, 2 * v * v, np.float32))
+        assert fake.pass_counts()["fetches"] == before + 1     # and of a run that has ended one copy is enough
+    s.shutdown()
+    s.close()
+
+
+@pytest.mark.parametrize("kind,pre", [(B.BASE, False), (B.HYBRID, True)])
+def test_a_fetch_in_the_middle_of_a_pass_and_an_input_behind_its_last_launch(fake, mocked, kind, pre):
+    name, d = mocked
+    exe = B.Executor.from_dir(d, name, kind)
+    run = exe.execute_preemptable if pre else exe.execute
+    c, seen = 3, []                                        # c: index of the storage of that name
+    for _ in range(3):                                     # c joins what a pass mirrors
+        set_inputs(exe.set_input_checked, 3.0)
+        run()
+        np.testing.assert_array_equal(exe.get_data(c, N), np.full(N, 3, np.float32))
+
+    def hook(where):
+        if where == 0:
+            seen.append(exe.get_output())
+        else:
+            exe.set_input_checked("c", np.full(N, 7, np.float32))
+
+    fake.set_pass_hook(hook)
+    set_inputs(exe.set_input_checked, 5.0)
+    run()
+    np.testing.assert_array_equal(seen, np.full((1, N), 18, np.float32))
+    for _ in range(2):
+        np.testing.assert_array_equal(exe.get_output(), np.full(N, 50, np.float32))
+        np.testing.assert_array_equal(exe.get_data(c, N), np.full(N, 7, np.float32))
+    exe.close()
