@@ -227,13 +227,15 @@ int reef_hal_graph_destroy(reef_graph_t g);
  *                memory of the pass's; host[i] is where range i is found after a run.
  *   pass_run:    waits for what `after` (may be NULL: the default stream) has been given, runs the
  *                launches in order and returns when the last has finished.  `fresh`: the caches may hold
- *                what the host or launches outside passes have changed since the last run.
+ *                what the host, copies, fills, pass_commit or launches outside passes have changed since
+ *                the last run.
  *   host_write:  stores into device memory from the host (device memory behind the PCIe window); returns 2
  *                where the backend cannot.  Nothing that reads the memory may be running; a pass run
  *                with `fresh` sees the bytes, and so does any launch after host_write_fence (which does
- *                nothing when no host_write came since the last one).
+ *                nothing when no host_write, memcpy_h2d or memset came since the last one).
  *   fetch:       copies ranges of device memory, one behind the other at multiples of 256 bytes, into
- *                pinned host memory with one launch, and waits for it; what has written them has finished.
+ *                pinned host memory with one launch, and waits for it; the kernels that have written them
+ *                have finished, and a host_write_fence has followed whatever else has.
  *                Returns 2 where the backend cannot. */
 typedef struct reef_pass_s* reef_pass_t;
 typedef struct reef_pass_launch {

@@ -123,10 +123,10 @@ Status ExecutorBase::init_executor_base(const char* json_file_path, GPUModule_t 
 Status ExecutorBase::load_param_from_file(const char* param_file_path) {
     std::unique_ptr<ModelParam> params(ModelParamParser::parse_from_file(param_file_path));
     if (!params) RETURN_STATUS(Status::NotFound);
-    {
-        std::lock_guard<std::mutex> lock(io_mtx);
-        current = nullptr;
-    }
+    std::lock_guard<std::mutex> lock(io_mtx);
+    current = nullptr;
+    inputs_set++;
+    host_wrote = true;
     for (size_t i = 0; i < storage.size(); i++) {
         auto it = params->find(model->storage[i].name);
         if (it == params->end()) continue;
@@ -165,10 +165,8 @@ Status ExecutorBase::set_input(int idx, const void* value, size_t len) {
     // The host stores straight into device memory: 602 KB in 15 us instead of 25 through the runtime's copy
     // (staging, copy engine, waiting for it), 1 KB in 2 us instead of 11.  The next run looks past the caches.
     const int rc = reef_hal_host_write(storage[idx], value, bytes);
-    if (rc == 0) {
-        host_wrote = true;
-        return Status::Succ;
-    }
+    host_wrote = true;
+    if (rc == 0) return Status::Succ;
     if (rc != 2) RETURN_STATUS(Status::Fail);
     GPU_RETURN_STATUS(reef_hal_memcpy_h2d(storage[idx], value, bytes));
     return Status::Succ;

@@ -97,6 +97,7 @@ protected:
     struct Pass {
         reef_pass_t handle = nullptr;
         bool tried = false;
+        bool fresh = true;     // it has not run since its blocks were uploaded
         Mirror mirror;         // filled by every run
     };
     // Runs the pass behind what `stream` has been given and waits for it.  *ran = false, and nothing done,
@@ -131,13 +132,13 @@ protected:
     reef_graph_t model_graph;
     Pass model_pass;
     // State of the storages (io_mtx: a client fetches results while the scheduler's thread runs the model).
-    // after_pass: the last thing that ran on them was a pass (which has finished); host_wrote: the host has stored
-    // into them past the caches; current: the mirror that is equal to them, or null.
+    // after_pass: the last thing that ran on them was a pass (which has finished); host_wrote: the host or the runtime's
+    // copies have stored into them past the caches (from the start: the arena's zeros); current: the mirror that is equal to them, or null.
     // A launch outside a pass returns before it has run, and only who has waited for its stream knows when it has:
     // busy holds the streams that may still run some.  While there are any, or a pass runs (passes_running), what a fetch
     // copies is good for that fetch only.  inputs_set counts set_input.
     std::mutex io_mtx;
-    bool after_pass = false, host_wrote = false;
+    bool after_pass = false, host_wrote = true;
     const Mirror* current = nullptr;
     std::vector<GPUStream_t> busy;
     int passes_running = 0;
@@ -168,7 +169,8 @@ Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, boo
     if (!p.handle) return Status::Succ;
     *ran = true;
     current = nullptr;
-    const int fresh = host_wrote || !after_pass;
+    const int fresh = host_wrote || !after_pass || p.fresh;
+    p.fresh = false;
     after_pass = host_wrote = false;
     runs++;
     passes_running++;

@@ -55,8 +55,8 @@ bool aql_pass_commit(AqlPass* p, std::string* err);
 // Adds a last launch that copies device ranges to host memory of the pass's: host[i] for range i.
 bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, const char** host, std::string* err);
 // Runs the recorded launches one after the other and returns when the last has finished.
-// fresh: the first launch drops what the caches hold of memory that others than finished kernels and
-// the runtime's copies have written (3 us: code and weights are fetched anew as well).
+// fresh: the first launch drops what the caches hold of memory that others than finished kernels have
+// written -- the host, the runtime's copies, aql_pass_commit (3 us: code and weights are fetched anew as well).
 // false and *err when the queue reported an error.
 bool aql_pass_run(AqlPass* p, bool fresh, std::string* err);
 void aql_pass_destroy(AqlPass* p);
@@ -64,9 +64,10 @@ void aql_pass_destroy(AqlPass* p);
 // Stores into device memory through the PCIe window, 45 GB/s; all of it has arrived when this returns.
 // Caches may still hold the old bytes.  false: the device says nothing of how to flush the window.
 bool aql_host_write(int device, void* dst, const void* src, size_t bytes);
-// Copies device ranges to pinned host memory, one behind the other at multiples of 256 bytes, and waits for it.
+// Copies device ranges to pinned host memory, one behind the other at multiples of 256 bytes, and waits for it: what
+// kernels have written, and what others have in front of the last aql_fence.
 bool aql_fetch(int device, const void* const* src, const size_t* bytes, size_t n, char* host, std::string* err);
-// Drops what the caches hold of bytes that aql_host_write has replaced.
+// Drops what the caches hold of bytes that the host or the runtime's copies have replaced.
 bool aql_fence(int device, std::string* err);
 
 }  // namespace hal

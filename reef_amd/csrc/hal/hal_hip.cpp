@@ -282,8 +282,20 @@ int h_free(reef_devptr_t p, int kind) {
     else HIPCHK(hipFree(p));
     return 0;
 }
-int h_memset(reef_devptr_t p, int byte, size_t n) { HIPCHK(hipMemset(p, byte, n)); return 0; }
-int h_h2d(reef_devptr_t d, const void* s, size_t n) { HIPCHK(hipMemcpy(d, s, n, hipMemcpyHostToDevice)); return 0; }
+// What has been stored into device memory by others than kernels (host_write, the runtime's copies and fills): how
+// many times, and how many of them the last fence covers.  Packets acquire at agent scope, which promises
+// nothing of such stores.
+std::atomic<uint64_t> g_host_writes{0}, g_host_writes_seen{0};
+int h_memset(reef_devptr_t p, int byte, size_t n) {
+    HIPCHK(hipMemset(p, byte, n));
+    g_host_writes.fetch_add(1);
+    return 0;
+}
+int h_h2d(reef_devptr_t d, const void* s, size_t n) {
+    HIPCHK(hipMemcpy(d, s, n, hipMemcpyHostToDevice));
+    g_host_writes.fetch_add(1);
+    return 0;
+}
 int h_d2h(void* d, reef_devptr_t s, size_t n) { HIPCHK(hipMemcpy(d, s, n, hipMemcpyDeviceToHost)); return 0; }
 int h_h2d_async(reef_devptr_t d, const void* s, size_t n, reef_stream_t st) {
     if (st) st->pending.store(true, std::memory_order_release);
@@ -779,7 +791,6 @@ int h_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char*
     reef_hal_set_error(("reef_hal_pass_mirror: " + err).c_str());
     return 1;
 }
-std::atomic<uint64_t> g_host_writes{0}, g_host_writes_seen{0};   // how many there were, how many of them the last fence covers
 int h_host_write(reef_devptr_t dst, const void* src, size_t n) {
     if (!g_host_visible || !reef::hal::aql_available(g_device)) return 2;
     // what the default stream still does with the memory comes first, as in front of a copy
@@ -790,7 +801,7 @@ int h_host_write(reef_devptr_t dst, const void* src, size_t n) {
 }
 int h_host_write_fence() {
     const uint64_t n = g_host_writes.load();
-    if (g_host_writes_seen.load() >= n) return 0;
+    if (g_host_writes_seen.load() >= n || !reef::hal::aql_available(g_device)) return 0;
     std::string err;
     if (reef::hal::aql_fence(g_device, &err)) {
         uint64_t seen = g_host_writes_seen.load();

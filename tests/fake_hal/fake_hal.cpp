@@ -78,7 +78,7 @@ long g_launches = 0, g_completed = 0, g_dropped = 0;
 struct LogEntry { std::string symbol; int stream; uint32_t grid, block, lds; };
 std::vector<LogEntry> g_log;
 int g_auto_progress = 1;  // kernels completed per stream_query
-bool g_passes = false, g_unseen = false;
+bool g_passes = false, g_host_writes = false, g_unseen = false;
 long g_pass_creates = 0, g_pass_runs = 0, g_fetches = 0, g_stale = 0, g_mallocs = 0, g_frees = 0;
 void (*g_pass_hook)(int) = nullptr;   // called with 0 in the middle of every pass and with 1 at its end
 
@@ -395,7 +395,7 @@ int f_pass_run(reef_pass_t p, reef_stream_t after, int fresh) {
 int f_pass_destroy(reef_pass_t p) { delete p; return 0; }
 int f_host_write(reef_devptr_t d, const void* s, size_t n) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
-    if (!g_passes) return 2;
+    if (!g_host_writes) return 2;
     std::memcpy(d, s, n);
     g_unseen = true;
     return 0;
@@ -456,11 +456,16 @@ void fake_hal_reset(void) {
     g_missing.clear();
     g_info_set = false;
     g_auto_progress = 1;
-    g_passes = g_unseen = false;
+    g_passes = g_host_writes = g_unseen = false;
     g_pass_creates = g_pass_runs = g_fetches = g_stale = g_mallocs = g_frees = 0;
     g_pass_hook = nullptr;
 }
-void fake_hal_set_passes(int on) { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_passes = on != 0; }
+// 1: passes, fetches and stores past the caches; 2: without the last
+void fake_hal_set_passes(int on) {
+    std::lock_guard<std::recursive_mutex> lock(g_mtx);
+    g_passes = on != 0;
+    g_host_writes = on == 1;
+}
 void fake_hal_set_pass_hook(void (*hook)(int)) { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_pass_hook = hook; }
 // pass_create, pass_run, fetch calls; packets that ran before the caches had been dropped; malloc, free calls
 void fake_hal_pass_counts(long out[6]) {

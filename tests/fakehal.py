@@ -109,9 +109,9 @@ class FakeHal:
     def set_missing(self, name):
         self.lib.fake_hal_set_missing(name.encode())
 
-    def set_passes(self, on=True):
-        """The backend records passes, stores past the caches and fetches (off after install)."""
-        self.lib.fake_hal_set_passes(int(on))
+    def set_passes(self, host_writes=True):
+        """The backend records passes and fetches (off after install), and stores past the caches or has to copy."""
+        self.lib.fake_hal_set_passes(1 if host_writes else 2)
 
     def set_pass_hook(self, fn):
         """`fn(0)` runs in the middle of every pass from now on, `fn(1)` at its end."""

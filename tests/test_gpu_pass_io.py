@@ -76,3 +76,31 @@ def test_a_mirrored_storage_that_is_written_is_read_back(model):
     e = np.exp(v - v.max(), dtype=np.float32)
     np.testing.assert_allclose(exe.get_output(), e / e.sum(), rtol=1e-5, atol=1e-7)
     exe.close()
+
+
+def test_parameters_loaded_again_between_passes(model, tmp_path):
+    """The runtime's copies replace what the last pass has left in the caches: small parameters and ones of 2 MiB."""
+    d, name, scores, _, _, _ = model
+    g = nets.resnet(18, image=(3, 64, 64), classes=100, name=name)
+    g.params = [(k, (a * np.float32(0.5)).astype(a.dtype) if a.dtype == np.float32 else a) for k, a in g.params]
+    halved = str(tmp_path / "halved")
+    g.write(halved)
+    files = ["%s/%s.param" % (p, name) for p in (d, halved)]
+    x = nets.image_input("passio", (3, 64, 64), 7)
+    want = []
+    for f in files:
+        ref = B.Executor.from_dir(d, name, B.BASE)
+        ref.load_param(f)
+        by_kernel(ref, x, ref.num_kernels())
+        want.append((ref.get_output(), ref.get_data(scores, 100)))
+        ref.close()
+    assert not np.array_equal(want[0][1], want[1][1])
+    exe = B.Executor.from_dir(d, name, B.BASE)
+    exe.set_input_checked("data", x)
+    for step in range(8):
+        exe.load_param(files[step % 2])
+        for _ in range(1 + step // 4):
+            exe.execute()
+        np.testing.assert_array_equal(exe.get_output(), want[step % 2][0])
+        np.testing.assert_array_equal(exe.get_data(scores, 100), want[step % 2][1])
+    exe.close()

@@ -1,5 +1,6 @@
 """What a model keeps between a run and the fetches behind it -- the mirror of the last run, what a fetch has copied --
 on the recording backend with passes switched on: a fetch returns what the storages hold, whenever it comes."""
+import os
 import time
 
 import numpy as np
@@ -88,4 +89,28 @@ def test_a_fetch_in_the_middle_of_a_pass_and_an_input_behind_its_last_launch(fak
     for _ in range(2):
         np.testing.assert_array_equal(exe.get_output(), np.full(N, 50, np.float32))
         np.testing.assert_array_equal(exe.get_data(c, N), np.full(N, 7, np.float32))
+    exe.close()
+
+
+@pytest.mark.parametrize("host_writes", [True, False])
+def test_packets_run_behind_whatever_was_stored_past_the_caches(fake, tmp_path, host_writes):
+    """Inputs, parameters that are loaded again and a pass's own argument blocks are stored by the host or the runtime's
+    copies: the first packets behind them drop the caches, those behind a pass of the same model do not."""
+    g = nets.resnet(18, image=(3, 32, 32), classes=16, name="tiny18")
+    d = write_model(g, tmp_path)
+    scores = g.kernels[-1]["args"][0]
+    fake.set_passes(host_writes)
+    exe = B.Executor.from_dir(d, g.name, B.BASE)
+    assert not exe.get_output(16).any()                    # the arena's zeros
+    for step in range(3):                                  # the scores join what the pass mirrors
+        exe.set_input_checked("data", nets.image_input("t", (3, 32, 32), step))
+        exe.execute()
+        exe.get_output(), exe.get_data(scores, 16)
+    exe.execute()
+    exe.load_param(os.path.join(d, g.name + ".param"))
+    exe.execute()
+    exe.load_param(os.path.join(d, g.name + ".param"))
+    exe.get_data(0, 3 * 32 * 32)
+    exe.execute()
+    assert fake.pass_counts()["stale"] == 0
     exe.close()
