@@ -223,8 +223,11 @@ int reef_hal_graph_destroy(reef_graph_t g);
  *   pass_block:  device address and size of the block of launch `i`, the host copy that pass_commit
  *                uploads (the caller may still write into it), and where in it the tail starts.
  *   pass_commit: uploads the blocks; needed before the first run.
- *   pass_mirror: (before pass_commit) adds a last launch that copies ranges of device memory to host
- *                memory of the pass's; host[i] is where range i is found after a run.
+ *   pass_mirror: adds a last launch that copies ranges of device memory to host memory of the pass's;
+ *                host[i] is where range i is found after a run.  The first call (before pass_commit)
+ *                allocates `reserve` bytes of host memory, or what its ranges take if that is more
+ *                (each rounded up to 256 bytes); a later call, between runs, mirrors other ranges
+ *                that fit into it, allocates nothing, and the next run has to be `fresh`.
  *   pass_run:    waits for what `after` (may be NULL: the default stream) has been given, runs the
  *                launches in order and returns when the last has finished.  `fresh`: the caches may hold
  *                what the host, copies, fills, pass_commit or launches outside passes have changed since
@@ -255,7 +258,7 @@ int reef_hal_pass_block(reef_pass_t p, size_t i, reef_pass_block* out);
 int reef_hal_pass_commit(reef_pass_t p);
 typedef struct reef_pass_range { const void* src; size_t bytes; } reef_pass_range;
 #define REEF_PASS_MAX_RANGES 8
-int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* ranges, size_t n, const char** host);
+int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* ranges, size_t n, size_t reserve, const char** host);
 int reef_hal_pass_run(reef_pass_t p, reef_stream_t after, int fresh);
 int reef_hal_host_write(reef_devptr_t dst, const void* src, size_t bytes);
 int reef_hal_host_write_fence(void);
@@ -317,7 +320,7 @@ typedef struct reef_hal_backend {
     int (*pass_commit)(reef_pass_t);
     int (*pass_run)(reef_pass_t, reef_stream_t, int);
     int (*pass_destroy)(reef_pass_t);
-    int (*pass_mirror)(reef_pass_t, const reef_pass_range*, size_t, const char**);
+    int (*pass_mirror)(reef_pass_t, const reef_pass_range*, size_t, size_t, const char**);
     int (*host_write)(reef_devptr_t, const void*, size_t);
     int (*host_write_fence)(void);
     int (*fetch)(const reef_pass_range*, size_t, void*);

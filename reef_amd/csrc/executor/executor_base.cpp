@@ -28,7 +28,14 @@ Status ExecutorBase::load_model_from_file(const char* json_file_path, const char
     GPU_RETURN_STATUS(reef_hal_init(0));
     GPUModule_t mod;
     GPU_RETURN_STATUS(reef_hal_module_load(co_file_path, &mod));
-    return this->load_model_from_GPU_module(json_file_path, mod);
+    RETURN_STATUS(this->load_model_from_GPU_module(json_file_path, mod));
+    return ready_model_pass();
+}
+
+Status ExecutorBase::ready_model_pass() {
+    if (use_graph) return Status::Succ;
+    std::lock_guard<std::mutex> lock(io_mtx);
+    return ready_pass(model_pass, [this](int i, Launch& l) { return make_launch(i, l); });
 }
 
 Status ExecutorBase::load_model_from_GPU_module(const char* json_file_path, GPUModule_t mod) {
@@ -200,7 +207,7 @@ constexpr size_t kMaxMirroredOutput = 4u << 20, kMaxWatched = 64 * 1024;   // la
 constexpr size_t kMaxWatch = 4;
 }
 
-// A small storage that is fetched after two different runs joins what the passes mirror.
+// A small storage that is fetched after two different runs joins what the passes mirror (mirror_watched).
 void ExecutorBase::note_fetch(size_t idx) {
     if (storage_bytes(idx) > kMaxWatched || watch.size() >= kMaxWatch) return;
     if (std::find(watch.begin(), watch.end(), idx) != watch.end()) return;
@@ -219,6 +226,36 @@ void ExecutorBase::list_mirrored(Mirror& m) const {
         }
     for (size_t idx : watch)
         if (!m.find(idx)) m.entries.push_back({idx, storage_bytes(idx), nullptr});
+}
+
+// Host memory that holds whatever list_mirrored may name in this model's life.
+size_t ExecutorBase::mirror_room() const {
+    size_t room = kMaxWatch * align_up<size_t>(kMaxWatched, 256);
+    for (size_t i = 0; i < model->storage.size(); i++)
+        if (model->storage[i].name == "output") {
+            if (storage_bytes(i) <= kMaxMirroredOutput) room += align_up<size_t>(storage_bytes(i), 256);
+            break;
+        }
+    return room;
+}
+
+// The pass mirrors what is watched by now.  In the fetch that found the storage missing, not in the next run: that one's
+// request pays for nothing, and in a scheduler it belongs to the real-time thread.  Caller holds io_mtx.
+Status ExecutorBase::mirror_watched(Pass& p) {
+    if (!p.handle || passes_running || p.mirror.watched == watch.size()) return Status::Succ;
+    Mirror m;
+    list_mirrored(m);
+    reef_pass_range ranges[REEF_PASS_MAX_RANGES];
+    const char* host[REEF_PASS_MAX_RANGES];
+    static_assert(1 + kMaxWatch <= REEF_PASS_MAX_RANGES, "a pass mirrors the output and the watched storages");
+    const size_t n = m.entries.size();
+    for (size_t i = 0; i < n; i++) ranges[i] = {storage[m.entries[i].idx], m.entries[i].bytes};
+    if (current == &p.mirror) current = nullptr;
+    GPU_RETURN_STATUS(reef_hal_pass_mirror(p.handle, ranges, n, mirror_room(), host));
+    for (size_t i = 0; i < n; i++) m.entries[i].host = host[i];
+    p.mirror = m;
+    p.fresh = true;
+    return Status::Succ;
 }
 
 // From the mirror; else, what is mirrored, all of it with one launch (8 us; the runtime's copy takes 12 to 15 for each),
@@ -241,6 +278,7 @@ Status ExecutorBase::fetch(size_t idx, void* out) {
         note_fetch(idx);
         list_mirrored(m);
     }
+    for (Pass* p : passes) RETURN_STATUS(mirror_watched(*p));
     const bool all = m.find(idx) != nullptr;
     if (!all) {
         m.entries.clear();
@@ -254,13 +292,8 @@ Status ExecutorBase::fetch(size_t idx, void* out) {
             total += align_up<size_t>(m.entries[i].bytes, 256);
         }
         if (current == &fetched) current = nullptr;
-        if (total > fetch_bytes) {
-            if (fetch_mem) reef_hal_free(fetch_mem, REEF_MEM_HOST_PINNED);
-            fetch_mem = nullptr;
-            fetch_bytes = 0;
-            GPU_RETURN_STATUS(reef_hal_malloc(total, REEF_MEM_HOST_PINNED, &fetch_mem));
-            fetch_bytes = total;
-        }
+        if (!fetch_mem) GPU_RETURN_STATUS(reef_hal_malloc(mirror_room(), REEF_MEM_HOST_PINNED, &fetch_mem));
+        if (total > mirror_room()) RETURN_STATUS(Status::OutOfRange);
         const int rc = reef_hal_fetch(ranges, m.entries.size(), fetch_mem);
         if (rc == 0) {
             const char* at = (const char*)fetch_mem;
@@ -452,15 +485,8 @@ Status ExecutorBase::record_pass(Pass& p, std::vector<Launch>& l) {
         const void* rec = cur.device + cur.tail;
         std::memcpy(cur.host + slot[i], &rec, sizeof(rec));
     }
-    list_mirrored(p.mirror);
-    std::vector<reef_pass_range> ranges;
-    for (const Mirror::Entry& e : p.mirror.entries) ranges.push_back({storage[e.idx], e.bytes});
-    if (!ranges.empty()) {
-        const char* host[REEF_PASS_MAX_RANGES];
-        static_assert(1 + kMaxWatch <= REEF_PASS_MAX_RANGES, "a pass mirrors the output and the watched storages");
-        GPU_RETURN_STATUS(reef_hal_pass_mirror(p.handle, ranges.data(), ranges.size(), host));
-        for (size_t i = 0; i < ranges.size(); i++) p.mirror.entries[i].host = host[i];
-    }
+    p.mirror.watched = ~(size_t)0;     // nothing yet
+    RETURN_STATUS(mirror_watched(p));
     GPU_RETURN_STATUS(reef_hal_pass_commit(p.handle));
     return Status::Succ;
 }

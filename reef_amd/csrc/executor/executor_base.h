@@ -97,13 +97,18 @@ protected:
     struct Pass {
         reef_pass_t handle = nullptr;
         bool tried = false;
-        bool fresh = true;     // it has not run since its blocks were uploaded
+        bool fresh = true;     // it has not run since one of its blocks was uploaded
         Mirror mirror;         // filled by every run
     };
     // Runs the pass behind what `stream` has been given and waits for it.  *ran = false, and nothing done,
     // where the backend cannot record one.
     template <class Make>
     Status run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran);
+    // Records the pass if that has not been tried yet: at load, so that no request pays for the code object, the
+    // allocations and the upload; a first run does it where a model was loaded without.  Caller holds io_mtx.
+    template <class Make>
+    Status ready_pass(Pass& p, const Make& make);
+    Status ready_model_pass();
     Status record_pass(Pass& p, std::vector<Launch>& launches);
     void drop_pass(Pass& p);
 public:
@@ -131,6 +136,7 @@ protected:
     bool use_graph;
     reef_graph_t model_graph;
     Pass model_pass;
+    std::vector<Pass*> passes{&model_pass};
     // State of the storages (io_mtx: a client fetches results while the scheduler's thread runs the model).
     // after_pass: the last thing that ran on them was a pass (which has finished); host_wrote: the host or the runtime's
     // copies have stored into them past the caches (from the start: the arena's zeros); current: the mirror that is equal to them, or null.
@@ -146,26 +152,31 @@ protected:
     bool at_rest() const { return busy.empty() && passes_running == 0; }
     Mirror fetched;                    // of the last fetch that was no pass's
     GPUDevicePtr_t fetch_mem = nullptr;   // pinned
-    size_t fetch_bytes = 0;
     std::vector<size_t> watch;         // storages fetched again and again
     size_t asked_idx = 0, asked_run = 0, runs = 0;
     void note_fetch(size_t idx);
     void list_mirrored(Mirror& m) const;
+    size_t mirror_room() const;
+    Status mirror_watched(Pass& p);
     Status fetch(size_t idx, void* out);
     void drop_graph();
 };
 
 template <class Make>
+Status ExecutorBase::ready_pass(Pass& p, const Make& make) {
+    if (p.tried) return Status::Succ;
+    std::vector<Launch> l(num_kernels());
+    for (size_t i = 0; i < l.size(); i++) RETURN_STATUS(make((int)i, l[i]));
+    RETURN_STATUS(record_pass(p, l));
+    p.tried = true;
+    return Status::Succ;
+}
+
+template <class Make>
 Status ExecutorBase::run_pass(Pass& p, const Make& make, GPUStream_t stream, bool* ran) {
     *ran = false;
     std::unique_lock<std::mutex> lock(io_mtx);
-    if (p.handle && p.mirror.watched != watch.size()) drop_pass(p);
-    if (!p.tried) {
-        std::vector<Launch> l(num_kernels());
-        for (size_t i = 0; i < l.size(); i++) RETURN_STATUS(make((int)i, l[i]));
-        RETURN_STATUS(record_pass(p, l));
-        p.tried = true;
-    }
+    RETURN_STATUS(ready_pass(p, make));
     if (!p.handle) return Status::Succ;
     *ran = true;
     current = nullptr;

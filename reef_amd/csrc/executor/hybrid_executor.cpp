@@ -13,7 +13,7 @@ static_assert(sizeof(reef_hal_completion) == 32 && offsetof(ReefBeArgs, preempte
 HybridExecutor::HybridExecutor()
     : preempt_mod(nullptr), trans_mod(nullptr), preempt_flag(nullptr), owns_flag(false),
       task_slot_base(nullptr), task_slots_host_empty(nullptr), task_slots_host(nullptr),
-      sync_ptr(nullptr), sync_bytes(0) {}
+      sync_ptr(nullptr), sync_bytes(0) { passes.push_back(&preempt_pass); }
 
 HybridExecutor::~HybridExecutor() {
     drop_pass(preempt_pass);
@@ -32,8 +32,9 @@ Status HybridExecutor::load_hybrid_model_from_file(const char* json_file_path,
     REEF_LOG_INFO("%s", trans_co_file_path);
     GPU_RETURN_STATUS(reef_hal_module_load(trans_co_file_path, &trans_module));
     GPU_RETURN_STATUS(reef_hal_module_load(preempt_co_file_path, &preempt_module));
-    return load_hybrid_model_from_GPU_module(json_file_path, profile_file_path, trans_module,
-                                             preempt_module);
+    RETURN_STATUS(load_hybrid_model_from_GPU_module(json_file_path, profile_file_path, trans_module,
+                                                    preempt_module));
+    return ready_model_pass();
 }
 
 Status HybridExecutor::load_hybrid_model_from_GPU_module(const char* json_file_path,
@@ -106,6 +107,11 @@ Status HybridExecutor::set_preempt_flag(GPUDevicePtr_t flag) {
     preempt_flag = flag;
     drop_pass(preempt_pass);   // its argument blocks name the old flag
     return Status::Succ;
+}
+
+Status HybridExecutor::prepare_preemptale() {
+    std::lock_guard<std::mutex> lock(io_mtx);
+    return ready_pass(preempt_pass, [this](int i, Launch& l) { return make_preempt_launch(i, l); });
 }
 
 Status HybridExecutor::execute_preemptale(GPUStream_t stream) {

@@ -391,6 +391,8 @@ struct AqlPass {
     hsa_signal_t done{};
     void* kernargs = nullptr;    // device memory, one 64-byte aligned block per launch
     char* mirror = nullptr;      // host memory, what aql_pass_mirror's launch fills
+    size_t mirror_bytes = 0;
+    bool mirrors = false;        // the last packet is that launch
     std::vector<char> host;      // the same as it is uploaded
     std::vector<size_t> at, tail;    // where a launch's block starts, and the caller's part inside it
     bool committed = false;
@@ -491,27 +493,43 @@ bool aql_fetch(int device, const void* const* src, const size_t* bytes, size_t n
     return aql_call(device, k, blocks, 256, &a, sizeof(a), nullptr, err);
 }
 
-bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, const char** host, std::string* err) {
-    if (p->mirror || p->packets.empty() || n == 0 || n > kBlitRanges) { *err = "bad number of ranges, or a second mirror"; return false; }
+bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, size_t reserve, const char** host,
+                     std::string* err) {
+    std::lock_guard<std::mutex> lock(p->mtx);      // no run is under way
+    if (p->packets.empty() || n > kBlitRanges) { *err = "bad number of ranges, or nothing to mirror behind"; return false; }
+    size_t total = 0;
+    for (size_t i = 0; i < n; ++i) total += (bytes[i] + 255) / 256 * 256;
+    if (!p->mirror) {
+        p->mirror_bytes = std::max(total, reserve);
+        void* m = nullptr;
+        const hipError_t e = hipHostMalloc(&m, std::max<size_t>(p->mirror_bytes, 256), hipHostMallocDefault);
+        if (e != hipSuccess) { *err = std::string("mirror: ") + hipGetErrorString(e); return false; }
+        p->mirror = (char*)m;
+    }
+    if (total > p->mirror_bytes) { *err = "the mirror has no room for these ranges"; return false; }
+    if (n == 0) return true;
     const AqlKernel* k = aql_kernel(blit_code().get(), device, "reef_blit_ranges", err);
     if (!k) return false;
     BlitArgs a;
-    size_t total = 0;
-    for (size_t i = 0; i < n; ++i) total += (bytes[i] + 255) / 256 * 256;
-    void* m = nullptr;
-    const hipError_t e = hipHostMalloc(&m, total, hipHostMallocDefault);
-    if (e != hipSuccess) { *err = std::string("mirror: ") + hipGetErrorString(e); return false; }
-    p->mirror = (char*)m;
     const uint32_t blocks = blit_args(&a, src, bytes, n, p->mirror);
     for (size_t i = 0; i < n; ++i) host[i] = a.range[i].dst;
     const uint32_t grid[3] = {blocks, 1, 1}, block[3] = {256, 1, 1};
     const size_t off = p->at.back();
     fill_kernarg(p->host.data() + off, *k, &a, sizeof(a), grid, block);
+    if (p->committed) {
+        const hipError_t e = hipMemcpy((char*)p->kernargs + off, p->host.data() + off, p->host.size() - off, hipMemcpyHostToDevice);
+        if (e != hipSuccess) { *err = std::string("mirror: ") + hipGetErrorString(e); return false; }
+    }
     hsa_kernel_dispatch_packet_t packet =
         dispatch_packet(*k, grid, block, 0, (char*)p->kernargs + off, HSA_FENCE_SCOPE_AGENT, HSA_FENCE_SCOPE_SYSTEM);
     packet.completion_signal = p->done;
-    p->packets.back().completion_signal = hsa_signal_t{};
-    p->packets.push_back(packet);
+    if (p->mirrors) {
+        p->packets.back() = packet;
+    } else {
+        p->packets.back().completion_signal = hsa_signal_t{};
+        p->packets.push_back(packet);
+        p->mirrors = true;
+    }
     return true;
 }
 

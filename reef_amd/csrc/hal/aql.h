@@ -52,8 +52,10 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
 bool aql_pass_block(AqlPass* p, size_t i, char** device, char** host, size_t* bytes, size_t* tail);
 // Uploads the blocks.
 bool aql_pass_commit(AqlPass* p, std::string* err);
-// Adds a last launch that copies device ranges to host memory of the pass's: host[i] for range i.
-bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, const char** host, std::string* err);
+// Adds a last launch that copies device ranges to host memory of the pass's: host[i] for range i.  The first call
+// allocates that memory, `reserve` bytes or more; a later one mirrors other ranges that fit into it.
+bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, size_t reserve, const char** host,
+                     std::string* err);
 // Runs the recorded launches one after the other and returns when the last has finished.
 // fresh: the first launch drops what the caches hold of memory that others than finished kernels have
 // written -- the host, the runtime's copies, aql_pass_commit (3 us: code and weights are fetched anew as well).

@@ -107,8 +107,8 @@ int reef_hal_pass_create(const reef_pass_launch* launches, size_t n, size_t tail
 }
 int reef_hal_pass_block(reef_pass_t p, size_t i, reef_pass_block* out) { return be()->pass_block ? be()->pass_block(p, i, out) : 1; }
 int reef_hal_pass_commit(reef_pass_t p) { return be()->pass_commit ? be()->pass_commit(p) : 1; }
-int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char** host) {
-    return be()->pass_mirror ? be()->pass_mirror(p, r, n, host) : 1;
+int reef_hal_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, size_t reserve, const char** host) {
+    return be()->pass_mirror ? be()->pass_mirror(p, r, n, reserve, host) : 1;
 }
 int reef_hal_pass_run(reef_pass_t p, reef_stream_t after, int fresh) { return be()->pass_run ? be()->pass_run(p, after, fresh) : 1; }
 int reef_hal_host_write(reef_devptr_t dst, const void* src, size_t bytes) { return be()->host_write ? be()->host_write(dst, src, bytes) : 2; }

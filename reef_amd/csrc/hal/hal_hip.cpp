@@ -781,13 +781,13 @@ int h_pass_commit(reef_pass_t p) {
     reef_hal_set_error(("reef_hal_pass_commit: " + err).c_str());
     return 1;
 }
-int h_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char** host) {
+int h_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, size_t reserve, const char** host) {
     const void* src[REEF_PASS_MAX_RANGES];
     size_t bytes[REEF_PASS_MAX_RANGES];
-    if (!p || !r || !host || n > REEF_PASS_MAX_RANGES) { reef_hal_set_error("reef_hal_pass_mirror: bad argument"); return 1; }
+    if (!p || (n && (!r || !host)) || n > REEF_PASS_MAX_RANGES) { reef_hal_set_error("reef_hal_pass_mirror: bad argument"); return 1; }
     for (size_t i = 0; i < n; ++i) { src[i] = r[i].src; bytes[i] = r[i].bytes; }
     std::string err;
-    if (reef::hal::aql_pass_mirror((reef::hal::AqlPass*)p, g_device, src, bytes, n, host, &err)) return 0;
+    if (reef::hal::aql_pass_mirror((reef::hal::AqlPass*)p, g_device, src, bytes, n, reserve, host, &err)) return 0;
     reef_hal_set_error(("reef_hal_pass_mirror: " + err).c_str());
     return 1;
 }

@@ -55,6 +55,7 @@ struct reef_pass_s {
     std::vector<char> host, device;   // argument blocks: as the caller fills them, as they were committed
     std::vector<reef_pass_range> ranges;
     std::vector<char> mirror;
+    bool unseen = false;              // its own blocks
 };
 
 namespace {
@@ -79,7 +80,7 @@ struct LogEntry { std::string symbol; int stream; uint32_t grid, block, lds; };
 std::vector<LogEntry> g_log;
 int g_auto_progress = 1;  // kernels completed per stream_query
 bool g_passes = false, g_host_writes = false, g_unseen = false;
-long g_pass_creates = 0, g_pass_runs = 0, g_fetches = 0, g_stale = 0, g_mallocs = 0, g_frees = 0;
+long g_pass_creates = 0, g_pass_runs = 0, g_fetches = 0, g_stale = 0, g_mallocs = 0, g_frees = 0, g_pass_mirrors = 0;
 void (*g_pass_hook)(int) = nullptr;   // called with 0 in the middle of every pass and with 1 at its end
 
 reef_stream_s* S(reef_stream_t s) { return s ? s : &g_null_stream; }
@@ -351,15 +352,21 @@ int f_pass_block(reef_pass_t p, size_t i, reef_pass_block* out) {
 int f_pass_commit(reef_pass_t p) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
     p->device.assign(p->host.begin(), p->host.end());
-    g_unseen = true;
+    p->unseen = true;
     return 0;
 }
-int f_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char** host) {
+int f_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, size_t reserve, const char** host) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
     p->ranges.assign(r, r + n);
     size_t total = 0;
     for (size_t i = 0; i < n; ++i) total += (r[i].bytes + 255) / 256 * 256;
-    p->mirror.assign(total, 0);
+    if (p->mirror.empty()) {
+        p->mirror.assign(total > reserve ? total : reserve, 0);
+    } else {
+        ++g_pass_mirrors;
+        p->unseen = true;
+        if (total > p->mirror.size()) return 1;
+    }
     total = 0;
     for (size_t i = 0; i < n; ++i) {
         host[i] = p->mirror.data() + total;
@@ -370,8 +377,8 @@ int f_pass_mirror(reef_pass_t p, const reef_pass_range* r, size_t n, const char*
 int f_pass_run(reef_pass_t p, reef_stream_t after, int fresh) {
     std::unique_lock<std::recursive_mutex> lock(g_mtx);
     drain(S(after));
-    if (fresh) g_unseen = false;
-    if (g_unseen) ++g_stale;
+    if (fresh) g_unseen = p->unseen = false;
+    if (g_unseen || p->unseen) ++g_stale;
     ++g_pass_runs;
     auto call_hook = [&](int where) {
         if (!g_pass_hook) return;
@@ -457,7 +464,7 @@ void fake_hal_reset(void) {
     g_info_set = false;
     g_auto_progress = 1;
     g_passes = g_host_writes = g_unseen = false;
-    g_pass_creates = g_pass_runs = g_fetches = g_stale = g_mallocs = g_frees = 0;
+    g_pass_creates = g_pass_runs = g_fetches = g_stale = g_mallocs = g_frees = g_pass_mirrors = 0;
     g_pass_hook = nullptr;
 }
 // 1: passes, fetches and stores past the caches; 2: without the last
@@ -467,10 +474,11 @@ void fake_hal_set_passes(int on) {
     g_host_writes = on == 1;
 }
 void fake_hal_set_pass_hook(void (*hook)(int)) { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_pass_hook = hook; }
-// pass_create, pass_run, fetch calls; packets that ran before the caches had been dropped; malloc, free calls
-void fake_hal_pass_counts(long out[6]) {
+// pass_create, pass_run, fetch calls; packets that ran before the caches had been dropped; malloc, free calls;
+// pass_mirror calls behind a pass's first
+void fake_hal_pass_counts(long out[7]) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
-    const long v[6] = {g_pass_creates, g_pass_runs, g_fetches, g_stale, g_mallocs, g_frees};
+    const long v[7] = {g_pass_creates, g_pass_runs, g_fetches, g_stale, g_mallocs, g_frees, g_pass_mirrors};
     std::memcpy(out, v, sizeof(v));
 }
 // Bytes from `p` to the end of the allocation that holds it (0 when unknown).

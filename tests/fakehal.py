@@ -119,9 +119,9 @@ class FakeHal:
         self.lib.fake_hal_set_pass_hook(self._hook)
 
     def pass_counts(self):
-        out = (ctypes.c_long * 6)()
+        out = (ctypes.c_long * 7)()
         self.lib.fake_hal_pass_counts(out)
-        return dict(zip(("creates", "runs", "fetches", "stale", "mallocs", "frees"), out))
+        return dict(zip(("creates", "runs", "fetches", "stale", "mallocs", "frees", "mirrors"), out))
 
     def log(self):
         out = []

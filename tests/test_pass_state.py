@@ -114,3 +114,54 @@ def test_packets_run_behind_whatever_was_stored_past_the_caches(fake, tmp_path, 
     exe.execute()
     assert fake.pass_counts()["stale"] == 0
     exe.close()
+
+
+@pytest.mark.parametrize("kind", [B.BASE, B.TRANS, B.HYBRID])
+def test_runs_record_and_allocate_nothing(fake, mocked, kind):
+    """Passes are recorded at load; a storage that joins what they mirror is added by the fetch that finds it missing."""
+    name, d = mocked
+    exe = B.Executor.from_dir(d, name, kind)
+    runs = [exe.execute] + ([exe.execute_preemptable] if kind == B.HYBRID else [])
+    assert fake.pass_counts()["creates"] == len(runs)
+    changing = ("creates", "mallocs", "frees", "mirrors")
+
+    def run(run_one):
+        before = fake.pass_counts()
+        run_one()
+        after = fake.pass_counts()
+        assert after["runs"] == before["runs"] + 1 and all(after[k] == before[k] for k in changing)
+
+    for step in range(12):
+        v = 2.0 + step
+        set_inputs(exe.set_input_checked, v)
+        if step == 5:                                      # not in the middle of a run
+            fake.set_pass_hook(lambda where: exe.get_data(2, N))
+        run(runs[step % len(runs)])
+        fake.set_pass_hook(lambda where: None)
+        for idx, want in ((4, 2 * v * v), (3, v), (2, 2 * v))[:1 + step // 3]:
+            np.testing.assert_array_equal(exe.get_data(idx, N), np.full(N, want, np.float32))
+    end = fake.pass_counts()
+    assert end["mirrors"] == 2 * len(runs) and end["stale"] == 0
+    set_inputs(exe.set_input_checked, 1.0)
+    run(runs[0])
+    for idx, want in ((4, 2), (3, 1), (2, 2)):             # all from the mirror
+        np.testing.assert_array_equal(exe.get_data(idx, N), np.full(N, want, np.float32))
+    assert fake.pass_counts()["fetches"] == end["fetches"]
+    exe.close()
+
+
+def test_a_scheduled_real_time_request_records_and_allocates_nothing(fake, mocked):
+    name, d = mocked
+    s = B.Scheduler(B.MODE_REEF)
+    m = s.load_model(d, name)
+    s.bind_model_queue(s.create_queue(B.QUEUE_RT), m)
+    s.run()
+    set_inputs(lambda k, x: s.set_input(m, x, k), 3.0)
+    before = fake.pass_counts()
+    assert before["creates"] == 1
+    s.wait_task(s.new_task(m))
+    after = fake.pass_counts()
+    assert after["runs"] == 1 and all(after[k] == before[k] for k in ("creates", "mallocs", "frees", "mirrors"))
+    np.testing.assert_array_equal(s.get_output(m, N), np.full(N, 18, np.float32))
+    s.shutdown()
+    s.close()
