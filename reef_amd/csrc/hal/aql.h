@@ -26,14 +26,9 @@ const AqlKernel* aql_kernel(AqlCode* code, int device, const char* name, std::st
 // One launch of `groups` workgroups of `threads`, waited for: it sees what finished kernels and the
 // runtime's copies have written (what a launch through the runtime sees; the runtime empties the caches in
 // front of a copy), and its results are visible everywhere when this returns.  Calls of several threads
-// run beside each other.  `resident`: device memory that holds aql_call_args' image of the same
-// arguments, or null (they are read from host memory then, 1.2 us later).
-constexpr size_t kAqlCallArgs = 512;
+// run beside each other.
 bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
-              const void* resident, std::string* err);
-// The argument block of such a launch.
-void aql_call_args(const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
-                   char (&image)[kAqlCallArgs]);
+              std::string* err);
 // Makes what one call in flight needs, so that a first call allocates nothing (one beside another does).
 bool aql_call_prepare(int device, std::string* err);
 

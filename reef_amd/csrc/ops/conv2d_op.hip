@@ -178,16 +178,6 @@ constexpr Kernel kKernels[] = {
 constexpr int kNumKernels = sizeof(kKernels) / sizeof(kKernels[0]);
 
 constexpr int kMaxDevices = 16;
-// Arguments that calls have come with, and whether they lie in device memory: a serving loop repeats its
-// calls, and a kernel's first read of an argument block in host memory is 1.2 us of a small layer's 12.
-struct KnownArgs {
-    ReefOpDesc desc;
-    int kernel = -1;
-    uint32_t tasks = 0, stamp = 0;
-    int users = 0;             // calls that read the device copy now
-    bool resident = false;
-};
-constexpr int kKnownSets = 32, kKnownWays = 2;
 struct DeviceState {
     bool ready = false;
     hipModule_t module = nullptr;
@@ -196,9 +186,6 @@ struct DeviceState {
     // the same kernels for launches that the call waits for (reef_ops_conv2d_wait); null: not available
     std::shared_ptr<reef::hal::AqlCode> aql;
     const reef::hal::AqlKernel* aql_fn[kNumKernels] = {};
-    KnownArgs known[kKnownSets][kKnownWays];
-    char* known_mem = nullptr;              // their device copies
-    uint32_t stamp = 0;
     // idle workspaces of reef_ops_conv2d, each laid out as `scratch`, counters zero
     std::vector<unsigned char*> pool;
 };
@@ -243,8 +230,6 @@ int ensure_device(DeviceState** out, bool may_set_up = true, int* device = nullp
                 if (!d.aql_fn[i]) d.aql.reset();
             }
             if (d.aql && !reef::hal::aql_call_prepare(dev, &why)) d.aql.reset();
-            void* m = nullptr;
-            if (d.aql && hipMalloc(&m, kKnownSets * kKnownWays * reef::hal::kAqlCallArgs) == hipSuccess) d.known_mem = (char*)m;
         }
         d.ready = true;
     }
@@ -414,48 +399,6 @@ int launch(const DeviceState& d, const Plan& p, hipStream_t stream) {
     return e == hipSuccess ? 0 : hip_fail(e, "hipModuleLaunchKernel");
 }
 
-// The device copy of these arguments, made when they come for the second time; null: none (yet).  What is
-// found is in use until release_args.
-const void* resident_args(DeviceState& d, const Plan& p, KnownArgs** found) {
-    *found = nullptr;
-    if (!d.known_mem) return nullptr;
-    uint64_t h = (uint64_t)p.kernel;
-    for (int i = 0; i < 5; ++i) h = (h ^ (uint64_t)p.desc.ptr[i]) * 0x9E3779B97F4A7C15ull;
-    std::lock_guard<std::mutex> lock(g_mtx);
-    KnownArgs* set = d.known[(h >> 40) % kKnownSets];
-    KnownArgs* victim = nullptr;
-    for (int i = 0; i < kKnownWays; ++i) {
-        KnownArgs& k = set[i];
-        if (k.kernel == p.kernel && k.tasks == p.tasks && std::memcmp(&k.desc, &p.desc, sizeof(p.desc)) == 0) {
-            char* at = d.known_mem + (&k - &d.known[0][0]) * reef::hal::kAqlCallArgs;
-            k.stamp = ++d.stamp;
-            if (!k.resident) {
-                char image[reef::hal::kAqlCallArgs];
-                reef::hal::aql_call_args(d.aql_fn[p.kernel], p.tasks, REEF_WG_THREADS, &p.desc, sizeof(p.desc), image);
-                if (hipMemcpy(at, image, sizeof(image), hipMemcpyHostToDevice) != hipSuccess) return nullptr;
-                k.resident = true;
-            }
-            k.users++;
-            *found = &k;
-            return at;
-        }
-        if (k.users == 0 && (!victim || k.stamp < victim->stamp)) victim = &k;
-    }
-    if (victim) {
-        victim->desc = p.desc;
-        victim->kernel = p.kernel;
-        victim->tasks = p.tasks;
-        victim->stamp = ++d.stamp;
-        victim->resident = false;
-    }
-    return nullptr;
-}
-void release_args(KnownArgs* k) {
-    if (!k) return;
-    std::lock_guard<std::mutex> lock(g_mtx);
-    k->users--;
-}
-
 // Launches on the default stream and returns when the result is there.  Work that the device was given
 // before (the layer's inputs among it) ends first; then the launch is one packet on a queue of this
 // library's own, whose completion the host sees 3 us earlier than it sees a stream go idle.
@@ -468,11 +411,8 @@ int launch_and_wait(DeviceState& d, int device, const Plan& p) {
     const hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
     std::string err;
-    KnownArgs* known;
-    const void* args = resident_args(d, p, &known);
-    if (!reef::hal::aql_call(device, d.aql_fn[p.kernel], p.tasks, REEF_WG_THREADS, &p.desc, sizeof(p.desc), args, &err))
+    if (!reef::hal::aql_call(device, d.aql_fn[p.kernel], p.tasks, REEF_WG_THREADS, &p.desc, sizeof(p.desc), &err))
         return fail("reef_ops_conv2d: " + err);     // (what the launch may still read stays in use)
-    release_args(known);
     return 0;
 }
 

@@ -62,3 +62,39 @@ def test_conv2d_op_rejects_bad_arguments():
     assert "bad shape" in B.last_error()
     assert B.ops_conv2d(B.Conv2dDesc(4, 2, 2, 4, 5, 5, 1, 1, 0, 0, 0), buf, buf, None, None, buf) == 1
     assert B.ops_conv2d(B.Conv2dDesc(4, 4, 4, 4, 1, 1, 1, 1, 0, 0, 9), buf, buf, None, None, buf) == 1
+
+
+def device_layer(case, seed):
+    """A layer of CASES' form with operands in device memory."""
+    cin, H, W, cout, k, s, p, act, has_bias, has_res = case
+    rng = np.random.default_rng(seed)
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    arrays = [rng.standard_normal((cin, H, W)), rng.standard_normal((cout, cin, k, k)) * np.sqrt(2.0 / (cin * k * k)),
+              rng.standard_normal(cout) if has_bias else None, rng.standard_normal((cout, Ho, Wo)) if has_res else None]
+    arrays = [a if a is None else a.astype(np.float32) for a in arrays]
+    bufs = [a if a is None else B.DeviceBuffer.from_array(a) for a in arrays]
+    return B.Conv2dDesc(cin, H, W, cout, k, k, s, s, p, p, act), arrays, bufs, (cout, Ho, Wo)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_a_call_runs_with_its_own_arguments_whatever_came_before(noalloc):
+    """Hundreds of calls in turn that differ in a pointer or two: each writes where it was told to, from what it was given."""
+    B.ops_init()
+    d, _, (x, w, _, _), shape = device_layer((64, 14, 14, 64, 1, 1, 0, 1, False, False), 1)
+    _, _, (x2, w2, _, _), _ = device_layer((64, 14, 14, 64, 1, 1, 0, 1, False, False), 2)
+    want = {}
+    for i, a in enumerate((x, x2)):
+        for j, b in enumerate((w, w2)):
+            o = B.DeviceBuffer(4 * int(np.prod(shape)))
+            assert B.ops_conv2d(d, a, b, None, None, o) == 0, B.last_error()
+            want[i, j] = o.to_array()
+    outs = [B.DeviceBuffer(4 * int(np.prod(shape))) for _ in range(70)]
+    for rep in range(4):
+        for o in outs:
+            o.fill(0xFF)
+        for n, o in enumerate(outs):
+            i, j = (n + rep) % 2, (n // 2 + rep) % 2
+            for _ in range(1 + n % 3):
+                assert B.ops_conv2d(d, (x, x2)[i], (w, w2)[j], None, None, o, noalloc=noalloc) == 0, B.last_error()
+        for n, o in enumerate(outs):
+            np.testing.assert_array_equal(o.to_array(), want[(n + rep) % 2, (n // 2 + rep) % 2])
