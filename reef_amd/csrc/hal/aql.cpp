@@ -357,14 +357,14 @@ bool aql_call_prepare(int device, std::string* err) {
 }
 
 bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
-              std::string* err) {
+              bool fresh, std::string* err) {
     if (std::max<size_t>(kernel->kernarg, kernarg_bytes) + sizeof(HiddenArgs) > kAqlCallArgs) { *err = "argument block too large"; return false; }
     Call* c = take_call(device, err);
     if (!c) return false;
     const uint32_t grid[3] = {groups, 1, 1}, block[3] = {threads, 1, 1};
     fill_kernarg(c->kernarg, *kernel, kernarg, kernarg_bytes, grid, block);
     hsa_kernel_dispatch_packet_t packet =
-        dispatch_packet(*kernel, grid, block, 0, c->kernarg, HSA_FENCE_SCOPE_AGENT, HSA_FENCE_SCOPE_SYSTEM);
+        dispatch_packet(*kernel, grid, block, 0, c->kernarg, fresh ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT, HSA_FENCE_SCOPE_SYSTEM);
     packet.completion_signal = c->done;
     hsa_signal_store_relaxed(c->done, 1);
     bool ok;
@@ -484,7 +484,7 @@ bool aql_fetch(int device, const void* const* src, const size_t* bytes, size_t n
     if (!k) return false;
     BlitArgs a;
     const uint32_t blocks = blit_args(&a, src, bytes, n, host);
-    return aql_call(device, k, blocks, 256, &a, sizeof(a), err);
+    return aql_call(device, k, blocks, 256, &a, sizeof(a), false, err);
 }
 
 bool aql_pass_mirror(AqlPass* p, int device, const void* const* src, const size_t* bytes, size_t n, size_t reserve, const char** host,

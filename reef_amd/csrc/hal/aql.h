@@ -23,12 +23,12 @@ std::shared_ptr<AqlCode> aql_code_from_file(const char* path);
 
 // A kernel of `code` (loaded on `device` if it is not yet), valid as long as the code is.  nullptr and *err: not found.
 const AqlKernel* aql_kernel(AqlCode* code, int device, const char* name, std::string* err);
-// One launch of `groups` workgroups of `threads`, waited for: it sees what finished kernels and the
-// runtime's copies have written (what a launch through the runtime sees; the runtime empties the caches in
-// front of a copy), and its results are visible everywhere when this returns.  Calls of several threads
-// run beside each other.
+// One launch of `groups` workgroups of `threads`, waited for: it sees what finished kernels have written --
+// and, `fresh`, what anybody else has (the caller's copies are other agents' stores to the device, which an acquire at
+// agent scope promises nothing of) -- and its results are visible everywhere when this returns.  Calls of several
+// threads run beside each other.
 bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t threads, const void* kernarg, size_t kernarg_bytes,
-              std::string* err);
+              bool fresh, std::string* err);
 // Makes what one call in flight needs, so that a first call allocates nothing (one beside another does).
 bool aql_call_prepare(int device, std::string* err);
 

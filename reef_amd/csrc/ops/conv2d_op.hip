@@ -411,7 +411,7 @@ int launch_and_wait(DeviceState& d, int device, const Plan& p) {
     const hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
     std::string err;
-    if (!reef::hal::aql_call(device, d.aql_fn[p.kernel], p.tasks, REEF_WG_THREADS, &p.desc, sizeof(p.desc), &err))
+    if (!reef::hal::aql_call(device, d.aql_fn[p.kernel], p.tasks, REEF_WG_THREADS, &p.desc, sizeof(p.desc), true, &err))
         return fail("reef_ops_conv2d: " + err);     // (what the launch may still read stays in use)
     return 0;
 }

@@ -1,6 +1,8 @@
 """reef_ops_conv2d: one fused convolution on plain device pointers (the call a kernel of the
 reference's fused_nn_conv2d_* family serves, resource/resnet152/resnet152.cu:35,376) against the
 CPU oracle, through the C-ABI.  Tolerance: 1e-4 of the output's largest magnitude (fp32)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -98,3 +100,30 @@ def test_a_call_runs_with_its_own_arguments_whatever_came_before(noalloc):
                 assert B.ops_conv2d(d, (x, x2)[i], (w, w2)[j], None, None, o, noalloc=noalloc) == 0, B.last_error()
         for n, o in enumerate(outs):
             np.testing.assert_array_equal(o.to_array(), want[(n + rep) % 2, (n // 2 + rep) % 2])
+
+
+@pytest.mark.parametrize("case", [(64, 14, 14, 64, 1, 1, 0, 1, True, True), (1024, 14, 14, 256, 1, 1, 0, 1, True, False),
+                                  (64, 112, 112, 64, 3, 1, 1, 0, True, True)])
+def test_a_call_sees_what_the_caller_has_uploaded_since_the_last(case):
+    """Operands that earlier calls have left in the caches are replaced by copies of up to 3 MiB, one at a time."""
+    B.ops_init()
+    d, _, first, shape = device_layer(case, 1)
+    sets = [device_layer(case, seed)[1:3] for seed in (1, 2)]
+    n = 4 * int(np.prod(shape))
+
+    def call(bufs, out, noalloc=False):
+        assert B.ops_conv2d(d, *bufs, out, noalloc=noalloc) == 0, B.last_error()
+        return out.to_array()
+
+    state = [0, 0, 0, 0]
+    out = B.DeviceBuffer(n)
+    for step in range(24):
+        operand = step % 4
+        if first[operand] is None:
+            continue
+        call(first, out, step % 3 == 0)
+        state[operand] ^= 1
+        a = sets[state[operand]][0][operand]
+        assert B.lib().reef_hal_memcpy_h2d(first[operand].ptr, a.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(a.nbytes)) == 0
+        mixed = [sets[s][1][k] for k, s in enumerate(state)]
+        np.testing.assert_array_equal(call(first, out, step % 3 == 0), call(mixed, B.DeviceBuffer(n)))
