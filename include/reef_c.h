@@ -211,8 +211,8 @@ int reef_ops_conv2d(const reef_conv2d_desc* c, const float* in, const float* w, 
  * serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.
  * The partial tiles and arrival counters of a split K live in a fixed array in device memory
  * that belongs to this library (4 MiB of partial tiles + 16384 counters per GPU, held until the
- * process ends; the counters are zero between calls); the call allocates and frees nothing,
- * enqueues the convolution and returns without waiting.  A layer whose
+ * process ends); the call allocates and frees nothing, enqueues the convolution -- a split one behind
+ * a small launch that clears its counters -- and returns without waiting.  A layer whose
  * split needs more than the array holds is refused with Status::Fail and a message saying so
  * (reef_ops_scratch_bytes() = bytes of partial tiles the array holds; the library's own choice
  * of split stays within it for every shape it accepts).  reef_ops_init must have
@@ -223,7 +223,9 @@ int reef_ops_conv2d_noalloc(const reef_conv2d_desc* c, const float* in, const fl
                             const float* residual, float* out, void* stream);
 size_t reef_ops_scratch_bytes(void);
 /* reef_ops_conv2d (noalloc 0) or reef_ops_conv2d_noalloc (1) on the default stream, behind everything the
- * device was given before; the output is complete when it returns. */
+ * device was given before; the output is complete when it returns.  Calls of several threads are
+ * safe: with noalloc 1 they have an array of their own beside reef_ops_conv2d_noalloc's, and those that
+ * split K take turns with it. */
 int reef_ops_conv2d_wait(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
                          const float* residual, float* out, int noalloc);
 /* Frees the idle workspaces of reef_ops_conv2d. */

@@ -28,9 +28,12 @@
 #include "reef_hal.h"
 #include "reef_kernels.h"
 
+// hal_device.hip
+int reef_hal_hip_fill(hipStream_t stream, void* p, int byte, size_t n);
+
 namespace {
 
-// ---- scratch of the allocation-free entry point -------------------------------------------
+// ---- scratch of the allocation-free entry points ------------------------------------------
 // [0, kCounterBytes): one arrival counter per output tile; [kCounterBytes, ..): partial tiles.
 constexpr size_t kCounterBytes = 64 * 1024;
 // The plan below splits K only where the partial tiles of all splits fit in here; the size check in
@@ -38,6 +41,8 @@ constexpr size_t kCounterBytes = 64 * 1024;
 constexpr size_t kWorkspaceBytes = 4u * 1024 * 1024;
 constexpr size_t kScratchBytes = kCounterBytes + kWorkspaceBytes;
 static __device__ __align__(256) __attribute__((used)) unsigned char scratch[kScratchBytes];
+// The waited calls' own: they take turns with it (DeviceState::wait_mtx), whatever callers do with streams.
+static __device__ __align__(256) __attribute__((used)) unsigned char wait_scratch[kScratchBytes];
 
 // ---- kernels ----------------------------------------------------------------------------------
 // What a kernel of a family needs of the filter.
@@ -183,6 +188,8 @@ struct DeviceState {
     hipModule_t module = nullptr;
     hipFunction_t fn[kNumKernels] = {};
     unsigned char* scratch_ptr = nullptr;   // device address of `scratch` on this GPU
+    unsigned char* wait_scratch_ptr = nullptr;
+    std::mutex wait_mtx;                    // held while a waited call uses wait_scratch
     // the same kernels for launches that the call waits for (reef_ops_conv2d_wait); null: not available
     std::shared_ptr<reef::hal::AqlCode> aql;
     const reef::hal::AqlKernel* aql_fn[kNumKernels] = {};
@@ -222,6 +229,9 @@ int ensure_device(DeviceState** out, bool may_set_up = true, int* device = nullp
         e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !p) return hip_fail(e, "hipGetSymbolAddress(scratch)");
         d.scratch_ptr = (unsigned char*)p;
+        e = hipGetSymbolAddress(&p, HIP_SYMBOL(wait_scratch));
+        if (e != hipSuccess || !p) return hip_fail(e, "hipGetSymbolAddress(wait_scratch)");
+        d.wait_scratch_ptr = (unsigned char*)p;
         if (reef::hal::aql_available(dev)) {
             std::string why;
             d.aql = reef::hal::aql_code_from_file(g_co_path.c_str());
@@ -456,7 +466,7 @@ void set_scratch(Plan* p, unsigned char* block) {
     p->desc.ptr[p->sync_slot] = block;
 }
 
-// The layer must fit the fixed array (the choice of split stays within it).
+// The layer must fit a fixed array (the choice of split stays within it).
 int check_scratch(const Plan& p) {
     if (p.ws_floats * 4 <= kWorkspaceBytes && (size_t)p.tiles * 4 <= kCounterBytes) return 0;
     char msg[200];
@@ -477,10 +487,17 @@ int run(const reef_conv2d_desc* c, const float* in, const float* w, const float*
     Plan p;
     if (int rc = make_plan(c, in, w, bias, residual, out, &p)) return rc;
     unsigned char* block = nullptr;
+    std::unique_lock<std::mutex> turn;
     if (p.split_k > 1) {
         if (int rc = check_scratch(p)) return rc;
-        if (fixed_scratch) set_scratch(&p, d->scratch_ptr);
-        else {
+        if (fixed_scratch && wait) {
+            turn = std::unique_lock<std::mutex>(d->wait_mtx);
+            set_scratch(&p, d->wait_scratch_ptr);       // its counters are zero at rest, as a pool block's
+        } else if (fixed_scratch) {
+            set_scratch(&p, d->scratch_ptr);
+            // Calls that overlap although they must not leave counts behind: this launch starts from zero all the same.
+            if (int rc = reef_hal_hip_fill(stream, d->scratch_ptr, 0, (size_t)p.tiles * 4)) return rc;
+        } else {
             if (int rc = take_block(d, &block)) return rc;
             set_scratch(&p, block);
         }

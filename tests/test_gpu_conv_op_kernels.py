@@ -40,7 +40,7 @@ def test_matches_oracle_call_after_call(case):
     B.ops_init()
     d, (x, w, b), out, ref = make(case)
     got = []
-    for noalloc in (False, False, True, True):      # host, then device copy of the arguments; pool, then fixed array
+    for noalloc in (False, False, True, True):      # pool, then fixed array; each again with what the last left
         out.fill(0xFF)
         assert B.ops_conv2d(d, x, w, b, None, out, noalloc=noalloc) == 0, B.last_error()
         got.append(out.to_array())

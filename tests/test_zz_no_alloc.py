@@ -6,7 +6,7 @@ import pytest
 
 from reef_amd import binding as B
 from tests.helpers import max_rel_err, REL_TOL
-from tests.test_gpu_conv_op import run_case, RNG
+from tests.test_gpu_conv_op import device_layer, run_case, RNG
 
 pytestmark = pytest.mark.gpu
 
@@ -53,9 +53,53 @@ def test_no_alloc_needs_init_and_states_its_limit():
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
                        cwd=__import__("os").path.dirname(__import__("os").path.dirname(__import__("os").path.abspath(__file__))))
     assert r.returncode == 0, (r.stdout, r.stderr)
-    # The size check of the entry point is a guard that no shape reaches today: its plan puts at most
-    # 256 workgroups on a split layer and a workgroup's tile has at most 64 x 64 outputs, so the
-    # partial tiles never exceed 256 x 4096 floats = the 4 MiB array, and a split layer has at most
-    # 128 tiles against 16384 counters.  The largest such layer goes through and matches:
+    # The size check of the entry point is a guard that no shape reaches today: the choice of kernel only
+    # considers splits whose partial tiles fit the 4 MiB array and that put at most 640 workgroups on a
+    # layer, so a split layer has at most 320 tiles against 16384 counters.  A deep one goes through
+    # and matches:
     B.ops_init()
     both((2048, 7, 7, 2048, 1, 1, 0, 0, False, False))
+
+
+def test_waited_calls_of_several_threads_do_not_share_their_scratch():
+    """Split layers of two sizes from four threads, beside calls on the default stream with the other fixed array: every
+    output holds the bits of the call made alone, and so does every call afterwards."""
+    import ctypes
+    import threading
+
+    B.ops_init()
+    layers = [device_layer(c, 5 + i) for i, c in enumerate(((1024, 14, 14, 256, 1, 1, 0, 1, True, False),
+                                                            (256, 7, 7, 64, 3, 1, 1, 1, True, True)))]
+    outs = [[B.DeviceBuffer(4 * int(np.prod(l[3]))) for l in layers] for _ in range(5)]
+    want = []
+    for l, o in zip(layers, outs[0]):
+        assert B.ops_conv2d(l[0], *l[2], o) == 0, B.last_error()
+        want.append(o.to_array())
+    bad = []
+
+    def waited(mine):
+        for rep in range(60):
+            k = (rep + mine) % 2
+            o = outs[mine][k]
+            if B.ops_conv2d(layers[k][0], *layers[k][2], o, noalloc=True) or not np.array_equal(o.to_array(), want[k]):
+                bad.append((mine, rep))
+
+    def on_the_stream():
+        L = B.lib()
+        for rep in range(60):
+            d, _, (x, w, bias, res), _ = layers[rep % 2]
+            o = outs[4][rep % 2]
+            st = L.reef_ops_conv2d_noalloc(ctypes.byref(d), x.ptr, w.ptr, bias.ptr if bias else None, res.ptr if res else None, o.ptr, None)
+            if st or not np.array_equal(o.to_array(), want[rep % 2]):
+                bad.append(("stream", rep))
+
+    threads = [threading.Thread(target=waited, args=(i,)) for i in range(4)] + [threading.Thread(target=on_the_stream)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for k, l in enumerate(layers):
+        for noalloc in (False, True):
+            assert B.ops_conv2d(l[0], *l[2], outs[0][k], noalloc=noalloc) == 0
+            np.testing.assert_array_equal(outs[0][k].to_array(), want[k])
