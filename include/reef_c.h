@@ -222,8 +222,8 @@ int reef_ops_conv2d(const reef_conv2d_desc* c, const float* in, const float* w, 
 int reef_ops_conv2d_noalloc(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
                             const float* residual, float* out, void* stream);
 size_t reef_ops_scratch_bytes(void);
-/* reef_ops_conv2d (noalloc 0) or reef_ops_conv2d_noalloc (1) on the default stream, behind everything the
- * device was given before; the output is complete when it returns.  Calls of several threads are
+/* reef_ops_conv2d (noalloc 0) or reef_ops_conv2d_noalloc (1) on the default stream: behind what that
+ * stream and the blocking streams were given before, beside what non-blocking streams run.  The output is complete when it returns.  Calls of several threads are
  * safe: with noalloc 1 they have an array of their own beside reef_ops_conv2d_noalloc's, and those that
  * split K take turns with it. */
 int reef_ops_conv2d_wait(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,

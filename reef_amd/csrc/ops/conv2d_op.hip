@@ -409,17 +409,18 @@ int launch(const DeviceState& d, const Plan& p, hipStream_t stream) {
     return e == hipSuccess ? 0 : hip_fail(e, "hipModuleLaunchKernel");
 }
 
-// Launches on the default stream and returns when the result is there.  Work that the device was given
-// before (the layer's inputs among it) ends first; then the launch is one packet on a queue of this
-// library's own, whose completion the host sees 3 us earlier than it sees a stream go idle.
+// Launches on the default stream and returns when the result is there.  What that stream waits for (its own work and
+// the blocking streams', the layer's inputs among it) ends first; then the launch is one packet on a queue of this
+// library's own, whose completion the host sees 3 us earlier than it sees a stream go idle.  Work of
+// non-blocking streams runs beside it, as beside a launch on the default stream.
 int launch_and_wait(DeviceState& d, int device, const Plan& p) {
     if (!d.aql) {
         if (int rc = launch(d, p, nullptr)) return rc;
-        const hipError_t e = hipDeviceSynchronize();
-        return e == hipSuccess ? 0 : hip_fail(e, "hipDeviceSynchronize");
+        const hipError_t e = hipStreamSynchronize(nullptr);
+        return e == hipSuccess ? 0 : hip_fail(e, "hipStreamSynchronize");
     }
-    const hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
+    const hipError_t e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
     std::string err;
     if (!reef::hal::aql_call(device, d.aql_fn[p.kernel], p.tasks, REEF_WG_THREADS, &p.desc, sizeof(p.desc), true, &err))
         return fail("reef_ops_conv2d: " + err);     // (what the launch may still read stays in use)

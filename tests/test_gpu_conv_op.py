@@ -127,3 +127,27 @@ def test_a_call_sees_what_the_caller_has_uploaded_since_the_last(case):
         assert B.lib().reef_hal_memcpy_h2d(first[operand].ptr, a.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(a.nbytes)) == 0
         mixed = [sets[s][1][k] for k, s in enumerate(state)]
         np.testing.assert_array_equal(call(first, out, step % 3 == 0), call(mixed, B.DeviceBuffer(n)))
+
+
+@pytest.mark.parametrize("case", [(64, 14, 14, 64, 1, 1, 0, 1, True, True), (1024, 14, 14, 256, 1, 1, 0, 1, True, False)])
+def test_a_waited_call_follows_the_default_stream_and_no_other(case):
+    B.ops_init()
+    L, size_t = B.lib(), ctypes.c_size_t
+    d, _, bufs, shape = device_layer(case, 3)
+    x, out = bufs[0], B.DeviceBuffer(4 * int(np.prod(shape)))
+    x.fill(0)
+    assert B.ops_conv2d(d, *bufs, out) == 0, B.last_error()
+    want = out.to_array()
+    x.fill(0xFF)
+    big, side, idle = B.DeviceBuffer(1 << 30), ctypes.c_void_p(), ctypes.c_int()
+    assert L.reef_hal_stream_create(0, ctypes.byref(side)) == 0      # a non-blocking one
+    assert L.reef_hal_device_sync() == 0
+    for _ in range(200):                                   # 1 GiB each: 30 ms and more
+        assert L.reef_hal_memset_async(big.ptr, 0, size_t(big.nbytes), side) == 0
+    for byte in (0xFF,) * 20 + (0,):                       # the default stream's last launch stores the input
+        assert L.reef_hal_memset_async(x.ptr, byte, size_t(x.nbytes), None) == 0
+    assert B.ops_conv2d(d, *bufs, out) == 0, B.last_error()
+    assert L.reef_hal_stream_query(side, ctypes.byref(idle)) == 0
+    np.testing.assert_array_equal(out.to_array(), want)
+    assert not idle.value
+    assert L.reef_hal_stream_destroy(side) == 0
