@@ -29,11 +29,13 @@ std::string hsa_text(hsa_status_t s, const char* what) {
 }
 
 // One hardware queue; passes of several threads interleave whole (the mutex is held while a
-// pass's packets are written, not while they run).
+// pass's packets are written, not while they run).  Every packet waits for the one in front of it (barrier bit), so
+// whoever submits behind another's packets waits for all of them: `load` counts those that have not ended.
 struct Queue {
     hsa_queue_t* q = nullptr;
     std::mutex mtx;
     std::atomic<int> error{0};
+    std::atomic<uint32_t> load{0};
 };
 void on_queue_error(hsa_status_t s, hsa_queue_t*, void* data) { ((Queue*)data)->error.store((int)s); }
 
@@ -45,15 +47,15 @@ constexpr size_t kAqlCallArgs = 512;     // the argument block of a single launc
 struct Call {
     hsa_signal_t done{};
     char* kernarg = nullptr;
-    Queue* queue = nullptr;
 };
 
 struct Device {
     bool tried = false, ok = false;
     hsa_agent_t agent{};
     volatile uint32_t* flush = nullptr;   // a store here pushes out what the host has stored into device memory
-    Queue* queues[kMaxQueues] = {};   // opened as passes need them, kept for the life of the process
-    unsigned next = 0;
+    Queue* queues[kMaxQueues] = {};   // one for each pass and call in flight until there are kMaxQueues, kept for the life of the process
+    std::atomic<unsigned> open{0};
+    std::mutex choose_mtx;
     std::vector<Call*> idle;     // calls that have ended, for the next ones: as many as ever ran at once
     std::mutex idle_mtx;
 };
@@ -103,23 +105,35 @@ bool set_up(int device) {
     return true;
 }
 
-// The next queue in turn.  Caller holds g_mtx.
-Queue* take_queue(Device& d, std::string* err) {
-    Queue*& q = d.queues[d.next % kMaxQueues];
-    if (!q) {
-        Queue* nq = new Queue;
-        const hsa_status_t s = hsa_queue_create(d.agent, kQueuePackets, HSA_QUEUE_TYPE_MULTI, on_queue_error, nq, UINT32_MAX,
-                                                UINT32_MAX, &nq->q);
-        if (s != HSA_STATUS_SUCCESS) {
-            delete nq;
-            *err = hsa_text(s, "hsa_queue_create");
-            return nullptr;
-        }
-        q = nq;
+// One more user of the device's queues.  Caller holds g_mtx.
+bool add_queue(Device& d, std::string* err) {
+    const unsigned n = d.open.load();
+    if (n == (unsigned)kMaxQueues) return true;
+    Queue* q = new Queue;
+    const hsa_status_t s = hsa_queue_create(d.agent, kQueuePackets, HSA_QUEUE_TYPE_MULTI, on_queue_error, q, UINT32_MAX,
+                                            UINT32_MAX, &q->q);
+    if (s != HSA_STATUS_SUCCESS) {
+        delete q;
+        *err = hsa_text(s, "hsa_queue_create");
+        return false;
     }
-    d.next++;
+    d.queues[n] = q;
+    d.open.store(n + 1);
+    return true;
+}
+
+// The queue that this many packets wait the least in; they count as its load until leave_queue.
+Queue* enter_queue(Device& d, uint32_t packets) {
+    std::lock_guard<std::mutex> lock(d.choose_mtx);
+    const unsigned n = d.open.load();
+    auto load = [](Queue* q) { return q->error.load() ? UINT32_MAX : q->load.load(); };
+    Queue* q = d.queues[0];
+    for (unsigned i = 1; i < n; ++i)
+        if (load(d.queues[i]) < load(q)) q = d.queues[i];
+    q->load.fetch_add(packets);
     return q;
 }
+void leave_queue(Queue* q, uint32_t packets) { q->load.fetch_sub(packets); }
 
 }  // namespace
 
@@ -332,18 +346,37 @@ Call* take_call(int device, std::string* err) {
     if (e != hipSuccess) { *err = std::string("argument block: ") + hipGetErrorString(e); return nullptr; }
     c->kernarg = (char*)p;
     const hsa_status_t s = hsa_signal_create(0, 0, nullptr, &c->done);
-    if (s == HSA_STATUS_SUCCESS) {
+    bool ok = s == HSA_STATUS_SUCCESS;
+    if (ok) {
         std::lock_guard<std::mutex> lock(g_mtx);
-        c->queue = take_queue(d, err);
+        ok = add_queue(d, err);
+        if (!ok) hsa_signal_destroy(c->done);
     } else {
         *err = hsa_text(s, "hsa_signal_create");
     }
-    if (!c->queue) {
-        if (s == HSA_STATUS_SUCCESS) hsa_signal_destroy(c->done);
+    if (!ok) {
         (void)hipHostFree(p);
         return nullptr;
     }
     return c.release();
+}
+
+// Submits a packet that signals c->done and waits for it; then the call is idle again.
+bool run_call(int device, Call* c, const hsa_kernel_dispatch_packet_t& packet, std::string* err) {
+    Device& d = g_devices[device];
+    hsa_signal_store_relaxed(c->done, 1);
+    Queue* w = enter_queue(d, 1);
+    bool ok;
+    {
+        std::lock_guard<std::mutex> submit(w->mtx);
+        ok = put_packet(*w, packet, true, err);
+    }
+    ok = ok && wait_done(*w, c->done, err);
+    leave_queue(w, 1);
+    if (!ok) return false;      // the device may still use what the call owns: it is not handed on
+    std::lock_guard<std::mutex> lock(d.idle_mtx);
+    d.idle.push_back(c);
+    return true;
 }
 
 }  // namespace
@@ -366,22 +399,11 @@ bool aql_call(int device, const AqlKernel* kernel, uint32_t groups, uint32_t thr
     hsa_kernel_dispatch_packet_t packet =
         dispatch_packet(*kernel, grid, block, 0, c->kernarg, fresh ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT, HSA_FENCE_SCOPE_SYSTEM);
     packet.completion_signal = c->done;
-    hsa_signal_store_relaxed(c->done, 1);
-    bool ok;
-    {
-        std::lock_guard<std::mutex> submit(c->queue->mtx);
-        ok = put_packet(*c->queue, packet, true, err);
-    }
-    ok = ok && wait_done(*c->queue, c->done, err);
-    if (!ok) return false;      // the device may still use what the call owns: it is not handed on
-    Device& d = g_devices[device];
-    std::lock_guard<std::mutex> lock(d.idle_mtx);
-    d.idle.push_back(c);
-    return true;
+    return run_call(device, c, packet, err);
 }
 
 struct AqlPass {
-    Queue* queue = nullptr;
+    int device = -1;
     hsa_signal_t done{};
     void* kernargs = nullptr;    // device memory, one 64-byte aligned block per launch
     char* mirror = nullptr;      // host memory, what aql_pass_mirror's launch fills
@@ -438,8 +460,8 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
     const hsa_status_t s = hsa_signal_create(0, 0, nullptr, &p->done);
     if (s != HSA_STATUS_SUCCESS) { *err = hsa_text(s, "hsa_signal_create"); return nullptr; }
     if (n) p->packets.back().completion_signal = p->done;
-    p->queue = take_queue(d, err);
-    return p->queue ? p.release() : nullptr;
+    p->device = device;
+    return add_queue(d, err) ? p.release() : nullptr;
 }
 
 bool aql_pass_block(AqlPass* p, size_t i, char** device, char** host, size_t* bytes, size_t* tail) {
@@ -549,35 +571,28 @@ bool aql_fence(int device, std::string* err) {
     static_assert(sizeof(b) == sizeof(hsa_kernel_dispatch_packet_t), "packets are of one size");
     hsa_kernel_dispatch_packet_t packet;
     std::memcpy(&packet, &b, sizeof(b));
-    hsa_signal_store_relaxed(c->done, 1);
-    bool ok;
-    {
-        std::lock_guard<std::mutex> submit(c->queue->mtx);
-        ok = put_packet(*c->queue, packet, true, err);
-    }
-    if (!ok || !wait_done(*c->queue, c->done, err)) return false;
-    std::lock_guard<std::mutex> lock(g_devices[device].idle_mtx);
-    g_devices[device].idle.push_back(c);
-    return true;
+    return run_call(device, c, packet, err);
 }
 
 bool aql_pass_run(AqlPass* p, bool fresh, std::string* err) {
     if (p->packets.empty()) return true;
     if (!p->committed) { *err = "the pass has not been committed"; return false; }
     std::lock_guard<std::mutex> lock(p->mtx);
-    Queue& w = *p->queue;
     uint16_t& first = p->packets[0].header;
     first = (uint16_t)((first & ~(3 << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE)) |
                        ((fresh ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT) << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE));
     hsa_signal_store_relaxed(p->done, 1);
+    const size_t n = p->packets.size();
+    Queue& w = *enter_queue(g_devices[p->device], (uint32_t)n);
+    bool ok = true;
     {
         std::lock_guard<std::mutex> submit(w.mtx);
-        const size_t n = p->packets.size();
         // the device starts on the first packets while the rest are written
-        for (size_t i = 0; i < n; ++i)
-            if (!put_packet(w, p->packets[i], i == n - 1 || (i & 31) == 3, err)) return false;
+        for (size_t i = 0; i < n && ok; ++i) ok = put_packet(w, p->packets[i], i == n - 1 || (i & 31) == 3, err);
     }
-    return wait_done(w, p->done, err);
+    ok = ok && wait_done(w, p->done, err);
+    leave_queue(&w, (uint32_t)n);
+    return ok;
 }
 
 void aql_pass_destroy(AqlPass* p) { delete p; }
