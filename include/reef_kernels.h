@@ -240,8 +240,9 @@ enum {
  *   reef_conv2d_u_<tile>    unaligned: im2col gather, any K
  *   reef_conv2d_d<R>_16x<BN>k4  direct: R = kh*kw taps compiled in (1, 3, 7, 9 for BN = 16, 32; 1, 9 for 16x64 and 32x32d4); operands go from memory
  *                           straight into 16x16x4 MFMAs, the four wavefronts split the input
- *                           channels.  d1 needs Cin % 8 == 0 (any stride); K_CHUNK is a multiple
- *                           of R (R > 1) or 8 (d1) and splits K on channel boundaries.
+ *                           channels.  d1 needs Cin % 4 == 0 (any stride; of a graph file's layers
+ *                           Cin % 8 == 0 is asked); K_CHUNK is a multiple of R (R > 1) or 4 (d1) and
+ *                           splits K on channel boundaries.
  *   reef_conv2d_f<R>_<direct tile>  (raw code object) direct, R = kw taps a filter row (3, 5, 7), any kh;
  *                           K_CHUNK is a multiple of 16 R.
  *   reef_conv2d_o1_<direct tile>    (raw code object) direct, 1x1, any Cin; K_CHUNK a multiple of 128.

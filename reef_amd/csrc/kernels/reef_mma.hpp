@@ -755,7 +755,7 @@ __device__ __forceinline__ bool conv2d_body(const ReefOpDesc& d_in, int task, ch
 //          R contiguous weights W[m][c + kq][0..R) and the R taps in[c + kq][iy(t)][ix(t)] of
 //          its output pixel; MFMA t multiplies tap t of four channels.  Tap offsets and their
 //          padding validity are fixed per lane for the whole kernel.
-//   R = 1: k slot kq covers eight channels c + 8 kq .. + 8: two 128-bit weight loads and eight
+//   R = 1: k slot kq covers four channels c + 4 kq .. + 4: one 128-bit weight load and four
 //          pixel loads; MFMA j multiplies channel j of each slot.  Any stride.
 // No LDS and no barrier inside the K loop, so NS steps of loads are in flight per wavefront
 // (a wavefront may have 63 vector-memory instructions outstanding; NS steps are up to 60 of
@@ -812,7 +812,7 @@ struct DirectGeom {
 // 16-lane row (kx = 0: from lane - 1, lane 0 from lane 15; kx = 2: from lane + 1, lane 13 from
 // lane 14), the three vertical taps are the rows g, g + 1, g + 2.  Every input value is fetched
 // once per tile instead of once per tap: G + 2 loads per step instead of 9 G, so the loads of
-// up to eight K steps are in flight per wavefront.  Lanes 14 and 15 compute columns nobody
+// several K steps are in flight per wavefront.  Lanes 14 and 15 compute columns nobody
 // stores.  Same sum order over k as the tap form (channel-major steps, taps in filter order).
 constexpr int kRowSeg = 14;
 __device__ __forceinline__ float lane_from_left(float v) {   // lane i <- lane (i - 1) mod 16 of its row
@@ -835,8 +835,8 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane i <- lane (
 // PRE (1-tap kernels only, symbols reef_conv2d_p1_*): the layer reads its input through a
 // per-channel scale, shift and ReLU -- the pre-activation of a DenseNet layer, which cannot be
 // folded into the producing convolution because every consumer of the concatenation has its own.
-// The eight input values a lane loads per step are eight consecutive channels, so their scales
-// and shifts are two 128-bit loads each; a channel past the split loads scale = shift = 0 and
+// The four input values a lane loads per step are four consecutive channels, so their scales
+// and shifts are one 128-bit load each; a channel past the split loads scale = shift = 0 and
 // contributes relu(0) = 0.  REEF_F_PRE_ACT; the two vectors follow the optional epilogue operands.
 //
 // PACKED (filters with several taps; symbols reef_conv2d_d<R>k_* / reef_conv2d_r9k_*): the weights

@@ -61,9 +61,12 @@ enum Family {
 //     c0 + w (c1 + c2 (r + ceil(r)) / 2 + c3 max(1, r)) + c4 r   (+ c5 + c6 split / 10 where K is split)
 // w: thousands of products per output of one workgroup, in whole steps; r: workgroups per CU.  c1 is the
 // serial chain of a workgroup, c2 and c3 the CU's matrix pipes and loads, c4 a workgroup's start and
-// end, c5 and c6 the fold.  Fitted per kernel to 36 000 launches of 1500 shapes (3..768 channels in, 8..768
-// out, images of 7..160, filters of 1, 3, 5, 7, strides 1 and 2), with which the choice is 1.2 % slower than
-// the fastest of every shape on average.  Against one tile per filter (16 x 32 at 1x1, two image rows
+// end, c5 and c6 the fold.  The 1x1, filter-row and image-row families are fitted per kernel to 36 000 launches of 1500
+// shapes (3..768 channels in, 8..768 out, images of 7..160, square filters of 1, 3, 5, 7, strides 1 and 2), with which
+// the choice is 1.2 % slower than the fastest of every shape on average.  Filters that none of them takes are not
+// among those shapes, and their rows are taken from others: the tap kernels' (3x1, 7x1) from the row
+// kernels of as many taps, the staged ones' from the fit of launches inside models ("n" in modelgen/tiling.py), aligned
+// and unaligned loaders and both strides alike.  Those rows order the tiles of one family only.  Against one tile per filter (16 x 32 at 1x1, two image rows
 // at 3x3, staged 64 x 64 at 5x5, 7x7 and odd channel counts), kernel times: 5x5 48 -> 64 at 35x35 31.9 ->
 // 8.1 us, 7x7 209 -> 15 at 12x85 43 -> 9.3, 1x1 161 -> 617 at 23x21 17 -> 5.2, 3x3 256 -> 256 at 112x112
 // 210 -> 144 (103 TFLOP/s of the 152 that fp32 MFMAs reach).

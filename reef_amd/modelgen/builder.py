@@ -587,7 +587,11 @@ class GraphBuilder:
 
     ATTENTION_MAX_SEQ, ATTENTION_MAX_HEAD_DIM, ATTENTION_ROWS = 128, 64, 8    # REEF_AT_* of include/reef_kernels.h
     ATTENTION_MMA_MAX_SEQ, ATTENTION_MMA_ROWS = 512, 16
-    ATTENTION_MMA_FROM = 12      # workgroups from which the matrix cores' form is taken; fewer: twice as many of eight rows
+    # Workgroups from which the matrix cores' form is taken: every launch of BERT-base, whose 12 heads are 12 row
+    # blocks or more (16 tokens 5.72 -> 5.32 us, 128 tokens 7.61 -> 6.22, back to back).  Below, launches of both
+    # forms last 4 to 7 us: heads of 32 and more are up to 1.3 us faster on the matrix cores there too (one head of 64,
+    # 128 tokens: 7.29 -> 6.02), heads of 4 to 16 over a few tokens up to 0.3 us slower (4.22 -> 4.54).
+    ATTENTION_MMA_FROM = 12
 
     @classmethod
     def attention_ok(cls, seq, head_dim, ld, ldo, offs):

@@ -786,3 +786,30 @@ def test_convolution_that_averages_its_own_output(tmp_path, case):
         e.execute_preemptable() if pre else e.execute()
         np.testing.assert_array_equal(e.get_output()[:cout], want, err_msg="flavour %s %s" % (kind, pre))
         e.close()
+
+
+@pytest.mark.parametrize("seq,heads,hd,masked", [(128, 12, 64, False), (128, 2, 64, True), (77, 3, 64, True), (9, 12, 4, False), (1, 1, 64, False)])
+def test_attention_on_the_vector_units(tmp_path, seq, heads, hd, masked):
+    """reef_attention over its whole range, also where the builder would take the matrix cores' form: the largest
+    launch, a row block with one row, the smallest head and a single token.  Tolerance as in the test above it."""
+    hid = heads * hd
+    g = MB.GraphBuilder("attv", weight_std=0.05)
+    qkv = g.input("x", (seq, 3 * hid))
+    mask = g.input("attention_mask", (seq,), "uint1") if masked else None
+    ctx = g.attention(qkv, seq, heads, hd, 3 * hid, 0, hid, 2 * hid, 1.0 / np.sqrt(hd), mask=mask, mma=False)
+    g.mark_output(ctx)
+    assert g.kernels[0]["name"].startswith("reef_attention#")
+    pad = np.zeros(seq, np.uint8)
+    pad[seq - seq // 4:] = 1
+    x = rnd(seq, 3 * hid)
+    exe, orc, model = run_both(g, tmp_path, {"x": x, "attention_mask": pad} if masked else {"x": x})
+    compare_storages(exe, orc, model, what="attention")
+    m = x.reshape(seq, 3, heads, hd).astype(np.float64)
+    sc = np.einsum("shd,thd->hst", m[:, 0], m[:, 1]) / np.sqrt(hd)
+    if masked:
+        sc[:, :, pad != 0] = -np.inf
+    pr = np.exp(sc - sc.max(-1, keepdims=True))
+    pr /= pr.sum(-1, keepdims=True)
+    want = np.einsum("hst,thd->shd", pr, m[:, 2]).reshape(seq, hid)
+    got = exe.get_data(ctx.idx, seq * hid).reshape(seq, hid)
+    assert np.isfinite(got).all() and np.abs(got - want).max() <= 1e-4 * np.abs(want).max()
