@@ -348,3 +348,58 @@ def test_more_best_effort_queues_than_feeder_threads(dirs):
             np.testing.assert_array_equal(s.get_output(m, 1000), ref)
         s.shutdown()
         s.close()
+
+
+def test_a_client_that_polls_reads_its_own_run_once_it_has_waited(dirs):
+    """Both models' results are fetched all the time, before, during and after their runs, while the best-effort model is
+    preempted and padded by the other's requests: whatever the fetches in between see, the ones behind wait_task hold
+    the bits of a solo run on the input that was set last."""
+    import threading
+
+    names = ("resnet50", "resnet18")                       # best effort, real time
+    xs = [nets.image_input("poll%d" % i, (3, 224, 224)) for i in range(2)]
+    scores, want = {}, {}
+    for n in names:
+        model = json.load(open(os.path.join(dirs[n], n + ".json")))
+        scores[n] = model["kernels"][-1]["args"][0]        # what the softmax reads
+        for i, x in enumerate(xs):
+            exe = B.Executor.from_dir(dirs[n], n, B.HYBRID)
+            exe.set_input_checked("data", x)
+            exe.execute()
+            want[n, i] = exe.get_output(), exe.get_data(scores[n], 1000)
+            exe.close()
+    s = B.Scheduler(B.MODE_REEF)
+    mids = {n: s.load_model(dirs[n], n) for n in names}
+    s.bind_model_queue(s.create_queue(B.QUEUE_BE), mids["resnet50"])
+    s.bind_model_queue(s.create_queue(B.QUEUE_RT), mids["resnet18"])
+    s.run()
+    stop, polled = threading.Event(), [0]
+
+    def poll():
+        while not stop.is_set():
+            for n in names:
+                s.get_output(mids[n], 1000)
+                s.get_data(mids[n], scores[n], 1000)
+            polled[0] += 1
+
+    th = threading.Thread(target=poll)
+    th.start()
+    preempted = 0
+    try:
+        for step in range(60):
+            for n in names:
+                assert s.set_input(mids[n], xs[step % 2], "data") == 0
+            be = s.new_task(mids["resnet50"])
+            rts = [s.new_task(mids["resnet18"]) for _ in range(1 + step % 3)]
+            for t in rts + [be]:
+                assert s.wait_task(t) == 0
+            preempted += s.task_info(be)["preempted"]
+            for n in names:
+                for _ in range(2):
+                    np.testing.assert_array_equal(s.get_output(mids[n], 1000), want[n, step % 2][0])
+                    np.testing.assert_array_equal(s.get_data(mids[n], scores[n], 1000), want[n, step % 2][1])
+    finally:
+        stop.set()
+        th.join()
+    assert polled[0] >= 60 and preempted
+    s.shutdown()
