@@ -58,7 +58,8 @@ int reef_executor_load_hybrid(reef_executor_t e, const char* json_path, const ch
     HybridExecutor* h = e->hybrid();
     if (!h) return Status::Fail;
     RETURN_STATUS(h->load_hybrid_model_from_file(json_path, profile_path, trans_co_path, be_co_path));
-    return h->prepare_preemptale();
+    h->prepare_preemptale();
+    return Status::Succ;
 }
 int reef_executor_load_param(reef_executor_t e, const char* p) { return e->exe->load_param_from_file(p); }
 int reef_executor_set_input(reef_executor_t e, const char* name, const void* data, size_t len) {

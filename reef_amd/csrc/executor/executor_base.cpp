@@ -29,13 +29,14 @@ Status ExecutorBase::load_model_from_file(const char* json_file_path, const char
     GPUModule_t mod;
     GPU_RETURN_STATUS(reef_hal_module_load(co_file_path, &mod));
     RETURN_STATUS(this->load_model_from_GPU_module(json_file_path, mod));
-    return ready_model_pass();
+    ready_model_pass();
+    return Status::Succ;
 }
 
-Status ExecutorBase::ready_model_pass() {
-    if (use_graph) return Status::Succ;
+void ExecutorBase::ready_model_pass() {
+    if (use_graph) return;
     std::lock_guard<std::mutex> lock(io_mtx);
-    return ready_pass(model_pass, [this](int i, Launch& l) { return make_launch(i, l); });
+    (void)ready_pass(model_pass, [this](int i, Launch& l) { return make_launch(i, l); });
 }
 
 Status ExecutorBase::load_model_from_GPU_module(const char* json_file_path, GPUModule_t mod) {

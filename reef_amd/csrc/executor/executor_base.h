@@ -108,7 +108,8 @@ protected:
     // allocations and the upload; a first run does it where a model was loaded without.  Caller holds io_mtx.
     template <class Make>
     Status ready_pass(Pass& p, const Make& make);
-    Status ready_model_pass();
+    // At load: what cannot be recorded now is tried again, and the reason reported, by the first run.
+    void ready_model_pass();
     Status record_pass(Pass& p, std::vector<Launch>& launches);
     void drop_pass(Pass& p);
 public:
@@ -167,7 +168,11 @@ Status ExecutorBase::ready_pass(Pass& p, const Make& make) {
     if (p.tried) return Status::Succ;
     std::vector<Launch> l(num_kernels());
     for (size_t i = 0; i < l.size(); i++) RETURN_STATUS(make((int)i, l[i]));
-    RETURN_STATUS(record_pass(p, l));
+    const Status st = record_pass(p, l);
+    if (st != Status::Succ) {
+        drop_pass(p);
+        return st;
+    }
     p.tried = true;
     return Status::Succ;
 }

@@ -34,7 +34,8 @@ Status HybridExecutor::load_hybrid_model_from_file(const char* json_file_path,
     GPU_RETURN_STATUS(reef_hal_module_load(preempt_co_file_path, &preempt_module));
     RETURN_STATUS(load_hybrid_model_from_GPU_module(json_file_path, profile_file_path, trans_module,
                                                     preempt_module));
-    return ready_model_pass();
+    ready_model_pass();
+    return Status::Succ;
 }
 
 Status HybridExecutor::load_hybrid_model_from_GPU_module(const char* json_file_path,
@@ -109,9 +110,9 @@ Status HybridExecutor::set_preempt_flag(GPUDevicePtr_t flag) {
     return Status::Succ;
 }
 
-Status HybridExecutor::prepare_preemptale() {
+void HybridExecutor::prepare_preemptale() {
     std::lock_guard<std::mutex> lock(io_mtx);
-    return ready_pass(preempt_pass, [this](int i, Launch& l) { return make_preempt_launch(i, l); });
+    (void)ready_pass(preempt_pass, [this](int i, Launch& l) { return make_preempt_launch(i, l); });
 }
 
 Status HybridExecutor::execute_preemptale(GPUStream_t stream) {

@@ -26,8 +26,8 @@ public:
                                              GPUModule_t trans_module, GPUModule_t preempt_module);
 
     Status execute_preemptale(GPUStream_t stream = GPUStreamDefault);  // spelling as in the reference
-    // For models whose best-effort flavour is run whole (a scheduler launches it kernel by kernel).
-    Status prepare_preemptale();
+    // At load, for models whose best-effort flavour is run whole (a scheduler launches it kernel by kernel).
+    void prepare_preemptale();
     Status set_preempt_flag(GPUDevicePtr_t flag);
 
     Status reset_task_slot_async(int kernel_offset, GPUStream_t stream);

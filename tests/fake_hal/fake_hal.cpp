@@ -81,6 +81,7 @@ std::vector<LogEntry> g_log;
 int g_auto_progress = 1;  // kernels completed per stream_query
 bool g_passes = false, g_host_writes = false, g_unseen = false;
 long g_pass_creates = 0, g_pass_runs = 0, g_fetches = 0, g_stale = 0, g_mallocs = 0, g_frees = 0, g_pass_mirrors = 0;
+int g_pass_failures = 0;           // pass_create calls that fail from now on
 void (*g_pass_hook)(int) = nullptr;   // called with 0 in the middle of every pass and with 1 at its end
 
 reef_stream_s* S(reef_stream_t s) { return s ? s : &g_null_stream; }
@@ -324,6 +325,11 @@ int f_graph_destroy(reef_graph_t g) { delete g; return 0; }
 int f_pass_create(const reef_pass_launch* l, size_t n, size_t tail, reef_pass_t* out) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);
     if (!g_passes) return 2;
+    if (g_pass_failures > 0) {
+        --g_pass_failures;
+        reef_hal_set_error("fake: no pass");
+        return 1;
+    }
     ++g_pass_creates;
     reef_pass_s* p = new reef_pass_s;
     for (size_t i = 0; i < n; ++i) {
@@ -466,7 +472,9 @@ void fake_hal_reset(void) {
     g_passes = g_host_writes = g_unseen = false;
     g_pass_creates = g_pass_runs = g_fetches = g_stale = g_mallocs = g_frees = g_pass_mirrors = 0;
     g_pass_hook = nullptr;
+    g_pass_failures = 0;
 }
+void fake_hal_set_pass_failures(int n) { std::lock_guard<std::recursive_mutex> lock(g_mtx); g_pass_failures = n; }
 // 1: passes, fetches and stores past the caches; 2: without the last
 void fake_hal_set_passes(int on) {
     std::lock_guard<std::recursive_mutex> lock(g_mtx);

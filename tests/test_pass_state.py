@@ -165,3 +165,16 @@ def test_a_scheduled_real_time_request_records_and_allocates_nothing(fake, mocke
     np.testing.assert_array_equal(s.get_output(m, N), np.full(N, 18, np.float32))
     s.shutdown()
     s.close()
+
+
+@pytest.mark.parametrize("kind", [B.BASE, B.HYBRID])
+def test_a_pass_that_cannot_be_recorded_at_load_is_reported_by_the_run(fake, mocked, kind):
+    name, d = mocked
+    fake.lib.fake_hal_set_pass_failures(3 if kind == B.HYBRID else 2)   # at load, and in the first run
+    exe = B.Executor.from_dir(d, name, kind)
+    set_inputs(exe.set_input_checked, 3.0)
+    with pytest.raises(B.ReefError):
+        exe.execute()
+    exe.execute()
+    np.testing.assert_array_equal(exe.get_output(), np.full(N, 18, np.float32))
+    exe.close()
