@@ -27,7 +27,8 @@
  *   be     K(ReefBeArgs a)  =  (completion record, int* preempted, int* task_slot, ReefOpDesc d)
  *          replaces script/best_effort_kernel.py:22-29: a workgroup leaves at
  *          once when *preempted != 0, re-polls the flag inside its main loop,
- *          and thread 0 adds 1 to *task_slot only when the workgroup completed.
+ *          and *task_slot has grown by the number of workgroups that completed
+ *          when the launch has ended (not before: see be_count_completed).
  *          The completion record (reef_hal.h) lets the launch-window stream the
  *          kernel runs on see it finish without a second device operation: every
  *          workgroup counts itself out as it leaves, preempted or not.

@@ -308,6 +308,16 @@ __device__ __forceinline__ void be_signal_exit(const ReefBeArgs& a, int t) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __hip_atomic_store(a.done_word, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// *task_slot counts the workgroups of a launch that completed, and is read when the launch has ended
+// (the scheduler's wait-based preemption synchronizes the stream first).  One add each costs: adds to
+// one address go through at about ten a microsecond, and a launch ends when its last add has (DenseNet-201 alone:
+// 1314 us a pass with them, 1144 without; 0.8 us a launch).  So the first workgroup adds the number of
+// workgroups, and one that leaves early takes itself off.
+__device__ __forceinline__ void be_count_completed(const ReefBeArgs& a, bool done) {
+    int n = done ? 0 : -1;
+    if ((blockIdx.x | blockIdx.y | blockIdx.z) == 0) n += a.tasks ? (int)a.tasks : (int)(gridDim.x * gridDim.y * gridDim.z);
+    if (n != 0) atomicAdd(a.task_slot, n);
+}
 }  // namespace
 namespace {
 // Ops whose body makes the first flag check of a best-effort workgroup itself, at a point where
@@ -327,6 +337,7 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         FlagPoll poll{a.preempted};                                                       \
         bool done = false;                                                                \
         if (a.tasks != 0 && blockIdx.x >= a.tasks) {                                      \
+            done = true;                                                                  \
             prefetch_lines((const ReefPrefetch*)a.desc.ptr[REEF_PREFETCH_SLOT], (int)(blockIdx.x - a.tasks)); \
         } else if (ChecksFlagItself<OP>::value) {                                                \
             done = OP::run(a.desc, (int)blockIdx.x, smem, poll);                          \
@@ -335,7 +346,7 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
             __syncthreads();                                                              \
             if (!s_pre) done = OP::run(a.desc, (int)blockIdx.x, smem, poll);              \
         }                                                                                 \
-        if (done && t == 0) atomicAdd(a.task_slot, 1);                                    \
+        if (t == 0) be_count_completed(a, done);                                          \
         be_signal_exit(a, t);                                                             \
     }
 #else
