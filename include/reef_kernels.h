@@ -206,7 +206,10 @@ enum {
     REEF_CONV_DST_OFF,   /* element offset added to dst (and out2): channel slice of a concat buffer */
     REEF_CONV_WPACK,     /* pointer slot of the packed copy of the weights (symbols ...d<R>k_ / r9k_), else 0:
                             [ceil(Cout/16)][ceil(Cin/4)][ceil(taps/4)][4 channels][16 rows][4 taps] floats,
-                            zero where a row, channel or tap does not exist; the last pointer of the kernel */
+                            zero where a row, channel or tap does not exist; the last pointer of the kernel.
+                            1-tap filters (d1_, p1_: either form; v1_, p1_v_) and v9_, by channels:
+                            [ceil(Cout/16)][ceil(Cin/16)][taps][4 slots][16 rows][4 channels], and a split starts
+                            at a multiple of 16 channels */
     REEF_CONV_NATTR
 };
 #define REEF_F_BIAS 1
@@ -273,6 +276,10 @@ enum {
                                   weights [P][COUT], projection bias [P].  A workgroup holds every channel of its G
                                   output rows x 14 columns: M_TILES = 1, N_TILES = ceil(HO / G) * ceil(WO / 14),
                                   TILE = REEF_TILE_R9G<G>, no split. */
+#define REEF_F_BOTH_SHARES 8192 /* with REEF_F_PAIR_FOLD, symbols v1_16x16k4, p1_v_16x16k4 and v9_g1: in a plain launch the first
+                                  M_TILES * N_TILES workgroups take a tile each, both shares of its split one after the
+                                  other, and the rest have nothing to do.  Cin = 2 shares of whole groups of 256 (v9: 64)
+                                  channels. */
 #define REEF_CONV_MODE_GENERAL 0
 #define REEF_CONV_MODE_POINTWISE 1
 #define REEF_CONV_MODE_UNALIGNED 2

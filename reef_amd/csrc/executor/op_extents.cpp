@@ -97,6 +97,7 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
     const bool fused = flags & REEF_F_FUSED_REDUCE;
     // the loader family is part of the symbol: what it was compiled for must be what the layer is
     const i64 K = cin * kh * kw, taps = kh * kw;
+    const bool packed1 = a[REEF_CONV_WPACK] != 0;   // the 1-tap direct kernels take packed weights and others alike
     const bool unit = kh == 1 && kw == 1 && a[REEF_CONV_PH] == 0 && a[REEF_CONV_PW] == 0;
     const std::string fam = symbol.substr(std::strlen("reef_conv2d_"));
     const std::string head = fam.substr(0, fam.find('_'));  // "d9", "d9k", "r9k", "pw", a tile for the general family
@@ -152,9 +153,20 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
                a[REEF_CONV_TILE] == REEF_TILE_R9G2 && a[REEF_CONV_M_TILES] == cdiv(M, 16) &&
                a[REEF_CONV_N_TILES] == cdiv(Ho, 2) * cdiv(Wo, 14) && a[REEF_CONV_ACT] <= REEF_ACT_RELU6 &&
                a[REEF_CONV_ACT2] <= REEF_ACT_RELU6;
+    } else if (fam.compare(0, 3, "v1_") == 0 || fam.compare(0, 4, "p1_v_") == 0) {
+        // 1x1 / stride 1 on packed weights, the input in 16-byte pieces
+        mode = fam[0] == 'p' ? REEF_CONV_MODE_DIRECT_PRE : REEF_CONV_MODE_DIRECT;
+        packed = true;
+        fits = unit && a[REEF_CONV_SH] == 1 && a[REEF_CONV_SW] == 1 && cin % 8 == 0;
     } else if (fam.compare(0, 3, "p1_") == 0) {
         mode = REEF_CONV_MODE_DIRECT_PRE;
+        packed = packed1;
         fits = unit && cin % 8 == 0 && (flags & REEF_F_PRE_ACT);
+    } else if (fam.compare(0, 3, "v9_") == 0) {
+        // the row form in steps of 16 channels a wavefront
+        mode = REEF_CONV_MODE_ROWS;
+        packed = true;
+        fits = kh == 3 && kw == 3 && a[REEF_CONV_SH] == 1 && a[REEF_CONV_SW] == 1 && a[REEF_CONV_PH] == 1 && a[REEF_CONV_PW] == 1;
     } else if (fam.compare(0, 2, "r9") == 0) {
         mode = REEF_CONV_MODE_ROWS;
         packed = head.back() == 'k';
@@ -163,7 +175,7 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
     } else if (fam[0] == 'd') {
         mode = REEF_CONV_MODE_DIRECT;
         const i64 compiled = std::atoi(fam.c_str() + 1);
-        packed = head.back() == 'k';
+        packed = compiled == 1 ? packed1 : head.back() == 'k';
         fits = compiled == taps && (taps > 1 || cin % 8 == 0);
     }
     if (!fits || mode != a[REEF_CONV_MODE] || ((flags & REEF_F_PRE_ACT) != 0) != (mode == REEF_CONV_MODE_DIRECT_PRE) ||
@@ -175,6 +187,15 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
         return;
     }
     if (packed != (a[REEF_CONV_WPACK] != 0)) { n.bad = "packed weights and symbol do not go together"; return; }
+    if (flags & REEF_F_BOTH_SHARES) {
+        const i64 share = a[REEF_CONV_K_CHUNK] / taps;
+        const bool v1 = fam == "v1_16x16k4" || fam == "p1_v_16x16k4";
+        if (!(v1 || fam == "v9_g1") || split != 2 || !fused || !(flags & REEF_F_PAIR_FOLD) || 2 * share != cin ||
+            a[REEF_CONV_K_CHUNK] % taps != 0 || share % (v1 ? 256 : 64) != 0) {
+            n.bad = "both shares in one workgroup: a split of two into alike shares of whole groups of channels";
+            return;
+        }
+    }
     if (a[REEF_CONV_K_CHUNK] <= 0 || split * a[REEF_CONV_K_CHUNK] < K) {
         n.bad = "the splits do not cover the reduction";
         return;
@@ -205,7 +226,9 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
     }
     if (a[REEF_CONV_WPACK] != 0) {
         if (a[REEF_CONV_WPACK] != (i64)n.slots.size()) { n.bad = "the packed weights are not the last operand"; return; }
-        n.f32("packed weights", cdiv(M, 16) * cdiv(cin, 4) * cdiv(kh * kw, 4) * 4 * 16 * 4);
+        const bool by_channels = taps == 1 || fam.compare(0, 3, "v9_") == 0;
+        if (by_channels && a[REEF_CONV_K_CHUNK] % (16 * taps) != 0) { n.bad = "a split of the packed weights starts inside a group of 16 channels"; return; }
+        n.f32("packed weights", by_channels ? cdiv(M, 16) * cdiv(cin, 16) * taps * 256 : cdiv(M, 16) * cdiv(cin, 4) * cdiv(taps, 4) * 256);
     }
     n.tasks = split * a[REEF_CONV_M_TILES] * a[REEF_CONV_N_TILES];
 }

@@ -32,6 +32,11 @@ namespace {
 __device__ __forceinline__ int conv_tasks(const ReefOpDesc& d) {
     return d.attr[REEF_CONV_SPLIT_K] * d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
 }
+// (a plain launch whose workgroups take both shares of a split: the others come last)
+__device__ __forceinline__ int conv_v_tasks(const ReefOpDesc& d) {
+    const int tiles = d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
+    return (d.attr[REEF_CONV_FLAGS] & REEF_F_BOTH_SHARES) ? tiles : tiles * d.attr[REEF_CONV_SPLIT_K];
+}
 __device__ __forceinline__ int gemm_tasks(const ReefOpDesc& d) {
     const int s = d.attr[REEF_GEMM_SPLIT_K];
     return d.attr[REEF_GEMM_BATCH] * d.attr[REEF_GEMM_M_TILES] * d.attr[REEF_GEMM_N_TILES] * (s > 1 ? s : 1);
@@ -68,6 +73,28 @@ struct OpConvDirect {
     template <class P>
     static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
         return conv2d_direct_body<R, TN, TM, PRE, ROWS, PACKED, FROWS, ODDC>(d, task, smem, p);
+    }
+};
+// 1x1 / stride 1 on packed weights, the input turned in LDS
+template <int TM, int TN, bool PRE = false>
+struct OpConvV1 {
+    REEF_TASKS(conv_v_tasks)
+    static constexpr int LDS = TileV1<TM, TN>::LDS_BYTES;
+    static constexpr bool CHECKS_FLAG_ITSELF = true;
+    template <class P>
+    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+        return conv2d_v1_body<TM, TN, PRE>(d, task, smem, p);
+    }
+};
+// 3x3 / stride 1 / padding 1 by image rows, in steps of 16 channels a wavefront
+template <int G>
+struct OpConvV9 {
+    REEF_TASKS(conv_v_tasks)
+    static constexpr int LDS = TileV9<G>::LDS_BYTES;
+    static constexpr bool CHECKS_FLAG_ITSELF = true;
+    template <class P>
+    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+        return conv2d_v9_body<G>(d, task, smem, p);
     }
 };
 // the same with the weights read from their packed copy
@@ -287,7 +314,7 @@ __device__ __forceinline__ bool dkp_walk(const ReefDkpArgs& a, DkpWalk& w) {
             prefetch_lines((const ReefPrefetch*)d.ptr[REEF_PREFETCH_SLOT], behind);   \
             return;                                                                   \
         }                                                                             \
-        OP::run(d, (int)blockIdx.x, smem, NoPoll{true});                              \
+        OP::run(d, (int)blockIdx.x, smem, NoPoll{true, true});                              \
     }
 #elif REEF_FLAVOUR == 1
 namespace {
@@ -367,7 +394,7 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         if (!dkp_walk(a, w)) return;                                                   \
         const ReefDkpSide& side = w.right ? a.r : a.l;                                 \
         for (int i = w.idx; i < w.end; i += w.step) {                                  \
-            OP::run(side.desc, i, smem, NoPoll{!w.right});                             \
+            OP::run(side.desc, i, smem, NoPoll{!w.right, false});                             \
             __syncthreads();                                                           \
         }                                                                              \
     }                                                                                  \
@@ -416,6 +443,16 @@ REEF_ENTRY(reef_conv2d_p1_16x32k4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 1 REEF
 REEF_ENTRY(reef_conv2d_p1_32x32d4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 2 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_d1_32x32d4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 2>)
 REEF_ENTRY(reef_conv2d_d9_32x32d4, OpConvDirect<9 REEF_COMMA 2 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_v1_16x16k4, OpConvV1<1 REEF_COMMA 1>)
+REEF_ENTRY(reef_conv2d_v1_16x32k4, OpConvV1<1 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_v1_16x64k4, OpConvV1<1 REEF_COMMA 4>)
+REEF_ENTRY(reef_conv2d_v1_32x32d4, OpConvV1<2 REEF_COMMA 2>)
+REEF_ENTRY(reef_conv2d_p1_v_16x16k4, OpConvV1<1 REEF_COMMA 1 REEF_COMMA true>)
+REEF_ENTRY(reef_conv2d_p1_v_16x32k4, OpConvV1<1 REEF_COMMA 2 REEF_COMMA true>)
+REEF_ENTRY(reef_conv2d_p1_v_32x32d4, OpConvV1<2 REEF_COMMA 2 REEF_COMMA true>)
+REEF_ENTRY(reef_conv2d_v9_g1, OpConvV9<1>)
+REEF_ENTRY(reef_conv2d_v9_g2, OpConvV9<2>)
+REEF_ENTRY(reef_conv2d_v9_g4, OpConvV9<4>)
 REEF_ENTRY(reef_conv2d_r9_g1, OpConvRows<1>)
 REEF_ENTRY(reef_conv2d_r9_g2, OpConvRows<2>)
 REEF_ENTRY(reef_conv2d_r9_g4, OpConvRows<4>)

@@ -784,8 +784,8 @@ struct DirectGeom {
     // B values a lane loads per step: every tap of every pixel group, or (row form) one value
     // per input row of the tile
     static constexpr int NB = ROWS ? TN + 2 : TN * RC;
-    // vector-memory instructions per step (PRE: two 128-bit loads each of input scale and shift)
-    static constexpr int LOADS = TM * ((RC / 4) + (RC % 4)) + NB + (PRE ? 2 * (RC / 4) : 0);
+    // vector-memory instructions per step (PRE: one that brings the input scales and shifts)
+    static constexpr int LOADS = TM * ((RC / 4) + (RC % 4)) + NB + (PRE ? 1 : 0);
     // Steps of loads in flight per wavefront.  All of them are issued before the first MFMA, and a
     // wavefront that is still issuing loads multiplies nothing: with 8 steps ahead (all of a 14x14
     // row-form layer at a split of two) cycle stamps showed 4600 cycles of issue, then 6600 of K loop
@@ -803,6 +803,191 @@ struct DirectGeom {
                             : NS_GEN;
 };
 
+// What a thread holds for the output elements it writes (element (h, g): row 16 h + t / 16, column 16 g + t % 16 of
+// the tile), and where its workgroup's share of K stands.
+template <int TM, int TN>
+struct DirectTail {
+    ConvEpilogue ep;
+    unsigned om[TM], ooff[TM][TN];           // row; byte offset of the element, kOutside without one
+    float e_bias[TM], e_sh2[TM], e_res[TM][TN];
+    int split, split_k, rem, flags, aux;     // aux: pointer slot of (workspace, arrival counters)
+    bool fused, to_ws;                       // split folded inside the launch; partial tile to the workspace
+    bool both;                               // this workgroup has both shares of a split of two (REEF_F_BOTH_SHARES)
+
+    // Epilogue operands, fetched behind the first K steps' loads.
+    __device__ __forceinline__ void fetch(const ReefOpDesc& d, unsigned MN4) {
+        const int* a = d.attr;
+        ep.next = 3;   // plain split-K launches carry no epilogue operands
+#pragma unroll
+        for (int h = 0; h < TM; ++h) {
+            e_bias[h] = e_sh2[h] = 0.0f;
+#pragma unroll
+            for (int g = 0; g < TN; ++g) e_res[h][g] = 0.0f;
+        }
+        if (to_ws) return;
+        ep.init(d, flags, a[REEF_CONV_ACT], a[REEF_CONV_ACT2], a[REEF_CONV_COUT], MN4, (unsigned)a[REEF_CONV_DST_OFF] * 4u);
+#pragma unroll
+        for (int h = 0; h < TM; ++h) {
+            if (ep.has_bias) e_bias[h] = buf_load(ep.bias, om[h] * 4u);
+            if (ep.has_dual) e_sh2[h] = buf_load(ep.shift2, om[h] * 4u);
+            if (ep.has_res) {
+#pragma unroll
+                for (int g = 0; g < TN; ++g) e_res[h][g] = buf_load(ep.res, ooff[h][g]);
+            }
+        }
+    }
+};
+
+// From the wavefronts' partial tiles to the output: added through LDS in wavefront order, then epilogue and
+// store, partial tile to the workspace, or the fold of a split K inside the launch.  False: the workgroup
+// leaves a preempted launch.
+// WSTRIDE: floats between the wavefronts' places in LDS; the flags lie behind the last.
+// first: the first share's sums where the workgroup has both (t.both).
+template <int TM, int TN, int WSTRIDE = TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, class Poll>
+__device__ __forceinline__ bool direct_tail(const ReefOpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN],
+                                            const DirectTail<TM, TN>& t, const Poll& poll, const f32x4* first = nullptr) {
+    typedef TileD16<TN, TM> TD;
+    float* smem = (float*)smem_raw;
+    int* sflag = (int*)(smem + 4 * WSTRIDE);
+    const int* a = d.attr;
+    const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+    const int M = a[REEF_CONV_COUT], N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
+    // partial tiles of this wavefront -> LDS; element j of a lane is row 4 * (lane / 16) + j.
+    // Each group of four rows is skewed by 16 floats so the four k slots write to different banks.
+    float* part = smem + wave * WSTRIDE;
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = acc[h][g][j];
+    if (first && t.both) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[TD::PART + (5 * kq + j) * 16 + i16] = (*first)[j];
+    }
+    __syncthreads();
+    if (Poll::enabled && *sflag) return false;
+    const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
+    float v[TM][TN];
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+            const float* e = mine + (h * TN + g) * TD::PART;
+            v[h][g] = ((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE];
+        }
+    if (first && t.both) {      // the shares' sums in split order, as where they meet
+        const float* e = mine + TD::PART;
+        v[0][0] = (((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE]) + v[0][0];
+    }
+    if (t.to_ws) {
+        const rsrc_t ws = make_rsrc((const float*)d.ptr[2] + (size_t)t.split * M * N, (unsigned)M * (unsigned)N * 4u);
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) buf_store(ws, t.ooff[h][g], v[h][g]);
+        return true;
+    }
+    if (!t.fused) {
+        if (t.flags & REEF_F_GAP_OUTPUT) {
+            // The global average of the layer's output instead of the output (a classifier's last
+            // convolution): one pixel tile covers the image, so the 16 lanes of an output row hold
+            // the whole row between them.  out[m] = sum over the pixels / N, pixels in ascending order
+            // within a lane, lanes folded pairwise.
+#pragma unroll
+            for (int h = 0; h < TM; ++h) {
+                float s = 0.0f;
+#pragma unroll
+                for (int g = 0; g < TN; ++g)
+                    if (t.ooff[h][g] != kOutside) s += t.ep.value(v[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h]);
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+                if ((threadIdx.x & 15) == 0 && t.om[h] < (unsigned)M) buf_store(t.ep.out, t.om[h] * 4u, s * (1.0f / (float)N));
+            }
+            return true;
+        }
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+                t.ep.finish(v[h][g], t.ooff[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h], t.e_sh2[h]);
+        return true;
+    }
+
+    // split-K folded inside the launch
+    const size_t MN = (size_t)M * N;
+    float* ws = (float*)d.ptr[t.aux];
+    if (t.split_k == 2 && (t.flags & REEF_F_PAIR_FOLD) && poll.pair_fold_ok()) {
+        // One exchange per output element.  A value is parked with its sign bit flipped: a sum
+        // of products that starts from +0 is never -0, so a parked value is never the empty
+        // slot's 0 (and a -0 is parked as +0, should one ever come).
+        unsigned* slots = (unsigned*)(ws + 2 * MN);
+        unsigned got[TM][TN];
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) {
+                got[h][g] = 0;
+                if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M) {
+                    unsigned mine = __float_as_uint(v[h][g]) ^ 0x80000000u;
+                    mine = mine ? mine : 0x80000000u;
+                    got[h][g] = __hip_atomic_exchange(&slots[t.ooff[h][g] >> 2], mine, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+                if (got[h][g] != 0) {   // second to arrive: the other half is here
+                    const float other = __uint_as_float(got[h][g] ^ 0x80000000u);
+                    const float sum = t.split == 0 ? v[h][g] + other : other + v[h][g];   // split order
+                    t.ep.finish(sum, t.ooff[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h], t.e_sh2[h]);
+                    __hip_atomic_store(&slots[t.ooff[h][g] >> 2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+        return true;
+    }
+    int* counters = (int*)d.ptr[t.aux + 1] + a[REEF_CONV_SYNC_OFF];
+    int* s_last = sflag + 1;
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g)
+            if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M)
+                store_agent(ws + (size_t)t.split * MN + (t.ooff[h][g] >> 2), v[h][g]);
+    // every store of this workgroup has completed at device scope before it counts in
+    partial_stores_done();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int old = __hip_atomic_fetch_add(&counters[t.rem], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *s_last = (old == t.split_k - 1);
+    }
+    __syncthreads();
+    if (!*s_last) return true;
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+            if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M) {
+                const float* src = ws + (t.ooff[h][g] >> 2);
+                float sum = 0.0f;
+                for (int s0 = 0; s0 < t.split_k; s0 += 4) {
+                    float p[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) p[j] = load_agent(src + (size_t)min(s0 + j, t.split_k - 1) * MN);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (s0 + j < t.split_k) sum = (s0 + j == 0) ? p[j] : sum + p[j];
+                }
+                t.ep.finish(sum, t.ooff[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h], t.e_sh2[h]);
+            }
+        }
+    if (threadIdx.x == 0)  // ready for the next run
+        __hip_atomic_store(&counters[t.rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
 // Row form (ROWS; 3x3 filters, stride 1, padding 1; symbols reef_conv2d_r9_g<G>[m2]): the tile is
 // G image rows x one 14-column segment of the output.  Pixel group g is image row y0 + g and the
 // 16 lanes of a k slot are the columns of the segment: lanes 0..13 hold columns x0 .. x0 + 13,
@@ -816,10 +1001,18 @@ struct DirectGeom {
 // stores.  Same sum order over k as the tap form (channel-major steps, taps in filter order).
 constexpr int kRowSeg = 14;
 __device__ __forceinline__ float lane_from_left(float v) {   // lane i <- lane (i - 1) mod 16 of its row
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xF, 0xF, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x121, 0xF, 0xF, true));
 }
 __device__ __forceinline__ float lane_from_right(float v) {  // lane i <- lane (i + 1) mod 16 of its row
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x12F, 0xF, 0xF, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x12F, 0xF, 0xF, true));
+}
+template <int I>
+__device__ __forceinline__ float lane_of_quad(float v) {     // every lane <- lane I of its quad
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), I * 0x55, 0xF, 0xF, true));
+}
+template <int I>
+__device__ __forceinline__ float lane_of_row(float v) {      // every lane <- lane I of its row of 16
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + I, 0xF, 0xF, true));
 }
 
 // TN > 1 widens the tile along the pixels: every weight value a lane has loaded is multiplied
@@ -835,8 +1028,10 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane i <- lane (
 // PRE (1-tap kernels only, symbols reef_conv2d_p1_*): the layer reads its input through a
 // per-channel scale, shift and ReLU -- the pre-activation of a DenseNet layer, which cannot be
 // folded into the producing convolution because every consumer of the concatenation has its own.
-// The four input values a lane loads per step are four consecutive channels, so their scales
-// and shifts are one 128-bit load each; a channel past the split loads scale = shift = 0 and
+// The four input values a lane loads per step are four consecutive channels; one 32-bit load brings
+// their scales to lanes 0..3 and their shifts to lanes 4..7 of the 16 lanes of a k slot, from where DPP
+// broadcasts hand them to the row (two 128-bit loads that every lane makes for itself hold the vector-memory
+// pipe for 40 cycles, this one for 15).  A channel past the split takes scale = shift = 0 and
 // contributes relu(0) = 0.  REEF_F_PRE_ACT; the two vectors follow the optional epilogue operands.
 //
 // PACKED (filters with several taps; symbols reef_conv2d_d<R>k_* / reef_conv2d_r9k_*): the weights
@@ -847,6 +1042,10 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane i <- lane (
 // (zero-padded to whole groups): the 64 lanes of a wavefront read 1 KiB contiguous, aligned, per
 // group of four taps.  Measured on the 3x3 layers of ResNet-152: 1.4 us less per launch.  The
 // model generator writes the copy as a parameter of its own; attr WPACK names its pointer slot.
+// A 1-tap filter's copy is [Cout / 16][Cin / 16][k slot][row][4 channels], and the same kernels take
+// either form (attr WPACK = 0: OIHW), since only the addresses differ.  The pipe resolves one line of a
+// 128-bit load a cycle and lane: 64 cycles for the 16 rows of an OIHW tile, whose neighbouring lanes lie in
+// different lines, 20 for a contiguous KiB (L2-resident, 8 wavefronts a CU).
 //
 // FROWS (symbols reef_conv2d_f<R>_*): R is the width of the filter and a k slot's channel is one row of one
 // channel's filter, number c * kh + ky.  The weights of a row of W are contiguous in that order too, so the
@@ -861,7 +1060,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
                                                    const Poll& poll) {
     static_assert(!PRE || R == 1, "the pre-activation form exists for 1-tap filters only");
     static_assert(!ROWS || R == 9, "the row form exists for 3x3 filters only");
-    static_assert(!PACKED || R > 1, "1-tap filters are read from OIHW as they are");
+    static_assert(!PACKED || R > 1, "the 1-tap kernels see from their attributes whether the weights are packed");
     static_assert(!FROWS || !(PRE || ROWS || PACKED), "filter rows are read from OIHW, tap by tap");
     static_assert(!ODDC || R == 1, "only the 1-tap kernels load several channels at once");
     typedef DirectGeom<R, TN, TM, PRE, ROWS> G;
@@ -904,10 +1103,12 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
     const unsigned HW4 = (unsigned)(H * W) * 4u;
     const unsigned MN4 = (unsigned)M * (unsigned)N * 4u;
 
-    // epilogue operands of the TM x TN output elements this thread writes (element (h, g): row
-    // 16 h + t / 16, column 16 g + t % 16 of the tile), fetched ahead of the K loop
     const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
-    unsigned om[TM], ooff[TM][TN];
+    DirectTail<TM, TN> tail;
+    tail.both = false;
+    tail.split = split; tail.split_k = split_k; tail.rem = rem; tail.flags = flags; tail.fused = fused; tail.to_ws = to_ws;
+    unsigned (&om)[TM] = tail.om;
+    unsigned (&ooff)[TM][TN] = tail.ooff;
 #pragma unroll
     for (int h = 0; h < TM; ++h) {
         om[h] = (unsigned)(m0 + 16 * h + orow);
@@ -929,31 +1130,37 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
                               : 3 + ((flags & REEF_F_BIAS) ? 1 : 0) + ((flags & REEF_F_RESIDUAL) ? 1 : 0) +
                                     ((flags & REEF_F_AFFINE) ? 2 : 0) + ((flags & REEF_F_DUAL) ? 2 : 0);
     // per-lane operand offsets
-    const rsrc_t rs_a = make_rsrc(d.ptr[1], (unsigned)M * (unsigned)K * 4u);
     const rsrc_t rs_b = make_rsrc(d.ptr[0], (unsigned)(FROWS ? a[REEF_CONV_CIN] : C) * HW4);
     const int lane_c = cb + (wave * 4 + kq) * G::CPL;     // first channel of this lane's k slot
     constexpr int G4 = (R + 3) / 4;                 // groups of four taps in the packed copy
     const unsigned C4 = (unsigned)(C + 3) / 4u;
-    const rsrc_t rs_ap = make_rsrc(d.ptr[PACKED ? a[REEF_CONV_WPACK] : 1],
-                                   PACKED ? (unsigned)((M + 15) / 16) * C4 * (unsigned)G4 * 1024u
-                                          : (unsigned)M * (unsigned)K * 4u);
+    const bool packed1 = R == 1 && !FROWS && !ODDC && a[REEF_CONV_WPACK] != 0;
+    const unsigned C16 = (unsigned)(C + 15) / 16u;
+    const void* wp = d.ptr[1];
+    if (PACKED || packed1) wp = d.ptr[a[REEF_CONV_WPACK]];
+    const rsrc_t rs_ap = make_rsrc(wp,
+                                   PACKED    ? (unsigned)((M + 15) / 16) * C4 * (unsigned)G4 * 1024u
+                                   : packed1 ? (unsigned)((M + 15) / 16) * C16 * 1024u
+                                             : (unsigned)M * (unsigned)K * 4u);
+    const unsigned step_a = packed1 ? 4096u : (unsigned)(G::STEP_C * R) * 4u;   // bytes from a step's weights to the next
     unsigned va[TM];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
         va[h] = PACKED ? (((unsigned)(m0 / 16 + h) * C4 + (unsigned)(cb / 4 + wave)) * (unsigned)G4) * 1024u
                              + (unsigned)lane * 16u
+              : packed1 ? ((unsigned)(m0 / 16 + h) * C16 + (unsigned)(cb / 16 + wave)) * 1024u + (unsigned)lane * 16u
                        : ((unsigned)(m0 + 16 * h + i16) * (unsigned)K + (unsigned)(lane_c * R)) * 4u;
     // steps this lane's k slot stays inside the channel range of the split
     const int lane_steps = lane_c < ce ? (ce - lane_c + G::STEP_C - 1) / G::STEP_C : 0;
 
     constexpr int NB = G::NB;
     float ra[NS][TM][RC], rb[NS][NB];
-    float rps[NS][PRE ? RC : 1], rpt[NS][PRE ? RC : 1];
+    float rp[PRE ? NS : 1];     // lanes 0..3 of a k slot: the scales of its channels, 4..7: the shifts
     auto load_a = [&](int s, int step) {
         // offsets are below kOutside (a power of two), so or-ing it in moves them outside
         const unsigned outm = step < lane_steps ? 0u : kOutside;
         const unsigned sa = PACKED ? (unsigned)step * (unsigned)(4 * G4) * 1024u      // uniform
-                                   : (unsigned)step * (unsigned)(G::STEP_C * R) * 4u;
+                                   : (unsigned)step * step_a;
         if (PACKED) {
 #pragma unroll
             for (int h = 0; h < TM; ++h) {
@@ -979,14 +1186,14 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
 #pragma unroll
             for (int q = 0; q < RC / 4; ++q) {
                 const f32x4 v = __builtin_bit_cast(
-                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_a, (int)(oa + 16u * q), (int)sa, 0));
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_ap, (int)(oa + 16u * q), (int)sa, 0));
                 ra[s][h][4 * q] = v[0]; ra[s][h][4 * q + 1] = v[1];
                 ra[s][h][4 * q + 2] = v[2]; ra[s][h][4 * q + 3] = v[3];
             }
 #pragma unroll
             for (int q = RC / 4 * 4; q < RC; ++q)
                 ra[s][h][q] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_raw_buffer_load_b32(rs_a, (int)(oa + 4u * q), (int)sa, 0));
+                    float, __builtin_amdgcn_raw_buffer_load_b32(rs_ap, (int)(oa + 4u * q), (int)sa, 0));
         }
     };
     // The weights first -- the cold stream, and their offsets need nothing of the pixel
@@ -1048,30 +1255,16 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
     }
     // operands that follow the optional epilogue operands: (pre-activation scale, shift), then
     // (workspace, arrival counters) of a folded split
-    const int aux = ep_next + (PRE ? 2 : 0);
-    const rsrc_t rs_ps = make_rsrc(d.ptr[PRE ? ep_next : 0], (unsigned)C * 4u);
-    const rsrc_t rs_pt = make_rsrc(d.ptr[PRE ? ep_next + 1 : 0], (unsigned)C * 4u);
-    const unsigned vpre = (unsigned)lane_c * 4u;
+    tail.aux = ep_next + (PRE ? 2 : 0);
+    const float* pre_s = (const float*)d.ptr[PRE ? ep_next : 0];
+    const float* pre_t = (const float*)d.ptr[PRE ? ep_next + 1 : 0];
+    const float* pre_at = ((i16 & 4) ? pre_t : pre_s) + (i16 & 3);
 
     auto load_b = [&](int s, int step) {
         const unsigned outm = step < lane_steps ? 0u : kOutside;
         const unsigned sb = (unsigned)step * (unsigned)G::STEP_C * HW4;         // uniform
-        if (PRE) {
-            const unsigned op = vpre | outm;
-            const unsigned sp = (unsigned)step * (unsigned)G::STEP_C * 4u;   // uniform
-#pragma unroll
-            for (int q = 0; q < RC / 4; ++q) {
-                const f32x4 sc = __builtin_bit_cast(
-                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_ps, (int)(op + 16u * q), (int)sp, 0));
-                const f32x4 sh = __builtin_bit_cast(
-                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_pt, (int)(op + 16u * q), (int)sp, 0));
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    rps[s][PRE ? 4 * q + e : 0] = sc[e];
-                    rpt[s][PRE ? 4 * q + e : 0] = sh[e];
-                }
-            }
-        }
+        // (a slot past the split takes the first channels' and drops them in mma_stage)
+        if (PRE) rp[PRE ? s : 0] = pre_at[step < lane_steps ? lane_c + step * G::STEP_C : 0];
         if (FROWS) {
 #pragma unroll
             for (int g = 0; g < TN; ++g) {
@@ -1116,28 +1309,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
         asm volatile("" ::: "memory");
     }
 
-    // epilogue operands of this thread's output elements, behind the first K steps' loads
-    ConvEpilogue ep;
-    ep.next = 3;   // plain split-K launches carry no epilogue operands
-    float e_bias[TM], e_sh2[TM], e_res[TM][TN];
-#pragma unroll
-    for (int h = 0; h < TM; ++h) {
-        e_bias[h] = e_sh2[h] = 0.0f;
-#pragma unroll
-        for (int g = 0; g < TN; ++g) e_res[h][g] = 0.0f;
-    }
-    if (!to_ws) {
-        ep.init(d, flags, a[REEF_CONV_ACT], a[REEF_CONV_ACT2], M, MN4, (unsigned)a[REEF_CONV_DST_OFF] * 4u);
-#pragma unroll
-        for (int h = 0; h < TM; ++h) {
-            if (ep.has_bias) e_bias[h] = buf_load(ep.bias, om[h] * 4u);
-            if (ep.has_dual) e_sh2[h] = buf_load(ep.shift2, om[h] * 4u);
-            if (ep.has_res) {
-#pragma unroll
-                for (int g = 0; g < TN; ++g) e_res[h][g] = buf_load(ep.res, ooff[h][g]);
-            }
-        }
-    }
+    tail.fetch(d, MN4);
 
     if (Poll::enabled) {
         // The flag check every best-effort workgroup makes before it does anything
@@ -1160,6 +1332,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
             acc[h][g][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             acc[h][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
+    int pre_left = lane_steps;      // PRE: steps of this lane's slot that are still to come
     int odd_left = C - lane_c;      // ODDC: channels of this lane's row from its slot of the next step on
     auto mma_stage = [&](int s) {
         if (ODDC) {
@@ -1189,11 +1362,14 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
             return;
         }
         if (PRE) {
+            const float p = pre_left-- > 0 ? rp[PRE ? s : 0] : 0.0f;
+            const float sc[4] = {lane_of_row<0>(p), lane_of_row<1>(p), lane_of_row<2>(p), lane_of_row<3>(p)};
+            const float sh[4] = {lane_of_row<4>(p), lane_of_row<5>(p), lane_of_row<6>(p), lane_of_row<7>(p)};
 #pragma unroll
             for (int g = 0; g < TN; ++g)
 #pragma unroll
                 for (int q = 0; q < RC; ++q)
-                    rb[s][ROWS ? 0 : g * RC + q] = fmaxf(fmaf(rb[s][ROWS ? 0 : g * RC + q], rps[s][PRE ? q : 0], rpt[s][PRE ? q : 0]), 0.0f);
+                    rb[s][ROWS ? 0 : g * RC + q] = fmaxf(fmaf(rb[s][ROWS ? 0 : g * RC + q], sc[q & 3], sh[q & 3]), 0.0f);
         }
 #pragma unroll
         for (int q = 0; q < RC; ++q)
@@ -1250,133 +1426,459 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
             if (it + s < nsteps) mma_stage(s);
     }
 
-    // partial tiles of this wavefront -> LDS; element j of a lane is row 4 * (lane / 16) + j.
-    // Each group of four rows is skewed by 16 floats so the four k slots write to different banks.
-    float* part = smem + wave * (TD::SUBS * TD::PART);
+    f32x4 sum[TM][TN];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
+    return direct_tail(d, smem_raw, wave, sum, tail, poll);
+}
+
+// ---- reef_conv2d_v1_<tile>, reef_conv2d_p1_v_<tile>: 1x1 filters, stride 1, whole cache lines ----------------
+// The direct form for 1x1 / stride 1 layers whose image is a multiple of 4 pixels, on packed weights.  What
+// differs is how the input gets into the matrix cores.  A lane of conv2d_direct_body loads its four MFMA
+// operands with four 32-bit loads, each of which takes the CU's vector-memory pipe 15 cycles for 256 bytes
+// (8 wavefronts a CU, L2-resident); a 128-bit load brings 1 KiB in 23 to 31.  Here the 64 lanes of a wavefront
+// load a step's block of 16 channels x 16 TN pixels as rows of 16-byte pieces, TN loads, and the block is turned
+// in LDS: [16 rows][16 TN pixels], written with one 128-bit store a load, read as the four (x TN) operands of the
+// MFMAs.  Row 4 q + kq holds channel 4 kq + q, and pixel group g of a row sits at g ^ (its kq's high bits), so
+// that the four k slots read different banks.  The block is the wavefront's own and LDS serves a wavefront
+// in order: no barrier.  It is turned one step ahead of the MFMAs that use it.
+// PRE (p1_v): input scale, shift and ReLU on the loaded values; a lane's values of a load belong to one channel,
+// whose scale and shift one 32-bit load brings to neighbouring lanes.
+// Sums run over the channels in the order of conv2d_direct_body.
+template <int TM, int TN>
+struct TileV1 {      // a wavefront's place: the turned block, then its partial tile (16x16: one of either share)
+    static constexpr int WSTRIDE = (TM * TN == 1 ? 2 : TM * TN) * TileD16<TN, TM>::PART;
+    static constexpr int LDS_BYTES = 4 * WSTRIDE * 4 + 16;
+};
+template <int TM, int TN, bool PRE, class Poll>
+__device__ __forceinline__ bool conv2d_v1_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll& poll) {
+    static_assert(TN == 1 || TN == 2 || TN == 4, "a row of the turned block is 64, 128 or 256 bytes");
+    static_assert(!PRE || TN < 4, "scales and shifts of two channels a lane at most");
+    typedef TileD16<TN, TM> TD;
+    // steps of loads in flight (6, 8 and 12 on 16x16: the same K loop on 1024 channels, whose end the L2 -> CU
+    // stream sets -- a 64-byte piece brings its 128-byte line -- and up to 1.5 % slower networks)
+    constexpr int NS = 4;
+    constexpr int LPR = 4 * TN;                    // lanes (16-byte pieces) of a row
+    float* smem = (float*)smem_raw;
+    constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
+    int* sflag = (int*)(smem + 4 * WSTRIDE);
+    const int* a = d.attr;
+    const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
+    const int split_k = a[REEF_CONV_SPLIT_K], n_tiles = a[REEF_CONV_N_TILES];
+    const int tiles = a[REEF_CONV_M_TILES] * n_tiles;
+    const int flags = a[REEF_CONV_FLAGS];
+    DirectTail<TM, TN> tail;
+    tail.flags = flags;
+    tail.split_k = split_k;
+    tail.fused = split_k > 1 && (flags & REEF_F_FUSED_REDUCE);
+    tail.to_ws = split_k > 1 && !tail.fused;
+    // tile and split of this workgroup, as in conv2d_direct_body
+    const int chunk = a[REEF_CONV_K_CHUNK];
+    const int share = chunk >> 6;            // steps of a share
+    tail.both = TD::SUBS == 1 && poll.plain && (flags & REEF_F_BOTH_SHARES);
+    int split = 0, rem;
+    if (tail.both) {
+        tail.fused = false;
+        rem = xcd_chunked(task, tiles);
+    } else {
+        rem = task = xcd_chunked(task, tiles * split_k);
+        if (split_k > 1) {
+            const int q = div_small(task, tail.fused ? split_k : tiles);
+            split = tail.fused ? task - q * split_k : q;
+            rem = tail.fused ? q : task - split * tiles;
+        }
+    }
+    const int mt = div_small(rem, n_tiles), nt = rem - mt * n_tiles;
+    const int m0 = mt * TD::BM, n0 = nt * TD::BN;
+    tail.split = split;
+    tail.rem = rem;
+    const int cb = split * chunk, ce = tail.both ? C : min(C, cb + chunk);
+    const int c0 = cb + 16 * wave;                                   // first channel of this wavefront
+    const int steps = c0 < ce ? (ce - c0 + 63) >> 6 : 0;             // its steps (uniform)
+    const unsigned HW4 = (unsigned)N * 4u, MN4 = (unsigned)M * HW4;
+
+    const unsigned C16 = (unsigned)(C + 15) / 16u;
+    const rsrc_t rs_a = make_rsrc(d.ptr[a[REEF_CONV_WPACK]], (unsigned)((M + 15) / 16) * C16 * 1024u);
+    unsigned va[TM];
+#pragma unroll
+    for (int h = 0; h < TM; ++h) va[h] = ((unsigned)(m0 / 16 + h) * C16 + (unsigned)(c0 / 16)) * 1024u + (unsigned)lane * 16u;
+    // channels from C on lie behind the buffer and read as zeros, and so does a row of tiles behind the last
+    const rsrc_t rs_b = make_rsrc(d.ptr[0], (unsigned)C * HW4);
+    const int row0 = lane / LPR, piece = lane % LPR;                 // row of this lane's first load
+    const int px = n0 + 4 * piece;
+    const int ch0 = c0 + 4 * (row0 & 3) + (row0 >> 2);               // load j: channel ch0 + j (TN 4), ch0 + 2 j (TN 2)
+    unsigned vb[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) vb[j] = px < N ? (unsigned)(ch0 + j * (TN == 2 ? 2 : 1)) * HW4 + (unsigned)px * 4u : kOutside;
+
+    const int ep_next = tail.to_ws ? 3
+                                   : 3 + ((flags & REEF_F_BIAS) ? 1 : 0) + ((flags & REEF_F_RESIDUAL) ? 1 : 0) +
+                                         ((flags & REEF_F_AFFINE) ? 2 : 0) + ((flags & REEF_F_DUAL) ? 2 : 0);
+    tail.aux = ep_next + (PRE ? 2 : 0);
+    // lanes 0, 1 of four: scale, shift of the first load's channel; 2, 3: of the second load's
+    const float* pre_s = (const float*)d.ptr[PRE ? ep_next : 0];
+    const float* pre_t = (const float*)d.ptr[PRE ? ep_next + 1 : 0];
+    const float* pre_at = (lane & 1) ? pre_t : pre_s;
+    int pre_c = ch0 + (TN == 2 ? (lane & 2) : 0);        // the same, in the next step to be loaded
+
+    f32x4 ra[NS][TM], rb[NS][TN];
+    float rp[PRE ? NS : 1];
+    auto load_step = [&](int s) {       // the next step's operands into stage s
+#pragma unroll
+        for (int h = 0; h < TM; ++h) {
+            ra[s][h] = buf_load4(rs_a, va[h]);
+            va[h] += 4096u;
+        }
+        if (PRE) {
+            rp[PRE ? s : 0] = pre_at[min(pre_c, C - 1)];
+            pre_c += 64;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            rb[s][j] = buf_load4(rs_b, vb[j]);
+            vb[j] += 64u * HW4;
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        load_step(s);
+        asm volatile("" ::: "memory");
+    }
+    const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
+#pragma unroll
+    for (int h = 0; h < TM; ++h) {
+        tail.om[h] = (unsigned)(m0 + 16 * h + orow);
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+            const unsigned on = (unsigned)(n0 + 16 * g + ocol);
+            tail.ooff[h][g] = on < (unsigned)N ? (tail.om[h] * (unsigned)N + on) * 4u : kOutside;
+        }
+    }
+    tail.fetch(d, MN4);
+    if (Poll::enabled) {        // the wrapper's flag check, as in conv2d_direct_body
+        if (threadIdx.x == 0) *sflag = poll.load();
+        __syncthreads();
+        if (*sflag) return false;
+    }
+    f32x4 acc[TM][TN][2];
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g) acc[h][g][0] = acc[h][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // the turned block lies where this wavefront's partial tile goes afterwards
+    float* blk = smem + wave * WSTRIDE;
+    auto swz = [](int kslot) { return TN == 4 ? kslot : TN == 2 ? kslot >> 1 : 0; };
+    float* wr = blk + row0 * (16 * TN) + (((piece >> 2) ^ swz(row0 & 3)) * 16) + (piece & 3) * 4;
+    const float* rd[TN];
+#pragma unroll
+    for (int g = 0; g < TN; ++g) rd[g] = blk + kq * (16 * TN) + ((g ^ swz(kq)) * 16) + i16;
+    float bt[2][TN][4];
+    int turn_c = ch0 + (TN == 2 ? (lane & 2) : 0);       // channel whose scale or shift this lane holds in the next step
+    auto turn = [&](int s, int to) {
+        if (PRE) {
+            const float p = turn_c < C ? rp[PRE ? s : 0] : 0.0f;     // channels past C: relu(0)
+            turn_c += 64;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const float sc = j == 0 ? lane_of_quad<0>(p) : lane_of_quad<2>(p);
+                const float sh = j == 0 ? lane_of_quad<1>(p) : lane_of_quad<3>(p);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rb[s][j][e] = fmaxf(fmaf(rb[s][j][e], sc, sh), 0.0f);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) *(f32x4*)(wr + j * 256) = rb[s][j];
+        __builtin_amdgcn_wave_barrier();      // (keeps the order; the hardware has it anyway)
 #pragma unroll
         for (int g = 0; g < TN; ++g)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = acc[h][g][0][j] + acc[h][g][1][j];
-    __syncthreads();
-    if (Poll::enabled && *sflag) return false;
-    const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
-    constexpr int WSTRIDE = TD::SUBS * TD::PART;   // one wavefront's partial tiles
-    float v[TM][TN];
+            for (int q = 0; q < 4; ++q) bt[to][g][q] = rd[g][q * 64 * TN];
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto mma = [&](int s, int from) {
 #pragma unroll
-    for (int h = 0; h < TM; ++h)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int g = 0; g < TN; ++g) {
-            const float* e = mine + (h * TN + g) * TD::PART;
-            v[h][g] = ((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE];
-        }
-    if (to_ws) {
-        const rsrc_t ws = make_rsrc((const float*)d.ptr[2] + (size_t)split * M * N, MN4);
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g) buf_store(ws, ooff[h][g], v[h][g]);
-        return true;
-    }
-    if (!fused) {
-        if (flags & REEF_F_GAP_OUTPUT) {
-            // The global average of the layer's output instead of the output (a classifier's last
-            // convolution): one pixel tile covers the image, so the 16 lanes of an output row hold
-            // the whole row between them.  out[m] = sum over the pixels / N, pixels in ascending order
-            // within a lane, lanes folded pairwise.
-#pragma unroll
-            for (int h = 0; h < TM; ++h) {
-                float s = 0.0f;
+            for (int h = 0; h < TM; ++h)
 #pragma unroll
                 for (int g = 0; g < TN; ++g)
-                    if (ooff[h][g] != kOutside) s += ep.value(v[h][g], om[h] * 4u, e_res[h][g], e_bias[h]);
-#pragma unroll
-                for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
-                if ((threadIdx.x & 15) == 0 && om[h] < (unsigned)M) buf_store(ep.out, om[h] * 4u, s * (1.0f / (float)N));
+                    acc[h][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], bt[from][g][q], acc[h][g][q & 1], 0, 0, 0);
+    };
+    static_assert(NS % 2 == 0, "the turned blocks alternate");
+    int pf = 0, it = 0;
+    bool left = false;
+    f32x4 first = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // (a share is whole groups: the first one ends between two turns of the loop.  Tested inside the loop it
+    // made the compiler move the accumulators in every turn: ResNet-152 816 -> 848 us, without any such layer.)
+    int until = TD::SUBS == 1 && tail.both ? share : 0x7fffffff;
+    if (steps > 0) turn(0, 0);
+    for (;;) {
+    for (; it + 2 * NS <= steps && it < until; it += NS) {
+        if (Poll::enabled) {
+            if (pf) {
+                *sflag = 1;
+                left = true;
+                break;
             }
-            return true;
+            pf = poll.load();
         }
 #pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g)
-                ep.finish(v[h][g], ooff[h][g], om[h] * 4u, e_res[h][g], e_bias[h], e_sh2[h]);
-        return true;
+        for (int s = 0; s < NS; ++s) {
+            if (s + 1 < NS) turn(s + 1, (s + 1) & 1);
+            mma(s, s & 1);
+            load_step(s);
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + 1 == NS) turn(0, 0);
+        }
     }
+    if (TD::SUBS != 1 || until != it || left) break;
+    first = acc[0][0][0] + acc[0][0][1];
+    acc[0][0][0] = acc[0][0][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    until = 0x7fffffff;
+    }
+    if (!left && it + NS <= steps) {
+        if (Poll::enabled && pf) {
+            *sflag = 1;
+            left = true;
+        } else {
+            if (Poll::enabled) pf = poll.load();
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (s + 1 < NS) turn(s + 1, (s + 1) & 1);
+                mma(s, s & 1);
+                if (it + s + NS < steps) load_step(s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            it += NS;
+            if (it < steps) turn(0, 0);
+        }
+    }
+    if (!left) {
+#pragma unroll
+        for (int s = 0; s < NS - 1; ++s)
+            if (it + s < steps) {
+                if (it + s + 1 < steps) turn(s + 1, (s + 1) & 1);
+                mma(s, s & 1);
+            }
+    }
+    f32x4 sum[TM][TN];
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
+    return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, TD::SUBS == 1 ? &first : nullptr);
+}
 
-    // split-K folded inside the launch
-    const size_t MN = (size_t)M * N;
-    float* ws = (float*)d.ptr[aux];
-    if (split_k == 2 && (flags & REEF_F_PAIR_FOLD) && poll.pair_fold_ok()) {
-        // One exchange per output element.  A value is parked with its sign bit flipped: a sum
-        // of products that starts from +0 is never -0, so a parked value is never the empty
-        // slot's 0 (and a -0 is parked as +0, should one ever come).
-        unsigned* slots = (unsigned*)(ws + 2 * MN);
-        unsigned got[TM][TN];
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g) {
-                got[h][g] = 0;
-                if (ooff[h][g] != kOutside && om[h] < (unsigned)M) {
-                    unsigned mine = __float_as_uint(v[h][g]) ^ 0x80000000u;
-                    mine = mine ? mine : 0x80000000u;
-                    got[h][g] = __hip_atomic_exchange(&slots[ooff[h][g] >> 2], mine, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g)
-                if (got[h][g] != 0) {   // second to arrive: the other half is here
-                    const float other = __uint_as_float(got[h][g] ^ 0x80000000u);
-                    const float sum = split == 0 ? v[h][g] + other : other + v[h][g];   // split order
-                    ep.finish(sum, ooff[h][g], om[h] * 4u, e_res[h][g], e_bias[h], e_sh2[h]);
-                    __hip_atomic_store(&slots[ooff[h][g] >> 2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-        return true;
-    }
-    int* counters = (int*)d.ptr[aux + 1] + a[REEF_CONV_SYNC_OFF];
-    int* s_last = sflag + 1;
-#pragma unroll
-    for (int h = 0; h < TM; ++h)
-#pragma unroll
-        for (int g = 0; g < TN; ++g)
-            if (ooff[h][g] != kOutside && om[h] < (unsigned)M)
-                store_agent(ws + (size_t)split * MN + (ooff[h][g] >> 2), v[h][g]);
-    // every store of this workgroup has completed at device scope before it counts in
-    partial_stores_done();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int old = __hip_atomic_fetch_add(&counters[rem], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *s_last = (old == split_k - 1);
-    }
-    __syncthreads();
-    if (!*s_last) return true;
-#pragma unroll
-    for (int h = 0; h < TM; ++h)
-#pragma unroll
-        for (int g = 0; g < TN; ++g) {
-            if (ooff[h][g] != kOutside && om[h] < (unsigned)M) {
-                const float* src = ws + (ooff[h][g] >> 2);
-                float sum = 0.0f;
-                for (int s0 = 0; s0 < split_k; s0 += 4) {
-                    float p[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) p[j] = load_agent(src + (size_t)min(s0 + j, split_k - 1) * MN);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (s0 + j < split_k) sum = (s0 + j == 0) ? p[j] : sum + p[j];
-                }
-                ep.finish(sum, ooff[h][g], om[h] * 4u, e_res[h][g], e_bias[h], e_sh2[h]);
-            }
+// ---- reef_conv2d_v9_g<G>: 3x3 / stride 1 / padding 1, whole cache lines --------------------------------------
+// The row form (ROWS above: G image rows x one 14-column segment x 16 output channels, halo columns in lanes 14
+// and 15, horizontal taps from the neighbouring lanes) in steps of 16 channels a wavefront instead of 4, so that every
+// load is 128 bits wide: the weights as 1 KiB pieces of a copy packed [Cout / 16][Cin / 16][9 taps][k slot][16 rows]
+// [4 channels], an input row as 16 channels x 64 bytes, turned in LDS as in conv2d_v1_body.  The row form's 32-bit
+// input loads and ninth tap take the vector-memory pipe 118 cycles for a step of 4 channels (g2), as long as
+// its MFMAs last a CU; these take a quarter less, and the row form of one row (g1) needs no split of K on a 14 x 14
+// image, whose exchange cost 2100 cycles of 14600.
+// The weights of a tap are loaded again as soon as its MFMAs have been issued, the input rows as soon as they are in
+// LDS: a step's loads have the whole step in front of them, and one step is the whole loop body.
+template <int G>
+struct TileV9 {
+    static constexpr int ROW = 20;                          // floats of a channel's row in LDS: 16 columns, a zero one, padding
+    static constexpr int BLOCK = (G + 2) * 16 * ROW;        // floats of a wavefront's rows; its partial tile goes there afterwards
+    static_assert(BLOCK >= G * TileD16<G, 1>::PART, "the partial tile fits the rows' place");
+    static constexpr int LDS_BYTES = 4 * BLOCK * 4 + 16;
+};
+template <int G, class Poll>
+__device__ __forceinline__ bool conv2d_v9_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll& poll) {
+    typedef TileV9<G> TV;
+    float* smem = (float*)smem_raw;
+    int* sflag = (int*)(smem + 4 * TV::BLOCK);
+    const int* a = d.attr;
+    const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], H = a[REEF_CONV_H], W = a[REEF_CONV_W];
+    const int N = H * W;
+    const int split_k = a[REEF_CONV_SPLIT_K], n_tiles = a[REEF_CONV_N_TILES];
+    const int tiles = a[REEF_CONV_M_TILES] * n_tiles;
+    const int flags = a[REEF_CONV_FLAGS];
+    DirectTail<1, G> tail;
+    tail.flags = flags;
+    tail.split_k = split_k;
+    tail.fused = split_k > 1 && (flags & REEF_F_FUSED_REDUCE);
+    tail.to_ws = split_k > 1 && !tail.fused;
+    // tile and split of this workgroup, as in conv2d_direct_body
+    const int c_chunk = a[REEF_CONV_K_CHUNK] / 9;
+    const int share = c_chunk >> 6;          // steps of a share
+    tail.both = G == 1 && poll.plain && (flags & REEF_F_BOTH_SHARES);
+    int split = 0, rem;
+    if (tail.both) {
+        tail.fused = false;
+        rem = xcd_chunked(task, tiles);
+    } else {
+        rem = task = xcd_chunked(task, tiles * split_k);
+        if (split_k > 1) {
+            const int q = div_small(task, tail.fused ? split_k : tiles);
+            split = tail.fused ? task - q * split_k : q;
+            rem = tail.fused ? q : task - split * tiles;
         }
-    if (threadIdx.x == 0)  // ready for the next run
-        __hip_atomic_store(&counters[rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
+    }
+    const int mt = div_small(rem, n_tiles), nt = rem - mt * n_tiles;
+    int seg = 0, yt = nt;
+    if (W > kRowSeg) {
+        const int segs = (W + kRowSeg - 1) / kRowSeg;
+        yt = div_small(nt, segs);
+        seg = nt - yt * segs;
+    }
+    const int m0 = mt * 16, y0 = yt * G, x0 = seg * kRowSeg;
+    tail.split = split;
+    tail.rem = rem;
+    const int cb = split * c_chunk, ce = tail.both ? C : min(C, cb + c_chunk);
+    const int c0 = cb + 16 * wave;
+    int steps = c0 < ce ? (ce - c0 + 63) >> 6 : 0;
+    const unsigned HW4 = (unsigned)N * 4u;
+
+    const unsigned C16 = (unsigned)(C + 15) / 16u;
+    const rsrc_t rs_a = make_rsrc(d.ptr[a[REEF_CONV_WPACK]], (unsigned)((M + 15) / 16) * C16 * 9216u);
+    unsigned va = ((unsigned)mt * C16 + (unsigned)(c0 / 16)) * 9216u + (unsigned)lane * 16u;
+    // channels from C on lie behind the buffer and read as zeros
+    const rsrc_t rs_b = make_rsrc(d.ptr[0], (unsigned)C * HW4);
+    const int row0 = lane >> 2;
+    const int s0 = x0 > 0 ? x0 - 1 : 0;                              // column of the image where the loaded rows start
+    unsigned vb[G + 2];
+#pragma unroll
+    for (int r = 0; r < G + 2; ++r) {
+        const int iy = y0 - 1 + r;
+        vb[r] = (unsigned)iy < (unsigned)H
+                    ? (unsigned)(c0 + 4 * (row0 & 3) + (row0 >> 2)) * HW4 + (unsigned)(iy * W + s0 + 4 * (lane & 3)) * 4u : kOutside;
+    }
+    f32x4 ra[9], rb[G + 2];
+    auto load_a = [&](int t) { ra[t] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_a, (int)va, t * 1024, 0)); };
+    auto load_b = [&]() {
+#pragma unroll
+        for (int r = 0; r < G + 2; ++r) {
+            rb[r] = buf_load4(rs_b, vb[r]);
+            vb[r] += 64u * HW4;
+        }
+    };
+    load_b();
+#pragma unroll
+    for (int t = 0; t < 9; ++t) load_a(t);
+
+    // the wavefront's block: rows [image row][4 q + kq][16 columns], channel 4 kq + q; column 16 is zero
+    float* blk = smem + wave * TV::BLOCK;
+#pragma unroll
+    for (int z = 0; z < ((G + 2) * 16 + 63) / 64; ++z)
+        if (z * 64 + lane < (G + 2) * 16) blk[(z * 64 + lane) * TV::ROW + 16] = 0.0f;
+    float* wr = blk + row0 * TV::ROW + (lane & 3) * 4;
+    const int col = i16 == 15 ? (x0 > 0 ? 0 : 16) : x0 + i16 < W ? x0 + i16 - s0 : 16;
+    const float* rd = blk + kq * TV::ROW + col;
+
+    const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
+    const int ep_next = tail.to_ws ? 3
+                                   : 3 + ((flags & REEF_F_BIAS) ? 1 : 0) + ((flags & REEF_F_RESIDUAL) ? 1 : 0) +
+                                         ((flags & REEF_F_AFFINE) ? 2 : 0) + ((flags & REEF_F_DUAL) ? 2 : 0);
+    tail.aux = ep_next;
+    tail.om[0] = (unsigned)(m0 + orow);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const bool ok = ocol < kRowSeg && x0 + ocol < W && y0 + g < H;
+        tail.ooff[0][g] = ok ? (tail.om[0] * (unsigned)N + (unsigned)((y0 + g) * W + x0 + ocol)) * 4u : kOutside;
+    }
+    tail.fetch(d, (unsigned)M * HW4);
+    if (Poll::enabled) {        // the wrapper's flag check, as in conv2d_direct_body
+        if (threadIdx.x == 0) *sflag = poll.load();
+        __syncthreads();
+        if (*sflag) return false;
+    }
+    f32x4 acc[1][G][2];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[0][g][0] = acc[0][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float in[G + 2][4];
+    auto turn = [&]() {                 // the loaded rows through LDS; on to the loads behind them
+#pragma unroll
+        for (int r = 0; r < G + 2; ++r) *(f32x4*)(wr + r * 16 * TV::ROW) = rb[r];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < G + 2; ++r)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) in[r][q] = rd[(r * 16 + 4 * q) * TV::ROW];
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto tap = [&](int t, const float (&v)[G + 2][4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                acc[0][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[t][q], v[g + t / 3][q], acc[0][g][q & 1], 0, 0, 0);
+    };
+    // The middle taps first, the neighbours' values formed behind them: then the loaded registers are free, and the
+    // next step's rows go through LDS under the outer taps.  (Formed next to its use, a neighbour's value waits for
+    // the MFMA that still reads its register: 58 cycles an MFMA.  All three taps read from LDS: 580 cycles a step.)
+    auto step = [&](auto more) {
+        float lf[G + 2][4], rt[G + 2][4];
+        if (more) va += 4 * 9216u;
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky) {
+            tap(3 * ky + 1, in);
+#pragma unroll
+            for (int r = ky; r < (ky < 2 ? ky + 1 : G + 2); ++r)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    lf[r][q] = lane_from_left(in[r][q]);
+                    rt[r][q] = lane_from_right(in[r][q]);
+                    asm volatile("" : "+v"(lf[r][q]), "+v"(rt[r][q]));
+                }
+            if (more) load_a(3 * ky + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (more) {
+            turn();
+            if (steps > 2) load_b();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int kx = 0; kx < 3; kx += 2)
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky) {
+                tap(3 * ky + kx, kx ? rt : lf);
+                if (more) load_a(3 * ky + kx);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    f32x4 first = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    struct Yes { constexpr operator bool() const { return true; } };
+    struct No { constexpr operator bool() const { return false; } };
+    int pf = 0;
+    bool left = false;
+    if (steps > 0) {
+        turn();
+        if (steps > 1) load_b();
+        if (G == 1 && tail.both) {
+            // (a loop of its own: one loop with the share's end inside cost the layers without shares 2 % of a pass)
+            for (const int rest = steps - share; steps > rest; --steps) step(Yes());
+            first = acc[0][0][0] + acc[0][0][1];
+            acc[0][0][0] = acc[0][0][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        for (; steps > 1; --steps) {
+            if (Poll::enabled) {
+                if (pf) {
+                    *sflag = 1;
+                    left = true;
+                    break;
+                }
+                pf = poll.load();
+            }
+            step(Yes());
+        }
+        if (!left) step(No());
+    }
+    f32x4 sum[1][G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) sum[0][g] = acc[0][g][0] + acc[0][g][1];
+    return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, G == 1 ? &first : nullptr);
 }
 
 // ---- reef_conv2d_xdw[2]_g<G>: 1x1 convolution, then depthwise 3x3, in one launch --------------

@@ -27,6 +27,7 @@ ACT_NONE, ACT_RELU, ACT_RELU6, ACT_GELU = 0, 1, 2, 3
 F_BIAS, F_RESIDUAL, F_AFFINE, F_DUAL, F_FUSED_REDUCE, F_PRE_ACT, F_PAIR_FOLD, F_DW_OUTPUT = 1, 2, 4, 8, 16, 32, 64, 128
 F_PROJ_OUTPUT = 4096
 F_POOL_OUTPUT, F_IN_SHIFT, F_POOL_SHIFT, F_GAP_OUTPUT = 256, 512, 1024, 2048
+F_BOTH_SHARES = 8192
 WG = 256
 
 
@@ -78,7 +79,7 @@ class GraphBuilder:
         self.unique_names = True
         # split-K folded inside the conv kernel (False: separate reef_splitk_reduce launch)
         self.fused_reduce = False
-        # multi-tap filters on the direct / row tiles also get a copy of their weights in the
+        # filters on the direct / row tiles also get a copy of their weights in the
         # layout those kernels load fastest (pack_conv_weights); parameter key = weight key + "k"
         self.pack_weights = True
         self.pair_fold = os.environ.get("REEF_PAIR_FOLD", "1") != "0"
@@ -234,7 +235,8 @@ class GraphBuilder:
         t = force or tiling.choose(M, N, K, fused=fused_reduce, pointwise=(kh, kw) == (1, 1),
                                    taps=kh * kw, direct=tiling.direct_ok(cin, kh, kw),
                                    rows=tiling.rows_ok(kh, kw, sh, sw, ph, pw), image=(Ho, Wo),
-                                   under_load=self.under_load, stride=max(sh, sw), pre_act=pre_act)
+                                   under_load=self.under_load, stride=max(sh, sw), pre_act=pre_act,
+                                   packed=self.pack_weights and w_arr is not None)
         if t.get("fused"):
             fused_reduce = True       # the measured table asks for the split folded into the launch
         pre = []
@@ -268,14 +270,22 @@ class GraphBuilder:
             mode, fam = 0, ""
         kname = "reef_conv2d_" + fam + t["tile"]
         packed = []
-        if self.pack_weights and w_arr is not None and (fam, t["tile"]) in PACKED_KERNELS:
+        # a launch has MAX_ARGS operands, the packed copy among them
+        others = 3 + len(opt) + len(pre) + (2 if t["split_k"] > 1 and fused_reduce else 0)
+        if self.pack_weights and w_arr is not None and (fam, t["tile"]) in PACKED_KERNELS and (kh * kw > 1 or others < MAX_ARGS):
             key = self.storage[w.idx]["name"] + "k"
-            arr = pack_conv_weights(w_arr.reshape(cout, cin, kh * kw))
+            v9 = fam == "r9_" and t["tile"] in tiling.V9_TILES
+            arr = pack_conv_weights(w_arr.reshape(cout, cin, kh * kw), by_channels=v9 or kh * kw == 1)
             pidx = self._storage(key, arr.size)
             self.graph_args.append(pidx)
             self.params.append((key, arr))
             packed = [pidx]
-            kname = "reef_conv2d_" + fam[:-1] + "k_" + t["tile"]
+            if v9:
+                kname = "reef_conv2d_v9_" + t["tile"]
+            elif kh * kw > 1:        # the 1-tap kernels take either form
+                kname = "reef_conv2d_" + fam[:-1] + "k_" + t["tile"]
+            elif tiling.v1_ok(kh, kw, sh, sw, ph, pw, N, t["tile"], cin, pre_act):
+                kname = "reef_conv2d_" + ("p1_v_" if pre else "v1_") + t["tile"]
             nbytes_pack = 4 * (arr.size - M * K)        # the copy is read instead of the original
         else:
             nbytes_pack = 0
@@ -298,6 +308,14 @@ class GraphBuilder:
             sync_idx, sync_off = self._sync_counters(t["m_tiles"] * t["n_tiles"])
             args = [x, w.idx, out.idx] + opt + pre + [ws.idx, sync_idx]
             flags |= F_PAIR_FOLD if pair else 0
+            share = t["k_chunk"] // (kh * kw)
+            # A split of two whose tiles alone give nearly every CU a workgroup gains nothing from twice as many that
+            # meet again (exchange: 2100 cycles).  ResNet-152's 71 such layers: 896 us of device time a pass where
+            # they meet (16x32 and two image rows a tile), 829 with both shares in one workgroup (16x16, one row).
+            if (pair and 2 * share == cin and t["m_tiles"] * t["n_tiles"] >= BOTH_SHARES_TILES
+                    and (share % 256 == 0 and kname in ("reef_conv2d_v1_16x16k4", "reef_conv2d_p1_v_16x16k4")
+                         or share % 64 == 0 and kname == "reef_conv2d_v9_g1")):
+                flags |= F_BOTH_SHARES
             attrs = base + [flags | F_FUSED_REDUCE, act, t["tile_id"], t["split_k"], t["k_chunk"],
                             t["m_tiles"], t["n_tiles"], act2, sync_off, mode, dst_off, len(args) if packed else 0]
             self._emit(kname, t["tasks"], args + packed, attrs, "conv2d", flops, nbytes + nbytes_pack, t["est_us"])
@@ -750,6 +768,11 @@ class GraphBuilder:
                 NG = (G + 2) if S == 1 else (2 * G + 1) * 2      # TileXdw: pixel groups of the 1x1 result
                 PS = (96 if S == 2 else 64 if G == 4 else 160) + 4     # a chunk of input channels per pixel / weight row
                 shared[n] = (NG * 16 * PS + 16 * PS + 16 * (NG * 16 + 20)) * 4 + 16
+            elif sym in ("reef_conv2d_v1_16x16k4", "reef_conv2d_p1_v_16x16k4"):
+                shared[n] = 4 * 2 * 320 * 4 + 16      # TileV1: a partial tile of either share
+            elif sym.startswith("reef_conv2d_v9_"):
+                # TileV9: four blocks of [image rows][16 channels][20 floats]
+                shared[n] = 4 * (tiling.ROW_TILES[sym.split("_")[-1]] + 2) * 16 * 20 * 4 + 16
             elif sym.startswith("reef_conv2d_") or sym.startswith("reef_gemm_"):
                 shared[n] = tiling.lds_bytes(sym.split("_")[-1])
                 if sym.startswith("reef_gemm_ntl_"):
@@ -801,21 +824,32 @@ class GraphBuilder:
         return base
 
 
+BOTH_SHARES_TILES = 192     # output tiles from which a workgroup takes both shares of a split of two
+MAX_ARGS = 9     # REEF_MAX_PTRS - 1: the last slot carries what a launch prefetches for the next one
+
 # (loader family prefix, tile) of the kernels that exist in a packed-weights form
 PACKED_KERNELS = {("r9_", "g1"), ("r9_", "g2"), ("r9_", "g4"), ("d9_", "16x16k4"), ("d9_", "16x32k4"),
                   ("d9_", "32x32d4"), ("d3_", "16x16k4"), ("d3_", "16x32k4"), ("d7_", "16x16k4"),
                   ("d7_", "16x32k4"), ("d25_", "16x16k4"), ("d25_", "16x32k4")}
+PACKED_KERNELS |= {("d1_", t) for t in tiling.DIRECT_TILES} | {("p1_", t) for t in tiling.PRE_ACT_TILES}
 
 
-def pack_conv_weights(w):
-    """[Cout][Cin][taps] weights -> the layout of attr REEF_CONV_WPACK:
-    [ceil(Cout/16)][ceil(Cin/4)][ceil(taps/4)][4 channels][16 rows][4 taps], zero-padded."""
+def pack_conv_weights(w, by_channels=False):
+    """[Cout][Cin][taps] weights -> the layouts of attr REEF_CONV_WPACK, zero-padded:
+    [ceil(Cout/16)][ceil(Cin/4)][ceil(taps/4)][4 channels][16 rows][4 taps], or by_channels
+    [ceil(Cout/16)][ceil(Cin/16)][taps][4 slots][16 rows][4 channels]."""
     M, C, R = w.shape
-    mt, c4, g4 = -(-M // 16), -(-C // 4), -(-R // 4)
-    pad = np.zeros((mt * 16, c4 * 4, g4 * 4), np.float32)
-    pad[:M, :C, :R] = w
-    # pad[mt*16 + i, c4*4 + kq, g*4 + j] -> out[mt, c4, g, kq, i, j]
-    out = pad.reshape(mt, 16, c4, 4, g4, 4).transpose(0, 2, 4, 3, 1, 5)
+    mt = -(-M // 16)
+    c, r = (-(-C // 16) * 16, R) if by_channels else (-(-C // 4) * 4, -(-R // 4) * 4)
+    if (mt * 16, c, r) != (M, C, R):
+        pad = np.zeros((mt * 16, c, r), np.float32)
+        pad[:M, :C, :R] = w
+    else:
+        pad = w
+    if by_channels:     # pad[mt*16 + i, c*16 + 4 kq + q, t] -> out[mt, c, t, kq, i, q]
+        out = pad.reshape(mt, 16, c // 16, 4, 4, r).transpose(0, 2, 5, 3, 1, 4)
+    else:               # pad[mt*16 + i, c*4 + kq, g*4 + j] -> out[mt, c, g, kq, i, j]
+        out = pad.reshape(mt, 16, c // 4, 4, r // 4, 4).transpose(0, 2, 4, 3, 1, 5)
     return np.ascontiguousarray(out).reshape(-1)
 
 

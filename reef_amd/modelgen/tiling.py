@@ -9,7 +9,7 @@ split-K to put a workgroup on every CU.
 """
 import math
 
-from .tuned import TUNED, TUNED_UNDER_LOAD, GEMM_UNDER_LOAD
+from .tuned import TUNED, TUNED_UNDER_LOAD, TUNED_PACKED, TUNED_PACKED_UNDER_LOAD, GEMM_UNDER_LOAD
 
 # name -> (id, BM, BN, relative MFMA efficiency of the inner loop, workgroups per CU)
 TILES = {
@@ -40,6 +40,7 @@ TILES = {
 }
 # matrix products only (reef_gemm_ntd_<tile>, reef_gemm_ntl_<tile>): name -> (id, BM, BN)
 GEMM_WIDE_TILES = {"32x48d4": (19, 32, 48), "48x48d4": (20, 48, 48), "64x64d4": (21, 64, 64)}
+V9_TILES = ("g1", "g2", "g4")      # row tiles that exist as reef_conv2d_v9_<tile>
 # row form: image rows per tile
 ROW_TILES = {"g1": 1, "g2": 2, "g4": 4, "g7": 7, "g2m2": 2, "g4m2": 4}
 ROW_SEG = 14
@@ -212,12 +213,14 @@ def _steps_time(bm, bn, eff, steps):
 
 
 def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, pointwise=False,
-           taps=1, direct=False, rows=False, image=None, under_load=False, stride=1, pre_act=False):
+           taps=1, direct=False, rows=False, image=None, under_load=False, stride=1, pre_act=False, packed=False):
     """Returns dict(tile, tile_id, BM, BN, split_k, k_chunk, m_tiles, n_tiles, tasks).
     Measured choices (tuned.py) win over the analytic model for the shapes they cover; an entry
     that names the direct tile counts only if the caller says the filter qualifies.
     under_load: the layer belongs to a model that shares the device with other streams; the
     entries measured for that case (TUNED_UNDER_LOAD) come before those measured alone.
+    packed: the layer's weights will be packed, so that it runs on the kernels that take whole cache lines
+    (v1_ok, the row tiles' v9): entries measured with those (TUNED_PACKED) come before the others.
     image: output rows and columns of a convolution (with stride, pre_act: the input goes through an
     activation of its own); shapes outside the table are then chosen by the measured cost of every
     tile (CONV_COST), those of a bare matrix product by the analytic model."""
@@ -226,6 +229,10 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
         hit = TUNED.get(key)
         if under_load and key in TUNED_UNDER_LOAD:
             hit = TUNED_UNDER_LOAD[key] + (hit[2] if hit is not None else 0.0,)
+        if packed and key in TUNED_PACKED:
+            hit = TUNED_PACKED[key] + (hit[2] if hit is not None else 0.0,)
+        if packed and under_load and key in TUNED_PACKED_UNDER_LOAD:
+            hit = TUNED_PACKED_UNDER_LOAD[key] + (hit[2] if hit is not None else 0.0,)
         if hit is not None and hit[0] in ROW_TILES:
             if rows and image is not None:
                 t = forced_rows(hit[0], M, image[0], image[1], K, abs(hit[1]))
@@ -240,7 +247,7 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
             t["fused"] = hit[1] < 0
             return t
     if allow_split and tiles is None and (image is not None or direct and M * N <= NUM_CUS * 4096):
-        return _choose_conv(M, N, K, taps, direct, rows and image is not None, image, stride, pointwise, pre_act)
+        return _choose_conv(M, N, K, taps, direct, rows and image is not None, image, stride, pointwise, pre_act, packed)
     best = None
     for name in (tiles or [t for t in TILES if t not in DIRECT_TILES and t not in ROW_TILES]):
         tid, bm, bn, eff, occ = TILES[name]
@@ -330,22 +337,51 @@ CONV_COST = {
     ("32x32k4", "p"): (4.406, 1, 2.163, 3.927, 1.29, 2.115, 0),
     ("32x32k4", "q"): (6.071, 2.839, 0, 10.58, 2.008, 1.917, 0),
 }
+# The same for the kernels on packed weights that take whole cache lines: "v" 1x1 (reef_conv2d_v1_*), "w" 3x3
+# (reef_conv2d_v9_*).  340 layer shapes of the same networks at 64 to 448, 3700 candidates; choosing by it costs
+# 5 % (1x1) and 2 % (3x3) on average against the measured best of a shape.
+CONV_COST_PACKED = {
+    ("16x16k4", "v"): (4.001, 0, 1.59, 0, 0.1832, 0, 1.203),
+    ("16x32k4", "v"): (3.821, 0, 3.041, 0, 0.2629, 0, 1.921),
+    ("16x64k4", "v"): (3.469, 0, 3.819, 2.785, 0.8784, 0, 3.612),
+    ("32x32d4", "v"): (3.444, 1.303, 2.86, 1.301, 0.7217, 0, 4.165),
+    ("g1", "w"): (3.502, 0.1328, 0.9924, 0.07493, 0.3518, 0, 2.982),
+    ("g2", "w"): (3.258, 0.2351, 1.289, 0.7421, 0.7164, 0, 4.338),
+    ("g4", "w"): (3.564, 0, 1.267, 2.714, 1.729, 0, 5.952),
+}
 PRE_ACT_LAUNCH_US = 6.0   # a pre-activation launch of its own, in front of a tile without the form
 
 
-def conv_kind(tile, taps, stride=1, pointwise=True):
+# Input channels from which a plain 1x1 layer of these tiles loads its input in 16-byte pieces; below, the kernel that
+# loads single values starts sooner.  Device time of whole passes: MobileNet-v2 (16x16k4, 144 to 576 channels)
+# 154.6 us with all of them in pieces, 153.4 from 256 channels, 152.5 from 512, 151.6 with none; ResNet-152 (16x32k4)
+# 836 with all, 832 from 65, 829 from 129 or 192, 842 from 257; ResNet-50 at 448 656 and 645 from 256.  Layers with
+# a pre-activation and 32x32d4 gain at every size (DenseNet-201's best-effort kernels 1037 us, 1041 from 512; ResNet-50 at
+# 448 645, 647 from 129, 654 from 513).
+V1_MIN_CIN = {"16x16k4": 640, "16x32k4": 256}
+
+
+def v1_ok(kh, kw, sh, sw, ph, pw, n_pixels, tile, cin, pre):
+    """Whether a 1x1 layer on packed weights loads its input in 16-byte pieces (reef_conv2d_v1_*)."""
+    return (kh, kw, sh, sw, ph, pw) == (1, 1, 1, 1, 0, 0) and n_pixels % 4 == 0 and (
+        pre or cin >= V1_MIN_CIN.get(tile, 0))
+
+
+def conv_kind(tile, taps, stride=1, pointwise=True, packed=False, n_pixels=0, cin=0, pre=False):
     if taps != 1:
-        return "9" if taps == 9 else "n"
+        return "w" if packed and tile in V9_TILES else "9" if taps == 9 else "n"
     if stride > 1:
         return "s"
-    return "1" if tile in DIRECT_TILES else "p" if pointwise else "q"
+    if tile in DIRECT_TILES:
+        return "v" if packed and n_pixels % 4 == 0 and (pre or cin >= V1_MIN_CIN.get(tile, 0)) else "1"
+    return "p" if pointwise else "q"
 
 
 def direct_cost(tile, geom, fused=True, kind="1"):
     """Microseconds of a launch of this geometry (forced, forced_rows) by CONV_COST."""
     s = geom["split_k"]
     r = geom["tasks"] / NUM_CUS
-    us = _cost(CONV_COST[(tile, kind)], geom["k_chunk"], geom["tasks"], s, (r + math.ceil(r)) / 2)
+    us = _cost((CONV_COST_PACKED if kind in "vw" else CONV_COST)[(tile, kind)], geom["k_chunk"], geom["tasks"], s, (r + math.ceil(r)) / 2)
     return us + T_REDUCE_LAUNCH if s > 1 and not fused else us
 
 
@@ -356,7 +392,7 @@ def _cost(c, depth, tasks, split, rounds):
     return t + c[5] + 0.1 * c[6] * split if split > 1 else t
 
 
-def _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act):
+def _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act, packed=False):
     """Cheapest tile and split of a convolution by CONV_COST; a split is folded inside the launch."""
     best = None
     pointwise = pointwise and stride == 1 and N % 4 == 0 and K % 4 == 0
@@ -365,8 +401,8 @@ def _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act)
             continue
         if tile in DIRECT_TILES and not (direct and taps in DIRECT_TAPS[tile]):
             continue
-        kind = conv_kind(tile, taps, stride, pointwise)
-        if (tile, kind) not in CONV_COST:
+        kind = conv_kind(tile, taps, stride, pointwise, packed and image is not None, N, K // taps, pre_act)
+        if (tile, kind) not in CONV_COST and (tile, kind) not in CONV_COST_PACKED:
             continue
         for s in (1, 2, 3, 4, 6, 8):
             g = forced_rows(tile, M, image[0], image[1], K, s) if tile in ROW_TILES else forced(tile, M, N, K, s, taps)

@@ -248,6 +248,32 @@ TUNED_UNDER_LOAD = {
     (128, 49, 1888, 1): ("16x16k4", -8),
 }
 
+# Entries that come before TUNED's for layers on packed weights, whose kernels take whole cache lines
+# (reef_conv2d_v1_*, reef_conv2d_v9_*).  Measured as whole passes of the network, the five cheapest choices of
+# tiling.CONV_COST_PACKED for every shape, kept where the pass is faster by more than 0.12 %: ResNet-152 911 -> 829 us
+# of device time (256 x 196 x 2304 39 of them, 256 x 196 x 1024 41: a workgroup takes both shares of their splits), Inception-v3
+# 462.3 -> 456.3, DenseNet-201 alone 912.8 -> 895.  Shapes that are not here keep TUNED's tile.
+TUNED_PACKED = {
+    (256, 196, 2304, 0): ("g1", -2),
+    (256, 196, 1024, 1): ("16x16k4", -2),
+    (512, 49, 4608, 0): ("g1", -2),
+    (2048, 49, 512, 1): ("32x32d4", 1),
+    (512, 49, 2048, 1): ("16x32k4", -2),
+    (320, 3136, 64, 1): ("16x32k4", 1),
+    (96, 1225, 576, 0): ("16x16k4", 1),
+    (704, 289, 768, 1): ("16x32k4", 1),
+    (768, 289, 768, 1): ("16x32k4", 1),
+    (80, 5329, 64, 1): ("16x32k4", 1),
+    (32, 784, 1152, 0): ("g1", 1),
+    (32, 3136, 1152, 0): ("g2", 1),
+}
+# The same under load (before TUNED_UNDER_LOAD): DenseNet-201's best-effort kernels, one pass alone 1144 -> 1037 us
+# and four passes side by side 1681 -> 1580; a split that meets on counters costs more than it saves now.
+TUNED_PACKED_UNDER_LOAD = {
+    (32, 49, 1152, 0): ("g1", 1),
+    (32, 196, 1152, 0): ("g1", 1),
+}
+
 # The same for the K-contiguous matrix products (tiling.choose_gemm(under_load=True)):
 # (M, N, K) -> (direct tile, split of K folded inside the launch).  BERT-base's FFN-down product in four,
 # which is the choice for a model alone as well.  Two clients of the network on two streams, inferences
