@@ -23,7 +23,7 @@ namespace reef_dev {
 
 // out = act(sum_{s ascending} ws[s] (+res)(+bias)(*scale+shift)); 4 elements per thread.
 template <int BATCH>
-__device__ __forceinline__ void splitk_reduce_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void splitk_reduce_body(const OpDesc& d, int task) {
     const int* a = d.attr;
     const int M = a[REEF_RED_M], N = a[REEF_RED_N], S = a[REEF_RED_SPLIT_K];
     const size_t MN = (size_t)M * N;
@@ -95,7 +95,7 @@ __device__ __forceinline__ float dw_taps(rsrc_t rs_in, rsrc_t rs_w, unsigned in_
     return acc;
 }
 
-__device__ __forceinline__ void dwconv2d_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void dwconv2d_body(const OpDesc& d, int task) {
     const int* a = d.attr;
     const int C = a[REEF_DW_C], H = a[REEF_DW_H], W = a[REEF_DW_W], Ho = a[REEF_DW_HO],
               Wo = a[REEF_DW_WO], kh = a[REEF_DW_KH], kw = a[REEF_DW_KW], sh = a[REEF_DW_SH],
@@ -128,7 +128,7 @@ __device__ __forceinline__ void dwconv2d_body(const ReefOpDesc& d, int task) {
     ((float*)d.ptr[2])[idx] = act_apply(acc, a[REEF_DW_ACT]);
 }
 
-__device__ __forceinline__ void pool2d_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void pool2d_body(const OpDesc& d, int task) {
     const int* a = d.attr;
     const int C = a[REEF_POOL_C], H = a[REEF_POOL_H], W = a[REEF_POOL_W], Ho = a[REEF_POOL_HO],
               Wo = a[REEF_POOL_WO], kh = a[REEF_POOL_KH], kw = a[REEF_POOL_KW],
@@ -192,7 +192,7 @@ __device__ __forceinline__ void pool2d_body(const ReefOpDesc& d, int task) {
 }
 
 // one wavefront per channel
-__device__ __forceinline__ void global_avgpool_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void global_avgpool_body(const OpDesc& d, int task) {
     const int C = d.attr[REEF_GAP_C], HW = d.attr[REEF_GAP_HW];
     const int c = task * 4 + (threadIdx.x >> 6);
     if (c >= C) return;
@@ -209,7 +209,7 @@ __device__ __forceinline__ void global_avgpool_body(const ReefOpDesc& d, int tas
     if ((threadIdx.x & 63) == 0) ((float*)d.ptr[1])[c] = s * (1.0f / (float)HW);
 }
 
-__device__ __forceinline__ void eltwise_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void eltwise_body(const OpDesc& d, int task) {
     const int* at = d.attr;
     const int C = at[REEF_ELT_C], inner = at[REEF_ELT_INNER], flags = at[REEF_ELT_FLAGS],
               act = at[REEF_ELT_ACT];
@@ -244,7 +244,7 @@ __device__ __forceinline__ void eltwise_body(const ReefOpDesc& d, int task) {
 }
 
 // GEMV: one wavefront per output neuron, 128-bit loads along k.
-__device__ __forceinline__ void dense_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void dense_body(const OpDesc& d, int task) {
     const int* a = d.attr;
     const int rows = a[REEF_DENSE_ROWS], in_f = a[REEF_DENSE_IN], out_f = a[REEF_DENSE_OUT],
               act = a[REEF_DENSE_ACT];
@@ -278,7 +278,7 @@ __device__ __forceinline__ void dense_body(const ReefOpDesc& d, int task) {
 }
 
 // one wavefront per row: max, exp, sum, divide
-__device__ __forceinline__ void softmax_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void softmax_body(const OpDesc& d, int task) {
     const int rows = d.attr[REEF_SM_ROWS], cols = d.attr[REEF_SM_COLS];
     const int r = task * 4 + (threadIdx.x >> 6);
     if (r >= rows) return;
@@ -329,7 +329,7 @@ __device__ __forceinline__ void softmax_body(const ReefOpDesc& d, int task) {
 // and sum are a few exchanges.  The values are fetched into registers while
 // the scores are computed and take the keys' place in LDS afterwards.  Every thread reaches
 // every barrier (rows and columns outside the tensor compute on zeros and are not stored).
-__device__ __forceinline__ void attention_body(const ReefOpDesc& d, int task, char* smem_raw) {
+__device__ __forceinline__ void attention_body(const OpDesc& d, int task, char* smem_raw) {
     const int* a = d.attr;
     const int S = a[REEF_AT_SEQ], HD = a[REEF_AT_HEAD_DIM];
     const int ld = a[REEF_AT_LD], ldo = a[REEF_AT_LDO];
@@ -445,7 +445,7 @@ __device__ __forceinline__ void attention_body(const ReefOpDesc& d, int task, ch
 }
 
 // one wavefront per row; two-pass mean / variance as the reference splits it
-__device__ __forceinline__ void layernorm_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void layernorm_body(const OpDesc& d, int task) {
     const int rows = d.attr[REEF_LN_ROWS], cols = d.attr[REEF_LN_COLS];
     const int r = task * 4 + (threadIdx.x >> 6);
     if (r >= rows) return;
@@ -503,7 +503,7 @@ __device__ __forceinline__ void layernorm_body(const ReefOpDesc& d, int task) {
     }
 }
 
-__device__ __forceinline__ void bias_gelu_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void bias_gelu_body(const OpDesc& d, int task) {
     const int rows = d.attr[REEF_GELU_ROWS], cols = d.attr[REEF_GELU_COLS];
     const float* x = (const float*)d.ptr[0];
     float* y = (float*)d.ptr[1];
@@ -516,7 +516,7 @@ __device__ __forceinline__ void bias_gelu_body(const ReefOpDesc& d, int task) {
     }
 }
 
-__device__ __forceinline__ void embedding_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void embedding_body(const OpDesc& d, int task) {
     const int seq = d.attr[REEF_EMB_SEQ], hidden = d.attr[REEF_EMB_HIDDEN],
               flags = d.attr[REEF_EMB_FLAGS];
     const long long* ids = (const long long*)d.ptr[0];
@@ -536,7 +536,7 @@ __device__ __forceinline__ void embedding_body(const ReefOpDesc& d, int task) {
     }
 }
 
-__device__ __forceinline__ void copy_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void copy_body(const OpDesc& d, int task) {
     const int count = d.attr[REEF_COPY_COUNT], dst_off = d.attr[REEF_COPY_DST_OFF];
     const float* in = (const float*)d.ptr[0];
     float* out = (float*)d.ptr[1] + dst_off;
@@ -550,7 +550,7 @@ __device__ __forceinline__ void copy_body(const ReefOpDesc& d, int task) {
 }
 
 // in [d0][d1][d2] -> out [d1][d0][d2] (+ bias[d1][d2])
-__device__ __forceinline__ void transpose_body(const ReefOpDesc& d, int task) {
+__device__ __forceinline__ void transpose_body(const OpDesc& d, int task) {
     const int d0 = d.attr[REEF_TR_D0], d1 = d.attr[REEF_TR_D1], d2 = d.attr[REEF_TR_D2];
     const float* in = (const float*)d.ptr[0];
     float* out = (float*)d.ptr[1];
@@ -572,7 +572,7 @@ __device__ __forceinline__ void transpose_body(const ReefOpDesc& d, int task) {
 // The reference's mocked model: logical block = task, 128 logical threads;
 // out[task*128 + t] = a[t] (+|*) b[task*128 + t]   (mocked_kernel.cu:9-27)
 template <bool MUL>
-__device__ __forceinline__ void mocked_body(const ReefOpDesc& d, int task, int t) {
+__device__ __forceinline__ void mocked_body(const OpDesc& d, int task, int t) {
     const float* a = (const float*)d.ptr[0];
     const float* b = (const float*)d.ptr[1];
     float* out = (float*)d.ptr[2];

@@ -14,6 +14,55 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kWave = 64;
 constexpr int kThreads = REEF_WG_THREADS;
 
+
+// A launch's descriptor, its attributes and first eight pointers in scalar registers.  A body that reads them one by
+// one from the argument block waits five or six times in a row, whenever what it reads next depends on what it has read:
+// 560 cycles from the first line of reef_conv2d_v9_g1 to its first load, 840 with the pass over the block's
+// lines that stood in front.  Here everything comes in one trip; no load crosses a line of a block that starts on one.  ResNet-152 826 -> 821 us of device time a pass, DenseNet-201 919 -> 901.
+struct OpPtrs {
+    const ReefOpDesc* m;
+    typedef int i32x16 __attribute__((ext_vector_type(16)));
+    i32x16 lo;
+    __device__ __forceinline__ void* operator[](int i) const {
+        if (__builtin_constant_p(i) && i < 8)
+            return (void*)((uint64_t)(uint32_t)lo[2 * i] | (uint64_t)(uint32_t)lo[2 * i + 1] << 32);
+        return m->ptr[i];       // a slot that the flags name
+    }
+};
+struct OpDesc {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    typedef int i32x8 __attribute__((ext_vector_type(8)));
+    OpPtrs ptr;
+    int attr[REEF_MAX_ATTRS];
+    // BEFORE: bytes of the argument block in front of the descriptor, whose first line comes along
+    template <int BEFORE>
+    __device__ __forceinline__ static OpDesc load(const ReefOpDesc& m) {
+        static_assert(REEF_MAX_ATTRS == 24 && offsetof(ReefOpDesc, attr) == 0x50, "the offsets below");
+        OpDesc d;
+        i32x4 a0, a3;
+        i32x8 a1, a2;
+        // (the pointers are needed last; in front of the attributes DenseNet-201 took 5 us more)
+#define REEF_DESC_LOADS "s_load_dwordx4 %[a0], %[m], 0x50\n\ts_load_dwordx8 %[a1], %[m], 0x60\n\t" \
+                        "s_load_dwordx8 %[a2], %[m], 0x80\n\ts_load_dwordx4 %[a3], %[m], 0xa0\n\ts_load_dwordx16 %[p], %[m], 0x0\n\t"
+#define REEF_DESC_REGS [a0] "=&s"(a0), [a1] "=&s"(a1), [a2] "=&s"(a2), [a3] "=&s"(a3), [p] "=&s"(d.ptr.lo)
+        if (BEFORE == 0) {
+            asm volatile(REEF_DESC_LOADS "s_waitcnt lgkmcnt(0)" : REEF_DESC_REGS : [m] "s"(&m));
+        } else {
+            int touched;
+            asm volatile(REEF_DESC_LOADS "s_load_dword %[t], %[f], 0x0\n\ts_waitcnt lgkmcnt(0)"
+                         : REEF_DESC_REGS, [t] "=&s"(touched) : [m] "s"(&m), [f] "s"((const char*)&m - BEFORE));
+        }
+#undef REEF_DESC_REGS
+#undef REEF_DESC_LOADS
+        d.ptr.m = &m;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { d.attr[i] = a0[i]; d.attr[20 + i] = a3[i]; }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { d.attr[4 + i] = a1[i]; d.attr[12 + i] = a2[i]; }
+        return d;
+    }
+};
+
 // ---- preemption polling -------------------------------------------------
 // The reference's best-effort wrapper reads *preempted once at block start
 // (script/best_effort_kernel.py:22-29) and relies on a patched driver to kill
@@ -119,10 +168,11 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// (Selected, not branched on: a chain of jumps per value stood behind every convolution.  With one epilogue for
+// all ways a tile is finished instead of three, ResNet-152 829 -> 826 us a pass, DenseNet-201 925 -> 919.)
 __device__ __forceinline__ float act_apply(float v, int act) {
-    if (act == REEF_ACT_RELU) return fmaxf(v, 0.0f);
-    if (act == REEF_ACT_RELU6) return fminf(fmaxf(v, 0.0f), 6.0f);
-    return v;
+    const float r = fminf(fmaxf(v, 0.0f), act == REEF_ACT_RELU6 ? 6.0f : __builtin_inff());
+    return act == REEF_ACT_RELU || act == REEF_ACT_RELU6 ? r : v;
 }
 
 __device__ __forceinline__ float gelu_erf(float x) {
@@ -206,7 +256,8 @@ struct Epilogue {
     const float* shift2;
     int act, act2;
     int next;  // first pointer slot after the optional operands
-    __device__ __forceinline__ void unpack(const ReefOpDesc& d, int first, int flags, int act_,
+    template <class D>
+    __device__ __forceinline__ void unpack(const D& d, int first, int flags, int act_,
                                            int act2_ = 0) {
         int p = first;
         bias = (flags & REEF_F_BIAS) ? (const float*)d.ptr[p++] : nullptr;

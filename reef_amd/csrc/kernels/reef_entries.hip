@@ -29,31 +29,31 @@ namespace {
 
 // Tasks of a plain launch, from its attributes: workgroups behind them prefetch for the next launch.
 // Ops without a count here are never given any.
-__device__ __forceinline__ int conv_tasks(const ReefOpDesc& d) {
+__device__ __forceinline__ int conv_tasks(const OpDesc& d) {
     return d.attr[REEF_CONV_SPLIT_K] * d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
 }
 // (a plain launch whose workgroups take both shares of a split: the others come last)
-__device__ __forceinline__ int conv_v_tasks(const ReefOpDesc& d) {
+__device__ __forceinline__ int conv_v_tasks(const OpDesc& d) {
     const int tiles = d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
     return (d.attr[REEF_CONV_FLAGS] & REEF_F_BOTH_SHARES) ? tiles : tiles * d.attr[REEF_CONV_SPLIT_K];
 }
-__device__ __forceinline__ int gemm_tasks(const ReefOpDesc& d) {
+__device__ __forceinline__ int gemm_tasks(const OpDesc& d) {
     const int s = d.attr[REEF_GEMM_SPLIT_K];
     return d.attr[REEF_GEMM_BATCH] * d.attr[REEF_GEMM_M_TILES] * d.attr[REEF_GEMM_N_TILES] * (s > 1 ? s : 1);
 }
-__device__ __forceinline__ int attention_tasks(const ReefOpDesc& d) {
+__device__ __forceinline__ int attention_tasks(const OpDesc& d) {
     return d.attr[REEF_AT_HEADS] * ((d.attr[REEF_AT_SEQ] + REEF_AT_ROWS - 1) / REEF_AT_ROWS);
 }
-__device__ __forceinline__ int attention_mma_tasks(const ReefOpDesc& d) {
+__device__ __forceinline__ int attention_mma_tasks(const OpDesc& d) {
     return d.attr[REEF_AT_HEADS] * ((d.attr[REEF_AT_SEQ] + REEF_AT_MM_ROWS - 1) / REEF_AT_MM_ROWS);
 }
-__device__ __forceinline__ int pool_tasks(const ReefOpDesc& d) {
+__device__ __forceinline__ int pool_tasks(const OpDesc& d) {
     return (d.attr[REEF_POOL_C] * d.attr[REEF_POOL_HO] * d.attr[REEF_POOL_WO] + kThreads - 1) / kThreads;
 }
-__device__ __forceinline__ int gap_tasks(const ReefOpDesc& d) { return (d.attr[REEF_GAP_C] + 3) / 4; }
-__device__ __forceinline__ int no_tasks(const ReefOpDesc&) { return 0x7fffffff; }
+__device__ __forceinline__ int gap_tasks(const OpDesc& d) { return (d.attr[REEF_GAP_C] + 3) / 4; }
+__device__ __forceinline__ int no_tasks(const OpDesc&) { return 0x7fffffff; }
 #define REEF_TASKS(FN) \
-    static __device__ __forceinline__ int tasks(const ReefOpDesc& d) { return FN(d); }
+    static __device__ __forceinline__ int tasks(const OpDesc& d) { return FN(d); }
 
 // ---- op functors: LDS need + body ------------------------------------------
 template <class T, int MODE = CONV_GENERAL>
@@ -61,7 +61,7 @@ struct OpConv {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = T::LDS_BYTES;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_body<T, MODE>(d, task, smem, p);
     }
 };
@@ -71,7 +71,7 @@ struct OpConvDirect {
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;   // the body makes the wrapper's first flag check
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_direct_body<R, TN, TM, PRE, ROWS, PACKED, FROWS, ODDC>(d, task, smem, p);
     }
 };
@@ -82,7 +82,7 @@ struct OpConvV1 {
     static constexpr int LDS = TileV1<TM, TN>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_v1_body<TM, TN, PRE>(d, task, smem, p);
     }
 };
@@ -93,7 +93,7 @@ struct OpConvV9 {
     static constexpr int LDS = TileV9<G>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_v9_body<G>(d, task, smem, p);
     }
 };
@@ -116,7 +116,7 @@ struct OpConvXdw {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileXdw<G, S>::LDS_BYTES;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_xdw_body<G, S>(d, task, smem, p);
     }
 };
@@ -127,7 +127,7 @@ struct OpConvBlock {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileBlk<G, S, STEM, MT, KC>::LDS_BYTES;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_block_body<G, S, STEM, MT, KC>(d, task, smem, p);
     }
 };
@@ -136,7 +136,7 @@ struct OpConvStemPool {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileSp7::LDS_BYTES;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_stem_pool_body(d, task, smem, p);
     }
 };
@@ -145,7 +145,7 @@ struct OpGemm {
     REEF_TASKS(gemm_tasks)
     static constexpr int LDS = T::LDS_BYTES + (LN_A ? 2 * T::BM * 4 : 0);   // + mean, rstd of the tile's rows
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return gemm_body<T, TRANS_B, LN_A>(d, task, smem, p);
     }
 };
@@ -155,7 +155,7 @@ struct OpGemmNtDirect {
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES + (LN ? 9 * 16 * TM * 4 : 0);   // + the rows' sums per wavefront, pivots
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P& p) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return gemm_nt_direct_body<TM, TN, LN>(d, task, smem, p);
     }
 };
@@ -164,7 +164,7 @@ struct OpGemmNtDirect {
         REEF_TASKS(TASKS)                                                                       \
         static constexpr int LDS = 0;                                                           \
         template <class P>                                                                      \
-        static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char*, const P&) { \
+        static __device__ __forceinline__ bool run(const OpDesc& d, int task, char*, const P&) { \
             CALL(d, task);                                                                      \
             return true;                                                                        \
         }                                                                                       \
@@ -173,7 +173,7 @@ struct OpAttention {
     REEF_TASKS(attention_tasks)
     static constexpr int LDS = REEF_AT_LDS_BYTES;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P&) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P&) {
         attention_body(d, task, smem);
         return true;
     }
@@ -182,7 +182,7 @@ struct OpAttentionMma {
     REEF_TASKS(attention_mma_tasks)
     static constexpr int LDS = REEF_AT_MM_LDS_BYTES;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char* smem, const P&) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P&) {
         attention_mma_body(d, task, smem);
         return true;
     }
@@ -206,7 +206,7 @@ struct OpMocked {
     REEF_TASKS(no_tasks)
     static constexpr int LDS = 0;
     template <class P>
-    static __device__ __forceinline__ bool run(const ReefOpDesc& d, int task, char*, const P&) {
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char*, const P&) {
 #if REEF_FLAVOUR == 2
         const int t = threadIdx.x;   // the padding flavour is launched with a flat workgroup
 #else
@@ -307,8 +307,8 @@ __device__ __forceinline__ bool dkp_walk(const ReefDkpArgs& a, DkpWalk& w) {
 #define REEF_ENTRY(NAME, OP)                                                          \
     extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS) NAME(ReefOpDesc) {  \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];               \
-        kernarg_warm<sizeof(ReefOpDesc)>();                                           \
-        const ReefOpDesc& d = kernarg_at<ReefOpDesc>(0);                              \
+        const ReefOpDesc& m = kernarg_at<ReefOpDesc>(0);                              \
+        const OpDesc d = OpDesc::load<0>(m);                                          \
         const int behind = (int)blockIdx.x - OP::tasks(d);                            \
         if (behind >= 0) {                                                            \
             prefetch_lines((const ReefPrefetch*)d.ptr[REEF_PREFETCH_SLOT], behind);   \
@@ -358,20 +358,20 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
     extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS) NAME(ReefBeArgs) {      \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];                   \
         __shared__ int s_pre;                                                             \
-        kernarg_warm<sizeof(ReefBeArgs)>();                                               \
         const ReefBeArgs& a = kernarg_at<ReefBeArgs>(0);                                  \
+        const OpDesc d = OpDesc::load<offsetof(ReefBeArgs, desc)>(a.desc);                \
         const int t = threadIdx.x + threadIdx.y * blockDim.x + threadIdx.z * blockDim.x * blockDim.y; \
         FlagPoll poll{a.preempted};                                                       \
         bool done = false;                                                                \
         if (a.tasks != 0 && blockIdx.x >= a.tasks) {                                      \
             done = true;                                                                  \
-            prefetch_lines((const ReefPrefetch*)a.desc.ptr[REEF_PREFETCH_SLOT], (int)(blockIdx.x - a.tasks)); \
+            prefetch_lines((const ReefPrefetch*)d.ptr[REEF_PREFETCH_SLOT], (int)(blockIdx.x - a.tasks)); \
         } else if (ChecksFlagItself<OP>::value) {                                                \
-            done = OP::run(a.desc, (int)blockIdx.x, smem, poll);                          \
+            done = OP::run(d, (int)blockIdx.x, smem, poll);                          \
         } else {                                                                          \
             if (t == 0) s_pre = poll.load();                                              \
             __syncthreads();                                                              \
-            if (!s_pre) done = OP::run(a.desc, (int)blockIdx.x, smem, poll);              \
+            if (!s_pre) done = OP::run(d, (int)blockIdx.x, smem, poll);              \
         }                                                                                 \
         if (t == 0) be_count_completed(a, done);                                          \
         be_signal_exit(a, t);                                                             \
@@ -394,7 +394,8 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         if (!dkp_walk(a, w)) return;                                                   \
         const ReefDkpSide& side = w.right ? a.r : a.l;                                 \
         for (int i = w.idx; i < w.end; i += w.step) {                                  \
-            OP::run(side.desc, i, smem, NoPoll{!w.right, false});                             \
+            const OpDesc d = OpDesc::load<0>(side.desc);                               \
+            OP::run(d, i, smem, NoPoll{!w.right, false});                             \
             __syncthreads();                                                           \
         }                                                                              \
     }                                                                                  \

@@ -502,32 +502,28 @@ struct ConvEpilogue {
     int act, act2;
     int next;         // first pointer slot after the optional operands
     unsigned doff4;   // byte offset of this layer's slice inside the output tensor(s)
-    __device__ __forceinline__ void init(const ReefOpDesc& d, int flags, int act_, int act2_, int M,
+    template <class D>
+    __device__ __forceinline__ void init(const D& d, int flags, int act_, int act2_, int M,
                                          unsigned MN4, unsigned doff4_) {
-        int p = 3;
+        // The slots follow from the flags alone, so the pointers come in one trip instead of one per operand that
+        // is there; a slot nobody fills is read, and its value not used.
         const unsigned M4 = (unsigned)M * 4u;
         doff4 = doff4_;
-        out = make_rsrc(d.ptr[2], doff4 + MN4);
         has_bias = flags & REEF_F_BIAS;
         has_res = flags & REEF_F_RESIDUAL;
         has_affine = flags & REEF_F_AFFINE;
         has_dual = flags & REEF_F_DUAL;
-        bias = res = scale = shift = out2 = shift2 = out;
-        if (has_bias) bias = make_rsrc(d.ptr[p++], M4);
-        if (has_res) res = make_rsrc(d.ptr[p++], MN4);
-        if (has_affine) {
-            scale = make_rsrc(d.ptr[p], M4);
-            shift = make_rsrc(d.ptr[p + 1], M4);
-            p += 2;
-        }
-        if (has_dual) {
-            out2 = make_rsrc(d.ptr[p], doff4 + MN4);
-            shift2 = make_rsrc(d.ptr[p + 1], M4);
-            p += 2;
-        }
+        const int p_res = 3 + (has_bias ? 1 : 0), p_aff = p_res + (has_res ? 1 : 0), p_dual = p_aff + (has_affine ? 2 : 0);
+        next = p_dual + (has_dual ? 2 : 0);
+        out = make_rsrc(d.ptr[2], doff4 + MN4);
+        bias = make_rsrc(d.ptr[3], M4);
+        res = make_rsrc(d.ptr[p_res], MN4);
+        scale = make_rsrc(d.ptr[p_aff], M4);
+        shift = make_rsrc(d.ptr[p_aff + 1], M4);
+        out2 = make_rsrc(d.ptr[p_dual], doff4 + MN4);
+        shift2 = make_rsrc(d.ptr[p_dual + 1], M4);
         act = act_;
         act2 = act2_;
-        next = p;
     }
     // off = (m * N + n) * 4 or outside; m4 = m * 4.  v = acc; v += residual; v += bias;
     // v = fma(v, scale, shift); act  -- then out2 = act2(out + shift2).
@@ -547,7 +543,7 @@ struct ConvEpilogue {
 };
 
 template <class T, int MODE, class Poll>
-__device__ __forceinline__ bool conv2d_body(const ReefOpDesc& d_in, int task, char* smem_raw,
+__device__ __forceinline__ bool conv2d_body(const OpDesc& d_in, int task, char* smem_raw,
                                             const Poll& poll) {
   int M, N, split_k, split, rem, m0, n0;
   float* smem = (float*)smem_raw;
@@ -561,7 +557,7 @@ __device__ __forceinline__ bool conv2d_body(const ReefOpDesc& d_in, int task, ch
   const WaveGeom<T> wg;
   const int r0 = wg.wk * T::RPW;   // first accumulator element this wavefront writes out
   {
-    const ReefOpDesc& d = d_in;
+    const OpDesc& d = d_in;
     const int* a = d.attr;
     M = a[REEF_CONV_COUT];
     N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
@@ -626,7 +622,7 @@ __device__ __forceinline__ bool conv2d_body(const ReefOpDesc& d_in, int task, ch
 
     // Everything the epilogue needs is re-read from the argument block here, so the
     // K loop does not carry the epilogue's pointers in scalar registers.
-    const ReefOpDesc* dp = &d_in;
+    const ReefOpDesc* dp = d_in.ptr.m;
     asm volatile("" : "+s"(dp));
     const ReefOpDesc& d = *dp;
     const int* a = d.attr;
@@ -815,7 +811,7 @@ struct DirectTail {
     bool both;                               // this workgroup has both shares of a split of two (REEF_F_BOTH_SHARES)
 
     // Epilogue operands, fetched behind the first K steps' loads.
-    __device__ __forceinline__ void fetch(const ReefOpDesc& d, unsigned MN4) {
+    __device__ __forceinline__ void fetch(const OpDesc& d, unsigned MN4) {
         const int* a = d.attr;
         ep.next = 3;   // plain split-K launches carry no epilogue operands
 #pragma unroll
@@ -844,7 +840,7 @@ struct DirectTail {
 // WSTRIDE: floats between the wavefronts' places in LDS; the flags lie behind the last.
 // first: the first share's sums where the workgroup has both (t.both).
 template <int TM, int TN, int WSTRIDE = TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, class Poll>
-__device__ __forceinline__ bool direct_tail(const ReefOpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN],
+__device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN],
                                             const DirectTail<TM, TN>& t, const Poll& poll, const f32x4* first = nullptr) {
     typedef TileD16<TN, TM> TD;
     float* smem = (float*)smem_raw;
@@ -889,102 +885,121 @@ __device__ __forceinline__ bool direct_tail(const ReefOpDesc& d, char* smem_raw,
             for (int g = 0; g < TN; ++g) buf_store(ws, t.ooff[h][g], v[h][g]);
         return true;
     }
-    if (!t.fused) {
-        if (t.flags & REEF_F_GAP_OUTPUT) {
-            // The global average of the layer's output instead of the output (a classifier's last
-            // convolution): one pixel tile covers the image, so the 16 lanes of an output row hold
-            // the whole row between them.  out[m] = sum over the pixels / N, pixels in ascending order
-            // within a lane, lanes folded pairwise.
+    if (!t.fused && (t.flags & REEF_F_GAP_OUTPUT)) {
+        // The global average of the layer's output instead of the output (a classifier's last
+        // convolution): one pixel tile covers the image, so the 16 lanes of an output row hold
+        // the whole row between them.  out[m] = sum over the pixels / N, pixels in ascending order
+        // within a lane, lanes folded pairwise.
 #pragma unroll
-            for (int h = 0; h < TM; ++h) {
-                float s = 0.0f;
+        for (int h = 0; h < TM; ++h) {
+            float s = 0.0f;
 #pragma unroll
-                for (int g = 0; g < TN; ++g)
-                    if (t.ooff[h][g] != kOutside) s += t.ep.value(v[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h]);
+            for (int g = 0; g < TN; ++g)
+                if (t.ooff[h][g] != kOutside) s += t.ep.value(v[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h]);
 #pragma unroll
-                for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
-                if ((threadIdx.x & 15) == 0 && t.om[h] < (unsigned)M) buf_store(t.ep.out, t.om[h] * 4u, s * (1.0f / (float)N));
-            }
-            return true;
+            for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+            if ((threadIdx.x & 15) == 0 && t.om[h] < (unsigned)M) buf_store(t.ep.out, t.om[h] * 4u, s * (1.0f / (float)N));
         }
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g)
-                t.ep.finish(v[h][g], t.ooff[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h], t.e_sh2[h]);
         return true;
     }
-
-    // split-K folded inside the launch
-    const size_t MN = (size_t)M * N;
-    float* ws = (float*)d.ptr[t.aux];
-    if (t.split_k == 2 && (t.flags & REEF_F_PAIR_FOLD) && poll.pair_fold_ok()) {
-        // One exchange per output element.  A value is parked with its sign bit flipped: a sum
-        // of products that starts from +0 is never -0, so a parked value is never the empty
-        // slot's 0 (and a -0 is parked as +0, should one ever come).
-        unsigned* slots = (unsigned*)(ws + 2 * MN);
-        unsigned got[TM][TN];
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g) {
-                got[h][g] = 0;
-                if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M) {
-                    unsigned mine = __float_as_uint(v[h][g]) ^ 0x80000000u;
-                    mine = mine ? mine : 0x80000000u;
-                    got[h][g] = __hip_atomic_exchange(&slots[t.ooff[h][g] >> 2], mine, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g)
-                if (got[h][g] != 0) {   // second to arrive: the other half is here
-                    const float other = __uint_as_float(got[h][g] ^ 0x80000000u);
-                    const float sum = t.split == 0 ? v[h][g] + other : other + v[h][g];   // split order
-                    t.ep.finish(sum, t.ooff[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h], t.e_sh2[h]);
-                    __hip_atomic_store(&slots[t.ooff[h][g] >> 2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-        return true;
-    }
-    int* counters = (int*)d.ptr[t.aux + 1] + a[REEF_CONV_SYNC_OFF];
-    int* s_last = sflag + 1;
+    // what this thread stores: its values, at their offsets (kOutside: none)
+    unsigned off[TM][TN];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
-        for (int g = 0; g < TN; ++g)
-            if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M)
-                store_agent(ws + (size_t)t.split * MN + (t.ooff[h][g] >> 2), v[h][g]);
-    // every store of this workgroup has completed at device scope before it counts in
-    partial_stores_done();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int old = __hip_atomic_fetch_add(&counters[t.rem], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *s_last = (old == t.split_k - 1);
+        for (int g = 0; g < TN; ++g) off[h][g] = t.ooff[h][g];
+    if (t.fused) {
+        // split-K folded inside the launch
+        const size_t MN = (size_t)M * N;
+        float* ws = (float*)d.ptr[t.aux];
+        if (t.split_k == 2 && (t.flags & REEF_F_PAIR_FOLD) && poll.pair_fold_ok()) {
+            // One exchange per output element.  A value is parked with its sign bit flipped: a sum
+            // of products that starts from +0 is never -0, so a parked value is never the empty
+            // slot's 0 (and a -0 is parked as +0, should one ever come).
+            unsigned* slots = (unsigned*)(ws + 2 * MN);
+            unsigned got[TM][TN];
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) {
+                    got[h][g] = 0;
+                    if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M) {
+                        unsigned mine = __float_as_uint(v[h][g]) ^ 0x80000000u;
+                        mine = mine ? mine : 0x80000000u;
+                        got[h][g] = __hip_atomic_exchange(&slots[t.ooff[h][g] >> 2], mine, __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+            bool any = false;
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) {
+                    off[h][g] = kOutside;
+                    if (got[h][g] != 0) {   // second to arrive: the other half is here
+                        const float other = __uint_as_float(got[h][g] ^ 0x80000000u);
+                        v[h][g] = t.split == 0 ? v[h][g] + other : other + v[h][g];   // split order
+                        off[h][g] = t.ooff[h][g];
+                        any = true;
+                        __hip_atomic_store(&slots[t.ooff[h][g] >> 2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+            if (!any) return true;
+        } else {
+            int* counters = (int*)d.ptr[t.aux + 1] + a[REEF_CONV_SYNC_OFF];
+            int* s_last = sflag + 1;
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g)
+                    if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M)
+                        store_agent(ws + (size_t)t.split * MN + (t.ooff[h][g] >> 2), v[h][g]);
+            // every store of this workgroup has completed at device scope before it counts in
+            partial_stores_done();
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                const int old = __hip_atomic_fetch_add(&counters[t.rem], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *s_last = (old == t.split_k - 1);
+            }
+            __syncthreads();
+            if (!*s_last) return true;
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) {
+                    if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M) {
+                        const float* src = ws + (t.ooff[h][g] >> 2);
+                        float sum = 0.0f;
+                        for (int s0 = 0; s0 < t.split_k; s0 += 4) {
+                            float p[4];
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) p[j] = load_agent(src + (size_t)min(s0 + j, t.split_k - 1) * MN);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                if (s0 + j < t.split_k) sum = (s0 + j == 0) ? p[j] : sum + p[j];
+                        }
+                        v[h][g] = sum;
+                    }
+                }
+            if (threadIdx.x == 0)  // ready for the next run
+                __hip_atomic_store(&counters[t.rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
-    __syncthreads();
-    if (!*s_last) return true;
+    // one epilogue for all of them
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) {
-            if (t.ooff[h][g] != kOutside && t.om[h] < (unsigned)M) {
-                const float* src = ws + (t.ooff[h][g] >> 2);
-                float sum = 0.0f;
-                for (int s0 = 0; s0 < t.split_k; s0 += 4) {
-                    float p[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) p[j] = load_agent(src + (size_t)min(s0 + j, t.split_k - 1) * MN);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (s0 + j < t.split_k) sum = (s0 + j == 0) ? p[j] : sum + p[j];
-                }
-                t.ep.finish(sum, t.ooff[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h], t.e_sh2[h]);
-            }
+            v[h][g] = t.ep.value(v[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h]);
+            buf_store(t.ep.out, off[h][g] + t.ep.doff4, v[h][g]);
         }
-    if (threadIdx.x == 0)  // ready for the next run
-        __hip_atomic_store(&counters[t.rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t.ep.has_dual) {
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+                buf_store(t.ep.out2, off[h][g] + t.ep.doff4, act_apply(v[h][g] + t.e_sh2[h], t.ep.act2));
+    }
     return true;
 }
 
@@ -1056,7 +1071,7 @@ __device__ __forceinline__ float lane_of_row(float v) {      // every lane <- la
 // ODDC (1-tap kernels; symbols reef_conv2d_o1_*): Cin is no multiple of 4.  The last 128-bit load of a row
 // of weights reaches into the next row; those values are dropped in front of the MFMAs.
 template <int R, int TN, int TM, bool PRE, bool ROWS, bool PACKED, bool FROWS, bool ODDC, class Poll>
-__device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int task, char* smem_raw,
+__device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task, char* smem_raw,
                                                    const Poll& poll) {
     static_assert(!PRE || R == 1, "the pre-activation form exists for 1-tap filters only");
     static_assert(!ROWS || R == 9, "the row form exists for 3x3 filters only");
@@ -1068,7 +1083,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const ReefOpDesc& d_in, int t
     constexpr int RC = G::RC, NS = G::NS;
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * TD::SUBS * TD::PART);
-    const ReefOpDesc& d = d_in;
+    const OpDesc& d = d_in;
     const int* a = d.attr;
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1453,13 +1468,15 @@ struct TileV1 {      // a wavefront's place: the turned block, then its partial 
     static constexpr int LDS_BYTES = 4 * WSTRIDE * 4 + 16;
 };
 template <int TM, int TN, bool PRE, class Poll>
-__device__ __forceinline__ bool conv2d_v1_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll& poll) {
+__device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
     static_assert(TN == 1 || TN == 2 || TN == 4, "a row of the turned block is 64, 128 or 256 bytes");
     static_assert(!PRE || TN < 4, "scales and shifts of two channels a lane at most");
     typedef TileD16<TN, TM> TD;
     // steps of loads in flight (6, 8 and 12 on 16x16: the same K loop on 1024 channels, whose end the L2 -> CU
     // stream sets -- a 64-byte piece brings its 128-byte line -- and up to 1.5 % slower networks)
-    constexpr int NS = 4;
+    // steps of loads in flight (with a pre-activation in 2 more wavefronts fit: DenseNet-201 901 -> 891 us of device time a
+    // pass, 1022 -> 1016 as a best-effort model; without one ResNet-152 takes 826 us in 4 and 878 in 2)
+    constexpr int NS = PRE ? 2 : 4;
     constexpr int LPR = 4 * TN;                    // lanes (16-byte pieces) of a row
     float* smem = (float*)smem_raw;
     constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
@@ -1692,7 +1709,7 @@ struct TileV9 {
     static constexpr int LDS_BYTES = 4 * BLOCK * 4 + 16;
 };
 template <int G, class Poll>
-__device__ __forceinline__ bool conv2d_v9_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll& poll) {
+__device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
     typedef TileV9<G> TV;
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * TV::BLOCK);
@@ -1935,7 +1952,7 @@ struct TileXdw {
 };
 
 template <int G, int S, class Poll>
-__device__ __forceinline__ bool conv2d_xdw_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll&) {
+__device__ __forceinline__ bool conv2d_xdw_body(const OpDesc& d, int task, char* smem_raw, const Poll&) {
     typedef TileXdw<G, S> T;
     constexpr int R = T::R, NG = T::NG, GW = T::GW, JM = T::CK / 16;
     float* smem = (float*)smem_raw;
@@ -2211,7 +2228,7 @@ __device__ __forceinline__ void blk_stage_store(const float (&v)[(COUNT + kThrea
 }
 
 template <int G, int S, bool STEM, int MT, int KC, class Poll>
-__device__ __forceinline__ bool conv2d_block_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll&) {
+__device__ __forceinline__ bool conv2d_block_body(const OpDesc& d, int task, char* smem_raw, const Poll&) {
     typedef TileBlk<G, S, STEM, MT, KC> T;
     constexpr int R = T::R, NG = T::NG, KF = T::KF, KP = T::KP;
     static_assert(!STEM || S == 1, "the stem form has a stride-1 depthwise stage");
@@ -2519,7 +2536,7 @@ struct TileSp7 {
 };
 
 template <class Poll>
-__device__ __forceinline__ bool conv2d_stem_pool_body(const ReefOpDesc& d, int task, char* smem_raw, const Poll&) {
+__device__ __forceinline__ bool conv2d_stem_pool_body(const OpDesc& d, int task, char* smem_raw, const Poll&) {
     typedef TileSp7 T;
     float* patch = (float*)smem_raw;
     float* E = patch + T::PATCH;
@@ -2668,7 +2685,7 @@ struct LnOut {
     f32x4 v, g, b;
     rsrc_t ra, rg, rb;
     // p: first of c1, c2, gamma, beta, A' in the pointer slots
-    __device__ __forceinline__ void init(const ReefOpDesc& d, int p, const float* A, int M_, int K, int lda, int m0_, int BM, int nt, int n_tiles) {
+    __device__ __forceinline__ void init(const OpDesc& d, int p, const float* A, int M_, int K, int lda, int m0_, int BM, int nt, int n_tiles) {
         out = (d.attr[REEF_GEMM_FLAGS] & REEF_GEMM_F_LN_OUT) ? (float*)d.ptr[p + 4] : nullptr;
         M = M_;
         m0 = m0_;
@@ -2747,7 +2764,7 @@ struct LnOut {
 // A and A' are [M][K] with leading dimension lda and no offset; no batch.
 // ptr: A, Wg, C, bias (optional), residual (optional), c1, c2, gamma, beta, A' (optional).
 template <class T, bool TRANS_B, bool LN_A, class Poll>
-__device__ __forceinline__ bool gemm_body(const ReefOpDesc& d, int task, char* smem_raw,
+__device__ __forceinline__ bool gemm_body(const OpDesc& d, int task, char* smem_raw,
                                           const Poll& poll) {
     const int* a = d.attr;
     const int M = a[REEF_GEMM_M], N = a[REEF_GEMM_N], K = a[REEF_GEMM_K];
@@ -2881,7 +2898,7 @@ __device__ __forceinline__ bool gemm_body(const ReefOpDesc& d, int task, char* s
 // on 32x32: 170 MB out of L2, 6.3 TB/s), and they go with (BM + BN) / (BM BN): 64x64 22.0 -> 17.9 us there,
 // 32x48 12.1 -> 10.2 at 128 x 2304 x 768, 48x48 27.4 -> 22.4 at 384 x 3072 x 768.
 template <int TM, int TN, bool LN, class Poll>
-__device__ __forceinline__ bool gemm_nt_direct_body(const ReefOpDesc& d, int task, char* smem_raw,
+__device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, char* smem_raw,
                                                     const Poll& poll) {
     typedef TileD16<TN, TM> TD;
     constexpr bool BIG = TM * TN > 4;
@@ -3278,7 +3295,7 @@ __device__ __forceinline__ void attention_scores(rsrc_t rk, const f32x4 (&q)[4],
     }
 }
 
-__device__ __forceinline__ void attention_mma_body(const ReefOpDesc& d, int task, char* smem_raw) {
+__device__ __forceinline__ void attention_mma_body(const OpDesc& d, int task, char* smem_raw) {
     constexpr int ROWS = REEF_AT_MM_ROWS;
     const int* a = d.attr;
     const int S = a[REEF_AT_SEQ], HD = a[REEF_AT_HEAD_DIM], heads = a[REEF_AT_HEADS];
