@@ -437,7 +437,9 @@ enum { REEF_TR_D0 = 0, REEF_TR_D1, REEF_TR_D2, REEF_TR_FLAGS, REEF_TR_NATTR };
  *       lda, ldb, ldc, strideA, strideB, strideC (elements), then offA, offB, offC: where the
  *       first matrix starts inside its storage, in elements (absent = 0; multiples of 4 like the
  *       strides) -- several operands can share one storage, e.g. Q, K and V as column blocks of
- *       one [tokens][3 * hidden] projection.
+ *       one [tokens][3 * hidden] projection.  ldb = 0 (direct kernels, batch 1, offB 0): B is the packed
+ *       copy of the weights, [ceil(N/16)][ceil(K/16)][4 slots][16 columns][4 k] floats, zero where a
+ *       column or k does not exist; its storage is named as the weights' with "pk" behind it.
  * tasks = batch * m_tiles * n_tiles.
  *
  * reef_gemm_ntl_<tile> (staged tiles; direct tiles with K a multiple of 8; trans_b = 1, batch 1, flags has REEF_GEMM_F_LN): the product

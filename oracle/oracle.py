@@ -438,6 +438,14 @@ class GraphOracle:
             alpha = _bits_to_float(alpha_bits)
             bias = P[3] if flags & 1 else None
             A, B, C = P[0][oA:], P[1][oB:], P[2][oC:]
+            if ldb == 0 or flags & 2:
+                names = [t["name"] for t in self.model["storage"]]
+                wname = names[k["args"][1]]
+            if ldb == 0:                                      # packed copy: the weights as the reference has them are kept
+                assert wname.endswith("pk"), wname            # under its name without "pk"
+                wname, ldb = wname[:-2], K
+                if not flags & 2:
+                    B = self.storage[names.index(wname)]
             p = 3 + (flags & 1)
             R = None
             if flags & 8:                                     # residual, laid out as C is
@@ -454,9 +462,8 @@ class GraphOracle:
                 if flags & 4:
                     np.lib.stride_tricks.as_strided(P[p + 4], (M, K), (lda * 4, 4))[:, :] = normed
                 A, lda = normed.reshape(-1), K
-                wname = self.model["storage"][k["args"][1]]["name"]
                 assert wname.endswith("gk"), wname
-                B = self.storage[[t["name"] for t in self.model["storage"]].index(wname[:-2])]
+                B = self.storage[names.index(wname[:-2])]
             for bi in range(batch):
                 Am = np.lib.stride_tricks.as_strided(A[bi * sA:], (M, K), (lda * 4, 4))
                 if trans_b:

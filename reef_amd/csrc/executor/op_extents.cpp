@@ -251,7 +251,7 @@ void splitk_reduce(const Attrs& a, Needs& n) {
 void gemm(const std::string& symbol, const Attrs& a, Needs& n) {
     if (a.v.size() <= (size_t)REEF_GEMM_STRIDE_C) { n.bad = "too few attributes for a matrix product"; return; }
     if (!all_positive(a, {REEF_GEMM_BATCH, REEF_GEMM_M, REEF_GEMM_N, REEF_GEMM_K, REEF_GEMM_M_TILES,
-                          REEF_GEMM_N_TILES, REEF_GEMM_LDA, REEF_GEMM_LDB, REEF_GEMM_LDC})) {
+                          REEF_GEMM_N_TILES, REEF_GEMM_LDA, REEF_GEMM_LDC}) || a[REEF_GEMM_LDB] < 0) {
         n.bad = "a dimension of the matrix product is not positive";
         return;
     }
@@ -266,10 +266,18 @@ void gemm(const std::string& symbol, const Attrs& a, Needs& n) {
         return;
     }
     n.f32("A", a[REEF_GEMM_OFF_A] + b1 * a[REEF_GEMM_STRIDE_A] + (M - 1) * a[REEF_GEMM_LDA] + K);
-    if (trans_b) n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (N - 1) * a[REEF_GEMM_LDB] + K);
+    const i64 fl = a[REEF_GEMM_FLAGS];
+    if (a[REEF_GEMM_LDB] == 0) {
+        // packed weights: the tiles that have the form: the direct ones
+        static const char* const kDirect[] = {"_16x16k4", "_16x32k4", "_32x32d4", "_32x48d4", "_48x48d4", "_64x64d4"};
+        bool ok = false;
+        for (const char* t : kDirect)
+            ok = ok || symbol == std::string("reef_gemm_ntd") + t || symbol == std::string("reef_gemm_ntl") + t;
+        if (!ok || !trans_b || b1 != 0 || a[REEF_GEMM_OFF_B] != 0) { n.bad = "packed weights: only the direct kernels take them, without a batch and an offset"; return; }
+        n.f32("packed B", cdiv(N, 16) * cdiv(K, 16) * 256);
+    } else if (trans_b) n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (N - 1) * a[REEF_GEMM_LDB] + K);
     else n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (K - 1) * a[REEF_GEMM_LDB] + N);
     n.f32("C", a[REEF_GEMM_OFF_C] + b1 * a[REEF_GEMM_STRIDE_C] + (M - 1) * a[REEF_GEMM_LDC] + N);
-    const i64 fl = a[REEF_GEMM_FLAGS];
     const i64 c_elems = a[REEF_GEMM_OFF_C] + b1 * a[REEF_GEMM_STRIDE_C] + (M - 1) * a[REEF_GEMM_LDC] + N;
     if (fl & REEF_GEMM_F_BIAS) n.f32("bias", N);
     if (fl & REEF_GEMM_F_RES) n.f32("residual", c_elems);

@@ -2897,15 +2897,21 @@ __device__ __forceinline__ bool gemm_body(const OpDesc& d, int task, char* smem_
 // eight and keep one accumulator per sub-tile.  A CU's loads are what bounds these products (384 x 2304 x 768
 // on 32x32: 170 MB out of L2, 6.3 TB/s), and they go with (BM + BN) / (BM BN): 64x64 22.0 -> 17.9 us there,
 // 32x48 12.1 -> 10.2 at 128 x 2304 x 768, 48x48 27.4 -> 22.4 at 384 x 3072 x 768.
-template <int TM, int TN, bool LN, class Poll>
-__device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, char* smem_raw,
-                                                    const Poll& poll) {
+//
+// PK (ldb = 0): B is the packed copy of a weight matrix, [ceil(N / 16)][ceil(K / 16)][k slot][16 columns]
+// [4 k], whose loads are contiguous KiBs, and the rows of A are loaded as 16-byte pieces (lane / 4 = row) and turned in
+// LDS as the input of conv2d_v1_body is: 20 and 23 to 31 cycles of the vector-memory pipe a KiB instead of 64.  BERT-base at
+// 128 tokens, six layers, 331 -> 297 us of device time a pass; at 384, four layers, 439 -> 402.
+template <int TM, int TN, bool LN, bool PK, class Poll>
+__device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, char* smem_raw,
+                                                   const Poll& poll) {
     typedef TileD16<TN, TM> TD;
-    constexpr bool BIG = TM * TN > 4;
+    constexpr bool BIG = TM * TN > 4 || PK;
     constexpr int KL = BIG ? 4 : 8;        // k values per lane and step
     constexpr int KSTEP = 16 * KL;         // k values of a step
     constexpr int AC = BIG ? 1 : 2;        // accumulators per sub-tile: enough for no MFMA to wait for the one in front
-    constexpr int NS = 3;      // steps of loads in flight (6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
+    // steps of loads in flight (unpacked, 6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
+    constexpr int NS = PK ? 4 : 3;
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * TD::SUBS * TD::PART);
     const int* a = d.attr;
@@ -2978,10 +2984,17 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
     const int nsteps = (k_hi - k_lo + KSTEP - 1) / KSTEP;
     const int lane_steps = lane_k < k_hi ? (k_hi - lane_k + KSTEP - 1) / KSTEP : 0;
     unsigned va[TM], vb[TN];
+    const int row0 = lane >> 2, ld_k = k_lo + wave * 16 + (lane & 3) * 4;      // PK: row and first k of this lane's piece of A
+    const int ld_steps = ld_k < k_hi ? (k_hi - ld_k + KSTEP - 1) / KSTEP : 0;
+    const unsigned K16 = (unsigned)(K + 15) / 16u;
+    const rsrc_t rs_bp = make_rsrc(d.ptr[1], PK ? (unsigned)((N + 15) / 16) * K16 * 1024u : 0u);
 #pragma unroll
-    for (int h = 0; h < TM; ++h) va[h] = ((unsigned)(m0 + 16 * h + i16) * lda + (unsigned)lane_k) * 4u;
+    for (int h = 0; h < TM; ++h)
+        va[h] = PK ? ((unsigned)(m0 + 16 * h + row0) * lda + (unsigned)ld_k) * 4u : ((unsigned)(m0 + 16 * h + i16) * lda + (unsigned)lane_k) * 4u;
 #pragma unroll
-    for (int g = 0; g < TN; ++g) vb[g] = ((unsigned)(n0 + 16 * g + i16) * ldb + (unsigned)lane_k) * 4u;
+    for (int g = 0; g < TN; ++g)
+        vb[g] = PK ? ((unsigned)(n0 / 16 + g) * K16 + (unsigned)(k_lo / 16 + wave)) * 1024u + (unsigned)lane * 16u
+                   : ((unsigned)(n0 + 16 * g + i16) * ldb + (unsigned)lane_k) * 4u;
 
     float ra[NS][TM][KL], rb[NS][TN][KL];
     auto load_slot = [&](float (&dst)[KL], rsrc_t rs, unsigned off, unsigned soff) {
@@ -2993,6 +3006,18 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
         }
     };
     auto load_step = [&](int s, int step) {
+        if (PK) {
+            // (a step behind this wavefront's last brings a neighbour's weights, which nothing multiplies)
+            const unsigned outp = step < ld_steps ? 0u : kOutside;
+#pragma unroll
+            for (int g = 0; g < TN; ++g) {
+                load_slot(rb[s][g], rs_bp, vb[g], 0u);
+                vb[g] += 4096u;
+            }
+#pragma unroll
+            for (int h = 0; h < TM; ++h) load_slot(ra[s][h], rs_a, va[h] | outp, (unsigned)step * 256u);
+            return;
+        }
         const unsigned outm = step < lane_steps ? 0u : kOutside;
         const unsigned so = (unsigned)step * (unsigned)KSTEP * 4u;   // uniform
 #pragma unroll
@@ -3022,8 +3047,28 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
 #pragma unroll
             for (int e = 0; e < AC; ++e) acc[h][g][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
+    // PK: the rows of A through LDS, one step ahead of the MFMAs: row r at 16 r, its piece p at p ^ (r / 4), so that the
+    // sixteen lanes of a k slot read different banks; where this wavefront's partial tile goes afterwards
+    float* blk = smem + wave * (TD::SUBS * TD::PART);
+    float* wr = blk + row0 * 16 + ((lane & 3) ^ (row0 >> 2)) * 4;
+    const float* rd = blk + i16 * 16 + (kq ^ (i16 >> 2)) * 4;
+    f32x4 at[PK ? 2 : 1][TM];
+    auto turn = [&](int s, int to) {
+#pragma unroll
+        for (int h = 0; h < TM; ++h) *(f32x4*)(wr + h * 256) = f32x4{ra[s][h][0], ra[s][h][1], ra[s][h][2], ra[s][h][3]};
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int h = 0; h < TM; ++h) at[PK ? to : 0][h] = *(const f32x4*)(rd + h * 256);
+        __builtin_amdgcn_wave_barrier();
+    };
     int ln_step = 0;
     auto mma_stage = [&](int s) {
+        if (PK) {
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) ra[s][h][q] = at[PK ? s & 1 : 0][h][q];
+        }
         if (LN) {
             const float in = ln_step++ < lane_steps ? 1.0f : 0.0f;     // values outside K were loaded as zeros: 0 - 0
 #pragma unroll
@@ -3048,9 +3093,12 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
     };
     int pf = 0, it = 0;
     bool left = false;
+    // this wavefront's own steps where their loads are its own
+    const int steps = PK ? (k_lo + 16 * wave < k_hi ? (k_hi - k_lo - 16 * wave + KSTEP - 1) / KSTEP : 0) : nsteps;
+    if (PK && steps > 0) turn(0, 0);
     // (groups whose refills all exist, then the last whole group with the refills the remaining steps
     // need and no others, as in the convolution)
-    for (; it + 2 * NS <= nsteps; it += NS) {
+    for (; it + 2 * NS <= steps; it += NS) {
         if (Poll::enabled) {
             if (pf) {
                 *sflag = 1;
@@ -3061,12 +3109,14 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
+            if (PK && s + 1 < NS) turn(s + 1, (s + 1) & 1);
             mma_stage(s);
             load_step(s, it + s + NS);
             __builtin_amdgcn_sched_barrier(0);
+            if (PK && s + 1 == NS) turn(0, 0);
         }
     }
-    if (!left && it + NS <= nsteps) {
+    if (!left && it + NS <= steps) {
         if (Poll::enabled && pf) {
             *sflag = 1;
             left = true;
@@ -3074,17 +3124,22 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
             if (Poll::enabled) pf = poll.load();
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
+                if (PK && s + 1 < NS) turn(s + 1, (s + 1) & 1);
                 mma_stage(s);
-                if (it + s + NS < nsteps) load_step(s, it + s + NS);
+                if (it + s + NS < steps) load_step(s, it + s + NS);
                 __builtin_amdgcn_sched_barrier(0);
             }
             it += NS;
+            if (PK && it < steps) turn(0, 0);
         }
     }
     if (!left) {
 #pragma unroll
         for (int s = 0; s < NS - 1; ++s)
-            if (it + s < nsteps) mma_stage(s);
+            if (it + s < steps) {
+                if (PK && it + s + 1 < steps) turn(s + 1, (s + 1) & 1);
+                mma_stage(s);
+            }
     }
 
     float* sums = smem + 4 * TD::SUBS * TD::PART + 4;      // LN: [wavefront][row][2], then the pivots [row]
@@ -3236,6 +3291,12 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
     if (threadIdx.x == 0)  // ready for the next run
         __hip_atomic_store(&counters[rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
+}
+
+template <int TM, int TN, bool LN, class Poll>
+__device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
+    if (d.attr[REEF_GEMM_LDB] == 0) return gemm_nt_direct_run<TM, TN, LN, true>(d, task, smem_raw, poll);
+    return gemm_nt_direct_run<TM, TN, LN, false>(d, task, smem_raw, poll);
 }
 
 // ---- reef_attention_m16: softmax(alpha Q K^T (masked)) V of all heads in one launch, on the matrix cores ----

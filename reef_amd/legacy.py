@@ -116,6 +116,7 @@ def import_model(ref_json_path, table=None, name=None, input_shape=None):
     elif isinstance(table, str):
         table = json.load(open(table))
     g = MB.GraphBuilder(model_name)
+    g.pack_weights = False        # the parameters' values are the directory's, not the builder's
     g.unique_names = True
     g.fused_reduce = True
     g.storage = [dict(s) for s in ref["storage"]]

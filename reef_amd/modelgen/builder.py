@@ -67,6 +67,7 @@ class GraphBuilder:
         self.kernels = []
         self.graph_args = []
         self.params = []               # (key, float32 array)
+        self._packed = {}              # key -> packed copy of a product's weights
         self._param_pos = {}           # storage index of a parameter -> its place in params
         self.flops = 0                 # algorithmic FLOPs of contractions
         self.kernel_flops = []         # per kernel call
@@ -79,8 +80,8 @@ class GraphBuilder:
         self.unique_names = True
         # split-K folded inside the conv kernel (False: separate reef_splitk_reduce launch)
         self.fused_reduce = False
-        # filters on the direct / row tiles also get a copy of their weights in the
-        # layout those kernels load fastest (pack_conv_weights); parameter key = weight key + "k"
+        # filters on the direct / row tiles and weights of direct products also get a copy of their weights
+        # in the layout those kernels load fastest (pack_conv_weights); parameter key = weight key + "k" or "pk"
         self.pack_weights = True
         self.pair_fold = os.environ.get("REEF_PAIR_FOLD", "1") != "0"
 
@@ -129,6 +130,13 @@ class GraphBuilder:
         self.graph_args.append(idx)
         self.params.append((key, arr))
         return Tensor(idx, (arr.size,))
+
+    def packed_matrix(self, b, N, K):
+        """The packed copy of weights b [N][K] for the direct products (ldb = 0), one per matrix."""
+        key = self.storage[b.idx]["name"] + "pk"
+        if key not in self._packed:
+            self._packed[key] = self.derived_param(key, pack_conv_weights(self.param_array(b).reshape(N, K, 1), by_channels=True))
+        return self._packed[key]
 
     def _sync_counters(self, n):
         """Reserves n counters in the model's sync storage; returns (storage idx, first counter)."""
@@ -676,13 +684,18 @@ class GraphBuilder:
         if ln is not None:
             assert trans_b and batch == 1 and off_a == 0, "the LayerNorm form: one K-contiguous B, A without offset"
             assert force_tile is None or force_tile in self.LN_GEMM_TILES, "no LayerNorm form of this tile"
+        # weights of a model generated here also as the copy that the direct kernels load fastest
+        packed = direct_ok and self.pack_weights and batch == 1 and off_b == 0 and ldb == K and b.idx in self._param_pos
         if force_tile is not None:
             t = tiling.forced(force_tile, M, N, K, 1)
         else:
-            t = tiling.choose_product(M, N, K, batch, direct_ok, under_load=self.under_load, ln=ln is not None)
+            t = tiling.choose_product(M, N, K, batch, direct_ok, under_load=self.under_load, ln=ln is not None, packed=packed)
         direct = t["tile"] in tiling.GEMM_DIRECT_TILES or t["tile"] in tiling.GEMM_WIDE_TILES
         assert direct_ok or not direct, "this GEMM has no direct form"
         args = [a.idx, b.idx, out.idx]
+        packed = packed and direct
+        if packed and ln is None:
+            args[1] = self.packed_matrix(b, N, K).idx
         if ln is not None:
             # Wg = W gamma (column k scaled by gamma[k]); c1 = its row sums; c2 = W beta
             assert ldb == K and off_b == 0, "the LayerNorm form takes the weight matrix whole"
@@ -691,12 +704,14 @@ class GraphBuilder:
             bt = self.param_array(ln["beta"]).astype(np.float64)
             wkey = self.storage[b.idx]["name"]
             Wg = (W * gm[None, :]).astype(np.float32)
-            args[1] = self.derived_param(wkey + "gk", Wg).idx      # the storage named wkey keeps W itself
+            # the storage named wkey keeps W itself
+            args[1] = (self.derived_param(wkey + "gkpk", pack_conv_weights(Wg[:, :, None], by_channels=True)) if packed
+                       else self.derived_param(wkey + "gk", Wg)).idx
             ln = dict(ln, c1=self.derived_param(wkey + "sk", Wg.astype(np.float64).sum(axis=1)),
                       c2=self.derived_param(wkey + "tk", W @ bt))
         flags = 0
         if bias is not None:
-            flags = 1
+            flags |= 1
             args.append(bias.idx)
         if res is not None:
             flags |= 8
@@ -733,7 +748,7 @@ class GraphBuilder:
         self._emit("reef_gemm_%s_%s" % ("ntl" if ln is not None else "ntd" if direct else "nt" if trans_b else "nn", t["tile"]),
                    tasks, args,
                    [batch, M, N, K, 1 if trans_b else 0, flags, act, float_bits(alpha), t["tile_id"],
-                    t["m_tiles"], t["n_tiles"], lda, ldb, ldc, stride_a, stride_b, stride_c,
+                    t["m_tiles"], t["n_tiles"], lda, 0 if packed else ldb, ldc, stride_a, stride_b, stride_c,
                     off_a, off_b, off_c] + ((attrs_ln or [0]) + attrs_split if attrs_split else attrs_ln),
                    "gemm", flops, 4 * batch * (M * K + N * K + M * N), t["est_us"])
         return out

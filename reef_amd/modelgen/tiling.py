@@ -115,18 +115,35 @@ GEMM_COST = {
     ("64x32k2", False): (4.431, 12.06, 0, 0, 0.5025, 0, 0),
     ("64x32k2", True): (5.956, 3.589, 7.457, 1.34, 0.4235, 0, 0),
 }
+# The same for the direct kernels on packed weights (reef_kernels.h, ldb = 0): 13 sequence lengths of 16 to 512 times 16
+# layer shapes of 256 to 4096 columns and depth, 4279 launches.  It picks within 4.3 % of the fastest launch on average, by
+# GEMM_COST 11 %: BERT-base at 128, six layers, 300 us of device time a pass by GEMM_COST and 285 by this (297 with the
+# FFN-down product as in GEMM_UNDER_LOAD); at 384, four layers, 433 and 402 (in turn, unpacked: 331 and 439).
+GEMM_COST_PACKED = {
+    ("16x16k4", False): (3.735, 0, 0.1841, 1.183, 0.01631, 0, 3.281),
+    ("16x16k4", True): (3.942, 0, 0.07655, 1.525, 0.2484, 0, 0),
+    ("16x32k4", False): (3.405, 0, 1.262, 0.9671, 0.2277, 0, 4.159),
+    ("16x32k4", True): (3.852, 0, 1.346, 1.298, 0.4132, 0, 0),
+    ("32x32d4", False): (3.05, 0, 3.095, 1.396, 0.7459, 0, 6.121),
+    ("32x48d4", False): (3.086, 0.716, 5.058, 0.7567, 1.084, 0, 7.42),
+    ("32x48d4", True): (4.614, 0, 5.885, 1.29, 0.7968, 0, 0),
+    ("48x48d4", False): (3.429, 0, 6.574, 2.962, 1.658, 0, 9.302),
+    ("48x48d4", True): (4.494, 0, 12.44, 0, 1.871, 0, 0),
+    ("64x64d4", False): (3.374, 0, 16.25, 0, 4.555, 0, 14.41),
+    ("64x64d4", True): (5.874, 0, 19.3, 0, 1.903, 0, 0),
+}
 GEMM_COST_MIN, GEMM_COST_MAX_OUT = 256, 512 * 4096     # columns and depth from which, outputs up to which it was measured
 
 
-def choose_product(M, N, K, batch=1, direct_ok=False, under_load=False, ln=False):
+def choose_product(M, N, K, batch=1, direct_ok=False, under_load=False, ln=False, packed=False):
     """Tile (and split of K, gemm_split) of a matrix product: inside the measured range by GEMM_COST, outside
     it by choose_gemm (behind a LayerNorm: the staged 32x32k4, which takes every shape).
-    under_load: as in choose_gemm."""
-    if under_load and direct_ok and not ln and batch == 1 and (M, N, K) in GEMM_UNDER_LOAD:
-        return choose_gemm(M, N, K, batch, direct_ok, under_load)
+    under_load: as in choose_gemm.  packed: the direct kernels will find packed weights (GEMM_COST_PACKED)."""
+    if (under_load or packed) and direct_ok and not ln and batch == 1 and (M, N, K) in GEMM_UNDER_LOAD:
+        return choose_gemm(M, N, K, batch, direct_ok, True)
     if batch == 1 and direct_ok and min(N, K) >= GEMM_COST_MIN and M * N <= GEMM_COST_MAX_OUT:
         best = None
-        for (tile, through_ln), c in GEMM_COST.items():
+        for (tile, through_ln), c in (GEMM_COST_PACKED if packed else GEMM_COST).items():
             if through_ln != ln:
                 continue
             staged = tile not in DIRECT_TILES and tile not in GEMM_WIDE_TILES
