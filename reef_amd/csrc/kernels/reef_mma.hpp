@@ -837,11 +837,12 @@ struct DirectTail {
 // From the wavefronts' partial tiles to the output: added through LDS in wavefront order, then epilogue and
 // store, partial tile to the workspace, or the fold of a split K inside the launch.  False: the workgroup
 // leaves a preempted launch.
-// WSTRIDE: floats between the wavefronts' places in LDS; the flags lie behind the last.
+// WSTRIDE: floats between the wavefronts' places in LDS; the flags (one a wavefront) lie behind the last.
+// stop: this wavefront has seen the preemption flag.
 // first: the first share's sums where the workgroup has both (t.both).
 template <int TM, int TN, int WSTRIDE = TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, class Poll>
 __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN],
-                                            const DirectTail<TM, TN>& t, const Poll& poll, const f32x4* first = nullptr) {
+                                            const DirectTail<TM, TN>& t, const Poll& poll, bool stop, const f32x4* first = nullptr) {
     typedef TileD16<TN, TM> TD;
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * WSTRIDE);
@@ -862,8 +863,9 @@ __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int
 #pragma unroll
         for (int j = 0; j < 4; ++j) part[TD::PART + (5 * kq + j) * 16 + i16] = (*first)[j];
     }
+    if (Poll::enabled && lane == 0) sflag[wave] = stop;
     __syncthreads();
-    if (Poll::enabled && *sflag) return false;
+    if (Poll::enabled && (sflag[0] | sflag[1] | sflag[2] | sflag[3])) return false;
     const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
     float v[TM][TN];
 #pragma unroll
@@ -1082,9 +1084,14 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     typedef TileD16<TN, TM> TD;
     constexpr int RC = G::RC, NS = G::NS;
     float* smem = (float*)smem_raw;
-    int* sflag = (int*)(smem + 4 * TD::SUBS * TD::PART);
     const OpDesc& d = d_in;
     const int* a = d.attr;
+    // The flag check every best-effort workgroup makes before it does anything
+    // (script/best_effort_kernel.py:22-29): read by every wavefront in front of its first loads, looked at where the K
+    // loop looks at it anyway and where the wavefronts meet behind it.  A workgroup that finds the flag raised has only
+    // read.  (Looked at behind the first loads, with a barrier, every launch waited for all of them before its
+    // first MFMA: DenseNet-201 1017 -> 980 us of device time a pass.)
+    const int raised = Poll::enabled ? poll.load() : 0;
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = FROWS ? a[REEF_CONV_KH] : 1;
@@ -1326,15 +1333,6 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
 
     tail.fetch(d, MN4);
 
-    if (Poll::enabled) {
-        // The flag check every best-effort workgroup makes before it does anything
-        // (script/best_effort_kernel.py:22-29) is made here, with the first loads of the K loop
-        // already on their way: its trip to memory hides behind theirs instead of standing in
-        // front of them.  A workgroup that finds the flag raised has only read.
-        if (threadIdx.x == 0) *sflag = poll.load();
-        __syncthreads();
-        if (*sflag) return false;
-    }
 
     // Whole groups of NS steps with no condition inside (a loop with per-step conditions gets
     // reordered around the loads), then the remaining steps, whose loads are already under way.
@@ -1395,7 +1393,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
                     acc[h][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][ROWS ? 0 : g * RC + q],
                                                                             acc[h][g][q & 1], 0, 0, 0);
     };
-    int pf = 0;
+    int pf = raised;
     int it = 0;
     bool left = false;
     // (groups whose refills all exist; the last whole group follows with the refills the remaining
@@ -1404,9 +1402,8 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     for (; it + 2 * NS <= nsteps; it += NS) {
         if (Poll::enabled) {
             // the flag is read one group ahead; a wavefront that sees it tells the others
-            // through LDS and all of them leave after the barrier below
+            // through LDS and all of them leave where they meet
             if (pf) {
-                *sflag = 1;
                 left = true;
                 break;
             }
@@ -1422,7 +1419,6 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     }
     if (!left && it + NS <= nsteps) {
         if (Poll::enabled && pf) {
-            *sflag = 1;
             left = true;
         } else {
             if (Poll::enabled) pf = poll.load();
@@ -1446,7 +1442,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
-    return direct_tail(d, smem_raw, wave, sum, tail, poll);
+    return direct_tail(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
 // ---- reef_conv2d_v1_<tile>, reef_conv2d_p1_v_<tile>: 1x1 filters, stride 1, whole cache lines ----------------
@@ -1480,8 +1476,8 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     constexpr int LPR = 4 * TN;                    // lanes (16-byte pieces) of a row
     float* smem = (float*)smem_raw;
     constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
-    int* sflag = (int*)(smem + 4 * WSTRIDE);
     const int* a = d.attr;
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
@@ -1576,11 +1572,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
         }
     }
     tail.fetch(d, MN4);
-    if (Poll::enabled) {        // the wrapper's flag check, as in conv2d_direct_body
-        if (threadIdx.x == 0) *sflag = poll.load();
-        __syncthreads();
-        if (*sflag) return false;
-    }
     f32x4 acc[TM][TN][2];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
@@ -1627,7 +1618,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
                     acc[h][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], bt[from][g][q], acc[h][g][q & 1], 0, 0, 0);
     };
     static_assert(NS % 2 == 0, "the turned blocks alternate");
-    int pf = 0, it = 0;
+    int pf = raised, it = 0;
     bool left = false;
     f32x4 first = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // (a share is whole groups: the first one ends between two turns of the loop.  Tested inside the loop it
@@ -1638,7 +1629,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     for (; it + 2 * NS <= steps && it < until; it += NS) {
         if (Poll::enabled) {
             if (pf) {
-                *sflag = 1;
                 left = true;
                 break;
             }
@@ -1660,7 +1650,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     }
     if (!left && it + NS <= steps) {
         if (Poll::enabled && pf) {
-            *sflag = 1;
             left = true;
         } else {
             if (Poll::enabled) pf = poll.load();
@@ -1688,7 +1677,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
-    return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, TD::SUBS == 1 ? &first : nullptr);
+    return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, left || raised, TD::SUBS == 1 ? &first : nullptr);
 }
 
 // ---- reef_conv2d_v9_g<G>: 3x3 / stride 1 / padding 1, whole cache lines --------------------------------------
@@ -1712,8 +1701,8 @@ template <int G, class Poll>
 __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
     typedef TileV9<G> TV;
     float* smem = (float*)smem_raw;
-    int* sflag = (int*)(smem + 4 * TV::BLOCK);
     const int* a = d.attr;
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], H = a[REEF_CONV_H], W = a[REEF_CONV_W];
@@ -1805,11 +1794,6 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
         tail.ooff[0][g] = ok ? (tail.om[0] * (unsigned)N + (unsigned)((y0 + g) * W + x0 + ocol)) * 4u : kOutside;
     }
     tail.fetch(d, (unsigned)M * HW4);
-    if (Poll::enabled) {        // the wrapper's flag check, as in conv2d_direct_body
-        if (threadIdx.x == 0) *sflag = poll.load();
-        __syncthreads();
-        if (*sflag) return false;
-    }
     f32x4 acc[1][G][2];
 #pragma unroll
     for (int g = 0; g < G; ++g) acc[0][g][0] = acc[0][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1868,7 +1852,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     f32x4 first = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     struct Yes { constexpr operator bool() const { return true; } };
     struct No { constexpr operator bool() const { return false; } };
-    int pf = 0;
+    int pf = raised;
     bool left = false;
     if (steps > 0) {
         turn();
@@ -1882,7 +1866,6 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
         for (; steps > 1; --steps) {
             if (Poll::enabled) {
                 if (pf) {
-                    *sflag = 1;
                     left = true;
                     break;
                 }
@@ -1895,7 +1878,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     f32x4 sum[1][G];
 #pragma unroll
     for (int g = 0; g < G; ++g) sum[0][g] = acc[0][g][0] + acc[0][g][1];
-    return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, G == 1 ? &first : nullptr);
+    return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, left || raised, G == 1 ? &first : nullptr);
 }
 
 // ---- reef_conv2d_xdw[2]_g<G>: 1x1 convolution, then depthwise 3x3, in one launch --------------
@@ -2915,6 +2898,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * TD::SUBS * TD::PART);
     const int* a = d.attr;
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M = a[REEF_GEMM_M], N = a[REEF_GEMM_N], K = a[REEF_GEMM_K];
@@ -3030,15 +3014,6 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
         load_step(s, s);
         asm volatile("" ::: "memory");
     }
-    if (Poll::enabled) {
-        // The flag check every best-effort workgroup makes before it does anything
-        // (script/best_effort_kernel.py:22-29) is made here, with the first loads of the K loop
-        // already on their way: its trip to memory hides behind theirs instead of standing in
-        // front of them.  A workgroup that finds the flag raised has only read.
-        if (threadIdx.x == 0) *sflag = poll.load();
-        __syncthreads();
-        if (*sflag) return false;
-    }
     f32x4 acc[TM][TN][AC];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
@@ -3091,7 +3066,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
                     acc[h][g][q % AC] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][g][q],
                                                                              acc[h][g][q % AC], 0, 0, 0);
     };
-    int pf = 0, it = 0;
+    int pf = raised, it = 0;
     bool left = false;
     // this wavefront's own steps where their loads are its own
     const int steps = PK ? (k_lo + 16 * wave < k_hi ? (k_hi - k_lo - 16 * wave + KSTEP - 1) / KSTEP : 0) : nsteps;
@@ -3101,7 +3076,6 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     for (; it + 2 * NS <= steps; it += NS) {
         if (Poll::enabled) {
             if (pf) {
-                *sflag = 1;
                 left = true;
                 break;
             }
@@ -3118,7 +3092,6 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     }
     if (!left && it + NS <= steps) {
         if (Poll::enabled && pf) {
-            *sflag = 1;
             left = true;
         } else {
             if (Poll::enabled) pf = poll.load();
@@ -3167,8 +3140,9 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = AC == 2 ? acc[h][g][0][j] + acc[h][g][AC - 1][j] : acc[h][g][0][j];
+    if (Poll::enabled && lane == 0) sflag[wave] = left || raised;
     __syncthreads();
-    if (Poll::enabled && *sflag) return false;
+    if (Poll::enabled && (sflag[0] | sflag[1] | sflag[2] | sflag[3])) return false;
     const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
     constexpr int WSTRIDE = TD::SUBS * TD::PART;
     const float alpha = __int_as_float(a[REEF_GEMM_ALPHA_BITS]);
