@@ -405,7 +405,8 @@ enum {
  * for sequences of up to REEF_AT_MM_MAX_SEQ.  tasks = heads * ceil(seq / REEF_AT_MM_ROWS). */
 #define REEF_AT_MM_ROWS 16
 #define REEF_AT_MM_MAX_SEQ 512
-#define REEF_AT_MM_LDS_BYTES (4 * (REEF_AT_MM_ROWS * (REEF_AT_MM_MAX_SEQ + 4) + REEF_AT_MM_ROWS))
+/* scores, 1 / sum of each row, and a block of 16 x 16 values a wavefront */
+#define REEF_AT_MM_LDS_BYTES (4 * (REEF_AT_MM_ROWS * (REEF_AT_MM_MAX_SEQ + 4) + REEF_AT_MM_ROWS) + 4 * 1024)
 
 /* ---- reef_bias_gelu: out = gelu_erf(x + bias[col]).  ptr: x, out, bias(optional).
  * attr: rows, cols, flags.  tasks = ceil(rows*cols / 1024). */

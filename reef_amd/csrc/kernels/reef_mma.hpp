@@ -2884,7 +2884,7 @@ __device__ __forceinline__ bool gemm_body(const OpDesc& d, int task, char* smem_
 // PK (ldb = 0): B is the packed copy of a weight matrix, [ceil(N / 16)][ceil(K / 16)][k slot][16 columns]
 // [4 k], whose loads are contiguous KiBs, and the rows of A are loaded as 16-byte pieces (lane / 4 = row) and turned in
 // LDS as the input of conv2d_v1_body is: 20 and 23 to 31 cycles of the vector-memory pipe a KiB instead of 64.  BERT-base at
-// 128 tokens, six layers, 331 -> 297 us of device time a pass; at 384, four layers, 439 -> 402.
+// 128 tokens, six layers, 331 -> 305 us of device time a pass; at 384, four layers, 439 -> 402.
 template <int TM, int TN, bool LN, bool PK, class Poll>
 __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, char* smem_raw,
                                                    const Poll& poll) {
@@ -3276,18 +3276,20 @@ __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, c
 // ---- reef_attention_m16: softmax(alpha Q K^T (masked)) V of all heads in one launch, on the matrix cores ----
 // For sequences of up to REEF_AT_MM_MAX_SEQ.  A workgroup takes 16 query rows of one head.
 //   scores   the wavefronts take the key tiles (16 keys) in turn; Q and K come straight from memory into
-//            16x16x4 MFMAs, k slot kq holding elements 16 u + 4 kq .. + 3 of the head (a load of a wavefront
-//            reads 64 consecutive bytes of every row); the scores of the 16
+//            16x16x4 MFMAs, k slot kq holding elements 16 u + 4 kq .. + 3 of the head; the scores of the 16
 //            rows go to LDS (row stride 4 mod 64 floats: the four k slots' rows lie in different banks).
 //   softmax  16 threads a row; what stays in LDS is exp(s - max), its sum divides the result at the end.
 //   context  a wavefront forms 16 columns of the head for all rows: A = four probabilities per lane and
-//            128-bit LDS read, B = values straight from memory (64-byte pieces of their rows), the next 64
-//            keys' values on their way while these multiply, the first before the scores are formed.
-// Bound by latency (Q, K, V of a layer are in L2): 384 tokens, 12 heads of 64: 16.4 us against 14.5 + 6.3 + 9.4
+//            128-bit LDS read, B = the values, the next 64 keys' on their way while these multiply, the first
+//            before the scores are formed.
+// K and V are loaded as sixteen rows of four 16-byte pieces (lane / 4 = row), 17 to 31 cycles of the vector-memory pipe
+// a KiB, and turned into the operands' layout in a block of LDS of each wavefront's own.  (K with lane % 16 = row takes 64
+// cycles, V in single values 60: at 384 tokens 16.4 -> 15.0 us, BERT-base of four layers 402 -> 396 us a pass.)
+// Bound by latency (Q, K, V of a layer are in L2): 384 tokens, 12 heads of 64: 15.0 us against 14.5 + 6.3 + 9.4
 // for scores, softmax and context as launches of their own around two [12][384][384] tensors.
 template <int NT>
 __device__ __forceinline__ void attention_scores(rsrc_t rk, const f32x4 (&q)[4], const unsigned (&koff)[4], int ld, int S, int kq, int i16,
-                                                 int wave, int tiles, float alpha, const unsigned char* mask, float* P, int SP) {
+                                                 int wave, int tiles, float alpha, const unsigned char* mask, float* P, int SP, float* blk) {
     // NT: 128-bit loads per k slot (HD <= 16 NT)
     // two pairs of tiles: one is loaded while the other is multiplied
     f32x4 kb[2][2][NT];
@@ -3299,7 +3301,20 @@ __device__ __forceinline__ void attention_scores(rsrc_t rk, const f32x4 (&q)[4],
             for (int u = 0; u < NT; ++u) r[v][u] = buf_load4(rk, koff[u] + row);
         }
     };
-    auto multiply = [&](const f32x4 (&r)[2][NT], int tile) {
+    // A piece p of row r lies at p ^ (r / 4): the sixteen lanes of a k slot read different banks.
+    const int row0 = 4 * kq + (i16 >> 2);
+    float* wr = blk + row0 * 16 + ((i16 & 3) ^ kq) * 4;
+    const float* rd = blk + i16 * 16 + (kq ^ (i16 >> 2)) * 4;
+    auto multiply = [&](f32x4 (&r)[2][NT], int tile) {
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {      // a wavefront's LDS accesses stay in order
+                *(f32x4*)wr = r[v][u];
+                __builtin_amdgcn_wave_barrier();
+                r[v][u] = *(const f32x4*)rd;
+                __builtin_amdgcn_wave_barrier();
+            }
         f32x4 acc[2][2];
 #pragma unroll
         for (int v = 0; v < 2; ++v) acc[v][0] = acc[v][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -3352,32 +3367,34 @@ __device__ __forceinline__ void attention_mma_body(const OpDesc& d, int task, ch
     const int SP = chunks * 64 + 4;
     float* P = (float*)smem_raw;                              // [16][SP]
     float* inv = P + ROWS * SP;                               // [16]
+    float* blk = P + ROWS * (REEF_AT_MM_MAX_SEQ + 4) + ROWS + wave * 256;      // this wavefront's block to turn
+    const int row0 = lane >> 2, piece = lane & 3;             // of this lane's loads of K and V
 
     const int nt = (HD + 15) / 16;
     f32x4 q[4];
     unsigned koff[4];         // this lane's pieces of a row of its tile (offsets that are added, not selected: no branch per load)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        const unsigned k = (unsigned)(16 * u + 4 * kq);
-        koff[u] = ((unsigned)i16 * (unsigned)ld + k) * 4u + (k < (unsigned)HD ? 0u : kOutside);
-        q[u] = buf_load4(rq, koff[u] + (unsigned)m0 * (unsigned)ld * 4u);
+        const unsigned k = (unsigned)(16 * u + 4 * kq), kl = (unsigned)(16 * u + 4 * piece);
+        koff[u] = ((unsigned)row0 * (unsigned)ld + kl) * 4u + (kl < (unsigned)HD ? 0u : kOutside);
+        q[u] = buf_load4(rq, ((unsigned)(m0 + i16) * (unsigned)ld + k) * 4u + (k < (unsigned)HD ? 0u : kOutside));
     }
     const int col = wave * 16 + i16;                          // column of the head this lane forms
-    float vb[2][16];                                          // two chunks: one is loaded while the other is multiplied
-    const unsigned voff = ((unsigned)(kq * 4) * (unsigned)ld + (unsigned)col) * 4u + (col < HD ? 0u : kOutside);
-    auto load_v = [&](float (&v)[16], int chunk) {
+    f32x4 vb[2][4];                                           // two chunks: one is loaded while the other is multiplied
+    // row r of a turned block holds key 4 (r % 4) + r / 4, so that a k slot's four keys lie in rows of different banks
+    const int vcol = wave * 16 + 4 * piece;
+    const unsigned voff = ((unsigned)(4 * (row0 & 3) + (row0 >> 2)) * (unsigned)ld + (unsigned)vcol) * 4u + (vcol < HD ? 0u : kOutside);
+    auto load_v = [&](f32x4 (&v)[4], int chunk) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) v[g * 4 + t] = buf_load(rv, voff + (unsigned)((chunk * 64 + g * 16 + t) * ld) * 4u);
+        for (int g = 0; g < 4; ++g) v[g] = buf_load4(rv, voff + (unsigned)((chunk * 64 + g * 16) * ld) * 4u);
     };
     load_v(vb[0], 0);
     load_v(vb[1], 1);
 
-    if (nt == 4) attention_scores<4>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
-    else if (nt == 3) attention_scores<3>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
-    else if (nt == 2) attention_scores<2>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
-    else attention_scores<1>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP);
+    if (nt == 4) attention_scores<4>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP, blk);
+    else if (nt == 3) attention_scores<3>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP, blk);
+    else if (nt == 2) attention_scores<2>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP, blk);
+    else attention_scores<1>(rk, q, koff, ld, S, kq, i16, wave, tiles, alpha, mask, P, SP, blk);
     __syncthreads();
 
     {
@@ -3413,12 +3430,21 @@ __device__ __forceinline__ void attention_mma_body(const OpDesc& d, int task, ch
 
     f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
     const float* pr = P + i16 * SP + kq * 4;
-    auto multiply_v = [&](const float (&v)[16], int c) {
+    auto multiply_v = [&](const f32x4 (&v)[4], int c) {
+        float b[4][4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            *(f32x4*)(blk + row0 * 16 + piece * 4) = v[g];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int t = 0; t < 4; ++t) b[g][t] = blk[(4 * t + kq) * 16 + i16];
+            __builtin_amdgcn_wave_barrier();
+        }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const f32x4 p = *(const f32x4*)(pr + c * 64 + g * 16);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], v[g * 4 + t], acc[t & 1], 0, 0, 0);
+            for (int t = 0; t < 4; ++t) acc[t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], b[g][t], acc[t & 1], 0, 0, 0);
         }
     };
     for (int c = 0; c < chunks; c += 2) {
