@@ -17,8 +17,8 @@ constexpr int kThreads = REEF_WG_THREADS;
 
 // A launch's descriptor, its attributes and first eight pointers in scalar registers.  A body that reads them one by
 // one from the argument block waits five or six times in a row, whenever what it reads next depends on what it has read:
-// 560 cycles from the first line of reef_conv2d_v9_g1 to its first load, 840 with the pass over the block's
-// lines that stood in front.  Here everything comes in one trip; no load crosses a line of a block that starts on one.  ResNet-152 826 -> 821 us of device time a pass, DenseNet-201 919 -> 901.
+// 810 cycles from the start of reef_conv2d_v9_g1 to its first load, with the pass over the block's lines that stood in
+// front; 660 this way.  Here everything comes in one trip; no load crosses a line of a block that starts on one.  ResNet-152 826 -> 821 us of device time a pass, DenseNet-201 919 -> 901.
 struct OpPtrs {
     const ReefOpDesc* m;
     typedef int i32x16 __attribute__((ext_vector_type(16)));
