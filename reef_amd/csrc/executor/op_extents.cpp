@@ -230,6 +230,11 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
         if (by_channels && a[REEF_CONV_K_CHUNK] % (16 * taps) != 0) { n.bad = "a split of the packed weights starts inside a group of 16 channels"; return; }
         n.f32("packed weights", by_channels ? cdiv(M, 16) * cdiv(cin, 16) * taps * 256 : cdiv(M, 16) * cdiv(cin, 4) * cdiv(taps, 4) * 256);
     }
+    // half of a plain launch's workgroups lie behind its tasks then, and those read that slot as what to prefetch
+    if ((flags & REEF_F_BOTH_SHARES) && n.slots.size() > REEF_PREFETCH_SLOT) {
+        n.bad = "both shares in one workgroup: an operand in the slot of the prefetch record";
+        return;
+    }
     n.tasks = split * a[REEF_CONV_M_TILES] * a[REEF_CONV_N_TILES];
 }
 

@@ -320,7 +320,8 @@ class GraphBuilder:
             # A split of two whose tiles alone give nearly every CU a workgroup gains nothing from twice as many that
             # meet again (exchange: 2100 cycles).  ResNet-152's 71 such layers: 896 us of device time a pass where
             # they meet (16x32 and two image rows a tile), 829 with both shares in one workgroup (16x16, one row).
-            if (pair and 2 * share == cin and t["m_tiles"] * t["n_tiles"] >= BOTH_SHARES_TILES
+            # (Half of such a launch's workgroups lie behind its tasks, where operand slot 9 is the prefetch record's.)
+            if (pair and 2 * share == cin and len(args) + len(packed) <= MAX_ARGS and t["m_tiles"] * t["n_tiles"] >= BOTH_SHARES_TILES
                     and (share % 256 == 0 and kname in ("reef_conv2d_v1_16x16k4", "reef_conv2d_p1_v_16x16k4")
                          or share % 64 == 0 and kname == "reef_conv2d_v9_g1")):
                 flags |= F_BOTH_SHARES

@@ -13,7 +13,7 @@ import pytest
 
 from oracle import oracle as O
 from reef_amd import binding as B
-from reef_amd.modelgen import builder as MB
+from reef_amd.modelgen import builder as MB, tiling
 
 L = B.lib()
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -662,3 +662,27 @@ def test_a_stem_kernel_is_checked_against_its_storages(tmp_path):
     broken(lambda m: m["kernels"][0].__setitem__("name", "reef_conv2d_u_64x32k2#0"), "loader family")
     broken(lambda m: m["storage"][m["kernels"][0]["args"][2]].__setitem__("size", 24 * 10 * 11), "output")
     broken(lambda m: m["storage"][m["kernels"][0]["args"][4]].__setitem__("size", 2), "input shift")
+
+
+def test_the_slot_of_the_prefetch_record_is_no_operand_of_a_launch_with_workgroups_behind_its_tasks(tmp_path):
+    """Workgroups behind a plain launch's tasks read operand slot 9 as what to prefetch.  With both shares of a split in one
+    workgroup half of the grid is such: the layer below has ten operands, its packed weights in slot 9, and is not
+    built that way; a file that sets the flag (8192) on it is refused."""
+    g = MB.GraphBuilder("slotfmt")
+    x = g.input("x", (256, 14, 14))
+    r = g.input("r", (256, 14, 14))
+    f = tiling.forced_rows("g1", 256, 14, 14, 256 * 9, 2)
+    kw = dict(bias=True, residual=r, force=f, fused_reduce=True)
+    g.conv2d(x, 256, 3, 1, 1, dual_act=MB.ACT_RELU, **kw)
+    g.mark_output(g.conv2d(x, 256, 3, 1, 1, **kw))
+    base = g.write(str(tmp_path / "ok"), link_code_objects=False)
+    assert B.check_model(base + ".json") == (True, "")
+    model = json.load(open(base + ".json"))
+    k = model["kernels"][0]
+    assert k["name"].startswith("reef_conv2d_v9_g1#") and len(k["args"]) == 10 and k["attrs"][23] == 9
+    assert k["attrs"][12] & 64 and not k["attrs"][12] & 8192
+    k["attrs"][12] |= 8192
+    p = str(tmp_path / "flagged.json")
+    json.dump(model, open(p, "w"))
+    ok, why = B.check_model(p)
+    assert not ok and "prefetch" in why, why
