@@ -276,10 +276,8 @@ enum {
                                   weights [P][COUT], projection bias [P].  A workgroup holds every channel of its G
                                   output rows x 14 columns: M_TILES = 1, N_TILES = ceil(HO / G) * ceil(WO / 14),
                                   TILE = REEF_TILE_R9G<G>, no split. */
-#define REEF_F_BOTH_SHARES 8192 /* with REEF_F_PAIR_FOLD, symbols v1_16x16k4, p1_v_16x16k4 and v9_g1: in a plain launch the first
-                                  M_TILES * N_TILES workgroups take a tile each, both shares of its split one after the
-                                  other, and the rest have nothing to do.  Cin = 2 shares of whole groups of 256 (v9: 64)
-                                  channels. */
+/* 8192 is not used: model files may carry it beside REEF_F_PAIR_FOLD from a generator that asked for both shares of a
+   split of two in one workgroup, and run as any other split of two. */
 #define REEF_CONV_MODE_GENERAL 0
 #define REEF_CONV_MODE_POINTWISE 1
 #define REEF_CONV_MODE_UNALIGNED 2

@@ -187,15 +187,6 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
         return;
     }
     if (packed != (a[REEF_CONV_WPACK] != 0)) { n.bad = "packed weights and symbol do not go together"; return; }
-    if (flags & REEF_F_BOTH_SHARES) {
-        const i64 share = a[REEF_CONV_K_CHUNK] / taps;
-        const bool v1 = fam == "v1_16x16k4" || fam == "p1_v_16x16k4";
-        if (!(v1 || fam == "v9_g1") || split != 2 || !fused || !(flags & REEF_F_PAIR_FOLD) || 2 * share != cin ||
-            a[REEF_CONV_K_CHUNK] % taps != 0 || share % (v1 ? 256 : 64) != 0) {
-            n.bad = "both shares in one workgroup: a split of two into alike shares of whole groups of channels";
-            return;
-        }
-    }
     if (a[REEF_CONV_K_CHUNK] <= 0 || split * a[REEF_CONV_K_CHUNK] < K) {
         n.bad = "the splits do not cover the reduction";
         return;
@@ -229,11 +220,6 @@ void conv2d(const std::string& symbol, const Attrs& a, Needs& n) {
         const bool by_channels = taps == 1 || fam.compare(0, 3, "v9_") == 0;
         if (by_channels && a[REEF_CONV_K_CHUNK] % (16 * taps) != 0) { n.bad = "a split of the packed weights starts inside a group of 16 channels"; return; }
         n.f32("packed weights", by_channels ? cdiv(M, 16) * cdiv(cin, 16) * taps * 256 : cdiv(M, 16) * cdiv(cin, 4) * cdiv(taps, 4) * 256);
-    }
-    // half of a plain launch's workgroups lie behind its tasks then, and those read that slot as what to prefetch
-    if ((flags & REEF_F_BOTH_SHARES) && n.slots.size() > REEF_PREFETCH_SLOT) {
-        n.bad = "both shares in one workgroup: an operand in the slot of the prefetch record";
-        return;
     }
     n.tasks = split * a[REEF_CONV_M_TILES] * a[REEF_CONV_N_TILES];
 }

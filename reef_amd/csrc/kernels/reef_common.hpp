@@ -77,13 +77,11 @@ struct NoPoll {
     // model: plain launches and the real-time side of a padded launch).  What a folded split of
     // two may leave between its two workgroups in the pair slots relies on it (REEF_F_PAIR_FOLD).
     bool completes = false;
-    bool plain = false;      // a plain launch: workgroup = task, and nobody else counts its workgroups
     __device__ __forceinline__ int load() const { return 0; }
     __device__ __forceinline__ bool pair_fold_ok() const { return completes; }
 };
 struct FlagPoll {
     static constexpr bool enabled = true;
-    static constexpr bool plain = false;
     const int* flag;
     __device__ __forceinline__ bool pair_fold_ok() const { return false; }
     __device__ __forceinline__ int load() const {
@@ -200,7 +198,6 @@ __device__ __forceinline__ void touch4(const char* a, const char* b, const char*
 // operands, the others the XCD's slice of the weights.
 __device__ __forceinline__ void prefetch_lines(const ReefPrefetch* r, int j) {
     constexpr int X = REEF_PREFETCH_WGS_UNIT;
-    if (!r || (unsigned)j >= r->wgs) return;      // behind the last
     const unsigned slot = (unsigned)j / X, per = r->wgs / X - 1, x = blockIdx.x % X, tid = threadIdx.x;
     const char* at[REEF_PREFETCH_SMALL];
     if (slot == per) {

@@ -32,11 +32,6 @@ namespace {
 __device__ __forceinline__ int conv_tasks(const OpDesc& d) {
     return d.attr[REEF_CONV_SPLIT_K] * d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
 }
-// (a plain launch whose workgroups take both shares of a split: the others come last)
-__device__ __forceinline__ int conv_v_tasks(const OpDesc& d) {
-    const int tiles = d.attr[REEF_CONV_M_TILES] * d.attr[REEF_CONV_N_TILES];
-    return (d.attr[REEF_CONV_FLAGS] & REEF_F_BOTH_SHARES) ? tiles : tiles * d.attr[REEF_CONV_SPLIT_K];
-}
 __device__ __forceinline__ int gemm_tasks(const OpDesc& d) {
     const int s = d.attr[REEF_GEMM_SPLIT_K];
     return d.attr[REEF_GEMM_BATCH] * d.attr[REEF_GEMM_M_TILES] * d.attr[REEF_GEMM_N_TILES] * (s > 1 ? s : 1);
@@ -78,7 +73,7 @@ struct OpConvDirect {
 // 1x1 / stride 1 on packed weights, the input turned in LDS
 template <int TM, int TN, bool PRE = false>
 struct OpConvV1 {
-    REEF_TASKS(conv_v_tasks)
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileV1<TM, TN>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
@@ -89,7 +84,7 @@ struct OpConvV1 {
 // 3x3 / stride 1 / padding 1 by image rows, in steps of 16 channels a wavefront
 template <int G>
 struct OpConvV9 {
-    REEF_TASKS(conv_v_tasks)
+    REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileV9<G>::LDS_BYTES;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
@@ -314,7 +309,7 @@ __device__ __forceinline__ bool dkp_walk(const ReefDkpArgs& a, DkpWalk& w) {
             prefetch_lines((const ReefPrefetch*)d.ptr[REEF_PREFETCH_SLOT], behind);   \
             return;                                                                   \
         }                                                                             \
-        OP::run(d, (int)blockIdx.x, smem, NoPoll{true, true});                              \
+        OP::run(d, (int)blockIdx.x, smem, NoPoll{true});                              \
     }
 #elif REEF_FLAVOUR == 1
 namespace {
@@ -395,7 +390,7 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         const ReefDkpSide& side = w.right ? a.r : a.l;                                 \
         for (int i = w.idx; i < w.end; i += w.step) {                                  \
             const OpDesc d = OpDesc::load<0>(side.desc);                               \
-            OP::run(d, i, smem, NoPoll{!w.right, false});                             \
+            OP::run(d, i, smem, NoPoll{!w.right});                             \
             __syncthreads();                                                           \
         }                                                                              \
     }                                                                                  \

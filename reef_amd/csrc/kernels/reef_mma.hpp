@@ -808,7 +808,6 @@ struct DirectTail {
     float e_bias[TM], e_sh2[TM], e_res[TM][TN];
     int split, split_k, rem, flags, aux;     // aux: pointer slot of (workspace, arrival counters)
     bool fused, to_ws;                       // split folded inside the launch; partial tile to the workspace
-    bool both;                               // this workgroup has both shares of a split of two (REEF_F_BOTH_SHARES)
 
     // Epilogue operands, fetched behind the first K steps' loads.
     __device__ __forceinline__ void fetch(const OpDesc& d, unsigned MN4) {
@@ -839,10 +838,9 @@ struct DirectTail {
 // leaves a preempted launch.
 // WSTRIDE: floats between the wavefronts' places in LDS; the flags (one a wavefront) lie behind the last.
 // stop: this wavefront has seen the preemption flag.
-// first: the first share's sums where the workgroup has both (t.both).
 template <int TM, int TN, int WSTRIDE = TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, class Poll>
 __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN],
-                                            const DirectTail<TM, TN>& t, const Poll& poll, bool stop, const f32x4* first = nullptr) {
+                                            const DirectTail<TM, TN>& t, const Poll& poll, bool stop) {
     typedef TileD16<TN, TM> TD;
     float* smem = (float*)smem_raw;
     int* sflag = (int*)(smem + 4 * WSTRIDE);
@@ -859,10 +857,6 @@ __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = acc[h][g][j];
-    if (first && t.both) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) part[TD::PART + (5 * kq + j) * 16 + i16] = (*first)[j];
-    }
     if (Poll::enabled && lane == 0) sflag[wave] = stop;
     __syncthreads();
     if (Poll::enabled && (sflag[0] | sflag[1] | sflag[2] | sflag[3])) return false;
@@ -875,10 +869,6 @@ __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int
             const float* e = mine + (h * TN + g) * TD::PART;
             v[h][g] = ((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE];
         }
-    if (first && t.both) {      // the shares' sums in split order, as where they meet
-        const float* e = mine + TD::PART;
-        v[0][0] = (((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE]) + v[0][0];
-    }
     if (t.to_ws) {
         const rsrc_t ws = make_rsrc((const float*)d.ptr[2] + (size_t)t.split * M * N, (unsigned)M * (unsigned)N * 4u);
 #pragma unroll
@@ -1127,7 +1117,6 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
 
     const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
     DirectTail<TM, TN> tail;
-    tail.both = false;
     tail.split = split; tail.split_k = split_k; tail.rem = rem; tail.flags = flags; tail.fused = fused; tail.to_ws = to_ws;
     unsigned (&om)[TM] = tail.om;
     unsigned (&ooff)[TM][TN] = tail.ooff;
@@ -1459,8 +1448,8 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
 // whose scale and shift one 32-bit load brings to neighbouring lanes.
 // Sums run over the channels in the order of conv2d_direct_body.
 template <int TM, int TN>
-struct TileV1 {      // a wavefront's place: the turned block, then its partial tile (16x16: one of either share)
-    static constexpr int WSTRIDE = (TM * TN == 1 ? 2 : TM * TN) * TileD16<TN, TM>::PART;
+struct TileV1 {      // a wavefront's place: the turned block, then its partial tile
+    static constexpr int WSTRIDE = TM * TN * TileD16<TN, TM>::PART;
     static constexpr int LDS_BYTES = 4 * WSTRIDE * 4 + 16;
 };
 template <int TM, int TN, bool PRE, class Poll>
@@ -1491,25 +1480,18 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     tail.to_ws = split_k > 1 && !tail.fused;
     // tile and split of this workgroup, as in conv2d_direct_body
     const int chunk = a[REEF_CONV_K_CHUNK];
-    const int share = chunk >> 6;            // steps of a share
-    tail.both = TD::SUBS == 1 && poll.plain && (flags & REEF_F_BOTH_SHARES);
-    int split = 0, rem;
-    if (tail.both) {
-        tail.fused = false;
-        rem = xcd_chunked(task, tiles);
-    } else {
-        rem = task = xcd_chunked(task, tiles * split_k);
-        if (split_k > 1) {
-            const int q = div_small(task, tail.fused ? split_k : tiles);
-            split = tail.fused ? task - q * split_k : q;
-            rem = tail.fused ? q : task - split * tiles;
-        }
+    task = xcd_chunked(task, tiles * split_k);
+    int split = 0, rem = task;
+    if (split_k > 1) {
+        const int q = div_small(task, tail.fused ? split_k : tiles);
+        split = tail.fused ? task - q * split_k : q;
+        rem = tail.fused ? q : task - split * tiles;
     }
     const int mt = div_small(rem, n_tiles), nt = rem - mt * n_tiles;
     const int m0 = mt * TD::BM, n0 = nt * TD::BN;
     tail.split = split;
     tail.rem = rem;
-    const int cb = split * chunk, ce = tail.both ? C : min(C, cb + chunk);
+    const int cb = split * chunk, ce = min(C, cb + chunk);
     const int c0 = cb + 16 * wave;                                   // first channel of this wavefront
     const int steps = c0 < ce ? (ce - c0 + 63) >> 6 : 0;             // its steps (uniform)
     const unsigned HW4 = (unsigned)N * 4u, MN4 = (unsigned)M * HW4;
@@ -1620,13 +1602,8 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     static_assert(NS % 2 == 0, "the turned blocks alternate");
     int pf = raised, it = 0;
     bool left = false;
-    f32x4 first = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // (a share is whole groups: the first one ends between two turns of the loop.  Tested inside the loop it
-    // made the compiler move the accumulators in every turn: ResNet-152 816 -> 848 us, without any such layer.)
-    int until = TD::SUBS == 1 && tail.both ? share : 0x7fffffff;
     if (steps > 0) turn(0, 0);
-    for (;;) {
-    for (; it + 2 * NS <= steps && it < until; it += NS) {
+    for (; it + 2 * NS <= steps; it += NS) {
         if (Poll::enabled) {
             if (pf) {
                 left = true;
@@ -1642,11 +1619,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
             __builtin_amdgcn_sched_barrier(0);
             if (s + 1 == NS) turn(0, 0);
         }
-    }
-    if (TD::SUBS != 1 || until != it || left) break;
-    first = acc[0][0][0] + acc[0][0][1];
-    acc[0][0][0] = acc[0][0][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    until = 0x7fffffff;
     }
     if (!left && it + NS <= steps) {
         if (Poll::enabled && pf) {
@@ -1677,7 +1649,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
-    return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, left || raised, TD::SUBS == 1 ? &first : nullptr);
+    return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
 // ---- reef_conv2d_v9_g<G>: 3x3 / stride 1 / padding 1, whole cache lines --------------------------------------
@@ -1717,19 +1689,12 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     tail.to_ws = split_k > 1 && !tail.fused;
     // tile and split of this workgroup, as in conv2d_direct_body
     const int c_chunk = a[REEF_CONV_K_CHUNK] / 9;
-    const int share = c_chunk >> 6;          // steps of a share
-    tail.both = G == 1 && poll.plain && (flags & REEF_F_BOTH_SHARES);
-    int split = 0, rem;
-    if (tail.both) {
-        tail.fused = false;
-        rem = xcd_chunked(task, tiles);
-    } else {
-        rem = task = xcd_chunked(task, tiles * split_k);
-        if (split_k > 1) {
-            const int q = div_small(task, tail.fused ? split_k : tiles);
-            split = tail.fused ? task - q * split_k : q;
-            rem = tail.fused ? q : task - split * tiles;
-        }
+    task = xcd_chunked(task, tiles * split_k);
+    int split = 0, rem = task;
+    if (split_k > 1) {
+        const int q = div_small(task, tail.fused ? split_k : tiles);
+        split = tail.fused ? task - q * split_k : q;
+        rem = tail.fused ? q : task - split * tiles;
     }
     const int mt = div_small(rem, n_tiles), nt = rem - mt * n_tiles;
     int seg = 0, yt = nt;
@@ -1741,7 +1706,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     const int m0 = mt * 16, y0 = yt * G, x0 = seg * kRowSeg;
     tail.split = split;
     tail.rem = rem;
-    const int cb = split * c_chunk, ce = tail.both ? C : min(C, cb + c_chunk);
+    const int cb = split * c_chunk, ce = min(C, cb + c_chunk);
     const int c0 = cb + 16 * wave;
     int steps = c0 < ce ? (ce - c0 + 63) >> 6 : 0;
     const unsigned HW4 = (unsigned)N * 4u;
@@ -1849,7 +1814,6 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
                 __builtin_amdgcn_sched_barrier(0);
             }
     };
-    f32x4 first = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     struct Yes { constexpr operator bool() const { return true; } };
     struct No { constexpr operator bool() const { return false; } };
     int pf = raised;
@@ -1857,12 +1821,6 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     if (steps > 0) {
         turn();
         if (steps > 1) load_b();
-        if (G == 1 && tail.both) {
-            // (a loop of its own: one loop with the share's end inside cost the layers without shares 2 % of a pass)
-            for (const int rest = steps - share; steps > rest; --steps) step(Yes());
-            first = acc[0][0][0] + acc[0][0][1];
-            acc[0][0][0] = acc[0][0][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
         for (; steps > 1; --steps) {
             if (Poll::enabled) {
                 if (pf) {
@@ -1878,7 +1836,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     f32x4 sum[1][G];
 #pragma unroll
     for (int g = 0; g < G; ++g) sum[0][g] = acc[0][g][0] + acc[0][g][1];
-    return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, left || raised, G == 1 ? &first : nullptr);
+    return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
 // ---- reef_conv2d_xdw[2]_g<G>: 1x1 convolution, then depthwise 3x3, in one launch --------------

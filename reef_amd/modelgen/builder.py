@@ -27,7 +27,6 @@ ACT_NONE, ACT_RELU, ACT_RELU6, ACT_GELU = 0, 1, 2, 3
 F_BIAS, F_RESIDUAL, F_AFFINE, F_DUAL, F_FUSED_REDUCE, F_PRE_ACT, F_PAIR_FOLD, F_DW_OUTPUT = 1, 2, 4, 8, 16, 32, 64, 128
 F_PROJ_OUTPUT = 4096
 F_POOL_OUTPUT, F_IN_SHIFT, F_POOL_SHIFT, F_GAP_OUTPUT = 256, 512, 1024, 2048
-F_BOTH_SHARES = 8192
 WG = 256
 
 
@@ -316,15 +315,6 @@ class GraphBuilder:
             sync_idx, sync_off = self._sync_counters(t["m_tiles"] * t["n_tiles"])
             args = [x, w.idx, out.idx] + opt + pre + [ws.idx, sync_idx]
             flags |= F_PAIR_FOLD if pair else 0
-            share = t["k_chunk"] // (kh * kw)
-            # A split of two whose tiles alone give nearly every CU a workgroup gains nothing from twice as many that
-            # meet again (exchange: 2100 cycles).  ResNet-152's 71 such layers: 896 us of device time a pass where
-            # they meet (16x32 and two image rows a tile), 829 with both shares in one workgroup (16x16, one row).
-            # (Half of such a launch's workgroups lie behind its tasks, where operand slot 9 is the prefetch record's.)
-            if (pair and 2 * share == cin and len(args) + len(packed) <= MAX_ARGS and t["m_tiles"] * t["n_tiles"] >= BOTH_SHARES_TILES
-                    and (share % 256 == 0 and kname in ("reef_conv2d_v1_16x16k4", "reef_conv2d_p1_v_16x16k4")
-                         or share % 64 == 0 and kname == "reef_conv2d_v9_g1")):
-                flags |= F_BOTH_SHARES
             attrs = base + [flags | F_FUSED_REDUCE, act, t["tile_id"], t["split_k"], t["k_chunk"],
                             t["m_tiles"], t["n_tiles"], act2, sync_off, mode, dst_off, len(args) if packed else 0]
             self._emit(kname, t["tasks"], args + packed, attrs, "conv2d", flops, nbytes + nbytes_pack, t["est_us"])
@@ -784,8 +774,6 @@ class GraphBuilder:
                 NG = (G + 2) if S == 1 else (2 * G + 1) * 2      # TileXdw: pixel groups of the 1x1 result
                 PS = (96 if S == 2 else 64 if G == 4 else 160) + 4     # a chunk of input channels per pixel / weight row
                 shared[n] = (NG * 16 * PS + 16 * PS + 16 * (NG * 16 + 20)) * 4 + 16
-            elif sym in ("reef_conv2d_v1_16x16k4", "reef_conv2d_p1_v_16x16k4"):
-                shared[n] = 4 * 2 * 320 * 4 + 16      # TileV1: a partial tile of either share
             elif sym.startswith("reef_conv2d_v9_"):
                 # TileV9: four blocks of [image rows][16 channels][20 floats]
                 shared[n] = 4 * (tiling.ROW_TILES[sym.split("_")[-1]] + 2) * 16 * 20 * 4 + 16
@@ -840,7 +828,6 @@ class GraphBuilder:
         return base
 
 
-BOTH_SHARES_TILES = 192     # output tiles from which a workgroup takes both shares of a split of two
 MAX_ARGS = 9     # REEF_MAX_PTRS - 1: the last slot carries what a launch prefetches for the next one
 
 # (loader family prefix, tile) of the kernels that exist in a packed-weights form

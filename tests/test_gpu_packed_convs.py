@@ -92,3 +92,30 @@ def test_3x3_on_weights_packed_by_channels(tmp_path, tile, shape, split, fused):
     exe, orc, model = run_both(g, tmp_path, inputs)
     compare_storages(exe, orc, model, what="v9 %s %s x%d%s" % (tile, shape, split, " fused" if fused else ""))
     flavours_agree(exe, g, tmp_path, inputs)
+
+
+def test_the_bit_of_a_retired_mode_changes_nothing(tmp_path):
+    """Model files may carry flag 8192 on splits of two (reef_kernels.h): with and without it the same bits, in all
+    flavours, also where ten operands leave no slot for a prefetch record."""
+    shape = (256, 14, 14)
+    inputs = {"data": rnd(*shape), "res": rnd(*shape)}
+    held = []
+    for bit in (0, 8192):
+        g = MB.GraphBuilder("bit")
+        x, r = g.input("data", shape), g.input("res", shape)
+        rows = dict(force=tiling.forced_rows("g1", 256, 14, 14, 256 * 9, 2), fused_reduce=True)
+        y, z = g.conv2d(x, 256, 3, 1, 1, bias=True, residual=r, dual_act=MB.ACT_RELU, **rows)
+        one = dict(force=tiling.forced("16x16k4", 256, 196, 1024, 2, 1), fused_reduce=True)
+        cat = g.temp((1024, 14, 14))
+        g.conv2d(z, 1024, 1, 1, 0, out=cat)
+        g.mark_output(g.conv2d(cat, 256, 1, 1, 0, residual=y, **one))
+        split = [k for k in g.kernels if k["attrs"][12] & 64]
+        assert len(split) == 2 and len(split[0]["args"]) == 10
+        for k in split:
+            k["attrs"][12] |= bit
+        exe, orc, model = run_both(g, tmp_path / str(bit), inputs)
+        compare_storages(exe, orc, model, what="flag %d" % bit)
+        flavours_agree(exe, g, tmp_path / str(bit), inputs)
+        held.append([exe.get_data(k["args"][2], g.storage[k["args"][2]]["size"]) for k in g.kernels])
+    for a, b in zip(*held):
+        np.testing.assert_array_equal(a, b)
