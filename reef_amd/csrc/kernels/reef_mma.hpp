@@ -1446,7 +1446,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
 // in order: no barrier.  It is turned one step ahead of the MFMAs that use it.
 // PRE (p1_v): input scale, shift and ReLU on the loaded values; a lane's values of a load belong to one channel,
 // whose scale and shift one 32-bit load brings to neighbouring lanes.
-// Sums run over the channels in the order of conv2d_direct_body.
+// Sums run over the channels in the order of conv2d_direct_body, in NA chains a sub-tile.
 template <int TM, int TN>
 struct TileV1 {      // a wavefront's place: the turned block, then its partial tile
     static constexpr int WSTRIDE = TM * TN * TileD16<TN, TM>::PART;
@@ -1462,6 +1462,9 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     // steps of loads in flight (with a pre-activation in 2 more wavefronts fit: DenseNet-201 901 -> 891 us of device time a
     // pass, 1022 -> 1016 as a best-effort model; without one ResNet-152 takes 826 us in 4 and 878 in 2)
     constexpr int NS = PRE ? 2 : 4;
+    // Sums of a sub-tile, MFMA by MFMA in turn.  The smallest tile runs deep layers without a split of K: with four it has
+    // the chains that two shares of two have, and their rounding (below v9, where it is measured).
+    constexpr int NA = TM * TN == 1 ? 4 : 2;
     constexpr int LPR = 4 * TN;                    // lanes (16-byte pieces) of a row
     float* smem = (float*)smem_raw;
     constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
@@ -1554,11 +1557,13 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
         }
     }
     tail.fetch(d, MN4);
-    f32x4 acc[TM][TN][2];
+    f32x4 acc[TM][TN][NA];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
-        for (int g = 0; g < TN; ++g) acc[h][g][0] = acc[h][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int g = 0; g < TN; ++g)
+#pragma unroll
+            for (int n = 0; n < NA; ++n) acc[h][g][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     // the turned block lies where this wavefront's partial tile goes afterwards
     float* blk = smem + wave * WSTRIDE;
@@ -1597,7 +1602,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
             for (int h = 0; h < TM; ++h)
 #pragma unroll
                 for (int g = 0; g < TN; ++g)
-                    acc[h][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], bt[from][g][q], acc[h][g][q & 1], 0, 0, 0);
+                    acc[h][g][q % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], bt[from][g][q], acc[h][g][q % NA], 0, 0, 0);
     };
     static_assert(NS % 2 == 0, "the turned blocks alternate");
     int pf = raised, it = 0;
@@ -1648,7 +1653,10 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
-        for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
+        for (int g = 0; g < TN; ++g) {
+            sum[h][g] = acc[h][g][0] + acc[h][g][1];
+            if (NA == 4) sum[h][g] += acc[h][g][NA - 2] + acc[h][g][NA - 1];
+        }
     return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
@@ -1672,6 +1680,10 @@ struct TileV9 {
 template <int G, class Poll>
 __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
     typedef TileV9<G> TV;
+    // Sums of a row.  One row a tile needs no split of K and has four, as many chains as two shares of two: ResNet-152's
+    // scores are 2.47e-7 off 64 bits then (v1 likewise; mean of ten pictures; split in two 2.52e-7, unsplit with two
+    // sums 2.86e-7).  Four cost ResNet-152 0.8 % of a pass and DenseNet-201 1.1 %.
+    constexpr int NA = G == 1 ? 4 : 2;
     float* smem = (float*)smem_raw;
     const int* a = d.attr;
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
@@ -1759,9 +1771,11 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
         tail.ooff[0][g] = ok ? (tail.om[0] * (unsigned)N + (unsigned)((y0 + g) * W + x0 + ocol)) * 4u : kOutside;
     }
     tail.fetch(d, (unsigned)M * HW4);
-    f32x4 acc[1][G][2];
+    f32x4 acc[G][NA];
 #pragma unroll
-    for (int g = 0; g < G; ++g) acc[0][g][0] = acc[0][g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int n = 0; n < NA; ++n) acc[g][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float in[G + 2][4];
     auto turn = [&]() {                 // the loaded rows through LDS; on to the loads behind them
 #pragma unroll
@@ -1778,7 +1792,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int g = 0; g < G; ++g)
-                acc[0][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[t][q], v[g + t / 3][q], acc[0][g][q & 1], 0, 0, 0);
+                acc[g][q % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[t][q], v[g + t / 3][q], acc[g][q % NA], 0, 0, 0);
     };
     // The middle taps first, the neighbours' values formed behind them: then the loaded registers are free, and the
     // next step's rows go through LDS under the outer taps.  (Formed next to its use, a neighbour's value waits for
@@ -1835,7 +1849,10 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     }
     f32x4 sum[1][G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) sum[0][g] = acc[0][g][0] + acc[0][g][1];
+    for (int g = 0; g < G; ++g) {
+        sum[0][g] = acc[g][0] + acc[g][1];
+        if (NA == 4) sum[0][g] += acc[g][NA - 2] + acc[g][NA - 1];
+    }
     return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
