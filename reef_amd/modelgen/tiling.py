@@ -9,7 +9,7 @@ split-K to put a workgroup on every CU.
 """
 import math
 
-from .tuned import TUNED, TUNED_UNDER_LOAD, TUNED_PACKED, TUNED_PACKED_UNDER_LOAD, GEMM_UNDER_LOAD
+from .tuned import TUNED, TUNED_UNDER_LOAD, GEMM_UNDER_LOAD
 
 # name -> (id, BM, BN, relative MFMA efficiency of the inner loop, workgroups per CU)
 TILES = {
@@ -237,7 +237,7 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
     under_load: the layer belongs to a model that shares the device with other streams; the
     entries measured for that case (TUNED_UNDER_LOAD) come before those measured alone.
     packed: the layer's weights will be packed, so that it runs on the kernels that take whole cache lines
-    (v1_ok, the row tiles' v9): entries measured with those (TUNED_PACKED) come before the others.
+    (v1_ok, the row tiles' v9), which the entries were not measured with: see over_entry.
     image: output rows and columns of a convolution (with stride, pre_act: the input goes through an
     activation of its own); shapes outside the table are then chosen by the measured cost of every
     tile (CONV_COST), those of a bare matrix product by the analytic model."""
@@ -246,22 +246,20 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
         hit = TUNED.get(key)
         if under_load and key in TUNED_UNDER_LOAD:
             hit = TUNED_UNDER_LOAD[key] + (hit[2] if hit is not None else 0.0,)
-        if packed and key in TUNED_PACKED:
-            hit = TUNED_PACKED[key] + (hit[2] if hit is not None else 0.0,)
-        if packed and under_load and key in TUNED_PACKED_UNDER_LOAD:
-            hit = TUNED_PACKED_UNDER_LOAD[key] + (hit[2] if hit is not None else 0.0,)
-        if hit is not None and hit[0] in ROW_TILES:
-            if rows and image is not None:
-                t = forced_rows(hit[0], M, image[0], image[1], K, abs(hit[1]))
-                t["est_us"] = hit[2]
-                t["fused"] = hit[1] < 0
-                return t
+        if hit is not None and hit[0] in ROW_TILES and not (rows and image is not None):
             hit = None
         if hit is not None and (hit[0] not in DIRECT_TILES or direct):
             # a negative split factor in the table: the split is folded inside the launch
-            t = forced(hit[0], M, N, K, abs(hit[1]), taps)
+            if hit[0] in ROW_TILES:
+                t = forced_rows(hit[0], M, image[0], image[1], K, abs(hit[1]))
+            else:
+                t = forced(hit[0], M, N, K, abs(hit[1]), taps)
             t["est_us"] = hit[2]
             t["fused"] = hit[1] < 0
+            if packed and image is not None:
+                best = _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act, True)
+                if over_entry(best, t, taps, stride, pointwise, N, K, pre_act):
+                    return best
             return t
     if allow_split and tiles is None and (image is not None or direct and M * N <= NUM_CUS * 4096):
         return _choose_conv(M, N, K, taps, direct, rows and image is not None, image, stride, pointwise, pre_act, packed)
@@ -400,6 +398,28 @@ def direct_cost(tile, geom, fused=True, kind="1"):
     r = geom["tasks"] / NUM_CUS
     us = _cost((CONV_COST_PACKED if kind in "vw" else CONV_COST)[(tile, kind)], geom["k_chunk"], geom["tasks"], s, (r + math.ceil(r)) / 2)
     return us + T_REDUCE_LAUNCH if s > 1 and not fused else us
+
+
+# Part of a tap-form entry's cost below which the row form on whole cache lines replaces it (over_entry).  DenseNet-201's
+# 32 x 3136 x 1152 (0.72: as a best-effort model 1004 -> 986 us) gains, Inception-v3's 96 x 1225 x 576 and 864 (0.89, 0.93:
+# 457.5 -> 461.2) lose.
+ROWS_OVER_TAPS = 0.85
+
+
+def over_entry(best, entry, taps, stride, pointwise, n_pixels, K, pre):
+    """Whether a layer on packed weights takes the cost rule's choice and not the measured entry of its shape: where
+    the choice is an unsplit kernel on whole cache lines and the entry splits K, or is a tap-form 3x3 kernel of a
+    higher cost.  The entries were measured before these kernels.  Their splits fill the device where a workgroup
+    waited for its loads; the kernels on whole lines wait less, and an exchange between two workgroups is 2100
+    cycles of 14 600.  Device time of a pass, entries only and by this rule: ResNet-152 911 -> 820 us, ResNet-50 313 -> 302,
+    ResNet-18 149.3 -> 145.7, DenseNet-201 902 -> 885 and 1110 -> 986 as a best-effort model, Inception-v3 456 -> 457.5;
+    with every entry replaced that way, split or not, ResNet-152 821, MobileNet-v2 149.4 -> 152.6 and Inception-v3 460.6."""
+    kind, was = (conv_kind(t["tile"], taps, stride, pointwise, True, n_pixels, K // taps, pre) for t in (best, entry))
+    if kind not in ("v", "w") or best["split_k"] > 1:
+        return False
+    if entry["split_k"] > 1:
+        return True
+    return was == "9" and (entry["tile"], was) in CONV_COST and best["est_us"] < ROWS_OVER_TAPS * direct_cost(entry["tile"], entry, True, was)
 
 
 def _cost(c, depth, tasks, split, rounds):

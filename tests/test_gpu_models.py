@@ -10,7 +10,7 @@ import pytest
 
 from oracle import oracle as O
 from reef_amd import binding as B
-from reef_amd.modelgen import nets
+from reef_amd.modelgen import nets, tiling
 from tests.helpers import compare_storages, max_rel_err, write_model, REL_TOL
 
 pytestmark = pytest.mark.gpu
@@ -177,14 +177,23 @@ def test_recorded_submission_replays_bit_identical(tmp_path, kind):
     assert not np.array_equal(a, np.zeros_like(a))
 
 
-def test_split_of_two_meets_in_the_pair_slots_or_on_the_counters_with_the_same_bits(tmp_path):
+def test_split_of_two_meets_in_the_pair_slots_or_on_the_counters_with_the_same_bits(tmp_path, monkeypatch):
     """A split of two folded inside the launch has two protocols (REEF_F_PAIR_FOLD): launches
     that run to completion (raw flavour, real-time side of the padding flavour) meet in the pair
     slots with one atomic exchange per element, preemptible launches on the arrival counters.
     Same sums in the same order: all three flavours hold the same bits, run after run and in any
     order on ONE executor (shared buffers), the pair slots and the counters are empty at rest,
     and a preemptible run that was cut short (flag raised) leaves the pair slots alone."""
-    g = nets.resnet(152)          # the benchmark network: 71 of its convolutions are such splits
+    real = tiling.choose
+
+    def in_two(M, N, K, **kw):    # the benchmark network with its layers of 256 channels at 14 x 14 split in two
+        t = real(M, N, K, **kw)
+        if (M, N) != (256, 196) or t["tile"] not in ("g1", "16x16k4"):
+            return t
+        return dict(tiling.forced_rows("g1", M, 14, 14, K, 2) if t["tile"] == "g1" else tiling.forced("16x16k4", M, N, K, 2, kw["taps"]),
+                    fused=True)
+    monkeypatch.setattr(tiling, "choose", in_two)
+    g = nets.resnet(152)
     pair = [k for k in g.kernels if k["name"].startswith("reef_conv2d") and k["attrs"][12] & 64]
     assert len(pair) >= 60, "the network must contain splits of two in the direct family"
     d = write_model(g, tmp_path)
