@@ -258,7 +258,7 @@ def choose(M, N, K, allow_split=True, tiles=None, max_split=32, fused=True, poin
             t["fused"] = hit[1] < 0
             if packed and image is not None:
                 best = _choose_conv(M, N, K, taps, direct, rows, image, stride, pointwise, pre_act, True)
-                if over_entry(best, t, taps, stride, pointwise, N, K, pre_act):
+                if over_entry(best, t, taps, stride, pointwise, N, K, pre_act, under_load):
                     return best
             return t
     if allow_split and tiles is None and (image is not None or direct and M * N <= NUM_CUS * 4096):
@@ -406,19 +406,20 @@ def direct_cost(tile, geom, fused=True, kind="1"):
 ROWS_OVER_TAPS = 0.85
 
 
-def over_entry(best, entry, taps, stride, pointwise, n_pixels, K, pre):
+def over_entry(best, entry, taps, stride, pointwise, n_pixels, K, pre, under_load):
     """Whether a layer on packed weights takes the cost rule's choice and not the measured entry of its shape: where
     the choice is an unsplit kernel on whole cache lines and the entry splits K, or is a tap-form 3x3 kernel of a
     higher cost.  The entries were measured before these kernels.  Their splits fill the device where a workgroup
     waited for its loads; the kernels on whole lines wait less, and an exchange between two workgroups is 2100
-    cycles of 14 600.  Device time of a pass, entries only and by this rule: ResNet-152 911 -> 820 us, ResNet-50 313 -> 302,
+    cycles of 14 600.  (A split of two of the same tile stays where the model is alone, where it is one exchange: DenseNet-201
+    885 us either way.  Under load it meets on counters: 996 -> 986.)  Device time of a pass, entries only and by this rule: ResNet-152 911 -> 820 us, ResNet-50 313 -> 302,
     ResNet-18 149.3 -> 145.7, DenseNet-201 902 -> 885 and 1110 -> 986 as a best-effort model, Inception-v3 456 -> 457.5;
     with every entry replaced that way, split or not, ResNet-152 821, MobileNet-v2 149.4 -> 152.6 and Inception-v3 460.6."""
     kind, was = (conv_kind(t["tile"], taps, stride, pointwise, True, n_pixels, K // taps, pre) for t in (best, entry))
     if kind not in ("v", "w") or best["split_k"] > 1:
         return False
     if entry["split_k"] > 1:
-        return True
+        return under_load or entry["split_k"] > 2 or entry["tile"] != best["tile"]
     return was == "9" and (entry["tile"], was) in CONV_COST and best["est_us"] < ROWS_OVER_TAPS * direct_cost(entry["tile"], entry, True, was)
 
 

@@ -59,16 +59,18 @@ def test_cost_table_names_tiles_and_kinds():
         assert tile in tiling.TILES and kind in "1s9npq"
 
 
-# (cout, cin, taps, image side): split entry and row form; the same for 1x1; an odd image, whose 1x1 layers have no kernel on
-# whole lines; tap-form entries whose cost is near the row form's and far above it; a staged entry
-@pytest.mark.parametrize("cout,cin,taps,side,replaced", [
-    (256, 256, 9, 14, True), (256, 1024, 1, 14, True), (512, 2048, 1, 7, False), (96, 96, 9, 35, False), (32, 128, 9, 56, True),
-    (320, 64, 1, 56, False)])
-def test_a_packed_layer_and_the_entry_of_its_shape(cout, cin, taps, side, replaced):
+# (cout, cin, taps, image side, under load): split entry and row form; the same for 1x1; an odd image, whose 1x1 layers have
+# no kernel on whole lines; tap-form entries whose cost is near the row form's and far above it; a staged entry; a split of
+# two of the same tile, alone and under load
+@pytest.mark.parametrize("cout,cin,taps,side,loaded,replaced", [
+    (256, 256, 9, 14, False, True), (256, 1024, 1, 14, False, True), (512, 2048, 1, 7, False, False), (96, 96, 9, 35, False, False),
+    (32, 128, 9, 56, False, True), (320, 64, 1, 56, False, False), (32, 128, 9, 14, False, False), (32, 128, 9, 14, True, True)])
+def test_a_packed_layer_and_the_entry_of_its_shape(cout, cin, taps, side, loaded, replaced):
     M, N, K = cout, side * side, cin * taps
-    kw = dict(fused=False, pointwise=taps == 1, taps=taps, direct=True, rows=taps == 9, image=(side, side))
+    kw = dict(fused=False, pointwise=taps == 1, taps=taps, direct=True, rows=taps == 9, image=(side, side), under_load=loaded)
     plain, packed = tiling.choose(M, N, K, **kw), tiling.choose(M, N, K, packed=True, **kw)
-    entry = tiling.TUNED[(M, N, K, int(taps == 1))]
+    key = (M, N, K, int(taps == 1))
+    entry = tiling.TUNED_UNDER_LOAD[key] if loaded and key in tiling.TUNED_UNDER_LOAD else tiling.TUNED[key]
     assert (plain["tile"], plain["split_k"], plain["fused"]) == (entry[0], abs(entry[1]), entry[1] < 0)
     assert (packed != plain) == replaced
     if replaced:
