@@ -2867,7 +2867,13 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     constexpr bool BIG = TM * TN > 4 || PK;
     constexpr int KL = BIG ? 4 : 8;        // k values per lane and step
     constexpr int KSTEP = 16 * KL;         // k values of a step
-    constexpr int AC = BIG ? 1 : 2;        // accumulators per sub-tile: enough for no MFMA to wait for the one in front
+    // Accumulators per sub-tile: enough for no MFMA to wait for the one in front, and chains no longer than those of the
+    // same tile on unpacked weights.  A packed 16x16 product has four: the cost table runs it with fewer shares of K than
+    // the unpacked tiles it replaces.  Distance of BERT-base's output from 64 bits at 16, 40, 90, 128 tokens: unpacked
+    // 2.66e-7, 2.98e-7, 2.97e-7, 3.72e-7; packed with one sum 3.26, 3.60, 4.33, 3.80; with these 2.48, 2.59, 2.84, 3.71.
+    // Device time of a pass with one sum and with these: 115.0 and 114.9 us, 135.6 and 135.7, 175.1 and 175.5, 321.3 and
+    // 319.4 (with four in the 16x32 tile and behind a LayerNorm too: 116, 137.6, 177.8, 327).
+    constexpr int AC = TM * TN > 4 ? 1 : PK && !LN && TM * TN == 1 ? 4 : 2;
     // steps of loads in flight (unpacked, 6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
     constexpr int NS = PK ? 4 : 3;
     float* smem = (float*)smem_raw;
@@ -3114,7 +3120,10 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
         for (int g = 0; g < TN; ++g)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = AC == 2 ? acc[h][g][0][j] + acc[h][g][AC - 1][j] : acc[h][g][0][j];
+                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] =
+                    AC == 4   ? (acc[h][g][0][j] + acc[h][g][1 % AC][j]) + (acc[h][g][2 % AC][j] + acc[h][g][AC - 1][j])
+                    : AC == 2 ? acc[h][g][0][j] + acc[h][g][AC - 1][j]
+                              : acc[h][g][0][j];
     if (Poll::enabled && lane == 0) sflag[wave] = left || raised;
     __syncthreads();
     if (Poll::enabled && (sflag[0] | sflag[1] | sflag[2] | sflag[3])) return false;
