@@ -93,7 +93,12 @@ class FakeHal:
         self.core.reef_gpuconfig_override_geometry(num_cus, num_xcds)
         self.events.clear()
         self.skipped = 0
+        self._stop_after = 0
         return self
+
+    def stop_after(self, n):
+        """Nothing ends by itself any more once `n` kernels from now have run (set_auto_progress lets it go on)."""
+        self._stop_after = n
 
     def remove(self):
         # objects created on this backend must be destroyed on it
@@ -165,6 +170,10 @@ class FakeHal:
                         "launch_params": [blocks, 1, 1, 256, 1, 1]})
 
     def _on_kernel(self, symbol, module_path, kernarg, nbytes, grid, block, lds, stream):
+        if self._stop_after:
+            self._stop_after -= 1
+            if self._stop_after == 0:
+                self.lib.fake_hal_set_auto_progress(0)
         symbol = symbol.decode()
         path = module_path.decode()
         flavour = "be" if path.endswith(".be.co") else "trans" if path.endswith(".trans.co") else "raw"

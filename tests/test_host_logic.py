@@ -193,11 +193,13 @@ def test_scheduler_preempt_rollback_and_idempotence(fake, small_dirs):
     s.set_input(be_mid, x, "data")
     for n in "abc":
         s.set_input(rt_mid, THREE, n)
+    fake.stop_after(3)            # the best-effort task is under way, and still is when the other arrives
     be_tid = s.new_task(be_mid)
     t0 = time.time()
     while fake.lib.fake_hal_completed() < 3 and time.time() - t0 < 10:
         time.sleep(0.0002)
     rt_tid = s.new_task(rt_mid)
+    fake.lib.fake_hal_set_auto_progress(1)
     assert s.wait_task(rt_tid) == 0 and s.wait_task(be_tid) == 0
     np.testing.assert_array_equal(s.get_output(rt_mid, 8192), np.full(8192, 18.0, np.float32))
     np.testing.assert_array_equal(s.get_output(be_mid, 16), ref)
