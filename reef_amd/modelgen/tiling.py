@@ -400,10 +400,11 @@ def direct_cost(tile, geom, fused=True, kind="1"):
     return us + T_REDUCE_LAUNCH if s > 1 and not fused else us
 
 
-# Part of a tap-form entry's cost below which the row form on whole cache lines replaces it (over_entry).  DenseNet-201's
-# 32 x 3136 x 1152 (0.72: as a best-effort model 1004 -> 986 us) gains, Inception-v3's 96 x 1225 x 576 and 864 (0.89, 0.93:
-# 457.5 -> 461.2) lose.
-ROWS_OVER_TAPS = 0.85
+# Part of a tap-form entry's cost below which the row form on whole cache lines replaces it (over_entry).  Gain: 32 x 784 x 1152
+# and 32 x 3136 x 1152 of DenseNet-201 (0.83, 0.72: as a best-effort model 1004 -> 986 us with the second), 512 x 49 x 4608 of
+# ResNet-152 (0.86).  Lose: Inception-v3's 384 x 64 x 4032 (0.875: 456.0 -> 457.5 us; its rows of 8 pixels fill 8 of 14
+# columns), 96 x 1225 x 576 and 864 (0.89, 0.93: 457.5 -> 461.2).
+ROWS_OVER_TAPS = 0.87
 
 
 def over_entry(best, entry, taps, stride, pointwise, n_pixels, K, pre, under_load):
@@ -412,15 +413,16 @@ def over_entry(best, entry, taps, stride, pointwise, n_pixels, K, pre, under_loa
     higher cost.  The entries were measured before these kernels.  Their splits fill the device where a workgroup
     waited for its loads; the kernels on whole lines wait less, and an exchange between two workgroups is 2100
     cycles of 14 600.  (A split of two of the same tile stays where the model is alone, where it is one exchange: DenseNet-201
-    885 us either way.  Under load it meets on counters: 996 -> 986.)  Device time of a pass, entries only and by this rule: ResNet-152 911 -> 820 us, ResNet-50 313 -> 302,
-    ResNet-18 149.3 -> 145.7, DenseNet-201 902 -> 885 and 1110 -> 986 as a best-effort model, Inception-v3 456 -> 457.5;
-    with every entry replaced that way, split or not, ResNet-152 821, MobileNet-v2 149.4 -> 152.6 and Inception-v3 460.6."""
+    885 us either way.  Under load it meets on counters: 996 -> 986.)  Device time of a pass, entries only and by
+    this rule: ResNet-152 911 -> 820 us, ResNet-50 313 -> 302, ResNet-18 149.3 -> 145.7, DenseNet-201 902 -> 885 and 1110 ->
+    986 as a best-effort model; with every entry replaced that way, split or not, ResNet-152 821, MobileNet-v2 149.4 ->
+    152.6 and Inception-v3 456 -> 460.6."""
     kind, was = (conv_kind(t["tile"], taps, stride, pointwise, True, n_pixels, K // taps, pre) for t in (best, entry))
     if kind not in ("v", "w") or best["split_k"] > 1:
         return False
-    if entry["split_k"] > 1:
-        return under_load or entry["split_k"] > 2 or entry["tile"] != best["tile"]
-    return was == "9" and (entry["tile"], was) in CONV_COST and best["est_us"] < ROWS_OVER_TAPS * direct_cost(entry["tile"], entry, True, was)
+    if was == "9":
+        return (entry["tile"], was) in CONV_COST and best["est_us"] < ROWS_OVER_TAPS * direct_cost(entry["tile"], entry, True, was)
+    return entry["split_k"] > 1 and (under_load or entry["split_k"] > 2 or entry["tile"] != best["tile"])
 
 
 def _cost(c, depth, tasks, split, rounds):

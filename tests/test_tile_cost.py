@@ -60,11 +60,11 @@ def test_cost_table_names_tiles_and_kinds():
 
 
 # (cout, cin, taps, image side, under load): split entry and row form; the same for 1x1; an odd image, whose 1x1 layers have
-# no kernel on whole lines; tap-form entries whose cost is near the row form's and far above it; a staged entry; a split of
+# no kernel on whole lines; tap-form entries, unsplit and split, whose cost is near the row form's and above it; a staged entry; a split of
 # two of the same tile, alone and under load
 @pytest.mark.parametrize("cout,cin,taps,side,loaded,replaced", [
     (256, 256, 9, 14, False, True), (256, 1024, 1, 14, False, True), (512, 2048, 1, 7, False, False), (96, 96, 9, 35, False, False),
-    (32, 128, 9, 56, False, True), (320, 64, 1, 56, False, False), (32, 128, 9, 14, False, False), (32, 128, 9, 14, True, True)])
+    (32, 128, 9, 56, False, True), (384, 448, 9, 8, False, False), (512, 512, 9, 7, False, True), (320, 64, 1, 56, False, False), (32, 128, 9, 14, False, False), (32, 128, 9, 14, True, True)])
 def test_a_packed_layer_and_the_entry_of_its_shape(cout, cin, taps, side, loaded, replaced):
     M, N, K = cout, side * side, cin * taps
     kw = dict(fused=False, pointwise=taps == 1, taps=taps, direct=True, rows=taps == 9, image=(side, side), under_load=loaded)
