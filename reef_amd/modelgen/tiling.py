@@ -117,8 +117,9 @@ GEMM_COST = {
 }
 # The same for the direct kernels on packed weights (reef_kernels.h, ldb = 0): 13 sequence lengths of 16 to 512 times 16
 # layer shapes of 256 to 4096 columns and depth, 4279 launches.  It picks within 4.3 % of the fastest launch on average, by
-# GEMM_COST 11 %: BERT-base at 128, six layers, 300 us of device time a pass by GEMM_COST and 285 by this (305 with the
-# FFN-down product as in GEMM_UNDER_LOAD); at 384, four layers, 433 and 402 (in turn, unpacked: 331 and 439).
+# GEMM_COST 11 %: BERT-base at 128, six layers, 300 us of device time a pass by GEMM_COST and 285 by this (unpacked 331); at
+# 384, four layers, 433 and 402 (unpacked 439).  With the FFN-down product as in GEMM_UNDER_LOAD, which comes first, a pass takes
+# 7 % more: see there.
 GEMM_COST_PACKED = {
     ("16x16k4", False): (3.735, 0, 0.1841, 1.183, 0.01631, 0, 3.281),
     ("16x16k4", True): (3.942, 0, 0.07655, 1.525, 0.2484, 0, 0),

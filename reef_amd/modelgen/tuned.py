@@ -257,8 +257,9 @@ TUNED_UNDER_LOAD = {
 # and 0.587 / 0.975-0.977 ms real-time p50 / p99, in three 1606-1607 and 0.587-0.590 / 0.987-1.033 -- the
 # 64 workgroups fewer buy the real-time model nothing.
 # On packed weights these are taken for a model alone too: a graph for one use and for the other is the same then, as
-# the checks of nets.bert ask.  (There 16x16k4 unsplit would give one client 1508 inferences per second and two 2380;
-# the split in four gives them 1456 and 2308.)
+# the checks of nets.bert ask.  They cost: the cost table would run the product unsplit on 16x16k4, a pass of twelve layers
+# 594 us instead of 634 alone, of six layers as a best-effort model 308 instead of 329; two clients 2380
+# inferences per second instead of 2308.
 GEMM_UNDER_LOAD = {
     (128, 768, 3072): ("32x48d4", 4),
 }
