@@ -55,6 +55,7 @@ template <class T, int MODE = CONV_GENERAL>
 struct OpConv {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = T::LDS_BYTES;
+    static constexpr int WAVES = T::BM * T::BN >= 128 * 128 ? 1 : 2;
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
         return conv2d_body<T, MODE>(d, task, smem, p);
@@ -64,6 +65,7 @@ template <int R, int TN = 1, int TM = 1, bool PRE = false, bool ROWS = false, bo
 struct OpConvDirect {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
+    static constexpr int WAVES = 2;
     static constexpr bool CHECKS_FLAG_ITSELF = true;   // the body makes the wrapper's first flag check
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
@@ -75,6 +77,7 @@ template <int TM, int TN, bool PRE = false>
 struct OpConvV1 {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileV1<TM, TN>::LDS_BYTES;
+    static constexpr int WAVES = 2;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
@@ -86,6 +89,7 @@ template <int G>
 struct OpConvV9 {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileV9<G>::LDS_BYTES;
+    static constexpr int WAVES = 2;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
@@ -297,10 +301,22 @@ __device__ __forceinline__ bool dkp_walk(const ReefDkpArgs& a, DkpWalk& w) {
 }  // namespace
 
 // ---- entry generators ---------------------------------------------------------
+// Wavefronts a SIMD at least (OP::WAVES, 1 if absent).  Where one is enough the compiler keeps accumulators in accumulation
+// registers and turns them over there: reef_conv2d_v9_g1 moved all sixteen once a step, behind the MFMAs that write them.
+// With two, 256 registers each, MFMAs add to ordinary registers and nothing moves: ResNet-152 844.7 -> 840.9 us a request,
+// ResNet-50 at 448 699.7 -> 694.4, DenseNet-201 as a best-effort model 1012.4 -> 1007.5.  Only the convolutions ask for it:
+// BERT-base at 128 tokens takes 349 instead of 343 with it in the products and the attention.
+namespace {
+template <class OP, class = void>
+struct WavesOf { static constexpr int value = 1; };
+template <class OP>
+struct WavesOf<OP, decltype((void)OP::WAVES)> { static constexpr int value = OP::WAVES; };
+}  // namespace
 #define REEF_COMMA ,
 #if REEF_FLAVOUR == 0
 #define REEF_ENTRY(NAME, OP)                                                          \
-    extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS) NAME(ReefOpDesc) {  \
+    constexpr int NAME##_waves = WavesOf<OP>::value;                                    \
+    extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS, NAME##_waves) NAME(ReefOpDesc) {  \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];               \
         const ReefOpDesc& m = kernarg_at<ReefOpDesc>(0);                              \
         const OpDesc d = OpDesc::load<0>(m);                                          \
@@ -350,7 +366,8 @@ template <class OP>
 struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static constexpr bool value = OP::CHECKS_FLAG_ITSELF; };
 }  // namespace
 #define REEF_ENTRY(NAME, OP)                                                              \
-    extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS) NAME(ReefBeArgs) {      \
+    constexpr int NAME##_waves = WavesOf<OP>::value;                                    \
+    extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS, NAME##_waves) NAME(ReefBeArgs) {      \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];                   \
         __shared__ int s_pre;                                                             \
         const ReefBeArgs& a = kernarg_at<ReefBeArgs>(0);                                  \
@@ -377,7 +394,8 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
 // (GPUConfig::get_kernel_address, src/reef/executor/hip/hip_impl.cpp:16-32) and passes to its
 // proxies as func_l / func_r.  A merge_framework_<n> proxy jumps there.
 #define REEF_ENTRY(NAME, OP)                                                           \
-    extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS) NAME(ReefDkpArgs) {  \
+    constexpr int NAME##_waves = WavesOf<OP>::value;                                    \
+    extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS, NAME##_waves) NAME(ReefDkpArgs) {  \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];                \
         kernarg_warm<sizeof(ReefDkpArgs)>();                                           \
         const ReefDkpArgs& a = kernarg_at<ReefDkpArgs>(0);                             \
