@@ -140,6 +140,7 @@ void leave_queue(Queue* q, uint32_t packets) { q->load.fetch_sub(packets); }
 struct AqlKernel {
     uint64_t object;
     uint32_t lds, scratch, kernarg;
+    bool through;      // its stores need no release (<name>_through)
 };
 
 // The implicit arguments a kernel may read behind its own (code object version 5): block counts and
@@ -205,6 +206,8 @@ struct AqlCode {
             if (s == HSA_STATUS_SUCCESS)
                 s = hsa_executable_symbol_get_info(sym, HSA_EXECUTABLE_SYMBOL_INFO_KERNEL_KERNARG_SEGMENT_SIZE, &k.kernarg);
             if (s != HSA_STATUS_SUCCESS) { *err = hsa_text(s, ("kernel " + name).c_str()); return false; }
+            hsa_executable_symbol_t mark;
+            k.through = hsa_executable_get_symbol_by_name(exe, (name + "_through").c_str(), &agent, &mark) == HSA_STATUS_SUCCESS;
             it = kernels.emplace(name, k).first;
         }
         *out = it->second;
@@ -452,9 +455,10 @@ AqlPass* aql_pass_create(int device, const AqlLaunch* launches, size_t n, size_t
     for (size_t i = 0; i < n; ++i) {
         const AqlLaunch& l = launches[i];
         // Launches follow one another (barrier) and see each other's results; the last makes its results
-        // visible to host and copy engines.
+        // visible to host and copy engines.  Kernels that write their results through to memory leave nothing to release
+        // to the launch behind them (0.25 us a launch; code objects of older model directories do, and are released).
         const int acquire = HSA_FENCE_SCOPE_AGENT;
-        const int release = i == n - 1 ? HSA_FENCE_SCOPE_SYSTEM : HSA_FENCE_SCOPE_AGENT;
+        const int release = i == n - 1 ? HSA_FENCE_SCOPE_SYSTEM : kernels[i].through ? HSA_FENCE_SCOPE_NONE : HSA_FENCE_SCOPE_AGENT;
         p->packets.push_back(dispatch_packet(kernels[i], l.grid, l.block, l.dyn_lds, (char*)p->kernargs + at[i], acquire, release));
     }
     const hsa_status_t s = hsa_signal_create(0, 0, nullptr, &p->done);

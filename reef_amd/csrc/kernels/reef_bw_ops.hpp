@@ -125,7 +125,7 @@ __device__ __forceinline__ void dwconv2d_body(const OpDesc& d, int task) {
         }
     }
     if (a[REEF_DW_FLAGS] & 1) acc += ((const float*)d.ptr[3])[c];
-    ((float*)d.ptr[2])[idx] = act_apply(acc, a[REEF_DW_ACT]);
+    store_out((float*)d.ptr[2] + idx, act_apply(acc, a[REEF_DW_ACT]));
 }
 
 __device__ __forceinline__ void pool2d_body(const OpDesc& d, int task) {
@@ -188,7 +188,7 @@ __device__ __forceinline__ void pool2d_body(const OpDesc& d, int task) {
     if (mode == 0) v = m;
     else v = s / (float)(a[REEF_POOL_COUNT_PAD] ? kh * kw : (cnt > 0 ? cnt : 1));
     if (a[REEF_POOL_FLAGS] & 1) v += ((const float*)d.ptr[2])[c];
-    ((float*)d.ptr[1])[idx] = act_apply(v, a[REEF_POOL_ACT]);
+    store_out((float*)d.ptr[1] + idx, act_apply(v, a[REEF_POOL_ACT]));
 }
 
 // one wavefront per channel
@@ -206,7 +206,7 @@ __device__ __forceinline__ void global_avgpool_body(const OpDesc& d, int task) {
         for (int i = threadIdx.x & 63; i < HW; i += 64) s += in[i];
     }
     s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0) ((float*)d.ptr[1])[c] = s * (1.0f / (float)HW);
+    if ((threadIdx.x & 63) == 0) store_out((float*)d.ptr[1] + c, s * (1.0f / (float)HW));
 }
 
 __device__ __forceinline__ void eltwise_body(const OpDesc& d, int task) {
@@ -230,7 +230,7 @@ __device__ __forceinline__ void eltwise_body(const OpDesc& d, int task) {
         if (shift) v += shift[c];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = act_apply(v[e], act);
-        *(f32x4*)(out + i0) = v;
+        buf_store4(make_rsrc(out, (unsigned)(total * 4)), (unsigned)(i0 * 4), v);
     } else {
         for (int e = 0; e < 4 && i0 + e < total; ++e) {
             const int c = div_index(i0 + e, inner);
@@ -238,7 +238,7 @@ __device__ __forceinline__ void eltwise_body(const OpDesc& d, int task) {
             if (b) v += b[i0 + e];
             if (scale) v *= scale[c];
             if (shift) v += shift[c];
-            out[i0 + e] = act_apply(v, act);
+            store_out(out + i0 + e, act_apply(v, act));
         }
     }
 }
@@ -272,7 +272,7 @@ __device__ __forceinline__ void dense_body(const OpDesc& d, int task) {
             float v = s + bias;
             if (act == REEF_ACT_RELU) v = fmaxf(v, 0.0f);
             else if (act == REEF_ACT_GELU) v = gelu_erf(v);
-            ((float*)d.ptr[2])[(size_t)r * out_f + o] = v;
+            store_out((float*)d.ptr[2] + (size_t)r * out_f + o, v);
         }
     }
 }
@@ -309,7 +309,7 @@ __device__ __forceinline__ void softmax_body(const OpDesc& d, int task) {
         s = wave_sum(s);
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-            if (lane + 64 * j < cols) y[lane + 64 * j] = val[j] / s;
+            if (lane + 64 * j < cols) store_out(y + lane + 64 * j, val[j] / s);
         return;
     }
     auto at = [&](int i) { return (mask && mask[i]) ? -INFINITY : x[i]; };
@@ -319,7 +319,7 @@ __device__ __forceinline__ void softmax_body(const OpDesc& d, int task) {
     float s = 0.0f;
     for (int i = lane; i < cols; i += 64) s += expf(at(i) - m);
     s = wave_sum(s);
-    for (int i = lane; i < cols; i += 64) y[i] = expf(at(i) - m) / s;
+    for (int i = lane; i < cols; i += 64) store_out(y + i, expf(at(i) - m) / s);
 }
 
 // Attention of one head for REEF_AT_ROWS query rows: scores, masked softmax and context without a
@@ -440,7 +440,7 @@ __device__ __forceinline__ void attention_body(const OpDesc& d, int task, char* 
         float* out = (float*)d.ptr[1] + (size_t)(m0 + r) * ldo + h * HD;
 #pragma unroll
         for (int j = 0; j < OC; ++j)
-            if (c + LANES * j < HD) out[c + LANES * j] = o2[j];
+            if (c + LANES * j < HD) store_out(out + c + LANES * j, o2[j]);
     }
 }
 
@@ -484,7 +484,7 @@ __device__ __forceinline__ void layernorm_body(const OpDesc& d, int task) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int i = lane + 64 * j;
-            if (i < cols) y[i] = (val[j] - mean) * inv * gm[j] + bt[j];
+            if (i < cols) store_out(y + i, (val[j] - mean) * inv * gm[j] + bt[j]);
         }
         return;
     }
@@ -499,7 +499,7 @@ __device__ __forceinline__ void layernorm_body(const OpDesc& d, int task) {
     const float inv = 1.0f / sqrtf(wave_sum(v) / (float)cols + eps);
     for (int i = lane; i < cols; i += 64) {
         const float dlt = (res ? x[i] + res[i] : x[i]) - mean;
-        y[i] = dlt * inv * gamma[i] + beta[i];
+        store_out(y + i, dlt * inv * gamma[i] + beta[i]);
     }
 }
 
@@ -512,7 +512,7 @@ __device__ __forceinline__ void bias_gelu_body(const OpDesc& d, int task) {
     const size_t i0 = ((size_t)task * kThreads + threadIdx.x) * 4;
     for (int e = 0; e < 4 && i0 + e < total; ++e) {
         const int c = (int)((i0 + e) - (size_t)div_index(i0 + e, cols) * cols);
-        y[i0 + e] = gelu_erf(x[i0 + e] + (bias ? bias[c] : 0.0f));
+        store_out(y + i0 + e, gelu_erf(x[i0 + e] + (bias ? bias[c] : 0.0f)));
     }
 }
 
@@ -532,7 +532,7 @@ __device__ __forceinline__ void embedding_body(const OpDesc& d, int task) {
         float v = tok[(size_t)ids[s] * hidden + h];
         if (pos) v += pos[i0 + e];
         if (seg) v += seg[h];
-        out[i0 + e] = v;
+        store_out(out + i0 + e, v);
     }
 }
 
@@ -543,9 +543,9 @@ __device__ __forceinline__ void copy_body(const OpDesc& d, int task) {
     const int i0 = (task * kThreads + threadIdx.x) * 4;
     if (i0 >= count) return;
     if (((count | dst_off) & 3) == 0) {
-        *(f32x4*)(out + i0) = *(const f32x4*)(in + i0);
+        buf_store4(make_rsrc(out, (unsigned)count * 4u), (unsigned)i0 * 4u, *(const f32x4*)(in + i0));
     } else {
-        for (int e = 0; e < 4 && i0 + e < count; ++e) out[i0 + e] = in[i0 + e];
+        for (int e = 0; e < 4 && i0 + e < count; ++e) store_out(out + i0 + e, in[i0 + e]);
     }
 }
 
@@ -565,7 +565,7 @@ __device__ __forceinline__ void transpose_body(const OpDesc& d, int task) {
         const int a = q - b * d0;
         float v = in[((size_t)a * d1 + b) * d2 + c];
         if (bias) v += bias[(size_t)b * d2 + c];
-        out[i] = v;
+        store_out(out + i, v);
     }
 }
 
@@ -577,7 +577,7 @@ __device__ __forceinline__ void mocked_body(const OpDesc& d, int task, int t) {
     const float* b = (const float*)d.ptr[1];
     float* out = (float*)d.ptr[2];
     const int i = task * 128 + t;
-    out[i] = MUL ? a[t] * b[i] : a[t] + b[i];
+    store_out(out + i, MUL ? a[t] * b[i] : a[t] + b[i]);
 }
 
 }  // namespace reef_dev

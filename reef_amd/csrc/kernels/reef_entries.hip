@@ -65,7 +65,8 @@ template <int R, int TN = 1, int TM = 1, bool PRE = false, bool ROWS = false, bo
 struct OpConvDirect {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileD16<TN, TM>::LDS_BYTES;
-    static constexpr int WAVES = 2;
+    static constexpr int WAVES = R == 25 || TM * TN >= 4 ? 1 : 2;      // (more than 256 registers with the flag checks)
+    static constexpr bool THROUGH = !(R == 1 && TM == 2 && !PRE);
     static constexpr bool CHECKS_FLAG_ITSELF = true;   // the body makes the wrapper's first flag check
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
@@ -78,6 +79,7 @@ struct OpConvV1 {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileV1<TM, TN>::LDS_BYTES;
     static constexpr int WAVES = 2;
+    static constexpr bool THROUGH = PRE;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
@@ -311,10 +313,14 @@ template <class OP, class = void>
 struct WavesOf { static constexpr int value = 1; };
 template <class OP>
 struct WavesOf<OP, decltype((void)OP::WAVES)> { static constexpr int value = OP::WAVES; };
+template <class OP, class = void>
+struct WritesThrough { static constexpr bool value = true; };
+template <class OP>
+struct WritesThrough<OP, decltype((void)OP::THROUGH)> { static constexpr bool value = OP::THROUGH; };
 }  // namespace
 #define REEF_COMMA ,
 #if REEF_FLAVOUR == 0
-#define REEF_ENTRY(NAME, OP)                                                          \
+#define REEF_KERNEL(NAME, OP)                                                         \
     constexpr int NAME##_waves = WavesOf<OP>::value;                                    \
     extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS, NAME##_waves) NAME(ReefOpDesc) {  \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];               \
@@ -326,6 +332,7 @@ struct WavesOf<OP, decltype((void)OP::WAVES)> { static constexpr int value = OP:
             return;                                                                   \
         }                                                                             \
         OP::run(d, (int)blockIdx.x, smem, NoPoll{true});                              \
+        partial_stores_done();                                                        \
     }
 #elif REEF_FLAVOUR == 1
 namespace {
@@ -365,7 +372,7 @@ struct ChecksFlagItself { static constexpr bool value = false; };
 template <class OP>
 struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static constexpr bool value = OP::CHECKS_FLAG_ITSELF; };
 }  // namespace
-#define REEF_ENTRY(NAME, OP)                                                              \
+#define REEF_KERNEL(NAME, OP)                                                             \
     constexpr int NAME##_waves = WavesOf<OP>::value;                                    \
     extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS, NAME##_waves) NAME(ReefBeArgs) {      \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];                   \
@@ -387,13 +394,14 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
         }                                                                                 \
         if (t == 0) be_count_completed(a, done);                                          \
         be_signal_exit(a, t);                                                             \
+        partial_stores_done();                                                            \
     }
 #else
 // Every entry also publishes the address of its first instruction in a device variable
 // <name>_entry: what the reference reads out of the kernel descriptor on the host
 // (GPUConfig::get_kernel_address, src/reef/executor/hip/hip_impl.cpp:16-32) and passes to its
 // proxies as func_l / func_r.  A merge_framework_<n> proxy jumps there.
-#define REEF_ENTRY(NAME, OP)                                                           \
+#define REEF_KERNEL(NAME, OP)                                                          \
     constexpr int NAME##_waves = WavesOf<OP>::value;                                    \
     extern "C" __global__ void __launch_bounds__(REEF_WG_THREADS, NAME##_waves) NAME(ReefDkpArgs) {  \
         __shared__ __align__(16) char smem[OP::LDS > 0 ? OP::LDS : 16];                \
@@ -411,9 +419,26 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
             OP::run(d, i, smem, NoPoll{!w.right});                             \
             __syncthreads();                                                           \
         }                                                                              \
+        partial_stores_done();                                                         \
     }                                                                                  \
     extern "C" __device__ __attribute__((used)) void* const NAME##_entry = (void*)NAME;
 #endif
+
+// REEF_ENTRY: every store of the kernel is written through (store_out, buf_store, atomics) and acknowledged before its
+// wavefront ends, which <name>_through tells recorded passes: nothing is left to release to the launch behind it.
+// REEF_ENTRY_RELEASED: results stay in L2 until the release at the end of the launch.  1x1 kernels on whole lines without a
+// pre-activation and 32x32 ones: on images whose rows end inside a line (14 x 14) their many results written through piece by
+// piece cost what the release does, or more (512 channels to 512 4.06 us a launch either way, ResNet-152 844 us a request, and
+// 859 with them written through).
+#define REEF_ENTRY(NAME, OP)                                                          \
+    using NAME##_op = OP;                                                             \
+    static_assert(WritesThrough<NAME##_op>::value, "REEF_ENTRY_RELEASED");            \
+    REEF_KERNEL(NAME, NAME##_op)                                                      \
+    extern "C" __device__ __attribute__((used)) const int NAME##_through = 1;
+#define REEF_ENTRY_RELEASED(NAME, OP)                                                 \
+    using NAME##_op = OP;                                                             \
+    static_assert(!WritesThrough<NAME##_op>::value, "REEF_ENTRY");                    \
+    REEF_KERNEL(NAME, NAME##_op)
 
 REEF_ENTRY(reef_conv2d_128x128, OpConv<Tile128x128>)
 REEF_ENTRY(reef_conv2d_128x64, OpConv<Tile128x64>)
@@ -455,12 +480,12 @@ REEF_ENTRY(reef_conv2d_d7_16x32k4, OpConvDirect<7 REEF_COMMA 2>)
 REEF_ENTRY(reef_conv2d_p1_16x16k4, OpConvDirect<1 REEF_COMMA 1 REEF_COMMA 1 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_p1_16x32k4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 1 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_p1_32x32d4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 2 REEF_COMMA true>)
-REEF_ENTRY(reef_conv2d_d1_32x32d4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 2>)
+REEF_ENTRY_RELEASED(reef_conv2d_d1_32x32d4, OpConvDirect<1 REEF_COMMA 2 REEF_COMMA 2>)
 REEF_ENTRY(reef_conv2d_d9_32x32d4, OpConvDirect<9 REEF_COMMA 2 REEF_COMMA 2>)
-REEF_ENTRY(reef_conv2d_v1_16x16k4, OpConvV1<1 REEF_COMMA 1>)
-REEF_ENTRY(reef_conv2d_v1_16x32k4, OpConvV1<1 REEF_COMMA 2>)
-REEF_ENTRY(reef_conv2d_v1_16x64k4, OpConvV1<1 REEF_COMMA 4>)
-REEF_ENTRY(reef_conv2d_v1_32x32d4, OpConvV1<2 REEF_COMMA 2>)
+REEF_ENTRY_RELEASED(reef_conv2d_v1_16x16k4, OpConvV1<1 REEF_COMMA 1>)
+REEF_ENTRY_RELEASED(reef_conv2d_v1_16x32k4, OpConvV1<1 REEF_COMMA 2>)
+REEF_ENTRY_RELEASED(reef_conv2d_v1_16x64k4, OpConvV1<1 REEF_COMMA 4>)
+REEF_ENTRY_RELEASED(reef_conv2d_v1_32x32d4, OpConvV1<2 REEF_COMMA 2>)
 REEF_ENTRY(reef_conv2d_p1_v_16x16k4, OpConvV1<1 REEF_COMMA 1 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_p1_v_16x32k4, OpConvV1<1 REEF_COMMA 2 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_p1_v_32x32d4, OpConvV1<2 REEF_COMMA 2 REEF_COMMA true>)
@@ -503,7 +528,7 @@ REEF_ENTRY(reef_conv2d_f7_32x32d4, OpConvFilterRows<7 REEF_COMMA 2 REEF_COMMA 2>
 REEF_ENTRY(reef_conv2d_o1_16x16k4, OpConvOdd<>)
 REEF_ENTRY(reef_conv2d_o1_16x32k4, OpConvOdd<2>)
 REEF_ENTRY(reef_conv2d_o1_16x64k4, OpConvOdd<4>)
-REEF_ENTRY(reef_conv2d_o1_32x32d4, OpConvOdd<2 REEF_COMMA 2>)
+REEF_ENTRY_RELEASED(reef_conv2d_o1_32x32d4, OpConvOdd<2 REEF_COMMA 2>)
 #endif
 REEF_ENTRY(reef_conv2d_xdw_g2, OpConvXdw<2>)
 REEF_ENTRY(reef_conv2d_xdw_g4, OpConvXdw<4>)

@@ -837,8 +837,8 @@ struct DirectTail {
 // store, partial tile to the workspace, or the fold of a split K inside the launch.  False: the workgroup
 // leaves a preempted launch.
 // WSTRIDE: floats between the wavefronts' places in LDS; the flags (one a wavefront) lie behind the last.
-// stop: this wavefront has seen the preemption flag.
-template <int TM, int TN, int WSTRIDE = TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, class Poll>
+// stop: this wavefront has seen the preemption flag.  AUX: how the results are stored (kThrough, or 0 for plain stores).
+template <int TM, int TN, int WSTRIDE = TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, int AUX = kThrough, class Poll>
 __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN],
                                             const DirectTail<TM, TN>& t, const Poll& poll, bool stop) {
     typedef TileD16<TN, TM> TD;
@@ -874,7 +874,7 @@ __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int
 #pragma unroll
         for (int h = 0; h < TM; ++h)
 #pragma unroll
-            for (int g = 0; g < TN; ++g) buf_store(ws, t.ooff[h][g], v[h][g]);
+            for (int g = 0; g < TN; ++g) buf_store<AUX>(ws, t.ooff[h][g], v[h][g]);
         return true;
     }
     if (!t.fused && (t.flags & REEF_F_GAP_OUTPUT)) {
@@ -890,7 +890,7 @@ __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int
                 if (t.ooff[h][g] != kOutside) s += t.ep.value(v[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h]);
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
-            if ((threadIdx.x & 15) == 0 && t.om[h] < (unsigned)M) buf_store(t.ep.out, t.om[h] * 4u, s * (1.0f / (float)N));
+            if ((threadIdx.x & 15) == 0 && t.om[h] < (unsigned)M) buf_store<AUX>(t.ep.out, t.om[h] * 4u, s * (1.0f / (float)N));
         }
         return true;
     }
@@ -983,14 +983,14 @@ __device__ __forceinline__ bool direct_tail(const OpDesc& d, char* smem_raw, int
 #pragma unroll
         for (int g = 0; g < TN; ++g) {
             v[h][g] = t.ep.value(v[h][g], t.om[h] * 4u, t.e_res[h][g], t.e_bias[h]);
-            buf_store(t.ep.out, off[h][g] + t.ep.doff4, v[h][g]);
+            buf_store<AUX>(t.ep.out, off[h][g] + t.ep.doff4, v[h][g]);
         }
     if (t.ep.has_dual) {
 #pragma unroll
         for (int h = 0; h < TM; ++h)
 #pragma unroll
             for (int g = 0; g < TN; ++g)
-                buf_store(t.ep.out2, off[h][g] + t.ep.doff4, act_apply(v[h][g] + t.e_sh2[h], t.ep.act2));
+                buf_store<AUX>(t.ep.out2, off[h][g] + t.ep.doff4, act_apply(v[h][g] + t.e_sh2[h], t.ep.act2));
     }
     return true;
 }
@@ -1431,7 +1431,8 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
-    return direct_tail(d, smem_raw, wave, sum, tail, poll, left || raised);
+    return direct_tail<TM, TN, TileD16<TN, TM>::SUBS * TileD16<TN, TM>::PART, R == 1 && TM == 2 && !PRE ? 0 : kThrough>(
+        d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
 // ---- reef_conv2d_v1_<tile>, reef_conv2d_p1_v_<tile>: 1x1 filters, stride 1, whole cache lines ----------------
@@ -1657,7 +1658,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
             sum[h][g] = acc[h][g][0] + acc[h][g][1];
             if (NA == 4) sum[h][g] += acc[h][g][NA - 2] + acc[h][g][NA - 1];
         }
-    return direct_tail<TM, TN, WSTRIDE>(d, smem_raw, wave, sum, tail, poll, left || raised);
+    return direct_tail<TM, TN, WSTRIDE, PRE ? kThrough : 0>(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
 // ---- reef_conv2d_v9_g<G>: 3x3 / stride 1 / padding 1, whole cache lines --------------------------------------
@@ -2831,7 +2832,7 @@ __device__ __forceinline__ bool gemm_body(const OpDesc& d, int task, char* smem_
                     if (act == REEF_ACT_RELU) v = fmaxf(v, 0.0f);
                     else if (act == REEF_ACT_GELU) v = gelu_erf(v);
                     if (R) v += R[(size_t)m * ldc + n];
-                    C[(size_t)m * ldc + n] = v;
+                    store_out(C + (size_t)m * ldc + n, v);
                 }
             }
         }
@@ -3444,7 +3445,7 @@ __device__ __forceinline__ void attention_mma_body(const OpDesc& d, int task, ch
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int r = 4 * kq + j;
-            if (m0 + r < S) out[(size_t)(m0 + r) * ldo] = (acc[0][j] + acc[1][j]) * inv[r];
+            if (m0 + r < S) store_out(out + (size_t)(m0 + r) * ldo, (acc[0][j] + acc[1][j]) * inv[r]);
         }
     }
 }
