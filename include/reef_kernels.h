@@ -439,6 +439,8 @@ enum { REEF_TR_D0 = 0, REEF_TR_D1, REEF_TR_D2, REEF_TR_FLAGS, REEF_TR_NATTR };
  *       one [tokens][3 * hidden] projection.  ldb = 0 (direct kernels, batch 1, offB 0): B is the packed
  *       copy of the weights, [ceil(N/16)][ceil(K/16)][4 slots][16 columns][4 k] floats, zero where a
  *       column or k does not exist; its storage is named as the weights' with "pk" behind it.
+ *       With REEF_GEMM_F_SPLIT it is [ceil(N/16)][ceil(K/32)][3][4 slots][16 columns][8] bf16: three values
+ *       whose sum is the weight, of k = 4 * slot + 0..3 and 16 + 4 * slot + 0..3 ("xpk").
  * tasks = batch * m_tiles * n_tiles.
  *
  * reef_gemm_ntl_<tile> (staged tiles; direct tiles with K a multiple of 8; trans_b = 1, batch 1, flags has REEF_GEMM_F_LN): the product
@@ -457,6 +459,7 @@ enum { REEF_TR_D0 = 0, REEF_TR_D1, REEF_TR_D2, REEF_TR_FLAGS, REEF_TR_NATTR };
 #define REEF_GEMM_F_LN_OUT 4
 #define REEF_GEMM_F_RES 8
 #define REEF_GEMM_F_PAIR_FOLD 16
+#define REEF_GEMM_F_SPLIT 32      /* with ldb = 0, tiles from 32x32 on: B is the split copy */
 /* K split across workgroups (reef_gemm_ntd_<tile>, batch 1; attrs split_k > 1, k_chunk a multiple
  * of 128): tasks = split_k * m_tiles * n_tiles, the split_k workgroups of a tile neighbours in
  * the task order.  The partial tiles meet inside the launch as those of the direct convolutions

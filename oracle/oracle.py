@@ -443,7 +443,7 @@ class GraphOracle:
                 wname = names[k["args"][1]]
             if ldb == 0:                                      # packed copy: the weights as the reference has them are kept
                 assert wname.endswith("pk"), wname            # under its name without "pk"
-                wname, ldb = wname[:-2], K
+                wname, ldb = wname[:-3] if wname.endswith("xpk") else wname[:-2], K     # ("xpk": the split copy)
                 if not flags & 2:
                     B = self.storage[names.index(wname)]
             p = 3 + (flags & 1)

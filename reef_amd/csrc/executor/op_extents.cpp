@@ -261,11 +261,12 @@ void gemm(const std::string& symbol, const Attrs& a, Needs& n) {
     if (a[REEF_GEMM_LDB] == 0) {
         // packed weights: the tiles that have the form: the direct ones
         static const char* const kDirect[] = {"_16x16k4", "_16x32k4", "_32x32d4", "_32x48d4", "_48x48d4", "_64x64d4"};
+        const bool split = fl & REEF_GEMM_F_SPLIT;
         bool ok = false;
-        for (const char* t : kDirect)
-            ok = ok || symbol == std::string("reef_gemm_ntd") + t || symbol == std::string("reef_gemm_ntl") + t;
+        for (int t = split ? 2 : 0; t < 6; ++t)      // (of 16 rows only as 32-bit values)
+            ok = ok || symbol == std::string("reef_gemm_ntd") + kDirect[t] || symbol == std::string("reef_gemm_ntl") + kDirect[t];
         if (!ok || !trans_b || b1 != 0 || a[REEF_GEMM_OFF_B] != 0) { n.bad = "packed weights: only the direct kernels take them, without a batch and an offset"; return; }
-        n.f32("packed B", cdiv(N, 16) * cdiv(K, 16) * 256);
+        n.f32("packed B", split ? cdiv(N, 16) * cdiv(K, 32) * 768 : cdiv(N, 16) * cdiv(K, 16) * 256);
     } else if (trans_b) n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (N - 1) * a[REEF_GEMM_LDB] + K);
     else n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (K - 1) * a[REEF_GEMM_LDB] + N);
     n.f32("C", a[REEF_GEMM_OFF_C] + b1 * a[REEF_GEMM_STRIDE_C] + (M - 1) * a[REEF_GEMM_LDC] + N);

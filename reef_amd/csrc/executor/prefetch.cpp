@@ -44,7 +44,8 @@ Weights weights_of(const KernelInfo& k, int op) {
             w.slot = 1;
             w.chunks = (uint32_t)std::max(attr(k, REEF_GEMM_N_TILES), 1);    // column tile j on XCD j mod 8
             w.interleaved = w.chunks % 8 == 0;
-            if (!w.interleaved) w.chunks = 1;                                // every XCD sees all of them
+            if (!w.interleaved && !(attr(k, REEF_GEMM_FLAGS) & REEF_GEMM_F_SPLIT)) w.chunks = 1;      // every XCD sees all of them
+            // (split weights: in contiguous runs then)
             break;
         case REEF_OP_DENSE:
             w.slot = 1;

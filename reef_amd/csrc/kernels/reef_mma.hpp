@@ -740,6 +740,60 @@ __device__ __forceinline__ bool conv2d_body(const OpDesc& d_in, int task, char* 
     }
 }
 
+// ---- products of 32-bit values on the bf16 matrix cores ------------------------------------------------------
+// A 32-bit value is the sum of three bf16 values exactly: h rounded to nearest, m the first eight bits of what is left
+// (cut off), l the rest, at most eight bits.  A product is h h + (h m + m h) + (m m + h l + l h); the terms left
+// out are 2^-24 of it and of either sign.  The matrix cores multiply bf16 16 times as fast as 32 bits (16x16x32 in 16
+// cycles, 16x16x4 in 32), so the six products of a tile take 96 cycles where 32-bit ones take 256; and VALU work goes
+// on beside a bf16 MFMA, while a 32-bit one holds it up (an MFMA and three VALU operations: 22 cycles and 51).  The
+// five small products have an accumulator of their own, so that what is rounded into the large one is h h alone, once per
+// 32 values of k and not once per 4: errors against 64 bits are half of those of two 32-bit chains (K = 768, normal: 1.58e-7
+// against 3.51e-7; after a ReLU 1.22e-7 against 2.51e-7; K = 2304: 2.9e-7 against 6.1e-7).
+// What has no such sum -- infinities, NaN, values that round to infinity -- makes every product it is in infinite or
+// NaN; the kernels form an element that comes out so again, in 32 bits.  (Below 2^-110 l falls under the smallest bf16:
+// such values keep 2^-133 absolute.)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+struct Planes { u32x4 h, m, l; };      // eight values
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+    bf16x2 r;
+    r[0] = (__bf16)a;
+    r[1] = (__bf16)b;
+    h = __builtin_bit_cast(unsigned, r);
+    // (v_dot2_f32_bf16 would take a half of h from a in one operation, but waits for the matrix cores: 33 cycles behind an MFMA)
+    a -= __uint_as_float(h << 16);
+    b -= __uint_as_float(h & 0xFFFF0000u);
+    m = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+    a -= __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+    b -= __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
+    l = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ Planes split_planes(const f32x4& a, const f32x4& b) {
+    Planes p;
+    unsigned h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const f32x4& v = i < 2 ? a : b;
+        split_pair(v[2 * (i & 1)], v[2 * (i & 1) + 1], h, m, l);
+        p.h[i] = h;
+        p.m[i] = m;
+        p.l[i] = l;
+    }
+    return p;
+}
+__device__ __forceinline__ void mma_bf16(const u32x4& a, const u32x4& b, f32x4& c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ void mma_split(const Planes& a, const Planes& b, f32x4& main, f32x4& rest) {
+    mma_bf16(a.m, b.m, rest);
+    mma_bf16(a.h, b.l, rest);
+    mma_bf16(a.l, b.h, rest);
+    mma_bf16(a.h, b.h, main);
+    mma_bf16(a.h, b.m, rest);
+    mma_bf16(a.m, b.h, rest);
+}
+
 // ---- reef_conv2d_d<R>: operands straight from memory into the matrix cores ----------------
 // A batch-1 layer is latency bound: every weight is used once per inference, so each K step of
 // the tiled kernels above waits a full memory round trip (global -> registers -> LDS -> barrier).
@@ -2852,7 +2906,7 @@ __device__ __forceinline__ bool gemm_body(const OpDesc& d, int task, char* smem_
 // staged tiles.  A lane adds what it loads of a row to sums of (a - p) and (a - p)^2 around a pivot p
 // (element 0 of the row); the sixteen lanes that share a row -- four k slots, four wavefronts -- meet in LDS.
 //
-// Tiles of more than four sub-tiles (32x48, 48x48, 64x64) load four k values per lane and step instead of
+// Unpacked, tiles of more than four sub-tiles (32x48, 48x48, 64x64) load four k values per lane and step instead of
 // eight and keep one accumulator per sub-tile.  A CU's loads are what bounds these products (384 x 2304 x 768
 // on 32x32: 170 MB out of L2, 6.3 TB/s), and they go with (BM + BN) / (BM BN): 64x64 22.0 -> 17.9 us there,
 // 32x48 12.1 -> 10.2 at 128 x 2304 x 768, 48x48 27.4 -> 22.4 at 384 x 3072 x 768.
@@ -2861,9 +2915,286 @@ __device__ __forceinline__ bool gemm_body(const OpDesc& d, int task, char* smem_
 // [4 k], whose loads are contiguous KiBs, and the rows of A are loaded as 16-byte pieces (lane / 4 = row) and turned in
 // LDS as the input of conv2d_v1_body is: 20 and 23 to 31 cycles of the vector-memory pipe a KiB instead of 64.  BERT-base at
 // 128 tokens, six layers, 331 -> 305 us of device time a pass; at 384, four layers, 439 -> 402.
+template <int TM, int TN>
+struct TileGd {      // a wavefront's place: its partial tile, the sums of its rows, pivots, flags
+    static constexpr int WSTRIDE = TM * TN * 320 + 3 * 16 * TM + 4;
+};
+// What a thread holds for the elements of C it writes (element (h, g): row 16 h + t / 16, column 16 g + t % 16 of the
+// tile), and what the product's LayerNorm needs.
+template <int TM, int TN, bool LN>
+struct GemmTail {
+    typedef TileD16<TN, TM> TD;
+    rsrc_t rs_a, rs_c;
+    unsigned ooff[TM][TN];
+    float e_bias[TN], e_res[TM][TN];
+    float pivot[LN ? TM : 1], ls1[LN ? TM : 1], ls2[LN ? TM : 1], e_c1[LN ? TN : 1], e_c2[LN ? TN : 1];
+    LnOut ln_out;
+    int M, N, K, lda, m0, n0, nt, rem, split, split_k, k_lo, k_hi;
+    bool has_bias, has_res;
+
+    // Tile and share of K of this workgroup.  CHUNKED: where the column tiles are no multiple of the XCDs, so that in row-major
+    // order every XCD would read all weights, they are dealt out in contiguous runs, the row tiles of one fastest (32x48,
+    // 448 x 4096 x 1024: 51.9 -> 29.7 us a launch).
+    template <bool CHUNKED>
+    __device__ __forceinline__ void place(const OpDesc& d, int task) {
+        const int* a = d.attr;
+        M = a[REEF_GEMM_M];
+        N = a[REEF_GEMM_N];
+        K = a[REEF_GEMM_K];
+        lda = a[REEF_GEMM_LDA];
+        const int n_tiles = a[REEF_GEMM_N_TILES], tiles = a[REEF_GEMM_M_TILES] * n_tiles;
+        // K split across workgroups (batch 1): the split_k workgroups of a tile are neighbours in the task order
+        split_k = !LN && a[REEF_GEMM_SPLIT_K] > 1 ? a[REEF_GEMM_SPLIT_K] : 1;
+        int mt, b = 0;
+        if (CHUNKED && (n_tiles & 7)) {
+            const int m_tiles = a[REEF_GEMM_M_TILES], id = xcd_chunked(task, tiles * split_k), q = div_small(id, m_tiles);
+            mt = id - q * m_tiles;
+            nt = split_k > 1 ? div_small(q, split_k) : q;
+            split = q - nt * split_k;
+            rem = mt * n_tiles + nt;
+        } else {
+            const int tile_task = split_k > 1 ? div_small(task, split_k) : task;
+            split = task - tile_task * split_k;
+            b = div_small(tile_task, tiles);
+            rem = tile_task - b * tiles;
+            mt = div_small(rem, n_tiles);
+            nt = rem - mt * n_tiles;
+        }
+        m0 = mt * TD::BM;
+        n0 = nt * TD::BN;
+        k_lo = split_k > 1 ? split * a[REEF_GEMM_K_CHUNK] : 0;
+        k_hi = split_k > 1 ? min(K, k_lo + a[REEF_GEMM_K_CHUNK]) : K;
+        batch = b;
+        rs_a = make_rsrc((const float*)d.ptr[0] + a[REEF_GEMM_OFF_A] + (size_t)b * a[REEF_GEMM_STRIDE_A],
+                         ((unsigned)(M - 1) * (unsigned)lda + (unsigned)K) * 4u);
+    }
+    // LN: the pivots of this lane's rows of A, for the sums.
+    __device__ __forceinline__ void fetch_pivots() {
+        if (!LN) return;
+#pragma unroll
+        for (int h = 0; h < TM; ++h) {
+            pivot[LN ? h : 0] = buf_load(rs_a, (unsigned)(m0 + 16 * h + (threadIdx.x & 15)) * (unsigned)lda * 4u);
+            ls1[LN ? h : 0] = ls2[LN ? h : 0] = 0.0f;
+        }
+    }
+    // Bias, residual and the LayerNorm's operands.
+    __device__ __forceinline__ void fetch(const OpDesc& d) {
+        const int* a = d.attr;
+        const unsigned ldc = (unsigned)a[REEF_GEMM_LDC];
+        const size_t at_c = (size_t)a[REEF_GEMM_OFF_C] + (size_t)batch * a[REEF_GEMM_STRIDE_C];
+        rs_c = make_rsrc((const float*)d.ptr[2] + at_c, ((unsigned)(M - 1) * ldc + (unsigned)N) * 4u);
+        has_bias = a[REEF_GEMM_FLAGS] & REEF_GEMM_F_BIAS;
+        has_res = a[REEF_GEMM_FLAGS] & REEF_GEMM_F_RES;
+        const rsrc_t rs_bias = make_rsrc(d.ptr[has_bias ? 3 : 2], (unsigned)N * 4u);
+        // the residual is laid out as C is; without one an empty buffer, whose loads give 0
+        const rsrc_t rs_res = make_rsrc((const float*)d.ptr[has_res ? (has_bias ? 4 : 3) : 2] + at_c,
+                                        has_res ? ((unsigned)(M - 1) * ldc + (unsigned)N) * 4u : 0u);
+        const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
+        const int lnp = 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0);
+        if (LN) {      // c1 and c2 of this thread's columns
+            const rsrc_t rs_c1 = make_rsrc(d.ptr[lnp], (unsigned)N * 4u), rs_c2 = make_rsrc(d.ptr[lnp + 1], (unsigned)N * 4u);
+#pragma unroll
+            for (int g = 0; g < TN; ++g) {
+                const unsigned n4 = (unsigned)(n0 + 16 * g + ocol) * 4u;
+                e_c1[LN ? g : 0] = buf_load(rs_c1, n4);
+                e_c2[LN ? g : 0] = buf_load(rs_c2, n4);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+            const unsigned n = (unsigned)(n0 + 16 * g + ocol);
+            e_bias[g] = has_bias ? buf_load(rs_bias, n * 4u) : 0.0f;
+#pragma unroll
+            for (int h = 0; h < TM; ++h) {
+                const unsigned m = (unsigned)(m0 + 16 * h + orow);
+                ooff[h][g] = n < (unsigned)N ? (m * ldc + n) * 4u : kOutside;
+                e_res[h][g] = buf_load(rs_res, ooff[h][g]);
+            }
+        }
+        if (LN) ln_out.init(d, lnp, (const float*)d.ptr[0], M, K, lda, m0, TD::BM, nt, a[REEF_GEMM_N_TILES]);
+    }
+    // `count` values of row 16 h + lane % 16 of A into the row's sums; in: 1, or 0 for values outside K, which read as 0.
+    template <class V>
+    __device__ __forceinline__ void ln_add(int h, const V& v, int count, float in) {
+        const float pv = pivot[LN ? h : 0] * in;
+#pragma unroll
+        for (int q = 0; q < count; ++q) {
+            const float dl = v[q] - pv;
+            ls1[LN ? h : 0] += dl;
+            ls2[LN ? h : 0] = fmaf(dl, dl, ls2[LN ? h : 0]);
+        }
+    }
+    // From the wavefronts' partial tiles to C.  WSTRIDE: floats between the wavefronts' places in LDS.  again(m, n): the element's sum over [k_lo, k_hi) in
+    // 32 bits, for one that came out of split operands as infinite or NaN.  False: the workgroup leaves a preempted launch.
+    template <int WSTRIDE, bool AGAIN, class Poll, class Again>
+    __device__ __forceinline__ bool finish(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN], const Poll& poll, bool stop,
+                                           const Again& again) {
+        float* smem = (float*)smem_raw;
+        const int* a = d.attr;
+        const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4, orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
+        float* sums = smem + TD::SUBS * TD::PART;              // LN: [row][2] in every wavefront's place, pivots [row] behind the first's
+        int* sflag = (int*)(sums + (LN ? 3 * TD::BM : 0));      // one in every place; in the first's a second
+        if (LN) {
+#pragma unroll
+            for (int h = 0; h < TM; ++h) {
+                float t1 = ls1[LN ? h : 0], t2 = ls2[LN ? h : 0];
+                t1 += __shfl_xor(t1, 16, 64);
+                t2 += __shfl_xor(t2, 16, 64);
+                t1 += __shfl_xor(t1, 32, 64);
+                t2 += __shfl_xor(t2, 32, 64);
+                if (kq == 0) {
+                    const int r = 16 * h + i16;
+                    sums[wave * WSTRIDE + r * 2] = t1;
+                    sums[wave * WSTRIDE + r * 2 + 1] = t2;
+                    if (wave == 0) sums[2 * TD::BM + r] = pivot[LN ? h : 0];
+                }
+            }
+        }
+        float* part = smem + wave * WSTRIDE;
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] = acc[h][g][j];
+        if (Poll::enabled && lane == 0) sflag[wave * WSTRIDE] = stop;
+        __syncthreads();
+        if (Poll::enabled && (sflag[0] | sflag[WSTRIDE] | sflag[2 * WSTRIDE] | sflag[3 * WSTRIDE])) return false;
+        const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
+        const float alpha = __int_as_float(a[REEF_GEMM_ALPHA_BITS]);
+        const int act = a[REEF_GEMM_ACT];
+        auto row_stats = [&](int r, float& mu, float& rs) {
+            float t1 = 0.0f, t2 = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                t1 += sums[w * WSTRIDE + r * 2];
+                t2 += sums[w * WSTRIDE + r * 2 + 1];
+            }
+            const float m1 = t1 / (float)K;                    // mean of a - pivot
+            mu = sums[2 * TD::BM + r] + m1;
+            rs = 1.0f / sqrtf(fmaxf(t2 / (float)K - m1 * m1, 0.0f) + __int_as_float(a[REEF_GEMM_LN_EPS_BITS]));
+        };
+        float e_mu[LN ? TM : 1], e_rs[LN ? TM : 1];
+        if (LN) {
+#pragma unroll
+            for (int h = 0; h < TM; ++h) row_stats(16 * h + orow, e_mu[LN ? h : 0], e_rs[LN ? h : 0]);
+            ln_out.write(row_stats);
+        }
+        auto store = [&](float sum, int h, int g) {
+            if (LN) sum = e_rs[LN ? h : 0] * (sum - e_mu[LN ? h : 0] * e_c1[LN ? g : 0]) + e_c2[LN ? g : 0];
+            float v = sum * alpha + e_bias[g];
+            if (act == REEF_ACT_RELU) v = fmaxf(v, 0.0f);
+            else if (act == REEF_ACT_GELU) v = gelu_erf(v);
+            buf_store(rs_c, ooff[h][g], v + e_res[h][g]);
+        };
+        float v[TM][TN];
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) {
+                const float* e = mine + (h * TN + g) * TD::PART;
+                v[h][g] = ((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE];
+            }
+        if (AGAIN) {
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g)
+                    if (!__builtin_isfinite(v[h][g]) && m0 + 16 * h + orow < M && n0 + 16 * g + ocol < N)
+                        v[h][g] = again(m0 + 16 * h + orow, n0 + 16 * g + ocol);
+        }
+        if (split_k == 1) {
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) store(v[h][g], h, g);
+            return true;
+        }
+
+        // The split_k partial tiles of an output tile meet inside the launch, as those of the direct
+        // convolutions do: a split of two through one exchange per element where every launch on the
+        // buffers runs to completion, otherwise partial tiles to the workspace, a count per tile,
+        // and the last arrival sums them in split order.  The sums and their order are the same.
+        // ptr: .., workspace (split_k [+1] regions of M x N), arrival counters.
+        const int aux = 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0);
+        const size_t MN = (size_t)M * N;
+        float* ws = (float*)d.ptr[aux];
+        unsigned widx[TM][TN];         // element m * N + n of a dense M x N region, ~0u outside the matrix
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) {
+                const unsigned m = (unsigned)(m0 + 16 * h + orow), n = (unsigned)(n0 + 16 * g + ocol);
+                widx[h][g] = (m < (unsigned)M && n < (unsigned)N) ? m * (unsigned)N + n : ~0u;
+            }
+        if (split_k == 2 && (a[REEF_GEMM_FLAGS] & REEF_GEMM_F_PAIR_FOLD) && poll.pair_fold_ok()) {
+            // a value is parked with its sign bit flipped, so a parked value is never the empty slot's 0
+            unsigned* slots = (unsigned*)(ws + 2 * MN);
+            unsigned got[TM][TN];
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) {
+                    got[h][g] = 0;
+                    if (widx[h][g] != ~0u) {
+                        unsigned parked = __float_as_uint(v[h][g]) ^ 0x80000000u;
+                        parked = parked ? parked : 0x80000000u;
+                        got[h][g] = __hip_atomic_exchange(&slots[widx[h][g]], parked, __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g)
+                    if (got[h][g] != 0) {   // second to arrive: the other half is here
+                        const float other = __uint_as_float(got[h][g] ^ 0x80000000u);
+                        store(split == 0 ? v[h][g] + other : other + v[h][g], h, g);   // split order
+                        __hip_atomic_store(&slots[widx[h][g]], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+            return true;
+        }
+        int* counters = (int*)d.ptr[aux + 1] + a[REEF_GEMM_SYNC_OFF];
+        int* s_last = sflag + 1;
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+                if (widx[h][g] != ~0u) store_agent(ws + (size_t)split * MN + widx[h][g], v[h][g]);
+        partial_stores_done();   // every store of this workgroup is acknowledged before it counts in
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int old = __hip_atomic_fetch_add(&counters[rem], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *s_last = (old == split_k - 1);
+        }
+        __syncthreads();
+        if (!*s_last) return true;
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+                if (widx[h][g] != ~0u) {
+                    const float* src = ws + widx[h][g];
+                    float sum = 0.0f;
+                    for (int s0 = 0; s0 < split_k; s0 += 4) {
+                        float p[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) p[j] = load_agent(src + (size_t)min(s0 + j, split_k - 1) * MN);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if (s0 + j < split_k) sum = (s0 + j == 0) ? p[j] : sum + p[j];
+                    }
+                    store(sum, h, g);
+                }
+        if (threadIdx.x == 0)  // ready for the next run
+            __hip_atomic_store(&counters[rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    }
+    int batch;
+};
+
 template <int TM, int TN, bool LN, bool PK, class Poll>
-__device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, char* smem_raw,
-                                                   const Poll& poll) {
+__device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
     typedef TileD16<TN, TM> TD;
     constexpr bool BIG = TM * TN > 4 || PK;
     constexpr int KL = BIG ? 4 : 8;        // k values per lane and step
@@ -2877,90 +3208,33 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     constexpr int AC = TM * TN > 4 ? 1 : PK && !LN && TM * TN == 1 ? 4 : 2;
     // steps of loads in flight (unpacked, 6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
     constexpr int NS = PK ? 4 : 3;
-    float* smem = (float*)smem_raw;
-    int* sflag = (int*)(smem + 4 * TD::SUBS * TD::PART);
-    const int* a = d.attr;
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int M = a[REEF_GEMM_M], N = a[REEF_GEMM_N], K = a[REEF_GEMM_K];
-    const int n_tiles = a[REEF_GEMM_N_TILES];
-    const int tiles = a[REEF_GEMM_M_TILES] * n_tiles;
-    // K split across workgroups (batch 1): the split_k workgroups of a tile are neighbours in the task order
-    const int split_k = !LN && a[REEF_GEMM_SPLIT_K] > 1 ? a[REEF_GEMM_SPLIT_K] : 1;
-    const int tile_task = split_k > 1 ? div_small(task, split_k) : task;
-    const int split = task - tile_task * split_k;
-    const int b = div_small(tile_task, tiles);
-    const int rem = tile_task - b * tiles;
-    const int mt = div_small(rem, n_tiles), nt = rem - mt * n_tiles;
-    const int m0 = mt * TD::BM, n0 = nt * TD::BN;
-    const unsigned lda = (unsigned)a[REEF_GEMM_LDA], ldb = (unsigned)a[REEF_GEMM_LDB],
-                   ldc = (unsigned)a[REEF_GEMM_LDC];
-    const rsrc_t rs_a = make_rsrc((const float*)d.ptr[0] + a[REEF_GEMM_OFF_A] + (size_t)b * a[REEF_GEMM_STRIDE_A],
-                                  ((unsigned)(M - 1) * lda + (unsigned)K) * 4u);
-    const rsrc_t rs_b = make_rsrc((const float*)d.ptr[1] + a[REEF_GEMM_OFF_B] + (size_t)b * a[REEF_GEMM_STRIDE_B],
-                                  ((unsigned)(N - 1) * ldb + (unsigned)K) * 4u);
-    const rsrc_t rs_c = make_rsrc((const float*)d.ptr[2] + a[REEF_GEMM_OFF_C] + (size_t)b * a[REEF_GEMM_STRIDE_C],
-                                  ((unsigned)(M - 1) * ldc + (unsigned)N) * 4u);
-    const bool has_bias = a[REEF_GEMM_FLAGS] & REEF_GEMM_F_BIAS, has_res = a[REEF_GEMM_FLAGS] & REEF_GEMM_F_RES;
-    const rsrc_t rs_bias = make_rsrc(d.ptr[has_bias ? 3 : 2], (unsigned)N * 4u);
-    // the residual is laid out as C is; without one an empty buffer, whose loads give 0
-    const rsrc_t rs_res = make_rsrc((const float*)d.ptr[has_res ? (has_bias ? 4 : 3) : 2] + a[REEF_GEMM_OFF_C] +
-                                        (size_t)b * a[REEF_GEMM_STRIDE_C],
-                                    has_res ? ((unsigned)(M - 1) * ldc + (unsigned)N) * 4u : 0u);
-
-    // the outputs of this thread and their bias, ahead of the K loop
-    const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
-    unsigned ooff[TM][TN];
-    float e_bias[TN], e_res[TM][TN];
-#pragma unroll
-    for (int g = 0; g < TN; ++g) {
-        const unsigned n = (unsigned)(n0 + 16 * g + ocol);
-        e_bias[g] = has_bias ? buf_load(rs_bias, n * 4u) : 0.0f;
-#pragma unroll
-        for (int h = 0; h < TM; ++h) {
-            const unsigned m = (unsigned)(m0 + 16 * h + orow);
-            ooff[h][g] = n < (unsigned)N ? (m * ldc + n) * 4u : kOutside;
-            e_res[h][g] = buf_load(rs_res, ooff[h][g]);
-        }
-    }
-
-    // LN: the pivots of this lane's rows of A (for the sums) and of its output rows, c1 and c2 of its columns
-    const int lnp = 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0);
-    LnOut ln_out;
-    float pivot[LN ? TM : 1], ls1[LN ? TM : 1], ls2[LN ? TM : 1], e_c1[LN ? TN : 1], e_c2[LN ? TN : 1];
-    if (LN) {
-        const rsrc_t rs_c1 = make_rsrc(d.ptr[lnp], (unsigned)N * 4u), rs_c2 = make_rsrc(d.ptr[lnp + 1], (unsigned)N * 4u);
-#pragma unroll
-        for (int h = 0; h < TM; ++h) {
-            pivot[LN ? h : 0] = buf_load(rs_a, (unsigned)(m0 + 16 * h + i16) * lda * 4u);
-            ls1[LN ? h : 0] = ls2[LN ? h : 0] = 0.0f;
-        }
-#pragma unroll
-        for (int g = 0; g < TN; ++g) {
-            const unsigned n4 = (unsigned)(n0 + 16 * g + ocol) * 4u;
-            e_c1[LN ? g : 0] = buf_load(rs_c1, n4);
-            e_c2[LN ? g : 0] = buf_load(rs_c2, n4);
-        }
-        ln_out.init(d, lnp, (const float*)d.ptr[0], M, K, (int)lda, m0, TD::BM, nt, n_tiles);
-    }
-    const int k_lo = split_k > 1 ? split * a[REEF_GEMM_K_CHUNK] : 0;        // this workgroup's part of K
-    const int k_hi = split_k > 1 ? min(K, k_lo + a[REEF_GEMM_K_CHUNK]) : K;
-    const int lane_k = k_lo + (wave * 4 + kq) * KL;  // first k of this lane's slot
-    const int nsteps = (k_hi - k_lo + KSTEP - 1) / KSTEP;
-    const int lane_steps = lane_k < k_hi ? (k_hi - lane_k + KSTEP - 1) / KSTEP : 0;
+    GemmTail<TM, TN, LN> t;
+    t.template place<false>(d, task);
+    t.fetch_pivots();
+    t.fetch(d);
+    const int* a = d.attr;
+    const unsigned ldb = (unsigned)a[REEF_GEMM_LDB];
+    const rsrc_t rs_b = make_rsrc((const float*)d.ptr[1] + a[REEF_GEMM_OFF_B] + (size_t)t.batch * a[REEF_GEMM_STRIDE_B],
+                                  ((unsigned)(t.N - 1) * ldb + (unsigned)t.K) * 4u);
+    const int lane_k = t.k_lo + (wave * 4 + kq) * KL;  // first k of this lane's slot
+    const int nsteps = (t.k_hi - t.k_lo + KSTEP - 1) / KSTEP;
+    const int lane_steps = lane_k < t.k_hi ? (t.k_hi - lane_k + KSTEP - 1) / KSTEP : 0;
     unsigned va[TM], vb[TN];
-    const int row0 = lane >> 2, ld_k = k_lo + wave * 16 + (lane & 3) * 4;      // PK: row and first k of this lane's piece of A
-    const int ld_steps = ld_k < k_hi ? (k_hi - ld_k + KSTEP - 1) / KSTEP : 0;
-    const unsigned K16 = (unsigned)(K + 15) / 16u;
-    const rsrc_t rs_bp = make_rsrc(d.ptr[1], PK ? (unsigned)((N + 15) / 16) * K16 * 1024u : 0u);
+    const int row0 = lane >> 2, ld_k = t.k_lo + wave * 16 + (lane & 3) * 4;      // PK: row and first k of this lane's piece of A
+    const int ld_steps = ld_k < t.k_hi ? (t.k_hi - ld_k + KSTEP - 1) / KSTEP : 0;
+    const unsigned K16 = (unsigned)(t.K + 15) / 16u;
+    const rsrc_t rs_bp = make_rsrc(d.ptr[1], PK ? (unsigned)((t.N + 15) / 16) * K16 * 1024u : 0u);
 #pragma unroll
     for (int h = 0; h < TM; ++h)
-        va[h] = PK ? ((unsigned)(m0 + 16 * h + row0) * lda + (unsigned)ld_k) * 4u : ((unsigned)(m0 + 16 * h + i16) * lda + (unsigned)lane_k) * 4u;
+        va[h] = PK ? ((unsigned)(t.m0 + 16 * h + row0) * (unsigned)t.lda + (unsigned)ld_k) * 4u
+                   : ((unsigned)(t.m0 + 16 * h + i16) * (unsigned)t.lda + (unsigned)lane_k) * 4u;
 #pragma unroll
     for (int g = 0; g < TN; ++g)
-        vb[g] = PK ? ((unsigned)(n0 / 16 + g) * K16 + (unsigned)(k_lo / 16 + wave)) * 1024u + (unsigned)lane * 16u
-                   : ((unsigned)(n0 + 16 * g + i16) * ldb + (unsigned)lane_k) * 4u;
+        vb[g] = PK ? ((unsigned)(t.n0 / 16 + g) * K16 + (unsigned)(t.k_lo / 16 + wave)) * 1024u + (unsigned)lane * 16u
+                   : ((unsigned)(t.n0 + 16 * g + i16) * ldb + (unsigned)lane_k) * 4u;
 
     float ra[NS][TM][KL], rb[NS][TN][KL];
     auto load_slot = [&](float (&dst)[KL], rsrc_t rs, unsigned off, unsigned soff) {
@@ -2981,13 +3255,13 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
                 vb[g] += 4096u;
             }
 #pragma unroll
-            for (int h = 0; h < TM; ++h) load_slot(ra[s][h], rs_a, va[h] | outp, (unsigned)step * 256u);
+            for (int h = 0; h < TM; ++h) load_slot(ra[s][h], t.rs_a, va[h] | outp, (unsigned)step * 256u);
             return;
         }
         const unsigned outm = step < lane_steps ? 0u : kOutside;
         const unsigned so = (unsigned)step * (unsigned)KSTEP * 4u;   // uniform
 #pragma unroll
-        for (int h = 0; h < TM; ++h) load_slot(ra[s][h], rs_a, va[h] | outm, so);
+        for (int h = 0; h < TM; ++h) load_slot(ra[s][h], t.rs_a, va[h] | outm, so);
 #pragma unroll
         for (int g = 0; g < TN; ++g) load_slot(rb[s][g], rs_b, vb[g] | outm, so);
     };
@@ -3006,7 +3280,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
         }
     // PK: the rows of A through LDS, one step ahead of the MFMAs: row r at 16 r, its piece p at p ^ (r / 4), so that the
     // sixteen lanes of a k slot read different banks; where this wavefront's partial tile goes afterwards
-    float* blk = smem + wave * (TD::SUBS * TD::PART);
+    float* blk = (float*)smem_raw + wave * TileGd<TM, TN>::WSTRIDE;
     float* wr = blk + row0 * 16 + ((lane & 3) ^ (row0 >> 2)) * 4;
     const float* rd = blk + i16 * 16 + (kq ^ (i16 >> 2)) * 4;
     f32x4 at[PK ? 2 : 1][TM];
@@ -3027,17 +3301,9 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
                 for (int q = 0; q < 4; ++q) ra[s][h][q] = at[PK ? s & 1 : 0][h][q];
         }
         if (LN) {
-            const float in = ln_step++ < lane_steps ? 1.0f : 0.0f;     // values outside K were loaded as zeros: 0 - 0
+            const float in = ln_step++ < lane_steps ? 1.0f : 0.0f;
 #pragma unroll
-            for (int h = 0; h < TM; ++h) {
-                const float pv = pivot[LN ? h : 0] * in;
-#pragma unroll
-                for (int q = 0; q < KL; ++q) {
-                    const float dl = ra[s][h][q] - pv;
-                    ls1[LN ? h : 0] += dl;
-                    ls2[LN ? h : 0] = fmaf(dl, dl, ls2[LN ? h : 0]);
-                }
-            }
+            for (int h = 0; h < TM; ++h) t.ln_add(h, ra[s][h], KL, in);
         }
 #pragma unroll
         for (int q = 0; q < KL; ++q)
@@ -3051,7 +3317,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     int pf = raised, it = 0;
     bool left = false;
     // this wavefront's own steps where their loads are its own
-    const int steps = PK ? (k_lo + 16 * wave < k_hi ? (k_hi - k_lo - 16 * wave + KSTEP - 1) / KSTEP : 0) : nsteps;
+    const int steps = PK ? (t.k_lo + 16 * wave < t.k_hi ? (t.k_hi - t.k_lo - 16 * wave + KSTEP - 1) / KSTEP : 0) : nsteps;
     if (PK && steps > 0) turn(0, 0);
     // (groups whose refills all exist, then the last whole group with the refills the remaining steps
     // need and no others, as in the convolution)
@@ -3096,166 +3362,180 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
                 mma_stage(s);
             }
     }
+    f32x4 sum[TM][TN];
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g)
+            sum[h][g] = AC == 1   ? acc[h][g][0]
+                        : AC == 2 ? acc[h][g][0] + acc[h][g][AC - 1]
+                                  : (acc[h][g][0] + acc[h][g][AC > 2 ? 1 : 0]) + (acc[h][g][AC > 2 ? 2 : 0] + acc[h][g][AC > 3 ? 3 : 0]);
+    return t.template finish<TileGd<TM, TN>::WSTRIDE, false>(d, smem_raw, wave, sum, poll, left || raised, [](int, int) { return 0.0f; });
+}
 
-    float* sums = smem + 4 * TD::SUBS * TD::PART + 4;      // LN: [wavefront][row][2], then the pivots [row]
-    if (LN) {
+// REEF_GEMM_F_SPLIT: B is stored as the three bf16 parts of each weight, and the parts of A are formed behind its turn through
+// LDS, a step of 32 values of k a wavefront ahead of the 16x16x32 products.  32-bit MFMAs bound these tiles before (32x48:
+// 1536 cycles of them a step of 2000); now a CU's loads do, weights being half as large again (13 KiB a wavefront and step
+// at 20 to 22 cycles a KiB and CU: 1090 of 1150).  Splitting the weights here as well, five or six VALU operations a value,
+// costs more than that load, and a 16-row tile shares a split row with too few columns: those stay in 32 bits (a split
+// ntd_16x32 11.8 us against 10.6 at 128 x 768 x 3072).  Two workgroups a CU (256 registers) are worth more than a wider tile:
+// us a launch, 32 bits and this, LayerNorm in front of the first two,
+//   128 x 2304 x 768 10.8 -> 9.5, 128 x 3072 x 768 12.0 -> 10.6, 128 x 768 x 3072 in four 13.3 -> 12.2,
+//   256 x 2304 x 768 16.4 -> 12.9, 256 x 768 x 3072 16.5 -> 13.1, 384 x 768 x 768 8.5 -> 7.4, 512 x 3072 x 768 29.7 -> 25.0.
+// BERT-base at 128 tokens, six layers, best effort: 340 -> 321 us a request; at 384, four layers: 447 -> 422.
+// Distance of the outputs from 64 bits: 3.7e-7 -> 2.4e-7 and 3.6e-7 -> 2.1e-7.
+template <int TM, int TN, bool LN, class Poll>
+__device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
+    constexpr int KSTEP = 128;                               // k values of a step, 32 a wavefront: one split product
+    constexpr int NS = 2;                                    // steps of loads in flight: what 256 registers hold
+    typedef TileD16<TN, TM> TD;
+    static_assert(TM * 512 <= TD::SUBS * TD::PART, "the turned rows fit where the partial tile goes");
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
+    const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    GemmTail<TM, TN, LN> t;
+    t.template place<true>(d, task);
+    t.fetch_pivots();
+    // what the epilogue needs, ahead of the K loop, unless registers run out for it
+    constexpr bool LATE = LN && TM * TN >= 16 && REEF_FLAVOUR == 2;
+    if (!LATE) t.fetch(d);
+    const int k0 = t.k_lo + 32 * wave;                                                   // first k of this wavefront
+    const int steps = k0 < t.k_hi ? (t.k_hi - k0 + KSTEP - 1) / KSTEP : 0;               // its steps (uniform)
+    const unsigned K32 = (unsigned)(t.K + 31) / 32u;
+    const rsrc_t rs_b = make_rsrc(d.ptr[1], (unsigned)((t.N + 15) / 16) * K32 * 3072u);
+    unsigned vb[TN];
+#pragma unroll
+    for (int g = 0; g < TN; ++g) vb[g] = ((unsigned)(t.n0 / 16 + g) * K32 + (unsigned)(k0 / 32)) * 3072u + (unsigned)lane * 16u;
+    // A: a load is eight rows of 128 bytes; piece p of row r goes to place p ^ (r % 8) of a row of 32 floats in LDS, so that
+    // the sixteen lanes of a k slot read different banks.  This lane's row and first k, and its steps that lie inside K.
+    const int row0 = lane >> 3, ld_k = k0 + (lane & 7) * 4;
+    const int ld_steps = ld_k < t.k_hi ? (t.k_hi - ld_k + KSTEP - 1) / KSTEP : 0;
+    unsigned va[2 * TM];
+#pragma unroll
+    for (int j = 0; j < 2 * TM; ++j) va[j] = ((unsigned)(t.m0 + 8 * j + row0) * (unsigned)t.lda + (unsigned)ld_k) * 4u;
+    f32x4 ra[NS][2 * TM];
+    u32x4 rb[NS][TN][3];
+    auto load_step = [&](int s, int step) {
+        const unsigned outp = step < ld_steps ? 0u : kOutside;
+#pragma unroll
+        for (int j = 0; j < 2 * TM; ++j)
+            ra[s][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(t.rs_a, (int)(va[j] | outp), step * 4 * KSTEP, 0));
+#pragma unroll
+        for (int g = 0; g < TN; ++g) {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                rb[s][g][e] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_b, (int)(vb[g] + 1024u * e), 0, 0));
+            vb[g] += 3072u * 4u;
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        load_step(s, s);
+        asm volatile("" ::: "memory");
+    }
+    f32x4 acc[TM][TN][2];
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) acc[h][g][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // the rows of A through LDS, one step ahead of the MFMAs; where this wavefront's partial tile goes afterwards
+    float* blk = (float*)smem_raw + wave * TileGd<TM, TN>::WSTRIDE;
+    float* wr = blk + row0 * 32 + ((lane & 7) ^ row0) * 4;
+    const float* rd0 = blk + i16 * 32 + (kq ^ (i16 & 7)) * 4;
+    const float* rd1 = blk + i16 * 32 + ((kq + 4) ^ (i16 & 7)) * 4;
+    f32x4 av[TM][2];
+    auto turn = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < 2 * TM; ++j) *(f32x4*)(wr + j * 256) = ra[s][j];
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int h = 0; h < TM; ++h) {
-            float t1 = ls1[LN ? h : 0], t2 = ls2[LN ? h : 0];
-            t1 += __shfl_xor(t1, 16, 64);
-            t2 += __shfl_xor(t2, 16, 64);
-            t1 += __shfl_xor(t1, 32, 64);
-            t2 += __shfl_xor(t2, 32, 64);
-            if (kq == 0) {
-                const int r = 16 * h + i16;
-                sums[(wave * TD::BM + r) * 2] = t1;
-                sums[(wave * TD::BM + r) * 2 + 1] = t2;
-                if (wave == 0) sums[4 * TD::BM * 2 + r] = pivot[LN ? h : 0];
+            av[h][0] = *(const f32x4*)(rd0 + h * 512);
+            av[h][1] = *(const f32x4*)(rd1 + h * 512);
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    int ln_k = k0 + 4 * kq;
+    Planes pa[TM];
+    auto split_rows = [&]() {
+        if (LN) {      // values outside K were loaded as zeros: 0 - 0
+            const float in0 = ln_k < t.K ? 1.0f : 0.0f, in1 = ln_k + 16 < t.K ? 1.0f : 0.0f;
+            ln_k += KSTEP;
+#pragma unroll
+            for (int h = 0; h < TM; ++h) {
+                t.ln_add(h, av[h][0], 4, in0);
+                t.ln_add(h, av[h][1], 4, in1);
             }
         }
-    }
-    float* part = smem + wave * (TD::SUBS * TD::PART);
 #pragma unroll
-    for (int h = 0; h < TM; ++h)
-#pragma unroll
-        for (int g = 0; g < TN; ++g)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                part[(h * TN + g) * TD::PART + (5 * kq + j) * 16 + i16] =
-                    AC == 4   ? (acc[h][g][0][j] + acc[h][g][1 % AC][j]) + (acc[h][g][2 % AC][j] + acc[h][g][AC - 1][j])
-                    : AC == 2 ? acc[h][g][0][j] + acc[h][g][AC - 1][j]
-                              : acc[h][g][0][j];
-    if (Poll::enabled && lane == 0) sflag[wave] = left || raised;
-    __syncthreads();
-    if (Poll::enabled && (sflag[0] | sflag[1] | sflag[2] | sflag[3])) return false;
-    const float* mine = smem + threadIdx.x + (threadIdx.x >> 6) * 16;
-    constexpr int WSTRIDE = TD::SUBS * TD::PART;
-    const float alpha = __int_as_float(a[REEF_GEMM_ALPHA_BITS]);
-    const int act = a[REEF_GEMM_ACT];
-    auto row_stats = [&](int r, float& mu, float& rs) {
-        float t1 = 0.0f, t2 = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            t1 += sums[(w * TD::BM + r) * 2];
-            t2 += sums[(w * TD::BM + r) * 2 + 1];
-        }
-        const float m1 = t1 / (float)K;                    // mean of a - pivot
-        mu = sums[4 * TD::BM * 2 + r] + m1;
-        rs = 1.0f / sqrtf(fmaxf(t2 / (float)K - m1 * m1, 0.0f) + __int_as_float(a[REEF_GEMM_LN_EPS_BITS]));
+        for (int h = 0; h < TM; ++h) pa[h] = split_planes(av[h][0], av[h][1]);
     };
-    float e_mu[LN ? TM : 1], e_rs[LN ? TM : 1];
-    if (LN) {
-#pragma unroll
-        for (int h = 0; h < TM; ++h) row_stats(16 * h + orow, e_mu[LN ? h : 0], e_rs[LN ? h : 0]);
-        ln_out.write(row_stats);
-    }
-    auto finish = [&](float sum, int h, int g) {
-        if (LN) sum = e_rs[LN ? h : 0] * (sum - e_mu[LN ? h : 0] * e_c1[LN ? g : 0]) + e_c2[LN ? g : 0];
-        float v = sum * alpha + e_bias[g];
-        if (act == REEF_ACT_RELU) v = fmaxf(v, 0.0f);
-        else if (act == REEF_ACT_GELU) v = gelu_erf(v);
-        buf_store(rs_c, ooff[h][g], v + e_res[h][g]);
-    };
-    float v[TM][TN];
-#pragma unroll
-    for (int h = 0; h < TM; ++h)
+    auto multiply = [&](int s) {
 #pragma unroll
         for (int g = 0; g < TN; ++g) {
-            const float* e = mine + (h * TN + g) * TD::PART;
-            v[h][g] = ((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE];
+            const Planes pb = {rb[s][g][0], rb[s][g][1], rb[s][g][2]};
+#pragma unroll
+            for (int h = 0; h < TM; ++h) mma_split(pa[h], pb, acc[h][g][0], acc[h][g][1]);
         }
-    if (split_k == 1) {
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g) finish(v[h][g], h, g);
-        return true;
-    }
-
-    // The split_k partial tiles of an output tile meet inside the launch, as those of the direct
-    // convolutions do: a split of two through one exchange per element where every launch on the
-    // buffers runs to completion, otherwise partial tiles to the workspace, a count per tile,
-    // and the last arrival sums them in split order.  The sums and their order are the same.
-    // ptr: .., workspace (split_k [+1] regions of M x N), arrival counters.
-    const int aux = 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0);
-    const size_t MN = (size_t)M * N;
-    float* ws = (float*)d.ptr[aux];
-    unsigned widx[TM][TN];         // element m * N + n of a dense M x N region, ~0u outside the matrix
-#pragma unroll
-    for (int h = 0; h < TM; ++h)
-#pragma unroll
-        for (int g = 0; g < TN; ++g) {
-            const unsigned m = (unsigned)(m0 + 16 * h + orow), n = (unsigned)(n0 + 16 * g + ocol);
-            widx[h][g] = (m < (unsigned)M && n < (unsigned)N) ? m * (unsigned)N + n : ~0u;
+    };
+    int pf = raised, it = 0;
+    bool left = false;
+    if (steps > 0) turn(0);
+    for (; it + NS < steps; it += NS) {
+        if (Poll::enabled) {
+            if (pf) {
+                left = true;
+                break;
+            }
+            pf = poll.load();
         }
-    if (split_k == 2 && (a[REEF_GEMM_FLAGS] & REEF_GEMM_F_PAIR_FOLD) && poll.pair_fold_ok()) {
-        // a value is parked with its sign bit flipped, so a parked value is never the empty slot's 0
-        unsigned* slots = (unsigned*)(ws + 2 * MN);
-        unsigned got[TM][TN];
 #pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g) {
-                got[h][g] = 0;
-                if (widx[h][g] != ~0u) {
-                    unsigned parked = __float_as_uint(v[h][g]) ^ 0x80000000u;
-                    parked = parked ? parked : 0x80000000u;
-                    got[h][g] = __hip_atomic_exchange(&slots[widx[h][g]], parked, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-#pragma unroll
-        for (int h = 0; h < TM; ++h)
-#pragma unroll
-            for (int g = 0; g < TN; ++g)
-                if (got[h][g] != 0) {   // second to arrive: the other half is here
-                    const float other = __uint_as_float(got[h][g] ^ 0x80000000u);
-                    finish(split == 0 ? v[h][g] + other : other + v[h][g], h, g);   // split order
-                    __hip_atomic_store(&slots[widx[h][g]], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-        return true;
+        for (int s = 0; s < NS; ++s) {
+            split_rows();
+            if (s + 1 < NS) turn(s + 1);
+            multiply(s);
+            load_step(s, it + s + NS);         // (a step behind this wavefront's last brings zeros and a neighbour's weights: not used)
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + 1 == NS) turn(0);
+        }
     }
-    int* counters = (int*)d.ptr[aux + 1] + a[REEF_GEMM_SYNC_OFF];
-    int* s_last = sflag + 1;
+    if (Poll::enabled && pf) left = true;
+    if (!left) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            if (it + s < steps) {
+                split_rows();
+                if (s + 1 < NS && it + s + 1 < steps) turn(s + 1);
+                multiply(s);
+            }
+    }
+    if (LATE) t.fetch(d);
+    f32x4 sum[TM][TN];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
-        for (int g = 0; g < TN; ++g)
-            if (widx[h][g] != ~0u) store_agent(ws + (size_t)split * MN + widx[h][g], v[h][g]);
-    partial_stores_done();   // every store of this workgroup is acknowledged before it counts in
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int old = __hip_atomic_fetch_add(&counters[rem], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *s_last = (old == split_k - 1);
-    }
-    __syncthreads();
-    if (!*s_last) return true;
-#pragma unroll
-    for (int h = 0; h < TM; ++h)
-#pragma unroll
-        for (int g = 0; g < TN; ++g)
-            if (widx[h][g] != ~0u) {
-                const float* src = ws + widx[h][g];
-                float sum = 0.0f;
-                for (int s0 = 0; s0 < split_k; s0 += 4) {
-                    float p[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) p[j] = load_agent(src + (size_t)min(s0 + j, split_k - 1) * MN);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (s0 + j < split_k) sum = (s0 + j == 0) ? p[j] : sum + p[j];
-                }
-                finish(sum, h, g);
-            }
-    if (threadIdx.x == 0)  // ready for the next run
-        __hip_atomic_store(&counters[rem], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
+        for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
+    const float* A = (const float*)d.ptr[0] + d.attr[REEF_GEMM_OFF_A];
+    const unsigned short* B = (const unsigned short*)d.ptr[1];
+    return t.template finish<TileGd<TM, TN>::WSTRIDE, true>(d, smem_raw, wave, sum, poll, left || raised, [&](int m, int n) {
+        float s = 0.0f;
+        for (int k = t.k_lo; k < t.k_hi; ++k) {
+            const unsigned short* w = B + ((size_t)(n >> 4) * K32 + (k >> 5)) * 1536 + (((k >> 2) & 3) * 16 + (n & 15)) * 8 + ((k >> 4) & 1) * 4 + (k & 3);
+            const float wv = (__uint_as_float((unsigned)w[0] << 16) + __uint_as_float((unsigned)w[512] << 16)) + __uint_as_float((unsigned)w[1024] << 16);
+            s = fmaf(A[(size_t)m * t.lda + k], wv, s);
+        }
+        return s;
+    });
 }
 
 template <int TM, int TN, bool LN, class Poll>
 __device__ __forceinline__ bool gemm_nt_direct_body(const OpDesc& d, int task, char* smem_raw, const Poll& poll) {
-    if (d.attr[REEF_GEMM_LDB] == 0) return gemm_nt_direct_run<TM, TN, LN, true>(d, task, smem_raw, poll);
-    return gemm_nt_direct_run<TM, TN, LN, false>(d, task, smem_raw, poll);
+    if (d.attr[REEF_GEMM_LDB] != 0) return gemm_nt_direct_run<TM, TN, LN, false>(d, task, smem_raw, poll);
+    if constexpr (TM > 1)
+        if (d.attr[REEF_GEMM_FLAGS] & REEF_GEMM_F_SPLIT) return gemm_split_run<TM, TN, LN>(d, task, smem_raw, poll);
+    return gemm_nt_direct_run<TM, TN, LN, true>(d, task, smem_raw, poll);
 }
 
 // ---- reef_attention_m16: softmax(alpha Q K^T (masked)) V of all heads in one launch, on the matrix cores ----

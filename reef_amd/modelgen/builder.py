@@ -130,11 +130,12 @@ class GraphBuilder:
         self.params.append((key, arr))
         return Tensor(idx, (arr.size,))
 
-    def packed_matrix(self, b, N, K):
-        """The packed copy of weights b [N][K] for the direct products (ldb = 0), one per matrix."""
-        key = self.storage[b.idx]["name"] + "pk"
+    def packed_matrix(self, b, N, K, split=False):
+        """The packed copy of weights b [N][K] for the direct products (ldb = 0), one per matrix and form."""
+        key = self.storage[b.idx]["name"] + ("xpk" if split else "pk")
         if key not in self._packed:
-            self._packed[key] = self.derived_param(key, pack_conv_weights(self.param_array(b).reshape(N, K, 1), by_channels=True))
+            W = self.param_array(b).reshape(N, K)
+            self._packed[key] = self.derived_param(key, split_matrix(W) if split else pack_conv_weights(W[:, :, None], by_channels=True))
         return self._packed[key]
 
     def _sync_counters(self, n):
@@ -685,8 +686,9 @@ class GraphBuilder:
         assert direct_ok or not direct, "this GEMM has no direct form"
         args = [a.idx, b.idx, out.idx]
         packed = packed and direct
+        split = packed and t["tile"] in tiling.GEMM_SPLIT_TILES
         if packed and ln is None:
-            args[1] = self.packed_matrix(b, N, K).idx
+            args[1] = self.packed_matrix(b, N, K, split).idx
         if ln is not None:
             # Wg = W gamma (column k scaled by gamma[k]); c1 = its row sums; c2 = W beta
             assert ldb == K and off_b == 0, "the LayerNorm form takes the weight matrix whole"
@@ -696,11 +698,12 @@ class GraphBuilder:
             wkey = self.storage[b.idx]["name"]
             Wg = (W * gm[None, :]).astype(np.float32)
             # the storage named wkey keeps W itself
-            args[1] = (self.derived_param(wkey + "gkpk", pack_conv_weights(Wg[:, :, None], by_channels=True)) if packed
+            args[1] = (self.derived_param(wkey + "gkxpk", split_matrix(Wg)) if split
+                       else self.derived_param(wkey + "gkpk", pack_conv_weights(Wg[:, :, None], by_channels=True)) if packed
                        else self.derived_param(wkey + "gk", Wg)).idx
             ln = dict(ln, c1=self.derived_param(wkey + "sk", Wg.astype(np.float64).sum(axis=1)),
                       c2=self.derived_param(wkey + "tk", W @ bt))
-        flags = 0
+        flags = 32 if split else 0
         if bias is not None:
             flags |= 1
             args.append(bias.idx)
@@ -854,6 +857,28 @@ def pack_conv_weights(w, by_channels=False):
     else:               # pad[mt*16 + i, c*4 + kq, g*4 + j] -> out[mt, c, g, kq, i, j]
         out = pad.reshape(mt, 16, c // 4, 4, r // 4, 4).transpose(0, 2, 4, 3, 1, 5)
     return np.ascontiguousarray(out).reshape(-1)
+
+
+def split_matrix(w):
+    """[N][K] weights -> the layout of REEF_GEMM_F_SPLIT: each value as the sum of three bf16 values (the first rounded to
+    nearest, or cut off where that would be infinite; the second the next eight bits; the third the rest),
+    [ceil(N/16)][ceil(K/32)][3 parts][4 slots][16 columns][8 values of k]: 4 * slot + 0..3 and 16 + 4 * slot + 0..3 of the 32."""
+    N, K = w.shape
+    n, k = -(-N // 16), -(-K // 32)
+    x = np.zeros((n * 16, k * 32), np.float32)
+    x[:N, :K] = w
+
+    u = x.view(np.uint32)
+    finite = (u & np.uint32(0x7F800000)) != np.uint32(0x7F800000)
+    near = (u + np.uint32(0x7FFF) + ((u >> np.uint32(16)) & np.uint32(1))) & np.uint32(0xFFFF0000)
+    fits = finite & ((near & np.uint32(0x7F800000)) != np.uint32(0x7F800000))
+    nan = ~finite & ((u & np.uint32(0x7FFFFF)) != 0)
+    h = np.where(fits, near, (u & np.uint32(0xFFFF0000)) | np.where(nan, np.uint32(0x400000), np.uint32(0)))
+    r = np.where(finite, x, np.float32(0)) - np.where(finite, h, np.uint32(0)).view(np.float32)
+    m = r.view(np.uint32) & np.uint32(0xFFFF0000)
+    l = (r - m.view(np.float32)).view(np.uint32) & np.uint32(0xFFFF0000)
+    parts = [(p >> np.uint32(16)).astype(np.uint16).reshape(n, 16, k, 2, 4, 4).transpose(0, 2, 4, 1, 3, 5) for p in (h, m, l)]
+    return np.ascontiguousarray(np.stack(parts, axis=2)).reshape(-1).view(np.float32)
 
 
 def write_params(path, params):

@@ -40,6 +40,7 @@ TILES = {
 }
 # matrix products only (reef_gemm_ntd_<tile>, reef_gemm_ntl_<tile>): name -> (id, BM, BN)
 GEMM_WIDE_TILES = {"32x48d4": (19, 32, 48), "48x48d4": (20, 48, 48), "64x64d4": (21, 64, 64)}
+GEMM_SPLIT_TILES = ("32x32d4",) + tuple(GEMM_WIDE_TILES)      # direct tiles that take packed weights as three bf16 parts
 V9_TILES = ("g1", "g2", "g4")      # row tiles that exist as reef_conv2d_v9_<tile>
 # row form: image rows per tile
 ROW_TILES = {"g1": 1, "g2": 2, "g4": 4, "g7": 7, "g2m2": 2, "g4m2": 4}
@@ -115,23 +116,23 @@ GEMM_COST = {
     ("64x32k2", False): (4.431, 12.06, 0, 0, 0.5025, 0, 0),
     ("64x32k2", True): (5.956, 3.589, 7.457, 1.34, 0.4235, 0, 0),
 }
-# The same for the direct kernels on packed weights (reef_kernels.h, ldb = 0): 13 sequence lengths of 16 to 512 times 16
-# layer shapes of 256 to 4096 columns and depth, 4279 launches.  It picks within 4.3 % of the fastest launch on average, by
-# GEMM_COST 11 %: BERT-base at 128, six layers, 300 us of device time a pass by GEMM_COST and 285 by this (unpacked 331); at
-# 384, four layers, 433 and 402 (unpacked 439).  With the FFN-down product as in GEMM_UNDER_LOAD, which comes first, a pass takes
-# 7 % more: see there.
+# The same for the direct kernels on packed weights (reef_kernels.h, ldb = 0; from 32x32 on split ones): 12 sequence lengths
+# of 16 to 512 times 13 layer shapes of 256 to 4096 columns and depth, 2087 launches.  It picks within 1.5 % of the fastest
+# launch on average, by the table of the same tiles on 32-bit weights 5.6 %.  The 16-row tiles that split K keep
+# the coefficients of that table (all measured anew: 1.0 %), which split the products of 8 to 64 rows finer or alike: with the
+# new ones a network of 24 rows is 7 % faster and its distance from 64 bits 3 % larger.
 GEMM_COST_PACKED = {
     ("16x16k4", False): (3.735, 0, 0.1841, 1.183, 0.01631, 0, 3.281),
-    ("16x16k4", True): (3.942, 0, 0.07655, 1.525, 0.2484, 0, 0),
+    ("16x16k4", True): (2.926, 0.7903, 1.179, 0.5716, 0.3408, 0, 0),
     ("16x32k4", False): (3.405, 0, 1.262, 0.9671, 0.2277, 0, 4.159),
-    ("16x32k4", True): (3.852, 0, 1.346, 1.298, 0.4132, 0, 0),
-    ("32x32d4", False): (3.05, 0, 3.095, 1.396, 0.7459, 0, 6.121),
-    ("32x48d4", False): (3.086, 0.716, 5.058, 0.7567, 1.084, 0, 7.42),
-    ("32x48d4", True): (4.614, 0, 5.885, 1.29, 0.7968, 0, 0),
-    ("48x48d4", False): (3.429, 0, 6.574, 2.962, 1.658, 0, 9.302),
-    ("48x48d4", True): (4.494, 0, 12.44, 0, 1.871, 0, 0),
-    ("64x64d4", False): (3.374, 0, 16.25, 0, 4.555, 0, 14.41),
-    ("64x64d4", True): (5.874, 0, 19.3, 0, 1.903, 0, 0),
+    ("16x32k4", True): (3.315, 0.4111, 1.854, 0.8625, 0.5116, 0, 0),
+    ("32x32d4", False): (2.774, 1.242, 1.86, 1.274, 0.8819, 0, 6.57),
+    ("32x48d4", False): (2.977, 0.7474, 3.161, 0.8269, 1.442, 0, 8.945),
+    ("32x48d4", True): (3.947, 0.9158, 2.47, 2.651, 1.316, 0, 0),
+    ("48x48d4", False): (2.441, 0, 6.958, 0, 3.176, 0, 11.35),
+    ("48x48d4", True): (3.385, 0, 8.917, 0, 2.992, 0, 0),
+    ("64x64d4", False): (2.969, 0, 9.973, 0, 5.348, 0, 16.48),
+    ("64x64d4", True): (3.781, 0, 14.86, 0, 3.562, 0, 0),
 }
 GEMM_COST_MIN, GEMM_COST_MAX_OUT = 256, 512 * 4096     # columns and depth from which, outputs up to which it was measured
 

@@ -1,0 +1,77 @@
+"""Matrix products on split weights (REEF_GEMM_F_SPLIT): the parts are the weight, and what has no parts in bf16 -- infinities,
+NaN, values that round to infinity -- comes out as it does on the weights themselves."""
+import os
+
+import numpy as np
+import pytest
+
+from reef_amd import binding as B
+from reef_amd.modelgen import builder as MB, tiling
+
+
+def bf16(u):
+    return (u.astype(np.uint32) << np.uint32(16)).view(np.float32)
+
+
+def test_parts_of_a_weight_add_up_to_it():
+    rng = np.random.default_rng(3)
+    n, k = 21, 72
+    w = rng.integers(0, 2 ** 32, (n, k), dtype=np.uint32).view(np.float32)
+    w[np.abs(w) < 2.0 ** -100] = 1.5        # (below 2^-110 the third part falls under the smallest bf16)
+    w[0, :8] = [np.inf, -np.inf, np.nan, 3.4028235e38, -3.4028235e38, 0.0, -0.0, 1 + 2.0 ** -23]
+    p = MB.split_matrix(w).view(np.uint16).reshape(2, 3, 3, 4, 16, 2, 4)     # tile, group of 32, part, slot, column, half, k
+    h, m, l = (bf16(p[:, :, i]) for i in range(3))
+    with np.errstate(invalid="ignore"):
+        back = (h + m) + l
+    back = back.transpose(0, 3, 1, 4, 2, 5).reshape(32, 96)
+    assert np.array_equal(back[:n, :k], w, equal_nan=True) and not back[n:].any() and not back[:, k:].any()
+    assert np.isfinite(h[np.isfinite(back).reshape(2, 16, 3, 2, 4, 4).transpose(0, 2, 4, 1, 3, 5)]).all()
+
+
+def product(d, name, tile, a, w, split, packed):
+    (m, k), n = a.shape, w.shape[0]
+    g = MB.GraphBuilder(name)
+    g.pack_weights = packed
+    wt = g.param((n, k), 0.5)
+    g.params[g._param_pos[wt.idx]][1][:] = w.reshape(-1)
+    out = g.gemm(g.input("a", (m, k)), wt, m, n, k, force_tile=tile, split_k=split)
+    g.mark_output(out)
+    assert bool(g.kernels[0]["attrs"][5] & 32) == packed
+    g.write(os.path.join(str(d), name))
+    exe = B.Executor.from_dir(os.path.join(str(d), name), name, B.BASE)
+    exe.set_input_checked("a", a)
+    exe.execute()
+    y = exe.get_data(out.idx, m * n).reshape(m, n).copy()
+    exe.close()
+    return y
+
+
+# column tiles that are a multiple of the XCDs and that are not, a split that ends inside a step, the smallest
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 4, 8, 1), (33, 17 * 48 + 4, 264, 1), (70, 8 * 48, 520, 3), (49, 100, 392, 2)])
+@pytest.mark.parametrize("tile", tiling.GEMM_SPLIT_TILES)
+def test_product_of_split_operands(tmp_path, tile, shape):
+    m, n, k, split = shape
+    if split > 1 and tiling.forced(tile, m, n, k, split)["split_k"] != split:
+        pytest.skip("too little depth for this split")
+    rng = np.random.default_rng(5)
+    a, w = rng.standard_normal((m, k)).astype(np.float32), (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    # k + 1 roundings of at most 2^-24 of the sum of magnitudes, and the terms left out: 2^-24 of each product
+    bound = (k + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).T.astype(np.float64))
+    y = product(tmp_path, "split", tile, a, w, split, True)
+    assert (np.abs(y - a.astype(np.float64) @ w.T.astype(np.float64)) <= bound).all()
+    # rows and columns with values that have no parts: one each, so that no sum depends on its order
+    a[m // 2, k // 2], w[n // 2, 3] = 3.4e38, np.inf
+    if m > 4:
+        a[0, 1], a[1, 2], a[2, k - 1], a[3, 0] = np.inf, np.nan, -np.inf, -3.4e38
+    if n > 4:
+        w[1, k - 2], w[2, 5] = np.nan, 3.4e38
+        w[2, :5] = w[2, 6:] = 0.0          # (its only product with the huge values is with itself)
+        a[:, 5] = np.clip(a[:, 5], -0.5, 0.5)
+    with np.errstate(all="ignore"):
+        want = product(tmp_path, "plain", tile, a, w, split, False)
+        y = product(tmp_path, "split2", tile, a, w, split, True)
+        same = np.isfinite(want)
+        assert np.array_equal(np.isnan(want), np.isnan(y)) and np.array_equal(want[np.isinf(want)], y[np.isinf(want)])
+        bound = 2 * (k + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).T.astype(np.float64))
+        assert (np.abs(y[same].astype(np.float64) - want[same]) <= bound[same]).all()
