@@ -162,6 +162,17 @@ struct OpGemmNtDirect {
         return gemm_nt_direct_body<TM, TN, LN>(d, task, smem, p);
     }
 };
+template <int G>
+struct OpConvX9 {
+    REEF_TASKS(conv_tasks)
+    static constexpr int LDS = TileX9<G>::LDS_BYTES;
+    static constexpr int WAVES = 2;
+    template <class P>
+    static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P&) {
+        conv2d_x9_body<G>(d, task, smem);
+        return true;
+    }
+};
 #define REEF_SIMPLE_OP(STRUCT, CALL, TASKS)                                                     \
     struct STRUCT {                                                                             \
         REEF_TASKS(TASKS)                                                                       \
@@ -547,6 +558,10 @@ REEF_ENTRY(reef_gemm_nt_32x32k4, OpGemm<Tile32x32k4 REEF_COMMA true>)
 REEF_ENTRY(reef_gemm_nt_64x32k2, OpGemm<Tile64x32k2 REEF_COMMA true>)
 REEF_ENTRY(reef_gemm_ntl_32x32k4, OpGemm<Tile32x32k4 REEF_COMMA true REEF_COMMA true>)
 REEF_ENTRY(reef_gemm_ntl_64x32k2, OpGemm<Tile64x32k2 REEF_COMMA true REEF_COMMA true>)
+#if REEF_FLAVOUR == 0      // layers called on plain pointers only (reef_ops_conv2d)
+REEF_ENTRY(reef_conv2d_x9_g4, OpConvX9<4>)
+REEF_ENTRY(reef_conv2d_x9_g7, OpConvX9<7>)
+#endif
 REEF_ENTRY(reef_gemm_ntd_16x16k4, OpGemmNtDirect<1 REEF_COMMA 1>)
 REEF_ENTRY(reef_gemm_ntd_16x32k4, OpGemmNtDirect<1 REEF_COMMA 2>)
 REEF_ENTRY(reef_gemm_ntd_32x32d4, OpGemmNtDirect<2 REEF_COMMA 2>)

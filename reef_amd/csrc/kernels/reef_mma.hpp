@@ -785,13 +785,18 @@ __device__ __forceinline__ Planes split_planes(const f32x4& a, const f32x4& b) {
 __device__ __forceinline__ void mma_bf16(const u32x4& a, const u32x4& b, f32x4& c) {
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
+// Product p of the six.
+__device__ __forceinline__ void mma_part(int p, const Planes& a, const Planes& b, f32x4& main, f32x4& rest) {
+    if (p == 0) mma_bf16(a.m, b.m, rest);
+    if (p == 1) mma_bf16(a.h, b.h, main);
+    if (p == 2) mma_bf16(a.h, b.l, rest);
+    if (p == 3) mma_bf16(a.l, b.h, rest);
+    if (p == 4) mma_bf16(a.h, b.m, rest);
+    if (p == 5) mma_bf16(a.m, b.h, rest);
+}
 __device__ __forceinline__ void mma_split(const Planes& a, const Planes& b, f32x4& main, f32x4& rest) {
-    mma_bf16(a.m, b.m, rest);
-    mma_bf16(a.h, b.l, rest);
-    mma_bf16(a.l, b.h, rest);
-    mma_bf16(a.h, b.h, main);
-    mma_bf16(a.h, b.m, rest);
-    mma_bf16(a.m, b.h, rest);
+#pragma unroll
+    for (int p = 0; p < 6; ++p) mma_part(p, a, b, main, rest);
 }
 
 // ---- reef_conv2d_d<R>: operands straight from memory into the matrix cores ----------------
@@ -1909,6 +1914,206 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
         if (NA == 4) sum[0][g] += acc[g][NA - 2] + acc[g][NA - 1];
     }
     return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, left || raised);
+}
+
+// ---- reef_conv2d_x9_g<G>: 3x3 / stride 1 / padding 1 on split operands --------------------------------------
+// A workgroup owns 64 output channels x G image rows x 16 columns, its wavefronts 16 channels each; all four multiply
+// the same piece of the image, which is split into its bf16 parts once, on its way into LDS: [part][row][4 k slots][18
+// columns][4 channels], 16 channels a step, two steps there at a time.  A lane of the column side reads four channels of a pixel
+// and part with one 64-bit load, the shifted taps from the neighbouring pixels; the 64 lanes read 512 bytes in a row.
+// The weights are split by the wavefront that uses them, 36 values a lane for 30 G MFMAs.  An MFMA multiplies 16
+// channels of two taps: left and middle of a filter row, the right ones of rows 0 and 1, and that of row 2 with a zero.
+// The weights come as the caller has them, a filter's 576 bytes of 16 channels in a row, loaded as pieces of 128
+// bytes and brought to their lanes through LDS (each lane from its own 144 bytes, a load touches 64 lines: seven rows of
+// the layer below take 90 us, and 78 without any loads of weights; in pieces of 64 bytes 120 instead of 108 on four rows).
+// 256 channels to 256 at 112 x 112: 144 us on 32-bit MFMAs (reef_conv2d_r9_g4m2, whose matrix pipes are full), 85 here, the
+// MFMAs busy 55 % of the time: the splits (264 VALU operations for 210 MFMAs a step), LDS and the barrier take the
+// rest, with a second workgroup on the CU to fill in.  Four rows are for layers that leave seven too few workgroups.
+// Distance from 64 bits there 1.6e-7 (32-bit MFMAs, eight sums a row: 2.2e-7), and below the other kernels' wherever this is chosen.
+template <int G>
+struct TileX9 {
+    static constexpr int SLOT = 18 * 8, ROW = 4 * SLOT, PART = (G + 2) * ROW, BUF = 3 * PART;      // bytes
+    static constexpr int WROW = 576 + 16, WEIGHTS = 2 * BUF;      // a filter's 16 channels, padding
+    static constexpr int LDS_BYTES = WEIGHTS + 64 * WROW;
+};
+// One output of a convolution in 32 bits.
+__device__ __forceinline__ float conv2d_element(const OpDesc& d, int m, int n) {
+    const int* a = d.attr;
+    const int C = a[REEF_CONV_CIN], H = a[REEF_CONV_H], W = a[REEF_CONV_W], kh = a[REEF_CONV_KH], kw = a[REEF_CONV_KW], Wo = a[REEF_CONV_WO];
+    const int y = div_small(n, Wo), x = n - y * Wo;
+    const int iy = y * a[REEF_CONV_SH] - a[REEF_CONV_PH], ix = x * a[REEF_CONV_SW] - a[REEF_CONV_PW];
+    const float* w = (const float*)d.ptr[1] + (size_t)m * C * kh * kw;
+    const float* in = (const float*)d.ptr[0];
+    float s = 0.0f;
+    for (int c = 0; c < C; ++c)
+        for (int ky = 0; ky < kh; ++ky)
+            for (int kx = 0; kx < kw; ++kx) {
+                const bool ok = (unsigned)(iy + ky) < (unsigned)H && (unsigned)(ix + kx) < (unsigned)W;
+                s = fmaf(*w++, ok ? in[((size_t)c * H + iy + ky) * W + ix + kx] : 0.0f, s);
+            }
+    return s;
+}
+template <int G>
+__device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* smem) {
+    typedef TileX9<G> TX;
+    constexpr int ITEMS = (G + 2) * 72, PER = (ITEMS + kThreads - 1) / kThreads;      // (row, 4 channels, pixel) of a step; a thread's
+    const int* a = d.attr;
+    const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], H = a[REEF_CONV_H], W = a[REEF_CONV_W], N = H * W;
+    const int n_tiles = a[REEF_CONV_N_TILES];
+    task = xcd_chunked(task, a[REEF_CONV_M_TILES] * n_tiles);
+    const int mt = div_small(task, n_tiles), nt = task - mt * n_tiles;
+    const int segs = (W + 15) >> 4, yt = div_small(nt, segs);
+    const int m0 = mt * 64 + wave * 16, y0 = yt * G, x0 = (nt - yt * segs) * 16;
+    const unsigned HW4 = (unsigned)N * 4u;
+    const int steps = (C + 15) >> 4;
+
+    // channels from C on (a multiple of 4) lie behind the buffer and read as zeros
+    const rsrc_t rs_b = make_rsrc(d.ptr[0], (unsigned)C * HW4);
+    unsigned vb[PER];
+    int wr[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = tid + kThreads * k, r = i / 72, q4 = (i - r * 72) / 18, px = i - r * 72 - q4 * 18;
+        const int iy = y0 - 1 + r, ix = x0 - 1 + px;
+        vb[k] = i < ITEMS && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W ? (unsigned)(4 * q4) * HW4 + (unsigned)(iy * W + ix) * 4u : kOutside;
+        wr[k] = i < ITEMS ? r * TX::ROW + q4 * TX::SLOT + px * 8 : -1;
+    }
+    // weights of channels from C on are the next row's, or lie behind the buffer: the image is 0 there
+    const rsrc_t rs_a = make_rsrc(d.ptr[1], (unsigned)M * (unsigned)C * 36u);
+    // load j < 8: eight rows (from row 8 on for j >= 4), 128 bytes each; load 8: the last 64 bytes of all
+    const unsigned row36 = (unsigned)C * 36u;
+    unsigned va[3] = {(unsigned)(m0 + (lane >> 3)) * row36 + (unsigned)(lane & 7) * 16u, 0, (unsigned)(m0 + (lane >> 2)) * row36 + 512u + (unsigned)(lane & 3) * 16u};
+    va[1] = va[0] + 8u * row36;
+    const int wa[2] = {(lane >> 3) * TX::WROW + (lane & 7) * 16, (lane >> 2) * TX::WROW + 512 + (lane & 3) * 16};
+    char* wts = smem + TX::WEIGHTS + wave * (16 * TX::WROW);
+    float rb[PER][4];
+    f32x4 ra[9];
+    auto load_image = [&]() {
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rb[k][q] = buf_load(rs_b, vb[k] + (unsigned)q * HW4);
+            vb[k] += 16u * HW4;
+        }
+    };
+    auto load_weights = [&]() {
+#pragma unroll
+        for (int j = 0; j < 9; ++j) {
+            ra[j] = buf_load4(rs_a, j == 8 ? va[2] : va[j >> 2] + 128u * (j & 3));
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) va[j] += 16u * 36u;
+    };
+    load_image();
+    load_weights();
+    // two sums of large products and one of small ones a row: chains no longer than those of the image-row kernels
+    f32x4 acc[G][3];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g][0] = acc[g][1] = acc[g][2] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const char* rd = smem + kq * TX::SLOT + i16 * 8;
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u32x4_at8 __attribute__((ext_vector_type(4), aligned(8)));
+    Planes w[5];
+    // taps of the two halves of an MFMA: left and middle of filter row 0, 1, 2; right of rows 0 and 1; right of row 2
+    auto split_weights = [&](bool more) {
+#pragma unroll
+        for (int j = 0; j < 9; ++j) *(f32x4*)(wts + (j == 8 ? wa[1] : wa[0] + (j >> 2) * (8 * TX::WROW) + (j & 3) * 128)) = ra[j];
+        __builtin_amdgcn_wave_barrier();
+        if (more) load_weights();
+        float v[36];
+#pragma unroll
+        for (int j = 0; j < 9; ++j) {
+            const f32x4 x = *(const f32x4*)(wts + i16 * TX::WROW + kq * 144 + j * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * j + e] = x[e];
+        }
+        __builtin_amdgcn_wave_barrier();
+        constexpr int TA[5] = {0, 3, 6, 2, -1}, TB[5] = {1, 4, 7, 5, 8};
+#pragma unroll
+        for (int p = 0; p < 5; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = e < 2 ? TA[p] : TB[p], q = 2 * (e & 1);
+                unsigned h = 0, m = 0, l = 0;
+                if (t >= 0) split_pair(v[t < 0 ? 0 : q * 9 + t], v[t < 0 ? 0 : (q + 1) * 9 + t], h, m, l);
+                w[p].h[e] = h;
+                w[p].m[e] = m;
+                w[p].l[e] = l;
+            }
+    };
+    split_weights(steps > 1);
+    for (int s = 0; s < steps; ++s) {
+        const int buf = (s & 1) * TX::BUF;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            unsigned h0, m0_, l0, h1, m1, l1;
+            split_pair(rb[k][0], rb[k][1], h0, m0_, l0);
+            split_pair(rb[k][2], rb[k][3], h1, m1, l1);
+            if (wr[k] >= 0) {
+                char* p = smem + buf + wr[k];
+                *(u32x2*)p = u32x2{h0, h1};
+                *(u32x2*)(p + TX::PART) = u32x2{m0_, m1};
+                *(u32x2*)(p + 2 * TX::PART) = u32x2{l0, l1};
+            }
+        }
+        __syncthreads();
+        if (s + 1 < steps) load_image();
+        const char* at = rd + buf;
+        Planes lc[2], rr[2];
+        auto read = [&](int r, int to) {      // left and middle pixels of image row r; right ones of rows r and r + 1
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                const char* x = at + p * TX::PART + r * TX::ROW;
+                u32x4& l = p == 0 ? lc[to].h : p == 1 ? lc[to].m : lc[to].l;
+                u32x4& rt = p == 0 ? rr[to].h : p == 1 ? rr[to].m : rr[to].l;
+                l = *(const u32x4_at8*)x;
+                if (r > G) continue;
+                const u32x2 a0 = *(const u32x2*)(x + 16), a1 = *(const u32x2*)(x + 16 + TX::ROW);
+                rt = u32x4{a0[0], a0[1], a1[0], a1[1]};
+            }
+        };
+        __builtin_amdgcn_s_setprio(2);      // (a wavefront of the other workgroup splits meanwhile: 2 to 6 % of a launch)
+        read(0, 0);
+#pragma unroll
+        for (int r = 0; r < G + 2; ++r) {
+            if (r + 1 < G + 2) read(r + 1, (r + 1) & 1);
+            const Planes& l = lc[r & 1];
+            const Planes& rt = rr[r & 1];
+            // product by product over the up to five pairs of this row, so that what adds to one accumulator is apart
+#pragma unroll
+            for (int p = 0; p < 6; ++p) {
+#pragma unroll
+                for (int o = 0; o < 5; ++o) {
+                    const int g = o < 3 ? r - o : r - (o - 3);
+                    if (g < 0 || g >= G || (o >= 3 && r > G)) continue;
+                    f32x4 (&c)[3] = acc[g < 0 ? 0 : g < G ? g : 0];
+                    mma_part(p, w[o], o < 3 ? l : rt, c[o & 1], c[2]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        if (s + 1 < steps) split_weights(s + 2 < steps);
+    }
+    ConvEpilogue ep;
+    ep.init(d, a[REEF_CONV_FLAGS], a[REEF_CONV_ACT], a[REEF_CONV_ACT2], M, (unsigned)M * HW4, (unsigned)a[REEF_CONV_DST_OFF] * 4u);
+    const int x = x0 + i16;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        f32x4 sum = (acc[g][0] + acc[g][1]) + acc[g][2];
+        const int n = (y0 + g) * W + x;
+        const bool ok = x < W && y0 + g < H;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int m = m0 + 4 * kq + j;
+            if (!__builtin_isfinite(sum[j]) && ok && m < M) sum[j] = conv2d_element(d, m, n);
+            const unsigned off = ok ? ((unsigned)m * (unsigned)N + (unsigned)n) * 4u : kOutside, m4 = (unsigned)m * 4u;
+            ep.finish(sum[j], off, m4, ep.has_res ? buf_load(ep.res, off) : 0.0f, ep.has_bias ? buf_load(ep.bias, m4) : 0.0f,
+                      ep.has_dual ? buf_load(ep.shift2, m4) : 0.0f);
+        }
+    }
 }
 
 // ---- reef_conv2d_xdw[2]_g<G>: 1x1 convolution, then depthwise 3x3, in one launch --------------

@@ -52,6 +52,7 @@ enum Family {
     kFamRows3,        // three taps a filter row, any filter height
     kFamRows5, kFamRows7,
     kFamImageRows,    // 3x3, stride 1, padding 1
+    kFamImagePatch,   // the same, Cin % 4 == 0
     kFamTaps3,        // three taps in all (a column of them: no row kernel)
     kFamTaps7,
     kFamStaged,       // any filter, K % 4 == 0
@@ -69,11 +70,13 @@ enum Family {
 // and unaligned loaders and both strides alike.  Those rows order the tiles of one family only.  Against one tile per filter (16 x 32 at 1x1, two image rows
 // at 3x3, staged 64 x 64 at 5x5, 7x7 and odd channel counts), kernel times: 5x5 48 -> 64 at 35x35 31.9 ->
 // 8.1 us, 7x7 209 -> 15 at 12x85 43 -> 9.3, 1x1 161 -> 617 at 23x21 17 -> 5.2, 3x3 256 -> 256 at 112x112
-// 210 -> 144 (103 TFLOP/s of the 152 that fp32 MFMAs reach).
+// 210 -> 144 (103 TFLOP/s of the 152 that fp32 MFMAs reach) -> 85 by
+// image patches, whose rows are fitted to 70 of those shapes, from 0.3 to 15 GFLOP, with 3 % on top: where
+// they are near the others, those stay.  They do not split K, so they are for layers with some 400 tiles of 64 channels.
 struct Kernel {
     const char* symbol;
     Family family;
-    int tile, bm, bn;      // bn: pixels, or image rows of a segment of 14 columns
+    int tile, bm, bn;      // bn: pixels, or image rows of a segment of 14 columns (image patches: 16)
     float cost[2][7];
 };
 constexpr Kernel kKernels[] = {
@@ -152,6 +155,12 @@ constexpr Kernel kKernels[] = {
     {"reef_conv2d_r9_g4m2", kFamImageRows, REEF_TILE_R9G4M2, 32, 4,
      {{4.523f, 1.487f, 6.196f, 1.782f, 1.556f, 2.73f, 4.828f},
       {4.523f, 1.487f, 6.196f, 1.782f, 1.556f, 2.73f, 4.828f}}},
+    {"reef_conv2d_x9_g4", kFamImagePatch, REEF_TILE_R9G4, 64, 4,
+     {{6.956f, 2.998f, 1.896f, 9.85f, 2.644f, 0.0f, 0.0f},
+      {6.956f, 2.998f, 1.896f, 9.85f, 2.644f, 0.0f, 0.0f}}},
+    {"reef_conv2d_x9_g7", kFamImagePatch, REEF_TILE_R9G7, 64, 7,
+     {{11.48f, 5.748f, 3.443f, 11.69f, 3.077f, 0.0f, 0.0f},
+      {11.48f, 5.748f, 3.443f, 11.69f, 3.077f, 0.0f, 0.0f}}},
     {"reef_conv2d_d3_16x16k4", kFamTaps3, REEF_TILE_16x16k4, 16, 16,
      {{2.736f, 1.138f, 2.177f, 0.0f, 0.19f, 1.27f, 1.775f},
       {2.659f, 0.768f, 2.581f, 0.802f, 0.127f, 1.249f, 1.713f}}},
@@ -273,6 +282,9 @@ bool takes(Family f, const reef_conv2d_desc* c) {
         case kFamRows3: return rows3;
         case kFamRows5: return rows5;
         case kFamRows7: return rows7;
+        case kFamImagePatch:
+            if (c->cin % 4 != 0) return false;
+            // as the image rows
         case kFamImageRows:
             return rows3 && c->kh == 3 && c->stride_h == 1 && c->stride_w == 1 && c->pad_h == 1 && c->pad_w == 1;
         case kFamTaps3: return taps == 3 && !rows3;
@@ -308,12 +320,15 @@ Geometry choose(const reef_conv2d_desc* c, int Ho, int Wo) {
             default: step = unit = 16 * taps; break;
         }
         const int m_tiles = (M + k.bm - 1) / k.bm;
-        const int n_tiles = k.family == kFamImageRows ? ((Ho + k.bn - 1) / k.bn) * ((Wo + 13) / 14) : (N + k.bn - 1) / k.bn;
+        const int n_tiles = k.family == kFamImageRows    ? ((Ho + k.bn - 1) / k.bn) * ((Wo + 13) / 14)
+                            : k.family == kFamImagePatch ? ((Ho + k.bn - 1) / k.bn) * ((Wo + 15) / 16)
+                                                         : (N + k.bn - 1) / k.bn;
         const long long tiles = (long long)m_tiles * n_tiles;
         for (int want : {1, 2, 3, 4, 6, 8, 12, 16}) {
             const long long share = ((K + want - 1) / want + unit - 1) / unit * unit;
             const int split = (int)((K + share - 1) / share);
             if (split != want) continue;
+            if (split > 1 && k.family == kFamImagePatch) break;
             if (split > 1 && (tiles * split > 640 || (size_t)split * M * N * 4 > kWorkspaceBytes)) break;
             const long long mine = std::min<long long>(share, K);
             const float w = (float)((mine + step - 1) / step * step) / 1000.0f, r = (float)(tiles * split) / 256.0f;
@@ -373,7 +388,7 @@ int make_plan(const reef_conv2d_desc* c, const float* in, const float* w,
     const Geometry& g = chosen(c, Ho, Wo);
     const Kernel& k = kKernels[g.kernel];
     const int split = g.split, tiles = g.m_tiles * g.n_tiles;
-    const int mode = k.family == kFamImageRows ? REEF_CONV_MODE_ROWS
+    const int mode = k.family == kFamImageRows || k.family == kFamImagePatch ? REEF_CONV_MODE_ROWS
                      : k.family == kFamStaged ? REEF_CONV_MODE_GENERAL
                      : k.family == kFamStagedOdd ? REEF_CONV_MODE_UNALIGNED
                                                  : REEF_CONV_MODE_DIRECT;

@@ -1,0 +1,72 @@
+"""Large 3x3 layers through reef_ops_conv2d (reef_conv2d_x9_g*): sizes that end inside a tile, a step of channels and a
+group of output channels, a residual, and values that have no parts in bf16."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from reef_amd import binding as B
+
+pytestmark = pytest.mark.gpu
+
+
+def run(x, w, b, res, act):
+    cin, H, W = x.shape
+    cout = w.shape[0]
+    d = B.Conv2dDesc(cin, H, W, cout, 3, 3, 1, 1, 1, 1, act)
+    bufs = [B.DeviceBuffer.from_array(a) if a is not None else None for a in (x, w, b, res)]
+    out = B.DeviceBuffer(cout * H * W * 4)
+    out.fill(0xFF)
+    assert B.ops_conv2d(d, bufs[0], bufs[1], bufs[2], bufs[3], out) == 0, B.last_error()
+    return out.to_array().reshape(cout, H, W)
+
+
+# cin, H, W, cout: whole tiles; every edge ragged; few channels in; one column behind a segment
+@pytest.mark.parametrize("case", [(256, 112, 112, 256), (252, 113, 83, 270), (44, 139, 111, 326), (84, 95, 97, 348)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_against_64_bits(case, residual):
+    B.ops_init()
+    cin, H, W, cout = case
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3, 3)) * np.sqrt(2.0 / (cin * 9))).astype(np.float32)
+    b = rng.standard_normal(cout).astype(np.float32)
+    res = rng.standard_normal((cout, H, W)).astype(np.float32) if residual else None
+    got = run(x, w, b, res, 1)
+    # some output channels, everywhere: the first and last of a wavefront and of the layer
+    rows = sorted({0, 15, 16, 63, cout // 64 * 64 % cout, cout - 1})
+    xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1)))
+    ab = np.abs(xp)
+    for m in rows:
+        want, mag = np.full((H, W), float(b[m])), np.full((H, W), abs(float(b[m])))
+        for i in range(3):
+            for j in range(3):
+                want += np.tensordot(w[m, :, i, j].astype(np.float64), xp[:, i:i + H, j:j + W], 1)
+                mag += np.tensordot(np.abs(w[m, :, i, j]).astype(np.float64), ab[:, i:i + H, j:j + W], 1)
+        if res is not None:
+            want += res[m]
+            mag += np.abs(res[m])
+        # a rounding of at most 2^-24 of the sum of magnitudes per product and one each for the epilogue's terms
+        assert (np.abs(got[m] - np.maximum(want, 0.0)) <= (9 * cin + 4) * 2.0 ** -24 * mag).all(), m
+
+
+def test_values_without_parts():
+    B.ops_init()
+    cin, H, W, cout = 256, 112, 112, 256
+    rng = np.random.default_rng(12)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3, 3)) * 0.02).astype(np.float32)
+    plain = run(x, w, None, None, 0)
+    x[3, 10, 20], x[5, 50, 60], x[255, 111, 111], x[0, 0, 0], x[17, 80, 30] = np.inf, np.nan, -np.inf, 3.4e38, -3.4e38
+    got = run(x, w, None, None, 0)
+    touched = np.zeros((H, W), bool)
+    for y, z in ((10, 20), (50, 60), (111, 111), (0, 0), (80, 30)):
+        touched[max(0, y - 1):y + 2, max(0, z - 1):z + 2] = True
+    np.testing.assert_array_equal(got[:, ~touched], plain[:, ~touched])
+    with np.errstate(all="ignore"):
+        want = O.conv2d(x, w, np.zeros(cout, np.float32), None, None, None, (1, 1), (1, 1), 1, 0, 6.0, False).reshape(cout, H, W)[:, touched]
+    got = got[:, touched]
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    # a value of 3.4e38 in the sum: its product decides
+    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-3)
