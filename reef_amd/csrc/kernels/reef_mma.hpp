@@ -1135,12 +1135,6 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     float* smem = (float*)smem_raw;
     const OpDesc& d = d_in;
     const int* a = d.attr;
-    // The flag check every best-effort workgroup makes before it does anything
-    // (script/best_effort_kernel.py:22-29): read by every wavefront in front of its first loads, looked at where the K
-    // loop looks at it anyway and where the wavefronts meet behind it.  A workgroup that finds the flag raised has only
-    // read.  (Looked at behind the first loads, with a barrier, every launch waited for all of them before its
-    // first MFMA: DenseNet-201 1017 -> 980 us of device time a pass.)
-    const int raised = Poll::enabled ? poll.load() : 0;
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = FROWS ? a[REEF_CONV_KH] : 1;
@@ -1441,7 +1435,15 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
                     acc[h][g][q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][ROWS ? 0 : g * RC + q],
                                                                             acc[h][g][q & 1], 0, 0, 0);
     };
-    int pf = raised;
+    // The flag check every best-effort workgroup makes before it does anything
+    // (script/best_effort_kernel.py:22-29): read by every wavefront behind its first loads, and looked at where the wavefronts
+    // meet behind the K loop; what the loop itself looks at are loads of its own, one round ahead.  A workgroup that finds
+    // the flag raised has only read.  Loads return in order, and the flag, which no cache holds, comes later than
+    // operands do: in front of them it held up the first MFMAs of every launch (DenseNet-201 as a best-effort model 990 us a
+    // request that way and 956 this way, BERT-base at 128 tokens 323 and 319; looked at with a barrier before the loop: 1017 of device time to 980).
+    asm volatile("" ::: "memory");
+    const int raised = Poll::enabled ? poll.load() : 0;
+    int pf = 0;
     int it = 0;
     bool left = false;
     // (groups whose refills all exist; the last whole group follows with the refills the remaining
@@ -1469,7 +1471,6 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
         if (Poll::enabled && pf) {
             left = true;
         } else {
-            if (Poll::enabled) pf = poll.load();
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 mma_stage(s);
@@ -1529,7 +1530,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     float* smem = (float*)smem_raw;
     constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
     const int* a = d.attr;
-    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
@@ -1665,7 +1665,9 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
                     acc[h][g][q % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], bt[from][g][q], acc[h][g][q % NA], 0, 0, 0);
     };
     static_assert(NS % 2 == 0, "the turned blocks alternate");
-    int pf = raised, it = 0;
+    asm volatile("" ::: "memory");
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
+    int pf = 0, it = 0;
     bool left = false;
     if (steps > 0) turn(0, 0);
     for (; it + 2 * NS <= steps; it += NS) {
@@ -1689,7 +1691,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
         if (Poll::enabled && pf) {
             left = true;
         } else {
-            if (Poll::enabled) pf = poll.load();
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 if (s + 1 < NS) turn(s + 1, (s + 1) & 1);
@@ -1746,7 +1747,6 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     constexpr int NA = G == 1 ? 4 : 2;
     float* smem = (float*)smem_raw;
     const int* a = d.attr;
-    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], H = a[REEF_CONV_H], W = a[REEF_CONV_W];
@@ -1890,7 +1890,9 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     };
     struct Yes { constexpr operator bool() const { return true; } };
     struct No { constexpr operator bool() const { return false; } };
-    int pf = raised;
+    asm volatile("" ::: "memory");
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
+    int pf = 0;
     bool left = false;
     if (steps > 0) {
         turn();
@@ -3413,7 +3415,6 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     constexpr int AC = TM * TN > 4 ? 1 : PK && !LN && TM * TN == 1 ? 4 : 2;
     // steps of loads in flight (unpacked, 6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
     constexpr int NS = PK ? 4 : 3;
-    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GemmTail<TM, TN, LN> t;
@@ -3519,7 +3520,9 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
                     acc[h][g][q % AC] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][g][q],
                                                                              acc[h][g][q % AC], 0, 0, 0);
     };
-    int pf = raised, it = 0;
+    asm volatile("" ::: "memory");
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
+    int pf = 0, it = 0;
     bool left = false;
     // this wavefront's own steps where their loads are its own
     const int steps = PK ? (t.k_lo + 16 * wave < t.k_hi ? (t.k_hi - t.k_lo - 16 * wave + KSTEP - 1) / KSTEP : 0) : nsteps;
@@ -3547,7 +3550,6 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
         if (Poll::enabled && pf) {
             left = true;
         } else {
-            if (Poll::enabled) pf = poll.load();
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 if (PK && s + 1 < NS) turn(s + 1, (s + 1) & 1);
@@ -3595,7 +3597,6 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     constexpr int NS = 2;                                    // steps of loads in flight: what 256 registers hold
     typedef TileD16<TN, TM> TD;
     static_assert(TM * 512 <= TD::SUBS * TD::PART, "the turned rows fit where the partial tile goes");
-    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GemmTail<TM, TN, LN> t;
@@ -3685,7 +3686,9 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
             for (int h = 0; h < TM; ++h) mma_split(pa[h], pb, acc[h][g][0], acc[h][g][1]);
         }
     };
-    int pf = raised, it = 0;
+    asm volatile("" ::: "memory");
+    const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
+    int pf = 0, it = 0;
     bool left = false;
     if (steps > 0) turn(0);
     for (; it + NS < steps; it += NS) {
