@@ -180,8 +180,30 @@ __device__ __forceinline__ float act_apply(float v, int act) {
     return act == REEF_ACT_RELU || act == REEF_ACT_RELU6 ? r : v;
 }
 
+// x Phi(x), without a branch: Phi is 0.5 + x P(x^2) inside +-sqrt(2) and 2^-Q(|x|) of the tail outside, to 5.65, behind which
+// the tail rounds away.  P and Q are least-maximum fits of degree 6 (4e-10 and 5e-10 of Phi).  With erff, both
+// of whose branches a wavefront takes, BERT-base takes 303.7 us of device time a pass (128 tokens, six layers) and 238.2 (200,
+// four), with this 302.2 and 236.3.  Against 64 bits, 2.6 million
+// values from -8 to 8: at most 3.9e-7 and for normal x 2.34e-8 rms; with a correctly rounded erf 4.5e-7 and 2.45e-8.
 __device__ __forceinline__ float gelu_erf(float x) {
-    return x * (0.5f + 0.5f * erff(x * 0.70710678f));
+    const float t = x * x, ax = fabsf(x);
+    float p = 4.35816162e-07f;
+    p = fmaf(p, t, -8.8618599e-06f);
+    p = fmaf(p, t, 0.00011467361f);
+    p = fmaf(p, t, -0.00118680997f);
+    p = fmaf(p, t, 0.00997338817f);
+    p = fmaf(p, t, -0.0664903596f);
+    p = fmaf(p, t, 0.398942292f);
+    float q = -3.34661963e-05f;
+    q = fmaf(q, ax, 0.000749707164f);
+    q = fmaf(q, ax, -0.00786463264f);
+    q = fmaf(q, ax, 0.0525563173f);
+    q = fmaf(q, ax, 0.460382402f);
+    q = fmaf(q, ax, 1.14973807f);
+    q = fmaf(q, ax, 1.00051022f);
+    const float tail = ax < 5.65f ? __builtin_amdgcn_exp2f(-q) : 0.0f;
+    const float outer = x < 0.0f ? tail : 1.0f - tail;
+    return x * (ax < 1.41421354f ? fmaf(x, p, 0.5f) : outer);
 }
 
 // ---- prefetching workgroups --------------------------------------------------------
