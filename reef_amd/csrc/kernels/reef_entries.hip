@@ -94,6 +94,7 @@ struct OpConvV9 {
     REEF_TASKS(conv_tasks)
     static constexpr int LDS = TileV9<G>::LDS_BYTES;
     static constexpr int WAVES = 2;
+    static constexpr bool THROUGH = false;
     static constexpr bool CHECKS_FLAG_ITSELF = true;
     template <class P>
     static __device__ __forceinline__ bool run(const OpDesc& d, int task, char* smem, const P& p) {
@@ -444,7 +445,8 @@ struct ChecksFlagItself<OP, decltype((void)OP::CHECKS_FLAG_ITSELF)> { static con
 // REEF_ENTRY_RELEASED: results stay in L2 until the release at the end of the launch.  1x1 kernels on whole lines without a
 // pre-activation and 32x32 ones: on images whose rows end inside a line (14 x 14) their many results written through piece by
 // piece cost what the release does, or more (512 channels to 512 4.06 us a launch either way, ResNet-152 844 us a request, and
-// 859 with them written through).
+// 859 with them written through).  3x3 kernels on whole lines likewise: ResNet-152 815 us of device time a pass, ResNet-50 at 448
+// 627, and 823 and 631 with those written through (DenseNet-201, whose 32 channels leave little behind, 866 and 857).
 #define REEF_ENTRY(NAME, OP)                                                          \
     using NAME##_op = OP;                                                             \
     static_assert(WritesThrough<NAME##_op>::value, "REEF_ENTRY_RELEASED");            \
@@ -504,9 +506,9 @@ REEF_ENTRY_RELEASED(reef_conv2d_v1_32x32d4, OpConvV1<2 REEF_COMMA 2>)
 REEF_ENTRY(reef_conv2d_p1_v_16x16k4, OpConvV1<1 REEF_COMMA 1 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_p1_v_16x32k4, OpConvV1<1 REEF_COMMA 2 REEF_COMMA true>)
 REEF_ENTRY(reef_conv2d_p1_v_32x32d4, OpConvV1<2 REEF_COMMA 2 REEF_COMMA true>)
-REEF_ENTRY(reef_conv2d_v9_g1, OpConvV9<1>)
-REEF_ENTRY(reef_conv2d_v9_g2, OpConvV9<2>)
-REEF_ENTRY(reef_conv2d_v9_g4, OpConvV9<4>)
+REEF_ENTRY_RELEASED(reef_conv2d_v9_g1, OpConvV9<1>)
+REEF_ENTRY_RELEASED(reef_conv2d_v9_g2, OpConvV9<2>)
+REEF_ENTRY_RELEASED(reef_conv2d_v9_g4, OpConvV9<4>)
 REEF_ENTRY(reef_conv2d_r9_g1, OpConvRows<1>)
 REEF_ENTRY(reef_conv2d_r9_g2, OpConvRows<2>)
 REEF_ENTRY(reef_conv2d_r9_g4, OpConvRows<4>)

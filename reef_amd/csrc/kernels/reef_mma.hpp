@@ -1441,7 +1441,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     // the flag raised has only read.  Loads return in order, and the flag, which no cache holds, comes later than
     // operands do: in front of them it held up the first MFMAs of every launch (DenseNet-201 as a best-effort model 990 us a
     // request that way and 956 this way, BERT-base at 128 tokens 323 and 319; looked at with a barrier before the loop: 1017 of device time to 980).
-    asm volatile("" ::: "memory");
+    if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;
     int pf = 0;
     int it = 0;
@@ -1665,7 +1665,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
                     acc[h][g][q % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], bt[from][g][q], acc[h][g][q % NA], 0, 0, 0);
     };
     static_assert(NS % 2 == 0, "the turned blocks alternate");
-    asm volatile("" ::: "memory");
+    if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0, it = 0;
     bool left = false;
@@ -1890,7 +1890,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     };
     struct Yes { constexpr operator bool() const { return true; } };
     struct No { constexpr operator bool() const { return false; } };
-    asm volatile("" ::: "memory");
+    if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0;
     bool left = false;
@@ -1915,7 +1915,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
         sum[0][g] = acc[g][0] + acc[g][1];
         if (NA == 4) sum[0][g] += acc[g][NA - 2] + acc[g][NA - 1];
     }
-    return direct_tail<1, G, TV::BLOCK>(d, smem_raw, wave, sum, tail, poll, left || raised);
+    return direct_tail<1, G, TV::BLOCK, 0>(d, smem_raw, wave, sum, tail, poll, left || raised);
 }
 
 // ---- reef_conv2d_x9_g<G>: 3x3 / stride 1 / padding 1 on split operands --------------------------------------
@@ -3520,7 +3520,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
                     acc[h][g][q % AC] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[s][h][q], rb[s][g][q],
                                                                              acc[h][g][q % AC], 0, 0, 0);
     };
-    asm volatile("" ::: "memory");
+    if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0, it = 0;
     bool left = false;
@@ -3686,7 +3686,7 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
             for (int h = 0; h < TM; ++h) mma_split(pa[h], pb, acc[h][g][0], acc[h][g][1]);
         }
     };
-    asm volatile("" ::: "memory");
+    if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0, it = 0;
     bool left = false;

@@ -25,7 +25,7 @@ def test_marked_kernels_write_through(flavour, tmp_path):
                            "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", "--input=" + code_object(flavour), "--output=" + elf])
     names = subprocess.check_output([os.path.join(LLVM, "llvm-readelf"), "-sW", elf], text=True)
     marked = set(re.findall(r" (\w+)_through$", names, re.M))
-    assert len(marked) > 80 and "reef_conv2d_v9_g1" in marked and "reef_softmax" in marked
+    assert len(marked) > 80 and "reef_conv2d_p1_v_16x16k4" in marked and "reef_softmax" in marked
     name, stores, plain, unwaited = None, 0, set(), set()
     waited = True
     for line in subprocess.Popen([os.path.join(LLVM, "llvm-objdump"), "-d", elf], stdout=subprocess.PIPE, text=True).stdout:
