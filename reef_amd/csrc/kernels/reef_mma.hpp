@@ -799,6 +799,30 @@ __device__ __forceinline__ void mma_split(const Planes& a, const Planes& b, f32x
     for (int p = 0; p < 6; ++p) mma_part(p, a, b, main, rest);
 }
 
+// Whether a value of this wavefront's tile is infinite or NaN (0 times a finite one is 0).
+template <int TM, int TN>
+__device__ __forceinline__ bool any_not_finite(const f32x4 (&v)[TM][TN]) {
+    float t = 0.0f;
+#pragma unroll
+    for (int h = 0; h < TM; ++h)
+#pragma unroll
+        for (int g = 0; g < TN; ++g)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t = fmaf(v[h][g][j], 0.0f, t);
+    return __any(t != 0.0f);
+}
+__device__ __forceinline__ void keep_finite(f32x4& v, const f32x4& other) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __builtin_isfinite(v[j]) ? v[j] : other[j];
+}
+// Value e (0 to 7) of the eight whose parts these are.
+__device__ __forceinline__ float planes_value(const u32x4& h, const u32x4& m, const u32x4& l, int e) {
+    const int i = e >> 1;
+    if (e & 1)
+        return (__uint_as_float(h[i] & 0xFFFF0000u) + __uint_as_float(m[i] & 0xFFFF0000u)) + __uint_as_float(l[i] & 0xFFFF0000u);
+    return (__uint_as_float(h[i] << 16) + __uint_as_float(m[i] << 16)) + __uint_as_float(l[i] << 16);
+}
+
 // ---- reef_conv2d_d<R>: operands straight from memory into the matrix cores ----------------
 // A batch-1 layer is latency bound: every weight is used once per inference, so each K step of
 // the tiled kernels above waits a full memory round trip (global -> registers -> LDS -> barrier).
@@ -3231,11 +3255,10 @@ struct GemmTail {
             ls2[LN ? h : 0] = fmaf(dl, dl, ls2[LN ? h : 0]);
         }
     }
-    // From the wavefronts' partial tiles to C.  WSTRIDE: floats between the wavefronts' places in LDS.  again(m, n): the element's sum over [k_lo, k_hi) in
-    // 32 bits, for one that came out of split operands as infinite or NaN.  False: the workgroup leaves a preempted launch.
-    template <int WSTRIDE, bool AGAIN, class Poll, class Again>
-    __device__ __forceinline__ bool finish(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN], const Poll& poll, bool stop,
-                                           const Again& again) {
+    // From the wavefronts' partial tiles to C.  WSTRIDE: floats between the wavefronts' places in LDS.  False: the
+    // workgroup leaves a preempted launch.
+    template <int WSTRIDE, class Poll>
+    __device__ __forceinline__ bool finish(const OpDesc& d, char* smem_raw, int wave, const f32x4 (&acc)[TM][TN], const Poll& poll, bool stop) {
         float* smem = (float*)smem_raw;
         const int* a = d.attr;
         const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4, orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
@@ -3302,14 +3325,6 @@ struct GemmTail {
                 const float* e = mine + (h * TN + g) * TD::PART;
                 v[h][g] = ((e[0] + e[WSTRIDE]) + e[2 * WSTRIDE]) + e[3 * WSTRIDE];
             }
-        if (AGAIN) {
-#pragma unroll
-            for (int h = 0; h < TM; ++h)
-#pragma unroll
-                for (int g = 0; g < TN; ++g)
-                    if (!__builtin_isfinite(v[h][g]) && m0 + 16 * h + orow < M && n0 + 16 * g + ocol < N)
-                        v[h][g] = again(m0 + 16 * h + orow, n0 + 16 * g + ocol);
-        }
         if (split_k == 1) {
 #pragma unroll
             for (int h = 0; h < TM; ++h)
@@ -3577,7 +3592,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
             sum[h][g] = AC == 1   ? acc[h][g][0]
                         : AC == 2 ? acc[h][g][0] + acc[h][g][AC - 1]
                                   : (acc[h][g][0] + acc[h][g][AC > 2 ? 1 : 0]) + (acc[h][g][AC > 2 ? 2 : 0] + acc[h][g][AC > 3 ? 3 : 0]);
-    return t.template finish<TileGd<TM, TN>::WSTRIDE, false>(d, smem_raw, wave, sum, poll, left || raised, [](int, int) { return 0.0f; });
+    return t.template finish<TileGd<TM, TN>::WSTRIDE>(d, smem_raw, wave, sum, poll, left || raised);
 }
 
 // REEF_GEMM_F_SPLIT: B is stored as the three bf16 parts of each weight, and the parts of A are formed behind its turn through
@@ -3725,17 +3740,62 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
-    const float* A = (const float*)d.ptr[0] + d.attr[REEF_GEMM_OFF_A];
-    const unsigned short* B = (const unsigned short*)d.ptr[1];
-    return t.template finish<TileGd<TM, TN>::WSTRIDE, true>(d, smem_raw, wave, sum, poll, left || raised, [&](int m, int n) {
-        float s = 0.0f;
-        for (int k = t.k_lo; k < t.k_hi; ++k) {
-            const unsigned short* w = B + ((size_t)(n >> 4) * K32 + (k >> 5)) * 1536 + (((k >> 2) & 3) * 16 + (n & 15)) * 8 + ((k >> 4) & 1) * 4 + (k & 3);
-            const float wv = (__uint_as_float((unsigned)w[0] << 16) + __uint_as_float((unsigned)w[512] << 16)) + __uint_as_float((unsigned)w[1024] << 16);
-            s = fmaf(A[(size_t)m * t.lda + k], wv, s);
+    if (raised) left = true;
+    // What is infinite or NaN, again on 32-bit MFMAs: this wavefront's share of K, operands straight from memory, the weights put
+    // together from their parts, and the flag polled as above.  (128 x 768 x 3072 in 32x48, preemptible, a NaN in every row: 71
+    // us a request instead of 30; formed element by element, a thread at a time, 3150.)
+    if (!left && any_not_finite(sum)) {
+        constexpr int AC = TM * TN > 4 ? 1 : 2;      // as the 32-bit product of the tile has
+        f32x4 again[TM][TN][AC];
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+#pragma unroll
+                for (int e = 0; e < AC; ++e) again[h][g][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        pf = 0;
+#pragma unroll 1
+        for (it = 0; it < steps; ++it) {
+            if (Poll::enabled && pf) {
+                left = true;
+                break;
+            }
+            const int k = k0 + it * KSTEP + 4 * kq;      // k to k + 3 and k + 16 to k + 19 are this lane's, of rows and of columns
+            const unsigned out0 = k < t.k_hi ? 0u : kOutside, out1 = k + 16 < t.k_hi ? 0u : kOutside;
+            f32x4 x[TM][2];
+            u32x4 w[TN][3];
+#pragma unroll
+            for (int h = 0; h < TM; ++h) {
+                const unsigned at = ((unsigned)(t.m0 + 16 * h + i16) * (unsigned)t.lda + (unsigned)k) * 4u;
+                x[h][0] = buf_load4(t.rs_a, at | out0);
+                x[h][1] = buf_load4(t.rs_a, (at + 64u) | out1);
+            }
+#pragma unroll
+            for (int g = 0; g < TN; ++g)
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    w[g][e] = __builtin_bit_cast(u32x4, buf_load4(rs_b, ((unsigned)(t.n0 / 16 + g) * K32 + (unsigned)(k0 / 32 + 4 * it)) * 3072u +
+                                                                            (unsigned)lane * 16u + 1024u * e));
+            if (Poll::enabled) {
+                asm volatile("" ::: "memory");
+                pf = poll.load();
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) {
+                    const float v = planes_value(w[g][0], w[g][1], w[g][2], e);
+#pragma unroll
+                    for (int h = 0; h < TM; ++h)
+                        again[h][g][e % AC] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[h][e >> 2][e & 3], v, again[h][g][e % AC], 0, 0, 0);
+                }
         }
-        return s;
-    });
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) keep_finite(sum[h][g], AC == 1 ? again[h][g][0] : again[h][g][0] + again[h][g][AC - 1]);
+    }
+    return t.template finish<TileGd<TM, TN>::WSTRIDE>(d, smem_raw, wave, sum, poll, left);
 }
 
 template <int TM, int TN, bool LN, class Poll>

@@ -1,12 +1,14 @@
 """Matrix products on split weights (REEF_GEMM_F_SPLIT): the parts are the weight, and what has no parts in bf16 -- infinities,
 NaN, values that round to infinity -- comes out as it does on the weights themselves."""
 import os
+import time
 
 import numpy as np
 import pytest
 
 from reef_amd import binding as B
 from reef_amd.modelgen import builder as MB, tiling
+from tests.test_gpu_packed_convs import flavours_agree
 
 
 def bf16(u):
@@ -75,3 +77,52 @@ def test_product_of_split_operands(tmp_path, tile, shape):
         assert np.array_equal(np.isnan(want), np.isnan(y)) and np.array_equal(want[np.isinf(want)], y[np.isinf(want)])
         bound = 2 * (k + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).T.astype(np.float64))
         assert (np.abs(y[same].astype(np.float64) - want[same]) <= bound[same]).all()
+
+
+def loaded(d, tile, a, w, kind):
+    (m, k), n = a.shape, w.shape[0]
+    g = MB.GraphBuilder("nan")
+    wt = g.param((n, k), 0.5)
+    g.params[g._param_pos[wt.idx]][1][:] = w.reshape(-1)
+    out = g.gemm(g.input("a", (m, k)), wt, m, n, k, force_tile=tile, split_k=1)
+    g.mark_output(out)
+    assert g.kernels[0]["attrs"][5] & 32
+    g.write(os.path.join(str(d), "nan"))
+    exe = B.Executor.from_dir(os.path.join(str(d), "nan"), "nan", kind)
+    exe.set_input_checked("a", a)
+    return g, exe, out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tiling.GEMM_SPLIT_TILES)
+def test_flavours_agree_on_values_without_parts(tmp_path, tile):
+    m, n, k = 70, 100, 392
+    rng = np.random.default_rng(6)
+    a, w = rng.standard_normal((m, k)).astype(np.float32), (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    a[0, 1], a[1, 2], a[2, k - 1], a[40, 200], w[n // 2, 3] = np.inf, np.nan, -np.inf, 3.4e38, np.inf
+    g, exe, out = loaded(tmp_path, tile, a, w, B.BASE)
+    exe.execute()
+    assert not np.isfinite(exe.get_data(out.idx, m * n)).all()
+    flavours_agree(exe, g, tmp_path, {"a": a})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", ["32x48d4", "64x64d4"])
+def test_values_without_parts_cost_one_more_pass_over_the_depth(tmp_path, tile):
+    """A best-effort launch whose data holds NaN must not keep the device to itself (an element at a time it took a hundred
+    times as long)."""
+    m, n, k = 128, 768, 3072
+    rng = np.random.default_rng(7)
+    a, w = rng.standard_normal((m, k)).astype(np.float32), (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    _, exe, _ = loaded(tmp_path, tile, a, w, B.HYBRID)
+    best = []
+    for x in (a, np.full_like(a, np.nan)):
+        exe.set_input_checked("a", x)
+        times = []
+        for _ in range(8):
+            t0 = time.perf_counter()
+            exe.execute_preemptable()
+            times.append(time.perf_counter() - t0)
+        best.append(min(times))
+    exe.close()
+    assert best[1] < 5 * best[0], best
