@@ -228,6 +228,9 @@ size_t reef_ops_scratch_bytes(void);
  * split K take turns with it. */
 int reef_ops_conv2d_wait(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
                          const float* residual, float* out, int noalloc);
+/* The kernel that the three run this layer on, and into how many shares of K it is split (split_k may be null).
+ * Null: they refuse the layer.  No device is needed. */
+const char* reef_ops_conv2d_kernel(const reef_conv2d_desc* c, int* split_k);
 /* Frees the idle workspaces of reef_ops_conv2d. */
 int reef_ops_release(void);
 

@@ -452,3 +452,12 @@ def ops_conv2d(desc, inp, w, bias, residual, out, noalloc=False):
     """reef_ops_conv2d / reef_ops_conv2d_noalloc on DeviceBuffers, default stream, waited for; returns the status."""
     return lib().reef_ops_conv2d_wait(ctypes.byref(desc), inp.ptr, w.ptr, bias.ptr if bias is not None else None,
                                       residual.ptr if residual is not None else None, out.ptr, 1 if noalloc else 0)
+
+
+def ops_conv2d_kernel(desc):
+    """(symbol of the kernel, split of K) that reef_ops_conv2d runs this layer on; None if it refuses the layer."""
+    f = lib().reef_ops_conv2d_kernel
+    f.restype = ctypes.c_char_p
+    split = ctypes.c_int()
+    name = f(ctypes.byref(desc), ctypes.byref(split))
+    return (name.decode(), split.value) if name else None

@@ -367,24 +367,32 @@ const Geometry& chosen(const reef_conv2d_desc* c, int Ho, int Wo) {
     return s.g;
 }
 
-int make_plan(const reef_conv2d_desc* c, const float* in, const float* w,
-              const float* bias, const float* residual, float* out, Plan* p) {
-    if (!c || !in || !w || !out) return fail("reef_ops_conv2d: null argument");
+// Whether the layer is one that the kernels take; its output's size.
+int check_shape(const reef_conv2d_desc* c, int* Ho, int* Wo) {
     if (c->cin <= 0 || c->cout <= 0 || c->h <= 0 || c->w <= 0 || c->kh <= 0 || c->kw <= 0 || c->stride_h <= 0 ||
         c->stride_w <= 0 || c->pad_h < 0 || c->pad_w < 0)
         return fail("reef_ops_conv2d: bad shape");
-    const int Ho = (c->h + 2 * c->pad_h - c->kh) / c->stride_h + 1;
-    const int Wo = (c->w + 2 * c->pad_w - c->kw) / c->stride_w + 1;
-    if (Ho <= 0 || Wo <= 0) return fail("reef_ops_conv2d: empty output");
+    *Ho = (c->h + 2 * c->pad_h - c->kh) / c->stride_h + 1;
+    *Wo = (c->w + 2 * c->pad_w - c->kw) / c->stride_w + 1;
+    if (*Ho <= 0 || *Wo <= 0) return fail("reef_ops_conv2d: empty output");
     if (c->act != REEF_ACT_NONE && c->act != REEF_ACT_RELU && c->act != REEF_ACT_RELU6)
         return fail("reef_ops_conv2d: unknown activation");
-    const int M = c->cout, N = Ho * Wo, taps = c->kh * c->kw;
-    const long long K = (long long)c->cin * taps;
+    const int M = c->cout, N = *Ho * *Wo;
+    const long long K = (long long)c->cin * c->kh * c->kw;
     if ((long long)M * N >= (1ll << 28) || K * M >= (1ll << 28) || (long long)c->cin * c->h * c->w >= (1ll << 28))
         return fail("reef_ops_conv2d: tensor of 1 GiB or more");
     // the kernels decode pixel, tile and task numbers with a float reciprocal that is exact below 2^22
     if (N >= (1 << 22) || (long long)c->h * c->w >= (1 << 22))
         return fail("reef_ops_conv2d: image of 4 Mi pixels or more");
+    return 0;
+}
+
+int make_plan(const reef_conv2d_desc* c, const float* in, const float* w,
+              const float* bias, const float* residual, float* out, Plan* p) {
+    if (!c || !in || !w || !out) return fail("reef_ops_conv2d: null argument");
+    int Ho = 0, Wo = 0;
+    if (int rc = check_shape(c, &Ho, &Wo)) return rc;
+    const int M = c->cout, N = Ho * Wo;
     const Geometry& g = chosen(c, Ho, Wo);
     const Kernel& k = kKernels[g.kernel];
     const int split = g.split, tiles = g.m_tiles * g.n_tiles;
@@ -563,6 +571,14 @@ int reef_ops_conv2d_noalloc(const reef_conv2d_desc* c, const float* in, const fl
 int reef_ops_conv2d_wait(const reef_conv2d_desc* c, const float* in, const float* w, const float* bias,
                          const float* residual, float* out, int noalloc) {
     return run(c, in, w, bias, residual, out, nullptr, noalloc != 0, true);
+}
+
+const char* reef_ops_conv2d_kernel(const reef_conv2d_desc* c, int* split_k) {
+    int Ho = 0, Wo = 0;
+    if (!c || check_shape(c, &Ho, &Wo)) return nullptr;
+    const Geometry& g = chosen(c, Ho, Wo);
+    if (split_k) *split_k = g.split;
+    return kKernels[g.kernel].symbol;
 }
 
 int reef_ops_release(void) {

@@ -20,12 +20,17 @@ def run(x, w, b, res, act):
     return out.to_array().reshape(cout, H, W)
 
 
-# cin, H, W, cout: whole tiles; every edge ragged; few channels in; one column behind a segment
-@pytest.mark.parametrize("case", [(256, 112, 112, 256), (252, 113, 83, 270), (44, 139, 111, 326), (84, 95, 97, 348)])
+# cin, H, W, cout, image rows: whole tiles; every edge ragged; few channels in; one column behind a segment; the same of four
+# rows a tile: every edge ragged; whole rows of tiles; one column and one output channel behind the last tile
+CASES = [(256, 112, 112, 256, 7), (252, 113, 83, 270, 7), (44, 139, 111, 326, 7), (84, 95, 97, 348, 7),
+         (120, 86, 56, 292, 4), (580, 12, 79, 717, 4), (192, 98, 29, 369, 4), (276, 23, 129, 257, 4)]
+
+
+@pytest.mark.parametrize("case", CASES)
 @pytest.mark.parametrize("residual", [False, True])
 def test_against_64_bits(case, residual):
     B.ops_init()
-    cin, H, W, cout = case
+    cin, H, W, cout, _ = case
     rng = np.random.default_rng(11)
     x = rng.standard_normal((cin, H, W)).astype(np.float32)
     w = (rng.standard_normal((cout, cin, 3, 3)) * np.sqrt(2.0 / (cin * 9))).astype(np.float32)

@@ -78,3 +78,13 @@ def test_a_packed_layer_and_the_entry_of_its_shape(cout, cin, taps, side, loaded
         assert kind in ("v", "w") and packed["split_k"] == 1 and not packed["fused"]
     else:
         assert packed == plain
+
+
+def test_the_layers_of_the_image_patch_tests_run_on_image_patches():
+    from reef_amd import binding as B
+    from tests.test_gpu_image_patches import CASES
+    assert {c[4] for c in CASES} == {4, 7}
+    for cin, H, W, cout, rows in CASES:
+        assert B.ops_conv2d_kernel(B.Conv2dDesc(cin, H, W, cout, 3, 3, 1, 1, 1, 1, 1)) == ("reef_conv2d_x9_g%d" % rows, 1)
+    assert B.ops_conv2d_kernel(B.Conv2dDesc(254, 112, 112, 256, 3, 3, 1, 1, 1, 1, 1))[0].startswith("reef_conv2d_r9_")
+    assert B.ops_conv2d_kernel(B.Conv2dDesc(4, 8, 8, 4, 3, 3, 0, 1, 1, 1, 0)) is None
