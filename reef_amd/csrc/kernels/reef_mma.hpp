@@ -1962,22 +1962,49 @@ struct TileX9 {
     static constexpr int WROW = 576 + 16, WEIGHTS = 2 * BUF;      // a filter's 16 channels, padding
     static constexpr int LDS_BYTES = WEIGHTS + 64 * WROW;
 };
-// One output of a convolution in 32 bits.
-__device__ __forceinline__ float conv2d_element(const OpDesc& d, int m, int n) {
-    const int* a = d.attr;
-    const int C = a[REEF_CONV_CIN], H = a[REEF_CONV_H], W = a[REEF_CONV_W], kh = a[REEF_CONV_KH], kw = a[REEF_CONV_KW], Wo = a[REEF_CONV_WO];
-    const int y = div_small(n, Wo), x = n - y * Wo;
-    const int iy = y * a[REEF_CONV_SH] - a[REEF_CONV_PH], ix = x * a[REEF_CONV_SW] - a[REEF_CONV_PW];
-    const float* w = (const float*)d.ptr[1] + (size_t)m * C * kh * kw;
-    const float* in = (const float*)d.ptr[0];
-    float s = 0.0f;
-    for (int c = 0; c < C; ++c)
-        for (int ky = 0; ky < kh; ++ky)
-            for (int kx = 0; kx < kw; ++kx) {
-                const bool ok = (unsigned)(iy + ky) < (unsigned)H && (unsigned)(ix + kx) < (unsigned)W;
-                s = fmaf(*w++, ok ? in[((size_t)c * H + iy + ky) * W + ix + kx] : 0.0f, s);
+// The outputs of a wavefront of conv2d_x9_body (16 channels from m0, G rows from y0, 16 columns from x0) on 32-bit MFMAs, operands
+// straight from memory: four channels a step, a lane the filter of one and the pixels of its column; sums are taken over
+// 32 channels at a time, two chains each.
+template <int G>
+__device__ __forceinline__ void conv2d_x9_again(rsrc_t rs_a, rsrc_t rs_b, int C, int H, int W, int m0, int y0, int x0, f32x4 (&sum)[G]) {
+    const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+    const unsigned HW4 = (unsigned)(H * W) * 4u;
+    unsigned at[G + 2][3];
+#pragma unroll
+    for (int r = 0; r < G + 2; ++r)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+            const int iy = y0 - 1 + r, ix = x0 - 1 + i16 + dx;
+            at[r][dx] = (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W ? (unsigned)kq * HW4 + (unsigned)(iy * W + ix) * 4u : kOutside;
+        }
+    const unsigned wat = ((unsigned)(m0 + i16) * (unsigned)C + (unsigned)kq) * 36u;
+#pragma unroll
+    for (int g = 0; g < G; ++g) sum[g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int c0 = 0; c0 < C; c0 += 32) {
+        f32x4 acc[G][2];
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g][0] = acc[g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int c = c0; c < min(c0 + 32, C); c += 4) {      // (C is a multiple of 4)
+            const f32x4 w0 = buf_load4(rs_a, wat + (unsigned)c * 36u), w1 = buf_load4(rs_a, wat + (unsigned)c * 36u + 16u);
+            const float w2 = buf_load(rs_a, wat + (unsigned)c * 36u + 32u);
+            float x[G + 2][3];
+#pragma unroll
+            for (int r = 0; r < G + 2; ++r)
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) x[r][dx] = buf_load(rs_b, at[r][dx] + (unsigned)c * HW4);
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const float w = t < 4 ? w0[t & 3] : t < 8 ? w1[t & 3] : w2;
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+                    acc[g][t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, x[g + t / 3][t % 3], acc[g][t & 1], 0, 0, 0);
             }
-    return s;
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) sum[g] += acc[g][0] + acc[g][1];
+    }
 }
 template <int G>
 __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* smem) {
@@ -2126,17 +2153,26 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
     ConvEpilogue ep;
     ep.init(d, a[REEF_CONV_FLAGS], a[REEF_CONV_ACT], a[REEF_CONV_ACT2], M, (unsigned)M * HW4, (unsigned)a[REEF_CONV_DST_OFF] * 4u);
     const int x = x0 + i16;
+    f32x4 sum[1][G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) sum[0][g] = (acc[g][0] + acc[g][1]) + acc[g][2];
+    // What is infinite or NaN, again in 32 bits (256 channels to 256 at 112 x 112, NaN everywhere: 246 us a call instead of
+    // 103; formed element by element, a thread at a time, 8300).
+    if (any_not_finite(sum)) {
+        f32x4 again[G];
+        conv2d_x9_again<G>(rs_a, rs_b, C, H, W, m0, y0, x0, again);
+#pragma unroll
+        for (int g = 0; g < G; ++g) keep_finite(sum[0][g], again[g]);
+    }
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        f32x4 sum = (acc[g][0] + acc[g][1]) + acc[g][2];
         const int n = (y0 + g) * W + x;
         const bool ok = x < W && y0 + g < H;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int m = m0 + 4 * kq + j;
-            if (!__builtin_isfinite(sum[j]) && ok && m < M) sum[j] = conv2d_element(d, m, n);
             const unsigned off = ok ? ((unsigned)m * (unsigned)N + (unsigned)n) * 4u : kOutside, m4 = (unsigned)m * 4u;
-            ep.finish(sum[j], off, m4, ep.has_res ? buf_load(ep.res, off) : 0.0f, ep.has_bias ? buf_load(ep.bias, m4) : 0.0f,
+            ep.finish(sum[0][g][j], off, m4, ep.has_res ? buf_load(ep.res, off) : 0.0f, ep.has_bias ? buf_load(ep.bias, m4) : 0.0f,
                       ep.has_dual ? buf_load(ep.shift2, m4) : 0.0f);
         }
     }

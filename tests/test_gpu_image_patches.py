@@ -1,5 +1,7 @@
 """Large 3x3 layers through reef_ops_conv2d (reef_conv2d_x9_g*): sizes that end inside a tile, a step of channels and a
 group of output channels, a residual, and values that have no parts in bf16."""
+import time
+
 import numpy as np
 import pytest
 
@@ -74,4 +76,45 @@ def test_values_without_parts():
     np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
     ok = np.isfinite(want)
     # a value of 3.4e38 in the sum: its product decides
+    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[4]])
+def test_values_without_parts_cost_one_more_pass_over_the_channels(case):
+    """NaN all over: an element at a time it took eighty times as long."""
+    B.ops_init()
+    cin, H, W, cout, _ = case
+    rng = np.random.default_rng(13)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w = B.DeviceBuffer.from_array((rng.standard_normal((cout, cin, 3, 3)) * 0.02).astype(np.float32))
+    d, out = B.Conv2dDesc(cin, H, W, cout, 3, 3, 1, 1, 1, 1, 0), B.DeviceBuffer(cout * H * W * 4)
+    best = []
+    for data in (x, np.full_like(x, np.nan)):
+        inp, times = B.DeviceBuffer.from_array(data), []
+        for _ in range(8):
+            t0 = time.perf_counter()
+            assert B.ops_conv2d(d, inp, w, None, None, out) == 0, B.last_error()
+            times.append(time.perf_counter() - t0)
+        best.append(min(times))
+    assert np.isnan(out.to_array()).all() and best[1] < 5 * best[0], best
+
+
+@pytest.mark.parametrize("case", [CASES[5], CASES[7]])
+def test_values_without_parts_at_the_edges(case):
+    """Infinities and NaN in the corners, in the last channel and in filters: the oracle's classes, everywhere."""
+    B.ops_init()
+    cin, H, W, cout, _ = case
+    rng = np.random.default_rng(14)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3, 3)) * 0.02).astype(np.float32)
+    x[0] = np.clip(x[0], -0.9, 0.9)      # (times 3.4e38 below the largest value: beside an infinity no sum depends on its order)
+    x[cin - 1, H - 1, W - 1], x[0, 0, 0], x[cin // 2, 0, W - 1], x[5, H - 1, 0], x[3, H // 2, 16] = np.inf, np.nan, -np.inf, 3.4e38, np.inf
+    # (filters in the middle tap: the pixels around the image are zeros that every kernel here multiplies, and the oracle leaves out)
+    w[cout - 1, cin - 1, 1, 1], w[17, 2, 1, 1], w[33, 0, 2, 0] = np.inf, np.nan, 3.4e38
+    got = run(x, w, None, None, 0)
+    with np.errstate(all="ignore"):
+        want = O.conv2d(x, w, np.zeros(cout, np.float32), None, None, None, (1, 1), (1, 1), 1, 0, 6.0, False).reshape(cout, H, W)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
     np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-3)
