@@ -749,14 +749,17 @@ __device__ __forceinline__ bool conv2d_body(const OpDesc& d_in, int task, char* 
 // five small products have an accumulator of their own, so that what is rounded into the large one is h h alone, once per
 // 32 values of k and not once per 4: errors against 64 bits are half of those of two 32-bit chains (K = 768, normal: 1.58e-7
 // against 3.51e-7; after a ReLU 1.22e-7 against 2.51e-7; K = 2304: 2.9e-7 against 6.1e-7).
-// What has no such sum -- infinities, NaN, values that round to infinity -- makes every product it is in infinite or
-// NaN; the kernels form an element that comes out so again, in 32 bits.  (Below 2^-110 l falls under the smallest bf16:
-// such values keep 2^-133 absolute.)
+// What has no such sum: infinities, NaN and values that round to infinity make every product that they are in infinite or
+// NaN; the kernels form a sum that comes out so again, in 32 bits.  Below 2^-110 l ends under the smallest bf16, 2^-133
+// (bf16 MFMAs keep denormals, and what is small only as a product loses nothing); the kernels see that by the bits for which l
+// has no room, and add the products of what is left over in 32 bits.  (Without: 5e-6 from 64 bits at 1e-35, 5e-4 at 1e-37.)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 struct Planes { u32x4 h, m, l; };      // eight values
-__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+// lost: has bits of its lower half set once a finite value was not the sum of its parts (one operation for both; written out,
+// because the compiler collects them behind others and runs out of registers: ntl_64x64).
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l, unsigned& lost) {
     bf16x2 r;
     r[0] = (__bf16)a;
     r[1] = (__bf16)b;
@@ -767,15 +770,16 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsign
     m = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
     a -= __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
     b -= __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
+    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a), "v"(b));
     l = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-__device__ __forceinline__ Planes split_planes(const f32x4& a, const f32x4& b) {
+__device__ __forceinline__ Planes split_planes(const f32x4& a, const f32x4& b, unsigned& lost) {
     Planes p;
     unsigned h, m, l;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const f32x4& v = i < 2 ? a : b;
-        split_pair(v[2 * (i & 1)], v[2 * (i & 1) + 1], h, m, l);
+        split_pair(v[2 * (i & 1)], v[2 * (i & 1) + 1], h, m, l, lost);
         p.h[i] = h;
         p.m[i] = m;
         p.l[i] = l;
@@ -814,6 +818,13 @@ __device__ __forceinline__ bool any_not_finite(const f32x4 (&v)[TM][TN]) {
 __device__ __forceinline__ void keep_finite(f32x4& v, const f32x4& other) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = __builtin_isfinite(v[j]) ? v[j] : other[j];
+}
+// What its parts leave of a value: 0 from 2^-110 on.
+__device__ __forceinline__ float left_over(float a) {
+    a -= (float)(__bf16)a;
+    a -= __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+    a -= __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+    return fabsf(a) < 0x1p-126f ? a : 0.0f;      // (0 for what has no parts)
 }
 // Value e (0 to 7) of the eight whose parts these are.
 __device__ __forceinline__ float planes_value(const u32x4& h, const u32x4& m, const u32x4& l, int e) {
@@ -2069,6 +2080,7 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     typedef unsigned u32x4_at8 __attribute__((ext_vector_type(4), aligned(8)));
     Planes w[5];
+    unsigned lost = 0;
     // taps of the two halves of an MFMA: left and middle of filter row 0, 1, 2; right of rows 0 and 1; right of row 2
     auto split_weights = [&](bool more) {
 #pragma unroll
@@ -2090,7 +2102,7 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
             for (int e = 0; e < 4; ++e) {
                 const int t = e < 2 ? TA[p] : TB[p], q = 2 * (e & 1);
                 unsigned h = 0, m = 0, l = 0;
-                if (t >= 0) split_pair(v[t < 0 ? 0 : q * 9 + t], v[t < 0 ? 0 : (q + 1) * 9 + t], h, m, l);
+                if (t >= 0) split_pair(v[t < 0 ? 0 : q * 9 + t], v[t < 0 ? 0 : (q + 1) * 9 + t], h, m, l, lost);
                 w[p].h[e] = h;
                 w[p].m[e] = m;
                 w[p].l[e] = l;
@@ -2102,8 +2114,8 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             unsigned h0, m0_, l0, h1, m1, l1;
-            split_pair(rb[k][0], rb[k][1], h0, m0_, l0);
-            split_pair(rb[k][2], rb[k][3], h1, m1, l1);
+            split_pair(rb[k][0], rb[k][1], h0, m0_, l0, lost);
+            split_pair(rb[k][2], rb[k][3], h1, m1, l1, lost);
             if (wr[k] >= 0) {
                 char* p = smem + buf + wr[k];
                 *(u32x2*)p = u32x2{h0, h1};
@@ -3244,7 +3256,7 @@ struct GemmTail {
             ls1[LN ? h : 0] = ls2[LN ? h : 0] = 0.0f;
         }
     }
-    // Bias, residual and the LayerNorm's operands.
+    // Bias and the LayerNorm's operands.
     __device__ __forceinline__ void fetch(const OpDesc& d) {
         const int* a = d.attr;
         const unsigned ldc = (unsigned)a[REEF_GEMM_LDC];
@@ -3253,9 +3265,6 @@ struct GemmTail {
         has_bias = a[REEF_GEMM_FLAGS] & REEF_GEMM_F_BIAS;
         has_res = a[REEF_GEMM_FLAGS] & REEF_GEMM_F_RES;
         const rsrc_t rs_bias = make_rsrc(d.ptr[has_bias ? 3 : 2], (unsigned)N * 4u);
-        // the residual is laid out as C is; without one an empty buffer, whose loads give 0
-        const rsrc_t rs_res = make_rsrc((const float*)d.ptr[has_res ? (has_bias ? 4 : 3) : 2] + at_c,
-                                        has_res ? ((unsigned)(M - 1) * ldc + (unsigned)N) * 4u : 0u);
         const int orow = threadIdx.x >> 4, ocol = threadIdx.x & 15;
         const int lnp = 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0);
         if (LN) {      // c1 and c2 of this thread's columns
@@ -3275,10 +3284,20 @@ struct GemmTail {
             for (int h = 0; h < TM; ++h) {
                 const unsigned m = (unsigned)(m0 + 16 * h + orow);
                 ooff[h][g] = n < (unsigned)N ? (m * ldc + n) * 4u : kOutside;
-                e_res[h][g] = buf_load(rs_res, ooff[h][g]);
             }
         }
         if (LN) ln_out.init(d, lnp, (const float*)d.ptr[0], M, K, lda, m0, TD::BM, nt, a[REEF_GEMM_N_TILES]);
+    }
+    // The residual, which is laid out as C is; without one an empty buffer, whose loads give 0.
+    __device__ __forceinline__ void fetch_residual(const OpDesc& d) {
+        const int* a = d.attr;
+        const size_t at_c = (size_t)a[REEF_GEMM_OFF_C] + (size_t)batch * a[REEF_GEMM_STRIDE_C];
+        const rsrc_t rs_res = make_rsrc((const float*)d.ptr[has_res ? (has_bias ? 4 : 3) : 2] + at_c,
+                                        has_res ? ((unsigned)(M - 1) * (unsigned)a[REEF_GEMM_LDC] + (unsigned)N) * 4u : 0u);
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) e_res[h][g] = buf_load(rs_res, ooff[h][g]);
     }
     // `count` values of row 16 h + lane % 16 of A into the row's sums; in: 1, or 0 for values outside K, which read as 0.
     template <class V>
@@ -3290,6 +3309,16 @@ struct GemmTail {
             ls1[LN ? h : 0] += dl;
             ls2[LN ? h : 0] = fmaf(dl, dl, ls2[LN ? h : 0]);
         }
+    }
+    // Where this thread's elements lie in C, again: not kept in registers through a K loop that needs them all.
+    __device__ __forceinline__ void place_out(const OpDesc& d) {
+        int self = threadIdx.x;
+        asm volatile("" : "+v"(self));
+        const unsigned ldc = (unsigned)d.attr[REEF_GEMM_LDC], at = (unsigned)(m0 + (self >> 4)) * ldc + (unsigned)(n0 + (self & 15));
+#pragma unroll
+        for (int h = 0; h < TM; ++h)
+#pragma unroll
+            for (int g = 0; g < TN; ++g) ooff[h][g] = n0 + 16 * g + (self & 15) < N ? (at + 16u * h * ldc + 16u * g) * 4u : kOutside;
     }
     // From the wavefronts' partial tiles to C.  WSTRIDE: floats between the wavefronts' places in LDS.  False: the
     // workgroup leaves a preempted launch.
@@ -3472,6 +3501,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     t.template place<false>(d, task);
     t.fetch_pivots();
     t.fetch(d);
+    t.fetch_residual(d);
     const int* a = d.attr;
     const unsigned ldb = (unsigned)a[REEF_GEMM_LDB];
     const rsrc_t rs_b = make_rsrc((const float*)d.ptr[1] + a[REEF_GEMM_OFF_B] + (size_t)t.batch * a[REEF_GEMM_STRIDE_B],
@@ -3653,9 +3683,11 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     GemmTail<TM, TN, LN> t;
     t.template place<true>(d, task);
     t.fetch_pivots();
-    // what the epilogue needs, ahead of the K loop, unless registers run out for it
+    // what the epilogue needs, ahead of the K loop, unless registers run out for it: behind a LayerNorm the residual comes late
+    // (a LayerNorm's products that have one are few)
     constexpr bool LATE = LN && TM * TN >= 16 && REEF_FLAVOUR == 2;
     if (!LATE) t.fetch(d);
+    if (!LN) t.fetch_residual(d);
     const int k0 = t.k_lo + 32 * wave;                                                   // first k of this wavefront
     const int steps = k0 < t.k_hi ? (t.k_hi - k0 + KSTEP - 1) / KSTEP : 0;               // its steps (uniform)
     const unsigned K32 = (unsigned)(t.K + 31) / 32u;
@@ -3716,6 +3748,7 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     };
     int ln_k = k0 + 4 * kq;
     Planes pa[TM];
+    unsigned lost = 0;
     auto split_rows = [&]() {
         if (LN) {      // values outside K were loaded as zeros: 0 - 0
             const float in0 = ln_k < t.K ? 1.0f : 0.0f, in1 = ln_k + 16 < t.K ? 1.0f : 0.0f;
@@ -3727,7 +3760,7 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
             }
         }
 #pragma unroll
-        for (int h = 0; h < TM; ++h) pa[h] = split_planes(av[h][0], av[h][1]);
+        for (int h = 0; h < TM; ++h) pa[h] = split_planes(av[h][0], av[h][1], lost);
     };
     auto multiply = [&](int s) {
 #pragma unroll
@@ -3770,17 +3803,23 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
                 multiply(s);
             }
     }
-    if (LATE) t.fetch(d);
     f32x4 sum[TM][TN];
 #pragma unroll
     for (int h = 0; h < TM; ++h)
 #pragma unroll
         for (int g = 0; g < TN; ++g) sum[h][g] = acc[h][g][0] + acc[h][g][1];
     if (raised) left = true;
-    // What is infinite or NaN, again on 32-bit MFMAs: this wavefront's share of K, operands straight from memory, the weights put
-    // together from their parts, and the flag polled as above.  (128 x 768 x 3072 in 32x48, preemptible, a NaN in every row: 71
-    // us a request instead of 30; formed element by element, a thread at a time, 3150.)
-    if (!left && any_not_finite(sum)) {
+    // What the parts of A leave over, and then what is infinite or NaN, on 32-bit MFMAs: this wavefront's share of K, operands
+    // straight from memory, the weights (which are the sum of their parts) put together, and the flag polled as above.
+    // (128 x 768 x 3072 in 32x48, preemptible, NaN in every row 63 us a request and values of 1e-36 75 us, instead of 31; NaN
+    // formed element by element, a thread at a time, 3150.)
+    const bool again_for[2] = {__any((lost & 0xFFFFu) != 0) != 0, any_not_finite(sum)};
+    int self = threadIdx.x & 63;
+    asm volatile("" : "+v"(self));      // (nothing of this is kept in registers through the loop above)
+    const int row = self & 15, slot = self >> 4;
+#pragma unroll 1
+    for (int whole = 0; whole < 2; ++whole) {
+        if (left || !(whole ? again_for[1] : again_for[0])) continue;
         constexpr int AC = TM * TN > 4 ? 1 : 2;      // as the 32-bit product of the tile has
         f32x4 again[TM][TN][AC];
 #pragma unroll
@@ -3796,13 +3835,13 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
                 left = true;
                 break;
             }
-            const int k = k0 + it * KSTEP + 4 * kq;      // k to k + 3 and k + 16 to k + 19 are this lane's, of rows and of columns
+            const int k = k0 + it * KSTEP + 4 * slot;      // k to k + 3 and k + 16 to k + 19 are this lane's, of rows and of columns
             const unsigned out0 = k < t.k_hi ? 0u : kOutside, out1 = k + 16 < t.k_hi ? 0u : kOutside;
             f32x4 x[TM][2];
             u32x4 w[TN][3];
 #pragma unroll
             for (int h = 0; h < TM; ++h) {
-                const unsigned at = ((unsigned)(t.m0 + 16 * h + i16) * (unsigned)t.lda + (unsigned)k) * 4u;
+                const unsigned at = ((unsigned)(t.m0 + 16 * h + row) * (unsigned)t.lda + (unsigned)k) * 4u;
                 x[h][0] = buf_load4(t.rs_a, at | out0);
                 x[h][1] = buf_load4(t.rs_a, (at + 64u) | out1);
             }
@@ -3811,11 +3850,15 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
 #pragma unroll
                 for (int e = 0; e < 3; ++e)
                     w[g][e] = __builtin_bit_cast(u32x4, buf_load4(rs_b, ((unsigned)(t.n0 / 16 + g) * K32 + (unsigned)(k0 / 32 + 4 * it)) * 3072u +
-                                                                            (unsigned)lane * 16u + 1024u * e));
+                                                                            (unsigned)self * 16u + 1024u * e));
             if (Poll::enabled) {
                 asm volatile("" ::: "memory");
                 pf = poll.load();
             }
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[h][e >> 2][e & 3] = whole ? x[h][e >> 2][e & 3] : left_over(x[h][e >> 2][e & 3]);
 #pragma unroll
             for (int e = 0; e < 8; ++e)
 #pragma unroll
@@ -3829,7 +3872,21 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
 #pragma unroll
         for (int h = 0; h < TM; ++h)
 #pragma unroll
-            for (int g = 0; g < TN; ++g) keep_finite(sum[h][g], AC == 1 ? again[h][g][0] : again[h][g][0] + again[h][g][AC - 1]);
+            for (int g = 0; g < TN; ++g) {
+                const f32x4 r = AC == 1 ? again[h][g][0] : again[h][g][0] + again[h][g][AC - 1];
+                if (whole) keep_finite(sum[h][g], r);
+                else sum[h][g] += r;
+            }
+    }
+    if (LATE) t.fetch(d);
+    t.place_out(d);
+    if (LN) {
+        if (t.has_res) t.fetch_residual(d);
+        else
+#pragma unroll
+            for (int h = 0; h < TM; ++h)
+#pragma unroll
+                for (int g = 0; g < TN; ++g) t.e_res[h][g] = 0.0f;
     }
     return t.template finish<TileGd<TM, TN>::WSTRIDE>(d, smem_raw, wave, sum, poll, left);
 }

@@ -131,12 +131,16 @@ class GraphBuilder:
         return Tensor(idx, (arr.size,))
 
     def packed_matrix(self, b, N, K, split=False):
-        """The packed copy of weights b [N][K] for the direct products (ldb = 0), one per matrix and form."""
-        key = self.storage[b.idx]["name"] + ("xpk" if split else "pk")
-        if key not in self._packed:
-            W = self.param_array(b).reshape(N, K)
-            self._packed[key] = self.derived_param(key, split_matrix(W) if split else pack_conv_weights(W[:, :, None], by_channels=True))
-        return self._packed[key]
+        """The packed copy of weights b [N][K] for the direct products (ldb = 0), one per matrix and form, and whether it is
+        the split one (of weights that are not the sum of their parts it is not)."""
+        W = self.param_array(b).reshape(N, K)
+        for split in (True, False) if split else (False,):
+            key = self.storage[b.idx]["name"] + ("xpk" if split else "pk")
+            if key not in self._packed:
+                arr = split_matrix(W) if split else pack_conv_weights(W[:, :, None], by_channels=True)
+                self._packed[key] = None if arr is None else self.derived_param(key, arr)
+            if self._packed[key] is not None:
+                return self._packed[key], split
 
     def _sync_counters(self, n):
         """Reserves n counters in the model's sync storage; returns (storage idx, first counter)."""
@@ -688,7 +692,8 @@ class GraphBuilder:
         packed = packed and direct
         split = packed and t["tile"] in tiling.GEMM_SPLIT_TILES
         if packed and ln is None:
-            args[1] = self.packed_matrix(b, N, K, split).idx
+            copy, split = self.packed_matrix(b, N, K, split)
+            args[1] = copy.idx
         if ln is not None:
             # Wg = W gamma (column k scaled by gamma[k]); c1 = its row sums; c2 = W beta
             assert ldb == K and off_b == 0, "the LayerNorm form takes the weight matrix whole"
@@ -697,8 +702,10 @@ class GraphBuilder:
             bt = self.param_array(ln["beta"]).astype(np.float64)
             wkey = self.storage[b.idx]["name"]
             Wg = (W * gm[None, :]).astype(np.float32)
+            parts = split_matrix(Wg) if split else None
+            split = parts is not None
             # the storage named wkey keeps W itself
-            args[1] = (self.derived_param(wkey + "gkxpk", split_matrix(Wg)) if split
+            args[1] = (self.derived_param(wkey + "gkxpk", parts) if split
                        else self.derived_param(wkey + "gkpk", pack_conv_weights(Wg[:, :, None], by_channels=True)) if packed
                        else self.derived_param(wkey + "gk", Wg)).idx
             ln = dict(ln, c1=self.derived_param(wkey + "sk", Wg.astype(np.float64).sum(axis=1)),
@@ -862,7 +869,8 @@ def pack_conv_weights(w, by_channels=False):
 def split_matrix(w):
     """[N][K] weights -> the layout of REEF_GEMM_F_SPLIT: each value as the sum of three bf16 values (the first rounded to
     nearest, or cut off where that would be infinite; the second the next eight bits; the third the rest),
-    [ceil(N/16)][ceil(K/32)][3 parts][4 slots][16 columns][8 values of k]: 4 * slot + 0..3 and 16 + 4 * slot + 0..3 of the 32."""
+    [ceil(N/16)][ceil(K/32)][3 parts][4 slots][16 columns][8 values of k]: 4 * slot + 0..3 and 16 + 4 * slot + 0..3 of the 32.
+    None where a finite weight is not the sum of its parts (below 2^-110, if it has bits under the smallest bf16)."""
     N, K = w.shape
     n, k = -(-N // 16), -(-K // 32)
     x = np.zeros((n * 16, k * 32), np.float32)
@@ -876,7 +884,9 @@ def split_matrix(w):
     h = np.where(fits, near, (u & np.uint32(0xFFFF0000)) | np.where(nan, np.uint32(0x400000), np.uint32(0)))
     r = np.where(finite, x, np.float32(0)) - np.where(finite, h, np.uint32(0)).view(np.float32)
     m = r.view(np.uint32) & np.uint32(0xFFFF0000)
-    l = (r - m.view(np.float32)).view(np.uint32) & np.uint32(0xFFFF0000)
+    l = (r - m.view(np.float32)).view(np.uint32)
+    if (l & np.uint32(0xFFFF)).any():
+        return None
     parts = [(p >> np.uint32(16)).astype(np.uint16).reshape(n, 16, k, 2, 4, 4).transpose(0, 2, 4, 1, 3, 5) for p in (h, m, l)]
     return np.ascontiguousarray(np.stack(parts, axis=2)).reshape(-1).view(np.float32)
 

@@ -126,3 +126,63 @@ def test_values_without_parts_cost_one_more_pass_over_the_depth(tmp_path, tile):
         best.append(min(times))
     exe.close()
     assert best[1] < 5 * best[0], best
+
+
+def test_weights_that_are_not_the_sum_of_their_parts_are_not_split():
+    w = np.full((20, 40), 0.5, np.float32)
+    for x, exact in ((2.0 ** -110 * (1 + 2.0 ** -23), True), (2.0 ** -111 * (1 + 2.0 ** -23), False), (2.0 ** -111 * (1 + 2.0 ** -22), True),
+                     (2.0 ** -133, True), (2.0 ** -134, False), (-1e-40, False), (2.0 ** -149, False)):
+        w[7, 11] = x
+        assert (MB.split_matrix(w) is not None) == exact, x
+        g = MB.GraphBuilder("tiny")
+        wt, gamma = g.param(w.shape, 0.5), g.param((40,), 0.5)
+        g.params[g._param_pos[wt.idx]][1][:] = w.reshape(-1)
+        g.params[g._param_pos[gamma.idx]][1][:] = 1.0
+        a = g.input("a", (33, 40))
+        for ln in (None, dict(gamma=gamma, beta=gamma)):
+            g.gemm(a, wt, 33, 20, 40, force_tile="32x48d4", ln=ln)
+            g.gemm(a, wt, 33, 20, 40, force_tile="16x32k4", ln=ln)
+        names = [g.storage[k["args"][1]]["name"] for k in g.kernels]
+        p = g.storage[wt.idx]["name"]
+        assert names == [p + s for s in (("xpk", "pk", "gkxpk", "gkpk") if exact else ("pk", "pk", "gkpk", "gkpk"))]
+        assert [bool(k["attrs"][5] & 32) for k in g.kernels] == [exact, False] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-28, 1e-30, 1e-32, 1e-34, 1e-36, 1e-38])
+@pytest.mark.parametrize("tile", tiling.GEMM_SPLIT_TILES)
+def test_small_operands_are_as_exact_as_in_32_bits(tmp_path, tile, scale):
+    """(At 1e-36 the parts of a value keep 15 bits of it.)  The errors are thousands of alike and independent ones: 1.1 for what their
+    root mean square is known to.  Beside it the roundings of sums near the smallest normal value, to 2^-149: a standard deviation
+    of 2^-149 / 12^0.5 each, a quarter, six and a quarter again for every four and 32 values of k in 32 bits, in parts and for
+    what these leave."""
+    m, n, k = 64, 256, 768
+    rng = np.random.default_rng(8)
+    a = (rng.standard_normal((m, k)) * scale).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    want = a.astype(np.float64) @ w.T.astype(np.float64)
+    errs = [np.linalg.norm(product(tmp_path, "p%d" % packed, tile, a, w, 1, packed).astype(np.float64) - want) / np.linalg.norm(want)
+            for packed in (False, True)]
+    small = 2.0 ** -149 / 12 ** 0.5 * (k / 4 + 6 * k / 32) ** 0.5 / np.sqrt((want ** 2).mean())
+    assert errs[1] <= 1.1 * errs[0] + small, (errs, small)
+    if scale > 1e-37:
+        assert errs[1] <= 0.8 * errs[0], errs      # (in parts the sums have a quarter of the roundings)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tiling.GEMM_SPLIT_TILES)
+def test_a_row_of_small_values_leaves_the_other_rows_alone(tmp_path, tile):
+    m, n, k = 70, 100, 392
+    rng = np.random.default_rng(9)
+    a, w = rng.standard_normal((m, k)).astype(np.float32), (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    whole = product(tmp_path, "whole", tile, a, w, 1, True)
+    small = [0, 15, 16, 37, m - 1]
+    a[small] *= np.float32(1e-36)
+    y = product(tmp_path, "small", tile, a, w, 1, True)
+    others = np.setdiff1d(np.arange(m), small)
+    np.testing.assert_array_equal(y[others], whole[others])
+    bound = (k + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).T.astype(np.float64))
+    assert (np.abs(y - a.astype(np.float64) @ w.T.astype(np.float64)) <= bound)[small].all()
+    g, exe, _ = loaded(tmp_path, tile, a, w, B.BASE)
+    exe.execute()
+    flavours_agree(exe, g, tmp_path, {"a": a})
