@@ -757,8 +757,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 struct Planes { u32x4 h, m, l; };      // eight values
-// lost: has bits of its lower half set once a finite value was not the sum of its parts (one operation for both; written out,
-// because the compiler collects them behind others and runs out of registers: ntl_64x64).
+// lost: has bits of its lower half set once a finite value was not the sum of its parts (one operation for both).  ORDERED: in
+// this place; the compiler collects them behind others, which the products have no registers for (ntl_64x64) and
+// image patches are faster with (256 channels to 256 at 112 x 112 95.3 us a call instead of 96.4).
+template <bool ORDERED = true>
 __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l, unsigned& lost) {
     bf16x2 r;
     r[0] = (__bf16)a;
@@ -770,7 +772,8 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsign
     m = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
     a -= __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
     b -= __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
-    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a), "v"(b));
+    if (ORDERED) asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a), "v"(b));
+    else lost |= __float_as_uint(a) | __float_as_uint(b);
     l = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 __device__ __forceinline__ Planes split_planes(const f32x4& a, const f32x4& b, unsigned& lost) {
@@ -1971,13 +1974,14 @@ template <int G>
 struct TileX9 {
     static constexpr int SLOT = 18 * 8, ROW = 4 * SLOT, PART = (G + 2) * ROW, BUF = 3 * PART;      // bytes
     static constexpr int WROW = 576 + 16, WEIGHTS = 2 * BUF;      // a filter's 16 channels, padding
-    static constexpr int LDS_BYTES = WEIGHTS + 64 * WROW;
+    static constexpr int FLAGS = WEIGHTS + 64 * WROW, LDS_BYTES = FLAGS + 16;      // a word a wavefront
 };
 // The outputs of a wavefront of conv2d_x9_body (16 channels from m0, G rows from y0, 16 columns from x0) on 32-bit MFMAs, operands
 // straight from memory: four channels a step, a lane the filter of one and the pixels of its column; sums are taken over
-// 32 channels at a time, two chains each.
+// 32 channels at a time, two chains each.  rest_x, rest_w: of what the parts of pixels, or of weights, leave over.
 template <int G>
-__device__ __forceinline__ void conv2d_x9_again(rsrc_t rs_a, rsrc_t rs_b, int C, int H, int W, int m0, int y0, int x0, f32x4 (&sum)[G]) {
+__device__ __forceinline__ void conv2d_x9_again(rsrc_t rs_a, rsrc_t rs_b, int C, int H, int W, int m0, int y0, int x0, bool rest_x, bool rest_w,
+                                                f32x4 (&sum)[G]) {
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const unsigned HW4 = (unsigned)(H * W) * 4u;
     unsigned at[G + 2][3];
@@ -2005,9 +2009,16 @@ __device__ __forceinline__ void conv2d_x9_again(rsrc_t rs_a, rsrc_t rs_b, int C,
             for (int r = 0; r < G + 2; ++r)
 #pragma unroll
                 for (int dx = 0; dx < 3; ++dx) x[r][dx] = buf_load(rs_b, at[r][dx] + (unsigned)c * HW4);
+            if (rest_x) {
+#pragma unroll
+                for (int r = 0; r < G + 2; ++r)
+#pragma unroll
+                    for (int dx = 0; dx < 3; ++dx) x[r][dx] = left_over(x[r][dx]);
+            }
 #pragma unroll
             for (int t = 0; t < 9; ++t) {
-                const float w = t < 4 ? w0[t & 3] : t < 8 ? w1[t & 3] : w2;
+                float w = t < 4 ? w0[t & 3] : t < 8 ? w1[t & 3] : w2;
+                if (rest_w) w = left_over(w);
 #pragma unroll
                 for (int g = 0; g < G; ++g)
                     acc[g][t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, x[g + t / 3][t % 3], acc[g][t & 1], 0, 0, 0);
@@ -2080,7 +2091,7 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     typedef unsigned u32x4_at8 __attribute__((ext_vector_type(4), aligned(8)));
     Planes w[5];
-    unsigned lost = 0;
+    unsigned lost_w = 0, lost_x = 0;
     // taps of the two halves of an MFMA: left and middle of filter row 0, 1, 2; right of rows 0 and 1; right of row 2
     auto split_weights = [&](bool more) {
 #pragma unroll
@@ -2102,7 +2113,7 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
             for (int e = 0; e < 4; ++e) {
                 const int t = e < 2 ? TA[p] : TB[p], q = 2 * (e & 1);
                 unsigned h = 0, m = 0, l = 0;
-                if (t >= 0) split_pair(v[t < 0 ? 0 : q * 9 + t], v[t < 0 ? 0 : (q + 1) * 9 + t], h, m, l, lost);
+                if (t >= 0) split_pair<false>(v[t < 0 ? 0 : q * 9 + t], v[t < 0 ? 0 : (q + 1) * 9 + t], h, m, l, lost_w);
                 w[p].h[e] = h;
                 w[p].m[e] = m;
                 w[p].l[e] = l;
@@ -2114,8 +2125,8 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             unsigned h0, m0_, l0, h1, m1, l1;
-            split_pair(rb[k][0], rb[k][1], h0, m0_, l0, lost);
-            split_pair(rb[k][2], rb[k][3], h1, m1, l1, lost);
+            split_pair<false>(rb[k][0], rb[k][1], h0, m0_, l0, lost_x);
+            split_pair<false>(rb[k][2], rb[k][3], h1, m1, l1, lost_x);
             if (wr[k] >= 0) {
                 char* p = smem + buf + wr[k];
                 *(u32x2*)p = u32x2{h0, h1};
@@ -2168,13 +2179,24 @@ __device__ __forceinline__ void conv2d_x9_body(const OpDesc& d, int task, char* 
     f32x4 sum[1][G];
 #pragma unroll
     for (int g = 0; g < G; ++g) sum[0][g] = (acc[g][0] + acc[g][1]) + acc[g][2];
-    // What is infinite or NaN, again in 32 bits (256 channels to 256 at 112 x 112, NaN everywhere: 246 us a call instead of
-    // 103; formed element by element, a thread at a time, 8300).
-    if (any_not_finite(sum)) {
+    // What the parts of a pixel (whichever wavefront split it) or of a weight leave over, and then what is infinite or NaN, in
+    // 32 bits (256 channels to 256 at 112 x 112, pixels of 1e-36 294 us a call and NaN everywhere 245 us, instead of 103;
+    // NaN formed element by element, a thread at a time, 8300).
+    int* flags = (int*)(smem + TX::FLAGS);
+    const bool mine = __any((lost_x & 0xFFFFu) != 0);
+    if (lane == 0) flags[wave] = mine;
+    __syncthreads();
+    const int again_for[3] = {flags[0] | flags[1] | flags[2] | flags[3], __any((lost_w & 0xFFFFu) != 0), any_not_finite(sum)};
+#pragma unroll 1
+    for (int what = 0; what < 3; ++what) {
+        if (!(what == 0 ? again_for[0] : what == 1 ? again_for[1] : again_for[2])) continue;
         f32x4 again[G];
-        conv2d_x9_again<G>(rs_a, rs_b, C, H, W, m0, y0, x0, again);
+        conv2d_x9_again<G>(rs_a, rs_b, C, H, W, m0, y0, x0, what == 0, what == 1, again);
 #pragma unroll
-        for (int g = 0; g < G; ++g) keep_finite(sum[0][g], again[g]);
+        for (int g = 0; g < G; ++g) {
+            if (what == 2) keep_finite(sum[0][g], again[g]);
+            else sum[0][g] += again[g];
+        }
     }
 #pragma unroll
     for (int g = 0; g < G; ++g) {

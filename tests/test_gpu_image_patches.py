@@ -118,3 +118,45 @@ def test_values_without_parts_at_the_edges(case):
     np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
     ok = np.isfinite(want)
     np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-3)
+
+
+# pixels, filters, both
+@pytest.mark.parametrize("scales", [(1e-33, 1.0), (1e-35, 1.0), (1e-37, 1.0), (1.0, 1e-35), (1e-18, 1e-17), (1e-36, 1e-1)])
+@pytest.mark.parametrize("case", [CASES[1], CASES[7]])
+def test_small_operands_are_as_exact_as_others(case, scales):
+    """(At 1e-36 the parts of a value keep 15 bits of it.)  Against the same layer on ordinary values; the errors are thousands of alike
+    and independent ones: 1.1 for what their root mean square is known to, and a rounding to 2^-149 for each of the sums that an
+    output goes through, three for nine channels' worth of 32-bit products."""
+    B.ops_init()
+    cin, H, W, cout, _ = case
+    rng = np.random.default_rng(15)
+    x0 = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w0 = (rng.standard_normal((cout, cin, 3, 3)) * 0.02).astype(np.float32)
+    rows, errs = [0, 16, cout - 1], []
+    for a, b in ((1.0, 1.0), scales):
+        x, w = (x0 * np.float64(a)).astype(np.float32), (w0 * np.float64(b)).astype(np.float32)
+        got = run(x, w, None, None, 0)[rows]
+        xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1)))
+        want = np.stack([sum(np.tensordot(w[m, :, i, j].astype(np.float64), xp[:, i:i + H, j:j + W], 1) for i in range(3) for j in range(3))
+                         for m in rows])
+        errs.append(np.linalg.norm(got - want) / np.linalg.norm(want))
+    small = 2.0 ** -149 / 12 ** 0.5 * (3 * cin) ** 0.5 / np.sqrt((want ** 2).mean())
+    assert errs[1] <= 1.1 * errs[0] + small, (errs, small)
+
+
+def test_a_small_pixel_among_others_changes_nothing_else():
+    B.ops_init()
+    cin, H, W, cout, _ = CASES[4]
+    rng = np.random.default_rng(16)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3, 3)) * 0.02).astype(np.float32)
+    x[7, 40, 20] = 0.0
+    plain = run(x, w, None, None, 0)
+    x[7, 40, 20] = 1.0000001e-38
+    np.testing.assert_array_equal(run(x, w, None, None, 0), plain)      # (far below a rounding of every sum)
+    # alone in its surroundings it is all there is
+    x[:, 38:43, 18:23] = 0.0
+    x[7, 40, 20] = 1.0000001e-36
+    got = run(x, w, None, None, 0)[:, 39:42, 19:22]
+    want = w[:, 7, ::-1, ::-1].astype(np.float64) * x[7, 40, 20].astype(np.float64)
+    assert (np.abs(got - want) <= 2.0 ** -22 * np.abs(want) + 3 * 2.0 ** -149).all()
