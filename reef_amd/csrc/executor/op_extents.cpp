@@ -266,6 +266,7 @@ void gemm(const std::string& symbol, const Attrs& a, Needs& n) {
         for (int t = split ? 2 : 0; t < 6; ++t)      // (of 16 rows only as 32-bit values)
             ok = ok || symbol == std::string("reef_gemm_ntd") + kDirect[t] || symbol == std::string("reef_gemm_ntl") + kDirect[t];
         if (!ok || !trans_b || b1 != 0 || a[REEF_GEMM_OFF_B] != 0) { n.bad = "packed weights: only the direct kernels take them, without a batch and an offset"; return; }
+        if (split && cdiv(N, 16) * cdiv(K, 32) * 3072 >= 1ll << 32) { n.bad = "split weights of 4 GiB or more (the kernels' offsets are 32 bits)"; return; }
         n.f32("packed B", split ? cdiv(N, 16) * cdiv(K, 32) * 768 : cdiv(N, 16) * cdiv(K, 16) * 256);
     } else if (trans_b) n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (N - 1) * a[REEF_GEMM_LDB] + K);
     else n.f32("B", a[REEF_GEMM_OFF_B] + b1 * a[REEF_GEMM_STRIDE_B] + (K - 1) * a[REEF_GEMM_LDB] + N);

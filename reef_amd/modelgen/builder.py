@@ -690,7 +690,7 @@ class GraphBuilder:
         assert direct_ok or not direct, "this GEMM has no direct form"
         args = [a.idx, b.idx, out.idx]
         packed = packed and direct
-        split = packed and t["tile"] in tiling.GEMM_SPLIT_TILES
+        split = packed and tiling.takes_split(t["tile"], N, K)
         if packed and ln is None:
             copy, split = self.packed_matrix(b, N, K, split)
             args[1] = copy.idx

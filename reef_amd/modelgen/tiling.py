@@ -41,6 +41,7 @@ TILES = {
 # matrix products only (reef_gemm_ntd_<tile>, reef_gemm_ntl_<tile>): name -> (id, BM, BN)
 GEMM_WIDE_TILES = {"32x48d4": (19, 32, 48), "48x48d4": (20, 48, 48), "64x64d4": (21, 64, 64)}
 GEMM_SPLIT_TILES = ("32x32d4",) + tuple(GEMM_WIDE_TILES)      # direct tiles that take packed weights as three bf16 parts
+GEMM_SPLIT_BYTES = 1 << 32         # their offsets are 32 bits: larger copies stay 32-bit values, which are two thirds of that
 V9_TILES = ("g1", "g2", "g4")      # row tiles that exist as reef_conv2d_v9_<tile>
 # row form: image rows per tile
 ROW_TILES = {"g1": 1, "g2": 2, "g4": 4, "g7": 7, "g2m2": 2, "g4m2": 4}
@@ -159,6 +160,11 @@ def choose_product(M, N, K, batch=1, direct_ok=False, under_load=False, ln=False
     if ln:
         return forced("32x32k4", M, N, K, 1)
     return choose_gemm(M, N, K, batch, direct_ok, under_load)
+
+
+def takes_split(tile, N, K):
+    """Whether the tile runs a product with [N][K] packed weights on three parts of each."""
+    return tile in GEMM_SPLIT_TILES and math.ceil(N / 16) * math.ceil(K / 32) * 3072 < GEMM_SPLIT_BYTES
 
 
 GEMM_PAIR_FOLD_LINES = 900.0    # what a split of two costs, in the cost rule's cache lines

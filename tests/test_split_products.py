@@ -1,5 +1,6 @@
 """Matrix products on split weights (REEF_GEMM_F_SPLIT): the parts are the weight, and what has no parts in bf16 -- infinities,
 NaN, values that round to infinity -- comes out as it does on the weights themselves."""
+import json
 import os
 import time
 
@@ -146,6 +147,34 @@ def test_weights_that_are_not_the_sum_of_their_parts_are_not_split():
         p = g.storage[wt.idx]["name"]
         assert names == [p + s for s in (("xpk", "pk", "gkxpk", "gkpk") if exact else ("pk", "pk", "gkpk", "gkpk"))]
         assert [bool(k["attrs"][5] & 32) for k in g.kernels] == [exact, False] * 2
+
+
+def test_split_weights_whose_offsets_need_more_than_32_bits(tmp_path, monkeypatch):
+    """131072 x 5461 are 4 GiB as parts and 2.7 as 32-bit values: the generator keeps the latter, and a model that names the former
+    is refused (its kernel would read the weights modulo 4 GiB)."""
+    assert tiling.takes_split("32x48d4", 131072, 5440) and not tiling.takes_split("32x48d4", 131072, 5464)
+    assert tiling.takes_split("64x64d4", 4096, 4096) and not tiling.takes_split("16x32k4", 64, 64)
+
+    def model(name):
+        g = MB.GraphBuilder(name)
+        w = g.param((96, 72), 0.5)
+        g.mark_output(g.gemm(g.input("a", (40, 72)), w, 40, 96, 72, force_tile="32x48d4"))
+        return g, json.load(open(g.write(str(tmp_path / name), link_code_objects=False) + ".json"))
+    g, m = model("fits")
+    assert g.kernels[0]["attrs"][5] == 32
+    monkeypatch.setattr(tiling, "GEMM_SPLIT_BYTES", 6 * 3 * 3072)
+    assert model("large")[0].kernels[0]["attrs"][5] == 0
+    k, N, K = m["kernels"][0], 131072, 5464
+    k["attrs"][2:4], k["attrs"][10], k["attrs"][11], k["attrs"][13] = [N, K], N // 48 + 1, K, N
+    k["launch_params"][0] = 2 * k["attrs"][10]
+    for i, n in zip(k["args"], (40 * K, N // 16 * 171 * 768, 40 * N)):
+        m["storage"][i]["size"] = n
+    for bad in (True, False):
+        if not bad:
+            k["attrs"][3] = k["attrs"][11] = 5440
+        json.dump(m, open(str(tmp_path / "m.json"), "w"))
+        ok, why = B.check_model(str(tmp_path / "m.json"))
+        assert ok != bad and ("4 GiB" in why) == bad, why
 
 
 @pytest.mark.gpu
