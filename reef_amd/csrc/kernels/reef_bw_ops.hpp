@@ -209,6 +209,13 @@ __device__ __forceinline__ void global_avgpool_body(const OpDesc& d, int task) {
     if ((threadIdx.x & 63) == 0) store_out((float*)d.ptr[1] + c, s * (1.0f / (float)HW));
 }
 
+// Four results of a thread whose workgroup writes kThreads of them from `first` on, of a tensor of `total` floats, in one
+// store.  (The resource is the workgroup's part: the tensor may have more than the 4 GiB that one spans.)
+__device__ __forceinline__ void store_four(float* out, size_t first, size_t total, f32x4 v) {
+    const size_t left = total - first;
+    buf_store4(make_rsrc(out + first, left < (size_t)kThreads * 4 ? (unsigned)left * 4u : kThreads * 16u), threadIdx.x * 16u, v);
+}
+
 __device__ __forceinline__ void eltwise_body(const OpDesc& d, int task) {
     const int* at = d.attr;
     const int C = at[REEF_ELT_C], inner = at[REEF_ELT_INNER], flags = at[REEF_ELT_FLAGS],
@@ -230,7 +237,7 @@ __device__ __forceinline__ void eltwise_body(const OpDesc& d, int task) {
         if (shift) v += shift[c];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = act_apply(v[e], act);
-        buf_store4(make_rsrc(out, (unsigned)(total * 4)), (unsigned)(i0 * 4), v);
+        store_four(out, (size_t)__builtin_amdgcn_readfirstlane(task) * kThreads * 4, total, v);
     } else {
         for (int e = 0; e < 4 && i0 + e < total; ++e) {
             const int c = div_index(i0 + e, inner);
@@ -543,7 +550,7 @@ __device__ __forceinline__ void copy_body(const OpDesc& d, int task) {
     const int i0 = (task * kThreads + threadIdx.x) * 4;
     if (i0 >= count) return;
     if (((count | dst_off) & 3) == 0) {
-        buf_store4(make_rsrc(out, (unsigned)count * 4u), (unsigned)i0 * 4u, *(const f32x4*)(in + i0));
+        store_four(out, (size_t)__builtin_amdgcn_readfirstlane(task) * kThreads * 4, (size_t)count, *(const f32x4*)(in + i0));
     } else {
         for (int e = 0; e < 4 && i0 + e < count; ++e) store_out(out + i0 + e, in[i0 + e]);
     }
