@@ -78,6 +78,7 @@ struct NoPoll {
     // two may leave between its two workgroups in the pair slots relies on it (REEF_F_PAIR_FOLD).
     bool completes = false;
     __device__ __forceinline__ int load() const { return 0; }
+    __device__ __forceinline__ int hint() const { return 0; }
     __device__ __forceinline__ bool pair_fold_ok() const { return completes; }
 };
 struct FlagPoll {
@@ -87,7 +88,21 @@ struct FlagPoll {
     __device__ __forceinline__ int load() const {
         return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    // The flag by way of the scalar cache, which waits for no vector load: what it was when the line was fetched.  No more
+    // than a hint, therefore: who acts on it asks load() first.  (volatile: fetched here, and not where it is used.)
+    __device__ __forceinline__ int hint() const {
+        const int* p = flag;
+        asm("" : "+s"(p));      // (or the compiler takes the value of a load() for it)
+        return *(const volatile __attribute__((address_space(4))) int*)p;
+    }
 };
+// Whether a wavefront leaves in front of its K loop.  `raised` (a load()) is waited for only where the hint says that it will
+// have something to say.
+__device__ __forceinline__ bool leaves_at_once(int hint, int raised) {
+    if (!hint) return false;
+    asm volatile("" : "+v"(raised));      // (a branch, not a choice between two values, both of which would be waited for)
+    return __builtin_amdgcn_readfirstlane(raised) != 0;
+}
 
 // Device-coherent accesses for data one workgroup hands to another inside a kernel
 // (split-K partial tiles).  The scope travels on the instruction, so no L2-wide

@@ -381,8 +381,8 @@ __device__ __forceinline__ void be_count_completed(const ReefBeArgs& a, bool don
 }
 }  // namespace
 namespace {
-// Ops whose body makes the first flag check of a best-effort workgroup itself, in front of its loads without
-// waiting for it (the direct families); for all others the wrapper makes it.
+// Ops whose body makes the first flag check of a best-effort workgroup itself, behind its first loads (the direct
+// families); for all others the wrapper makes it.
 template <class OP, class = void>
 struct ChecksFlagItself { static constexpr bool value = false; };
 template <class OP>

@@ -1176,6 +1176,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = FROWS ? a[REEF_CONV_KH] : 1;
+    const int hint = poll.hint();
     const int M = a[REEF_CONV_COUT], C = FROWS ? a[REEF_CONV_CIN] * kh : a[REEF_CONV_CIN];
     const int H = a[REEF_CONV_H], W = a[REEF_CONV_W], Wo = a[REEF_CONV_WO];
     const int N = a[REEF_CONV_HO] * Wo;
@@ -1477,17 +1478,20 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     // (script/best_effort_kernel.py:22-29): read by every wavefront behind its first loads, and looked at where the wavefronts
     // meet behind the K loop; what the loop itself looks at are loads of its own, one round ahead.  A workgroup that finds
     // the flag raised has only read.  Loads return in order, and the flag, which no cache holds, comes later than
-    // operands do: in front of them it held up the first MFMAs of every launch (DenseNet-201 as a best-effort model 990 us a
-    // request that way and 956 this way, BERT-base at 128 tokens 323 and 319; looked at with a barrier before the loop: 1017 of device time to 980).
+    // operands do: in front of them it held up the first MFMAs of every launch (DenseNet-201 as a best-effort model 1012 us a
+    // request that way; looked at with a barrier before the loop another 37 of device time).  So that a wavefront under a
+    // raised flag does not run a round first, it has a hint by way of the scalar cache, and waits for the load where that
+    // says so: 979 us a request (968 without the hint), and 16 streams are empty 62 us after the flag (71.5; 62.3 with
+    // the flag in front of the loads), four 16.5 (18.8; 17.1).
     if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;
     int pf = 0;
     int it = 0;
-    bool left = false;
+    bool left = leaves_at_once(hint, raised);
     // (groups whose refills all exist; the last whole group follows with the refills the remaining
     // steps need and no others: a load outside the buffer brings nothing but still takes its turn in
     // the vector-memory pipe, and a group of them cost a layer with nsteps == NS 1700 cycles)
-    for (; it + 2 * NS <= nsteps; it += NS) {
+    for (; !left && it + 2 * NS <= nsteps; it += NS) {
         if (Poll::enabled) {
             // the flag is read one group ahead; a wavefront that sees it tells the others
             // through LDS and all of them leave where they meet
@@ -1568,6 +1572,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     float* smem = (float*)smem_raw;
     constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
     const int* a = d.attr;
+    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
@@ -1706,9 +1711,9 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0, it = 0;
-    bool left = false;
-    if (steps > 0) turn(0, 0);
-    for (; it + 2 * NS <= steps; it += NS) {
+    bool left = leaves_at_once(hint, raised);
+    if (steps > 0 && !left) turn(0, 0);
+    for (; !left && it + 2 * NS <= steps; it += NS) {
         if (Poll::enabled) {
             if (pf) {
                 left = true;
@@ -1785,6 +1790,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     constexpr int NA = G == 1 ? 4 : 2;
     float* smem = (float*)smem_raw;
     const int* a = d.attr;
+    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], H = a[REEF_CONV_H], W = a[REEF_CONV_W];
@@ -1931,8 +1937,8 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0;
-    bool left = false;
-    if (steps > 0) {
+    bool left = leaves_at_once(hint, raised);
+    if (steps > 0 && !left) {
         turn();
         if (steps > 1) load_b();
         for (; steps > 1; --steps) {
@@ -3308,7 +3314,10 @@ struct GemmTail {
                 ooff[h][g] = n < (unsigned)N ? (m * ldc + n) * 4u : kOutside;
             }
         }
-        if (LN) ln_out.init(d, lnp, (const float*)d.ptr[0], M, K, lda, m0, TD::BM, nt, a[REEF_GEMM_N_TILES]);
+    }
+    // LN: this thread's share of the normalised rows.
+    __device__ __forceinline__ void fetch_rows(const OpDesc& d) {
+        if (LN) ln_out.init(d, 3 + (has_bias ? 1 : 0) + (has_res ? 1 : 0), (const float*)d.ptr[0], M, K, lda, m0, TD::BM, nt, d.attr[REEF_GEMM_N_TILES]);
     }
     // The residual, which is laid out as C is; without one an empty buffer, whose loads give 0.
     __device__ __forceinline__ void fetch_residual(const OpDesc& d) {
@@ -3517,6 +3526,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     constexpr int AC = TM * TN > 4 ? 1 : PK && !LN && TM * TN == 1 ? 4 : 2;
     // steps of loads in flight (unpacked, 6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
     constexpr int NS = PK ? 4 : 3;
+    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GemmTail<TM, TN, LN> t;
@@ -3524,6 +3534,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     t.fetch_pivots();
     t.fetch(d);
     t.fetch_residual(d);
+    t.fetch_rows(d);
     const int* a = d.attr;
     const unsigned ldb = (unsigned)a[REEF_GEMM_LDB];
     const rsrc_t rs_b = make_rsrc((const float*)d.ptr[1] + a[REEF_GEMM_OFF_B] + (size_t)t.batch * a[REEF_GEMM_STRIDE_B],
@@ -3626,13 +3637,13 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0, it = 0;
-    bool left = false;
+    bool left = leaves_at_once(hint, raised);
     // this wavefront's own steps where their loads are its own
     const int steps = PK ? (t.k_lo + 16 * wave < t.k_hi ? (t.k_hi - t.k_lo - 16 * wave + KSTEP - 1) / KSTEP : 0) : nsteps;
-    if (PK && steps > 0) turn(0, 0);
+    if (PK && steps > 0 && !left) turn(0, 0);
     // (groups whose refills all exist, then the last whole group with the refills the remaining steps
     // need and no others, as in the convolution)
-    for (; it + 2 * NS <= steps; it += NS) {
+    for (; !left && it + 2 * NS <= steps; it += NS) {
         if (Poll::enabled) {
             if (pf) {
                 left = true;
@@ -3700,6 +3711,7 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     constexpr int NS = 2;                                    // steps of loads in flight: what 256 registers hold
     typedef TileD16<TN, TM> TD;
     static_assert(TM * 512 <= TD::SUBS * TD::PART, "the turned rows fit where the partial tile goes");
+    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GemmTail<TM, TN, LN> t;
@@ -3795,9 +3807,9 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;      // the flag check, as in conv2d_direct_body
     int pf = 0, it = 0;
-    bool left = false;
-    if (steps > 0) turn(0);
-    for (; it + NS < steps; it += NS) {
+    bool left = leaves_at_once(hint, raised);
+    if (steps > 0 && !left) turn(0);
+    for (; !left && it + NS < steps; it += NS) {
         if (Poll::enabled) {
             if (pf) {
                 left = true;
@@ -3818,12 +3830,14 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     if (Poll::enabled && pf) left = true;
     if (!left) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
+        for (int s = 0; s < NS; ++s) {
             if (it + s < steps) {
                 split_rows();
                 if (s + 1 < NS && it + s + 1 < steps) turn(s + 1);
                 multiply(s);
             }
+            if (s == 0 && !LATE) t.fetch_rows(d);      // (into registers of operands that are multiplied)
+        }
     }
     f32x4 sum[TM][TN];
 #pragma unroll
@@ -3900,7 +3914,10 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
                 else sum[h][g] += r;
             }
     }
-    if (LATE) t.fetch(d);
+    if (LATE) {
+        t.fetch(d);
+        t.fetch_rows(d);
+    }
     t.place_out(d);
     if (LN) {
         if (t.has_res) t.fetch_residual(d);
