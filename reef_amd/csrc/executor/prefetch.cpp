@@ -81,10 +81,14 @@ std::vector<ReefPrefetch> plan_prefetch(const Model& model, const std::vector<vo
         size_t bytes = 0;
         const bool has = w.slot >= 0 && (size_t)w.slot < k.args.size() && is_param[k.args[(size_t)w.slot]];
         if (has) operand((size_t)w.slot, &r.base, &bytes);
-        // what one XCD is to hold: the activations of both launches live in its 4 MiB as well
-        constexpr size_t kMostPerXcd = 1536 * 1024;
+        // what one XCD is to hold: the activations of both launches live in its 4 MiB as well, and the launch in front lasts
+        // until the last line is there.  With split weights that shows from 1 MiB on: BERT-base, six layers of 128 tokens as a
+        // best-effort model, where QKV has 1.27 MiB of them an XCD and the FFN 1.69, 352 us a request with both, 320 with QKV's, 316
+        // with neither; four layers of 384 tokens 415, 410 and 403.  (In 32 bits they were 0.84 and 1.12.)
+        const bool split = op_from_symbol(symbol_of(k.name)) == REEF_OP_GEMM && (attr(k, REEF_GEMM_FLAGS) & REEF_GEMM_F_SPLIT);
+        const size_t most = split ? 1024 * 1024 : 1536 * 1024;
         size_t per_xcd = w.chunks == 1 ? bytes : bytes / 8;
-        if (per_xcd > kMostPerXcd) bytes = per_xcd = 0;
+        if (per_xcd > most) bytes = per_xcd = 0;
         if (bytes) {
             r.chunks = w.chunks;
             r.chunk_bytes = (uint32_t)(((bytes + w.chunks - 1) / w.chunks + 15) / 16 * 16);

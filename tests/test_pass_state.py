@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from reef_amd import binding as B
-from reef_amd.modelgen import nets
+from reef_amd.modelgen import builder as MB, nets
 from tests.fakehal import FakeHal
 from tests.helpers import write_model
 
@@ -177,4 +177,19 @@ def test_a_pass_that_cannot_be_recorded_at_load_is_reported_by_the_run(fake, moc
         exe.execute()
     exe.execute()
     np.testing.assert_array_equal(exe.get_output(), np.full(N, 18, np.float32))
+    exe.close()
+
+
+# columns of the second product, 768 deep: 0.84 and 1.27 MiB an XCD split, 1.31 and 1.69 MiB in 32 bits
+@pytest.mark.parametrize("n,tile,fits", [(1536, "32x48d4", True), (2304, "32x48d4", False), (3584, "16x32k4", True), (4608, "16x32k4", False)])
+def test_weights_that_the_launch_in_front_brings_in(fake, tmp_path, n, tile, fits):
+    g = MB.GraphBuilder("prefetch")
+    x = g.gemm(g.input("x", (16, 768)), g.param((768, 768), 0.03), 16, 768, 768, force_tile="16x32k4")
+    g.mark_output(g.gemm(x, g.param((n, 768), 0.03), 16, n, 768, force_tile=tile))
+    fake._run_desc = lambda *args: None                     # (only the launches matter)
+    exe = B.Executor.from_dir(write_model(g, tmp_path), g.name, B.BASE)
+    exe.set_input_checked("x", np.ones((16, 768), np.float32))
+    exe.execute()
+    workgroups = fake.events[-2][3] - g.kernels[0]["launch_params"][0]
+    assert workgroups == 8 + (8 * 6 if fits else 0)        # one of each XCD's for small operands, six for its weights
     exe.close()
