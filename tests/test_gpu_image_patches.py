@@ -160,3 +160,48 @@ def test_a_small_pixel_among_others_changes_nothing_else():
     got = run(x, w, None, None, 0)[:, 39:42, 19:22]
     want = w[:, 7, ::-1, ::-1].astype(np.float64) * x[7, 40, 20].astype(np.float64)
     assert (np.abs(got - want) <= 2.0 ** -22 * np.abs(want) + 3 * 2.0 ** -149).all()
+
+
+def exact(x, w, rows):
+    cin, H, W = x.shape
+    xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1)))
+    return np.stack([sum(np.tensordot(w[m, :, i, j].astype(np.float64), xp[:, i:i + H, j:j + W], 1) for i in range(3) for j in range(3)) for m in rows])
+
+
+# (wide layers and deep ones; sums of the image-row kernels are split over four wavefronts and, for the last, over workgroups)
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("relu", [False, True])
+def test_no_further_off_than_the_image_row_kernels(case, relu):
+    """The same layer with a channel of zeros more runs on 32-bit products.  The errors are thousands of alike and independent ones:
+    1.1 for what their root mean square is known to."""
+    B.ops_init()
+    cin, H, W, cout, rows = case
+    rng = np.random.default_rng(17)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    x = np.maximum(x, 0) if relu else x
+    w = (rng.standard_normal((cout, cin, 3, 3)) * np.sqrt(2.0 / (cin * 9))).astype(np.float32)
+    some = [0, 16, cout // 2, cout - 1]
+    want, errs = exact(x, w, some), []
+    for more in (1, 0):
+        xm, wm = np.pad(x, ((0, more), (0, 0), (0, 0))), np.pad(w, ((0, 0), (0, more), (0, 0), (0, 0)))
+        name = B.ops_conv2d_kernel(B.Conv2dDesc(cin + more, H, W, cout, 3, 3, 1, 1, 1, 1, 0))[0]
+        assert ("_x9_" in name) == (not more), name
+        errs.append(np.linalg.norm(run(xm, wm, None, None, 0)[some] - want) / np.linalg.norm(want))
+    assert errs[1] <= 1.1 * errs[0], errs
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[4], CASES[7]])
+def test_every_product_of_parts_is_there(case):
+    """Filters with one weight each, all 24 bits in use: an output is one product, whose parts leave out at most 2^-23 of it, and
+    is rounded when its sums meet, twice; without any of the six products four fifths of them are further off, up to 2^-16."""
+    B.ops_init()
+    cin, H, W, cout, _ = case
+    rng = np.random.default_rng(18)
+    x = np.ldexp(rng.integers(2 ** 23, 2 ** 24, (cin, H, W)) | 1, -23).astype(np.float32) * rng.choice((-1, 1), (cin, H, W)).astype(np.float32)
+    some = list(range(0, cout, 5))
+    for turn in range(2):
+        w = np.zeros((cout, cin, 3, 3), np.float32)
+        tap, ch = (np.arange(cout) + turn) % 9, (np.arange(cout) * 7 + 3 * turn) % cin       # every tap of every lane and k slot
+        w[np.arange(cout), ch, tap // 3, tap % 3] = np.ldexp(rng.integers(2 ** 23, 2 ** 24, cout) | 1, -23)
+        got, want = run(x, w, None, None, 0)[some], exact(x, w, some)
+        assert (np.abs(got - want) <= 2.0 ** -22 * np.abs(want)).all()

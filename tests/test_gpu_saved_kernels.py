@@ -1,12 +1,14 @@
 """Kernels that the generator no longer names and saved model files may: the row form on weights packed by taps
-(reef_conv2d_r9k_*), and the 1-tap kernels on weights as OIHW has them (reef_conv2d_d1_*, reef_conv2d_p1_* with no packed
-copy).  Every storage against the oracle, and the three flavours bit for bit."""
+(reef_conv2d_r9k_*), the 1-tap kernels on weights as OIHW has them (reef_conv2d_d1_*, reef_conv2d_p1_* with no packed
+copy), and matrix products of 32 rows and more on weights packed as 32-bit values.  Every storage against the oracle, and the
+three flavours bit for bit."""
 import numpy as np
 import pytest
 
 from reef_amd.modelgen import builder as MB, tiling
 from tests.helpers import compare_storages, run_both
 from tests.test_gpu_packed_convs import V9_SHAPES, flavours_agree
+from tests.test_gpu_packed_products import SHAPES as PRODUCT_SHAPES
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +73,29 @@ def test_pointwise_on_unpacked_weights(tmp_path, tile, shape, split, fused):
         {"reef_conv2d_p1_" + tile} if tile in tiling.PRE_ACT_TILES else set())
     assert not any(k["attrs"][23] for k in convs)
     check(g, tmp_path, cin, cout, H, W, "d1 %s %s x%d%s" % (tile, shape, split, " fused" if fused else ""))
+
+
+@pytest.mark.parametrize("split", [1, 2, 3])
+@pytest.mark.parametrize("shape", PRODUCT_SHAPES)
+@pytest.mark.parametrize("tile", list(tiling.GEMM_SPLIT_TILES))
+def test_product_on_weights_packed_as_32_bit_values(tmp_path, monkeypatch, tile, shape, split):
+    m, n, k = shape
+    if split > 1 and tiling.forced(tile, m, n, k, split)["split_k"] != split:
+        pytest.skip("too little depth for this split")
+    monkeypatch.setattr(tiling, "GEMM_SPLIT_TILES", ())
+    g = MB.GraphBuilder("pk32")
+    x, r = g.input("data", (m, k)), g.input("res", (m, n))
+    w, bias = g.param((n, k), 0.5), g.param((n,), 0.5)
+    g.gemm(x, w, m, n, k, bias=bias, act=MB.ACT_GELU, res=r, force_tile=tile, split_k=split)
+    plain = g.gemm(x, w, m, n, k, alpha=0.5, force_tile=tile, split_k=split)
+    if split == 1 and tile in g.LN_GEMM_TILES:
+        ln = dict(gamma=g.param((k,), 0.5), beta=g.param((k,), 0.5))
+        g.gemm(x, w, m, n, k, bias=bias, force_tile=tile, ln=dict(ln, out=g.temp((m, k))))
+        g.gemm(x, w, m, n, k, res=r, force_tile=tile, ln=ln)
+    g.mark_output(plain)
+    products = [c for c in g.kernels if c["op"] == "gemm"]
+    assert all(c["attrs"][12] == 0 and not c["attrs"][5] & 32 and c["name"].split("#")[0].endswith(tile) for c in products)
+    inputs = {"data": rnd(m, k), "res": rnd(m, n)}
+    exe, orc, model = run_both(g, tmp_path, inputs)
+    compare_storages(exe, orc, model, what="pk32 %s %s x%d" % (tile, shape, split))
+    flavours_agree(exe, g, tmp_path, inputs)

@@ -59,8 +59,8 @@ def test_product_of_split_operands(tmp_path, tile, shape):
         pytest.skip("too little depth for this split")
     rng = np.random.default_rng(5)
     a, w = rng.standard_normal((m, k)).astype(np.float32), (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
-    # k + 1 roundings of at most 2^-24 of the sum of magnitudes, and the terms left out: 2^-24 of each product
-    bound = (k + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).T.astype(np.float64))
+    # k + 1 roundings of at most 2^-24 of the sum of magnitudes, and the terms left out: at most 2^-23 of each product
+    bound = (k + 3) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).T.astype(np.float64))
     y = product(tmp_path, "split", tile, a, w, split, True)
     assert (np.abs(y - a.astype(np.float64) @ w.T.astype(np.float64)) <= bound).all()
     # rows and columns with values that have no parts: one each, so that no sum depends on its order
@@ -127,6 +127,20 @@ def test_values_without_parts_cost_one_more_pass_over_the_depth(tmp_path, tile):
         best.append(min(times))
     exe.close()
     assert best[1] < 5 * best[0], best
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tiling.GEMM_SPLIT_TILES)
+def test_every_product_of_parts_is_there(tmp_path, tile):
+    """Columns with one weight each, all 24 bits in use, a column for every k: an output is one product, whose parts leave out at
+    most 2^-23 of it, and is rounded when its sums meet, twice; without any of the six products four fifths of them are further
+    off, up to 2^-16."""
+    m, k = 49, 264
+    rng = np.random.default_rng(10)
+    a = (np.ldexp(rng.integers(2 ** 23, 2 ** 24, (m, k)) | 1, -23) * rng.choice((-1, 1), (m, k))).astype(np.float32)
+    w = np.diag(np.ldexp(rng.integers(2 ** 23, 2 ** 24, k) | 1, -23)).astype(np.float32)
+    want = a.astype(np.float64) * np.diag(w).astype(np.float64)
+    assert (np.abs(product(tmp_path, "one", tile, a, w, 1, True) - want) <= 2.0 ** -22 * np.abs(want)).all()
 
 
 def test_weights_that_are_not_the_sum_of_their_parts_are_not_split():
