@@ -322,8 +322,9 @@ __device__ __forceinline__ bool dkp_walk(const ReefDkpArgs& a, DkpWalk& w) {
 // Wavefronts a SIMD at least (OP::WAVES, 1 if absent).  Where one is enough the compiler keeps accumulators in accumulation
 // registers and turns them over there: reef_conv2d_v9_g1 moved all sixteen once a step, behind the MFMAs that write them.
 // With two, 256 registers each, MFMAs add to ordinary registers and nothing moves: ResNet-152 844.7 -> 840.9 us a request,
-// ResNet-50 at 448 699.7 -> 694.4, DenseNet-201 as a best-effort model 1012.4 -> 1007.5.  Only the convolutions ask for it:
-// BERT-base at 128 tokens takes 349 instead of 343 with it in the products and the attention.
+// ResNet-50 at 448 699.7 -> 694.4, DenseNet-201 as a best-effort model 1012.4 -> 1007.5.  The convolutions
+// ask for it, and products of 32 rows (OpGemmNtDirect); with it in the other products and the attention BERT-base at 128
+// tokens took 349 instead of 343.
 namespace {
 template <class OP, class = void>
 struct WavesOf { static constexpr int value = 1; };

@@ -743,7 +743,8 @@ __device__ __forceinline__ bool conv2d_body(const OpDesc& d_in, int task, char* 
 // ---- products of 32-bit values on the bf16 matrix cores ------------------------------------------------------
 // A 32-bit value is the sum of three bf16 values exactly: h rounded to nearest, m the first eight bits of what is left
 // (cut off), l the rest, at most eight bits.  A product is h h + (h m + m h) + (m m + h l + l h); the terms left
-// out are 2^-24 of it and of either sign.  The matrix cores multiply bf16 16 times as fast as 32 bits (16x16x32 in 16
+// out (m l, l m, l l) are below 2^-23 of it, a quarter of 2^-24 as a rule (root mean square), and of either sign where the
+// operands are.  The matrix cores multiply bf16 16 times as fast as 32 bits (16x16x32 in 16
 // cycles, 16x16x4 in 32), so the six products of a tile take 96 cycles where 32-bit ones take 256; and VALU work goes
 // on beside a bf16 MFMA, while a 32-bit one holds it up (an MFMA and three VALU operations: 22 cycles and 51).  The
 // five small products have an accumulator of their own, so that what is rounded into the large one is h h alone, once per
@@ -1972,10 +1973,11 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
 // The weights come as the caller has them, a filter's 576 bytes of 16 channels in a row, loaded as pieces of 128
 // bytes and brought to their lanes through LDS (each lane from its own 144 bytes, a load touches 64 lines: seven rows of
 // the layer below take 90 us, and 78 without any loads of weights; in pieces of 64 bytes 120 instead of 108 on four rows).
-// 256 channels to 256 at 112 x 112: 144 us on 32-bit MFMAs (reef_conv2d_r9_g4m2, whose matrix pipes are full), 85 here, the
-// MFMAs busy 55 % of the time: the splits (264 VALU operations for 210 MFMAs a step), LDS and the barrier take the
-// rest, with a second workgroup on the CU to fill in.  Four rows are for layers that leave seven too few workgroups.
-// Distance from 64 bits there 1.6e-7 (32-bit MFMAs, eight sums a row: 2.2e-7), and below the other kernels' wherever this is chosen.
+// 256 channels to 256 at 112 x 112: 144 us on 32-bit MFMAs (reef_conv2d_r9_g4m2, whose matrix pipes are full), 86 here, of which
+// a SIMD multiplies 39 (94 thousand cycles): the splits (264 VALU operations and the checks that they are exact for 210 MFMAs a
+// step), LDS and the barrier take the rest, with a second workgroup on the CU to fill in.  Four rows are for layers that
+// leave seven too few workgroups.  Distance from 64 bits there, normal values, 2.1e-7 (32-bit MFMAs, eight sums a row: 3.1e-7), and below
+// the other kernels' wherever this is chosen.
 template <int G>
 struct TileX9 {
     static constexpr int SLOT = 18 * 8, ROW = 4 * SLOT, PART = (G + 2) * ROW, BUF = 3 * PART;      // bytes
@@ -3696,8 +3698,8 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
 
 // REEF_GEMM_F_SPLIT: B is stored as the three bf16 parts of each weight, and the parts of A are formed behind its turn through
 // LDS, a step of 32 values of k a wavefront ahead of the 16x16x32 products.  32-bit MFMAs bound these tiles before (32x48:
-// 1536 cycles of them a step of 2000); now a CU's loads do, weights being half as large again (13 KiB a wavefront and step
-// at 20 to 22 cycles a KiB and CU: 1090 of 1150).  Splitting the weights here as well, five or six VALU operations a value,
+// 1536 cycles of them a step of 2000); now a CU's loads do, weights being half as large again (13 KiB a wavefront and step,
+// about 1090 cycles at 20 to 22 a KiB and CU; the matrix pipes are busy 14 % of a launch at 384 tokens).  Splitting the weights here as well, five or six VALU operations a value,
 // costs more than that load, and a 16-row tile shares a split row with too few columns: those stay in 32 bits (a split
 // ntd_16x32 11.8 us against 10.6 at 128 x 768 x 3072).  Two workgroups a CU (256 registers) are worth more than a wider tile:
 // us a launch, 32 bits and this, LayerNorm in front of the first two,
