@@ -1973,7 +1973,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
 // The weights come as the caller has them, a filter's 576 bytes of 16 channels in a row, loaded as pieces of 128
 // bytes and brought to their lanes through LDS (each lane from its own 144 bytes, a load touches 64 lines: seven rows of
 // the layer below take 90 us, and 78 without any loads of weights; in pieces of 64 bytes 120 instead of 108 on four rows).
-// 256 channels to 256 at 112 x 112: 144 us on 32-bit MFMAs (reef_conv2d_r9_g4m2, whose matrix pipes are full), 86 here, of which
+// 256 channels to 256 at 112 x 112: 144 us on 32-bit MFMAs (reef_conv2d_r9_g4m2, whose matrix pipes are full), 88 here, of which
 // a SIMD multiplies 39 (94 thousand cycles): the splits (264 VALU operations and the checks that they are exact for 210 MFMAs a
 // step), LDS and the barrier take the rest, with a second workgroup on the CU to fill in.  Four rows are for layers that
 // leave seven too few workgroups.  Distance from 64 bits there, normal values, 2.1e-7 (32-bit MFMAs, eight sums a row: 3.1e-7), and below

@@ -70,7 +70,7 @@ enum Family {
 // and unaligned loaders and both strides alike.  Those rows order the tiles of one family only.  Against one tile per filter (16 x 32 at 1x1, two image rows
 // at 3x3, staged 64 x 64 at 5x5, 7x7 and odd channel counts), kernel times: 5x5 48 -> 64 at 35x35 31.9 ->
 // 8.1 us, 7x7 209 -> 15 at 12x85 43 -> 9.3, 1x1 161 -> 617 at 23x21 17 -> 5.2, 3x3 256 -> 256 at 112x112
-// 210 -> 144 (103 TFLOP/s of the 152 that fp32 MFMAs reach) -> 86 by
+// 210 -> 144 (103 TFLOP/s of the 152 that fp32 MFMAs reach) -> 88 by
 // image patches, whose rows are fitted to 70 of those shapes, from 0.3 to 15 GFLOP, with 3 % on top: where
 // they are near the others, those stay.  They do not split K, so they are for layers with some 400 tiles of 64 channels.
 struct Kernel {
