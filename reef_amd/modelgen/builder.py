@@ -873,22 +873,36 @@ def split_matrix(w):
     None where a finite weight is not the sum of its parts (below 2^-110, if it has bits under the smallest bf16)."""
     N, K = w.shape
     n, k = -(-N // 16), -(-K // 32)
-    x = np.zeros((n * 16, k * 32), np.float32)
-    x[:N, :K] = w
-
+    if N % 16 or K % 32:
+        x = np.zeros((n * 16, k * 32), np.float32)
+        x[:N, :K] = w
+    else:
+        x = np.ascontiguousarray(w, np.float32)
+    top = np.uint32(0xFFFF0000)
     u = x.view(np.uint32)
-    finite = (u & np.uint32(0x7F800000)) != np.uint32(0x7F800000)
-    near = (u + np.uint32(0x7FFF) + ((u >> np.uint32(16)) & np.uint32(1))) & np.uint32(0xFFFF0000)
-    fits = finite & ((near & np.uint32(0x7F800000)) != np.uint32(0x7F800000))
-    nan = ~finite & ((u & np.uint32(0x7FFFFF)) != 0)
-    h = np.where(fits, near, (u & np.uint32(0xFFFF0000)) | np.where(nan, np.uint32(0x400000), np.uint32(0)))
-    r = np.where(finite, x, np.float32(0)) - np.where(finite, h, np.uint32(0)).view(np.float32)
-    m = r.view(np.uint32) & np.uint32(0xFFFF0000)
-    l = (r - m.view(np.float32)).view(np.uint32)
-    if (l & np.uint32(0xFFFF)).any():
+    h = u >> np.uint32(16)
+    h &= np.uint32(1)
+    h += np.uint32(0x7FFF)
+    h += u
+    h &= top
+    if max(x.max(), -x.min()) < 3.38e38:      # (nor NaN: every value has parts)
+        r = x - h.view(np.float32)
+    else:
+        exponent = np.uint32(0x7F800000)
+        finite = (u & exponent) != exponent
+        nan = ~finite & ((u & np.uint32(0x7FFFFF)) != 0)
+        h = np.where(finite & ((h & exponent) != exponent), h, (u & top) | np.where(nan, np.uint32(0x400000), np.uint32(0)))
+        r = np.where(finite, x, np.float32(0)) - np.where(finite, h, np.uint32(0)).view(np.float32)
+    m = r.view(np.uint32) & top
+    r -= m.view(np.float32)
+    l = r.view(np.uint32)
+    halves = lambda p: p.view(np.uint16).reshape(n, 16, k, 2, 4, 4, 2)
+    if halves(l)[..., 0].any():
         return None
-    parts = [(p >> np.uint32(16)).astype(np.uint16).reshape(n, 16, k, 2, 4, 4).transpose(0, 2, 4, 1, 3, 5) for p in (h, m, l)]
-    return np.ascontiguousarray(np.stack(parts, axis=2)).reshape(-1).view(np.float32)
+    out = np.empty((n, k, 3, 4, 16, 2, 4), np.uint16)
+    for i, p in enumerate((h, m, l)):
+        out[:, :, i] = halves(p)[..., 1].transpose(0, 2, 4, 1, 3, 5)
+    return out.reshape(-1).view(np.float32)
 
 
 def write_params(path, params):

@@ -31,6 +31,21 @@ def test_parts_of_a_weight_add_up_to_it():
     assert np.isfinite(h[np.isfinite(back).reshape(2, 16, 3, 2, 4, 4).transpose(0, 2, 4, 1, 3, 5)]).all()
 
 
+def test_parts_of_a_matrix_with_and_without_values_that_have_none():
+    rng = np.random.default_rng(4)
+    for n, k in ((48, 96), (17, 40)):
+        w = rng.standard_normal((n, k)).astype(np.float32)
+        w[3, 5], w[4, 7] = 3.37e38, -3.37e38
+        plain = MB.split_matrix(w)
+        for bad in (np.inf, -np.inf, np.nan, 3.4028235e38):
+            v = w.copy()
+            v[n - 1, k - 1] = bad
+            differ = np.flatnonzero(MB.split_matrix(v).view(np.uint16) != plain.view(np.uint16))
+            col, at = (n - 1) % 16, (k - 1) % 32                 # where the value's parts lie, by the layout's definition
+            first = ((n - 1) // 16 * -(-k // 32) + (k - 1) // 32) * 1536 + (at % 16 // 4 * 16 + col) * 8 + at // 16 * 4 + at % 4
+            assert differ.size and set(differ) <= {first, first + 512, first + 1024}
+
+
 def product(d, name, tile, a, w, split, packed):
     (m, k), n = a.shape, w.shape[0]
     g = MB.GraphBuilder(name)
