@@ -1,5 +1,6 @@
 """Large 3x3 layers through reef_ops_conv2d (reef_conv2d_x9_g*): sizes that end inside a tile, a step of channels and a
 group of output channels, a residual, and values that have no parts in bf16."""
+import ctypes
 import time
 
 import numpy as np
@@ -205,3 +206,24 @@ def test_every_product_of_parts_is_there(case):
         w[np.arange(cout), ch, tap // 3, tap % 3] = np.ldexp(rng.integers(2 ** 23, 2 ** 24, cout) | 1, -23)
         got, want = run(x, w, None, None, 0)[some], exact(x, w, some)
         assert (np.abs(got - want) <= 2.0 ** -22 * np.abs(want)).all()
+
+
+def test_operands_that_lie_on_four_bytes():
+    """A caller's tensors may start at any float; the filters are loaded sixteen bytes at a time."""
+    B.ops_init()
+    cin, H, W, cout, _ = CASES[7]
+    rng = np.random.default_rng(19)
+    x = rng.standard_normal((cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3, 3)) * 0.02).astype(np.float32)
+    b, res = rng.standard_normal(cout).astype(np.float32), rng.standard_normal((cout, H, W)).astype(np.float32)
+    want = run(x, w, b, res, 1)
+
+    class At:
+        def __init__(self, arr, skip):
+            self.buf = B.DeviceBuffer.from_array(np.concatenate([np.zeros(skip, np.float32), arr.reshape(-1)]))
+            self.ptr = ctypes.c_void_p(self.buf.ptr.value + 4 * skip)
+    for skip in (1, 2, 3):
+        ops = [At(a, skip) for a in (x, w, b, res, np.zeros_like(want))]
+        d = B.Conv2dDesc(cin, H, W, cout, 3, 3, 1, 1, 1, 1, 1)
+        assert B.ops_conv2d(d, *ops) == 0, B.last_error()
+        np.testing.assert_array_equal(ops[4].buf.to_array()[skip:].reshape(want.shape), want)
