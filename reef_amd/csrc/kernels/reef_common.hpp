@@ -89,7 +89,8 @@ struct FlagPoll {
         return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     // The flag by way of the scalar cache, which waits for no vector load: what it was when the line was fetched.  No more
-    // than a hint, therefore: who acts on it asks load() first.  (volatile: fetched here, and not where it is used.)
+    // than a hint, therefore: who acts on it asks load() first.  (volatile: fetched here, and not where it is used; called
+    // behind the last scalar load that operands wait for, so that it is on its way beside them.)
     __device__ __forceinline__ int hint() const {
         const int* p = flag;
         asm("" : "+s"(p));      // (or the compiler takes the value of a load() for it)

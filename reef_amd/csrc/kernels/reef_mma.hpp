@@ -1177,7 +1177,6 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = FROWS ? a[REEF_CONV_KH] : 1;
-    const int hint = poll.hint();
     const int M = a[REEF_CONV_COUT], C = FROWS ? a[REEF_CONV_CIN] * kh : a[REEF_CONV_CIN];
     const int H = a[REEF_CONV_H], W = a[REEF_CONV_W], Wo = a[REEF_CONV_WO];
     const int N = a[REEF_CONV_HO] * Wo;
@@ -1407,6 +1406,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
         load_a(s, step);
         load_b(s, step);
     };
+    const int hint = poll.hint();
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         load_b(s, s);
@@ -1482,7 +1482,7 @@ __device__ __forceinline__ bool conv2d_direct_body(const OpDesc& d_in, int task,
     // operands do: in front of them it held up the first MFMAs of every launch (DenseNet-201 as a best-effort model 1012 us a
     // request that way; looked at with a barrier before the loop another 37 of device time).  So that a wavefront under a
     // raised flag does not run a round first, it has a hint by way of the scalar cache, and waits for the load where that
-    // says so: 979 us a request (968 without the hint), and 16 streams are empty 62 us after the flag (71.5; 62.3 with
+    // says so: 977 us a request (968 without the hint), and 16 streams are empty 62 us after the flag (71.5; 62.3 with
     // the flag in front of the loads), four 16.5 (18.8; 17.1).
     if (Poll::enabled) asm volatile("" ::: "memory");
     const int raised = Poll::enabled ? poll.load() : 0;
@@ -1573,7 +1573,6 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
     float* smem = (float*)smem_raw;
     constexpr int WSTRIDE = TileV1<TM, TN>::WSTRIDE;
     const int* a = d.attr;
-    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], N = a[REEF_CONV_HO] * a[REEF_CONV_WO];
@@ -1645,6 +1644,7 @@ __device__ __forceinline__ bool conv2d_v1_body(const OpDesc& d, int task, char* 
             vb[j] += 64u * HW4;
         }
     };
+    const int hint = poll.hint();
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         load_step(s);
@@ -1791,7 +1791,6 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
     constexpr int NA = G == 1 ? 4 : 2;
     float* smem = (float*)smem_raw;
     const int* a = d.attr;
-    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = a[REEF_CONV_CIN], M = a[REEF_CONV_COUT], H = a[REEF_CONV_H], W = a[REEF_CONV_W];
@@ -1851,6 +1850,7 @@ __device__ __forceinline__ bool conv2d_v9_body(const OpDesc& d, int task, char* 
             vb[r] += 64u * HW4;
         }
     };
+    const int hint = poll.hint();
     load_b();
 #pragma unroll
     for (int t = 0; t < 9; ++t) load_a(t);
@@ -3528,7 +3528,6 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
     constexpr int AC = TM * TN > 4 ? 1 : PK && !LN && TM * TN == 1 ? 4 : 2;
     // steps of loads in flight (unpacked, 6: BERT-base +1.8 %, 4: +1.7 %, 2: +0.7 %, same process)
     constexpr int NS = PK ? 4 : 3;
-    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GemmTail<TM, TN, LN> t;
@@ -3587,6 +3586,7 @@ __device__ __forceinline__ bool gemm_nt_direct_run(const OpDesc& d, int task, ch
 #pragma unroll
         for (int g = 0; g < TN; ++g) load_slot(rb[s][g], rs_b, vb[g] | outm, so);
     };
+    const int hint = poll.hint();
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         load_step(s, s);
@@ -3713,7 +3713,6 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
     constexpr int NS = 2;                                    // steps of loads in flight: what 256 registers hold
     typedef TileD16<TN, TM> TD;
     static_assert(TM * 512 <= TD::SUBS * TD::PART, "the turned rows fit where the partial tile goes");
-    const int hint = poll.hint();
     const int lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GemmTail<TM, TN, LN> t;
@@ -3753,6 +3752,7 @@ __device__ __forceinline__ bool gemm_split_run(const OpDesc& d, int task, char* 
             vb[g] += 3072u * 4u;
         }
     };
+    const int hint = poll.hint();
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         load_step(s, s);
